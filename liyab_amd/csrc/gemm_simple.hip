@@ -1,7 +1,7 @@
 // out[M,N] = a[M,K] . w[N,K]^T (+ bias) with an epilogue: the plain tiled
 // product. It is the product of the true 32-bit path (32-bit operands, FMA
-// accumulation, no matrix-core reduced precision) and the fallback for
-// bfloat16 shapes the MFMA kernels refuse.
+// accumulation in 32 bits) and the fallback for bfloat16 shapes the MFMA
+// kernels refuse.
 //
 // Both operands are contiguous along K (a row of `w` is one output feature,
 // as the reference lays matrices out: include/liyab/types.h:165-184,
@@ -11,7 +11,7 @@
 // of 64; within a chunk one chain of fused multiply-adds over ascending k that
 // starts from zero; the chunks' sums added in ascending order. (Chunks, so that
 // a step of few rows, which has few output elements, can still spread one
-// element's sum over several waves: gemm_rowwise_f32_kernel below.)
+// element's sum over several waves: gemm_chunks_f32_kernel below.)
 #include <type_traits>
 
 #include "activations.h"
@@ -91,245 +91,285 @@ gemm_simple_kernel(OutT* __restrict__ out, int64_t ldo, const T* __restrict__ a,
     }
 }
 
-// The tiled kernel for large 32-bit products: tiles of 128 x 128, a thread 8 x 8 output elements (rows
-// ty * 4 + {0..3} and 64 + the same, columns likewise), so that a step of k costs four 16-byte reads from
-// LDS for 64 multiply-adds where the 64 x 64 tiles above read two for 16: there the reads set the pace
-// (35 TFLOP/s). The chains and the order of sums are the ones above, bit for bit.
-constexpr int BM2 = 128, BN2 = 128;
+// -- 32-bit operands ------------------------------------------------------------------------------------------
+//
+// The chains above on the matrix cores: v_mfma_f32_32x32x2 and _16x16x4 multiply and add in 32 bits, one
+// fused multiply-add after the other over ascending k (measured on random, tiny and subnormal operands:
+// 64,000 of 64,000 results have the bits of an fmaf chain; rounded once, or in another order, a third
+// differ), so a chunk's chain of 64 is 32 or 16 instructions and has the bits it had on the vector units, at
+// the matrix cores' 157 TFLOP/s, twice what vector multiply-adds reach that are not packed (these
+// stopped at 35-57 in practice).
+typedef __attribute__((ext_vector_type(4))) float f32x4_t;
+typedef __attribute__((ext_vector_type(2))) float f32x2_t;
+typedef __attribute__((ext_vector_type(16))) float f32x16_t;
 
+// What follows the sum, as in the kernel above.
 template <int EPI, bool EXACT>
+__device__ __forceinline__ float finish_f32(float v, bool has_bias, float bias) {
+    if (has_bias) v += bias;
+    if constexpr (EPI == kEpiGeluTanh) v = gelu_tanh(v);
+    if constexpr (EPI == kEpiGeluErf) v = EXACT ? gelu_erf_exact(v) : gelu_erf_fast(v);
+    return v;
+}
+
+// Four k of one row from a clamped address: with VEC one 16-byte load, else element by element (operands that are not
+// aligned for it, a K that is no multiple of 4). What lies past K becomes zero, which adds nothing to a chain, only where the
+// values go to LDS: a choice made at the load would be waited for there.
+template <bool VEC>
+__device__ __forceinline__ f32x4_t load4_f32(const float* __restrict__ row, int k, int K) {
+    if constexpr (VEC) return *reinterpret_cast<const f32x4_t*>(row + (k < K ? k : 0));
+    f32x4_t v;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = row[k + i < K ? k + i : 0];
+    return v;
+}
+__device__ __forceinline__ f32x4_t within_k(f32x4_t v, int k, int K) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = k + i < K ? v[i] : 0.0f;
+    return v;
+}
+
+// Many rows: tiles of 64 x 64 on four waves, a wave 32 x 32. The matrix cores set the pace (a stage of 32 k takes a compute
+// unit 1,024 cycles and 16 KB of operands), so operands go through registers into one of two stages in LDS while the
+// other is multiplied; they are asked for two stages ahead of their products (one stage ahead, a lone workgroup a
+// compute unit waited for them: 4 x 768 x 3,072, one tile deep, 81 us against 68). An instruction takes k = 2 s from lanes 0-31
+// and k = 2 s + 1 from lanes 32-63: rows lie in LDS with the even k of every eight in front of the odd ones, so that a lane
+// reads its k of four instructions in 16 bytes.
+// Measured, us, the 64 x 64 or 128 x 128 tiles or the row-wise kernel on vector units before: 1,222 rows, 768 -> 2,304 166 -> 50
+// (87 TFLOP/s), 768 -> 3,072 192 -> 66, 3,072 -> 768 357 -> 72, 768 -> 768 103 -> 21; 4,096 rows, 768 -> 3,072 349 -> 190 (102 TFLOP/s).
+// Tiles of 128 x 128 were no faster anywhere (4,096 x 3,072 x 768 192 us, 2,048 x 768 x 3,072 233 against 117), nor was a
+// stage's other work strung between its products by hand.
+constexpr int kTile = 64;
+
+template <int EPI, bool EXACT, bool VEC>
 __global__ void __launch_bounds__(256)
-gemm_simple128_f32_kernel(float* __restrict__ out, int64_t ldo, const float* __restrict__ a, int64_t lda, const float* __restrict__ w,
-                          const float* __restrict__ bias, float* __restrict__ residual, int64_t ldr, int M, int N, int K) {
-    __shared__ float As[BK][BM2 + 4];
-    __shared__ float Ws[BK][BN2 + 4];
-    const int tid = threadIdx.x;
-    const int m0 = blockIdx.y * BM2, n0 = blockIdx.x * BN2;
-    const int ty = tid / 16, tx = tid % 16;
-    const int lrow = tid / 4, lk = (tid % 4) * 4;  // this thread loads 4 k of rows lrow and lrow + 64
-    float acc[8][8] = {}, tot[8][8] = {};
-    for (int k0 = 0; k0 < K; k0 += BK) {
+gemm_tiled_f32_kernel(float* __restrict__ out, int64_t ldo, const float* __restrict__ a, int64_t lda, const float* __restrict__ w,
+                      const float* __restrict__ bias, float* __restrict__ residual, int64_t ldr, int M, int N, int K, int vec_out) {
+    constexpr int KS = 32, LD = KS + 4;         // k a stage; padded rows: 16 lanes' 16-byte reads fall into different banks
+    constexpr int STAGE = 2 * kTile * LD;       // the tile of a, then the tile of w
+    __shared__ __attribute__((aligned(16))) float smem[2 * STAGE];
+    const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64, li = lane % 32, g = lane / 32;
+    const int wm = wave / 2, wn = wave % 2;
+    // an XCD takes a stretch of the tiles in groups of eight rows of tiles, down the rows first: what its L2 holds of either
+    // operand is shared by the workgroups that run side by side
+    const int tiles_n = (N + kTile - 1) / kTile, tiles_m = (M + kTile - 1) / kTile, n_tiles = gridDim.x;
+    const int xcd = blockIdx.x % 8, tile_id = xcd * (n_tiles / 8) + min(xcd, n_tiles % 8) + blockIdx.x / 8;
+    const int first = tile_id / (8 * tiles_n) * 8, within = tile_id % (8 * tiles_n), rows = min(8, tiles_m - first);
+    const int m0 = (first + within % rows) * kTile, n0 = within / rows * kTile;
+    const int lrow = tid / 8, lk = (tid % 8) * 4;  // this thread loads 4 k of rows lrow and lrow + 32 of either tile
+    const float* src[4];
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const int m = m0 + lrow + 64 * h, n = n0 + lrow + 64 * h;
-            const float* p = a + static_cast<int64_t>(m) * lda + k0 + lk;
-            const float* q = w + static_cast<int64_t>(n) * K + k0 + lk;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const bool in = k0 + lk + i < K;
-                As[lk + i][lrow + 64 * h] = (m < M && in) ? p[i] : 0.0f;
-                Ws[lk + i][lrow + 64 * h] = (n < N && in) ? q[i] : 0.0f;
-            }
-        }
-        __syncthreads();
-#pragma unroll
-        for (int k = 0; k < BK; ++k) {
-            float av[8], wv[8];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                av[i] = As[k][ty * 4 + i];
-                av[4 + i] = As[k][64 + ty * 4 + i];
-                wv[i] = Ws[k][tx * 4 + i];
-                wv[4 + i] = Ws[k][64 + tx * 4 + i];
-            }
-#pragma unroll
-            for (int i = 0; i < 8; ++i)
-#pragma unroll
-                for (int j = 0; j < 8; ++j) acc[i][j] = fmaf(av[i], wv[j], acc[i][j]);
-        }
-        if ((k0 + BK) % kChunk == 0 || k0 + BK >= K) {  // the chunk's chain ends: its sum joins the others'
-#pragma unroll
-            for (int i = 0; i < 8; ++i)
-#pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    tot[i][j] += acc[i][j];
-                    acc[i][j] = 0.0f;
-                }
-        }
-        __syncthreads();
+    for (int i = 0; i < 2; ++i) {
+        src[i] = a + static_cast<int64_t>(min(m0 + lrow + 32 * i, M - 1)) * lda;
+        src[2 + i] = w + static_cast<int64_t>(min(n0 + lrow + 32 * i, N - 1)) * K;
     }
+    f32x4_t ring[2][4];
+    auto fetch = [&](int k0, int stage) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const int m = m0 + (i / 4) * 64 + ty * 4 + i % 4;
-        if (m >= M) continue;
+        for (int i = 0; i < 4; ++i) ring[stage][i] = load4_f32<VEC>(src[i], k0 + lk, K);
+    };
+    auto put = [&](int k0, int stage) {  // k = 8 q + {0, 2, 4, 6} at 8 q + 0 .. 3, the odd ones behind them
+        float* s = smem + stage * STAGE + lrow * LD + (lk & ~7) + (lk & 4) / 2;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const int n = n0 + (j / 4) * 64 + tx * 4 + j % 4;
-            if (n >= N) continue;
-            float v = tot[i][j];
-            if (bias != nullptr) v += bias[n];
-            if constexpr (EPI == kEpiGeluTanh) v = gelu_tanh(v);
-            if constexpr (EPI == kEpiGeluErf) v = EXACT ? gelu_erf_exact(v) : gelu_erf_fast(v);
-            if constexpr (EPI == kEpiResidual) {
-                residual[static_cast<int64_t>(m) * ldr + n] += v;
-            } else {
-                out[static_cast<int64_t>(m) * ldo + n] = v;
-            }
+        for (int i = 0; i < 4; ++i) {  // rows lrow and lrow + 32 of a, then of w
+            const f32x4_t v = within_k(ring[stage][i], k0 + lk, K);
+            *reinterpret_cast<f32x2_t*>(s + 32 * i * LD) = f32x2_t{v[0], v[2]};
+            *reinterpret_cast<f32x2_t*>(s + 32 * i * LD + 4) = f32x2_t{v[1], v[3]};
         }
+    };
+    f32x16_t acc, tot;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) tot[r] = 0.0f;
+    auto multiply = [&](int stage) {
+        const float* sa = smem + stage * STAGE + (wm * 32 + li) * LD + 4 * g;
+        const float* sw = smem + stage * STAGE + (kTile + wn * 32 + li) * LD + 4 * g;
+        f32x4_t fa[2], fw[2];  // the next eight k are read while these multiply
+        fa[0] = *reinterpret_cast<const f32x4_t*>(sa);
+        fw[0] = *reinterpret_cast<const f32x4_t*>(sw);
+#pragma unroll
+        for (int q = 0; q < KS / 8; ++q) {
+            if (q + 1 < KS / 8) {
+                fa[(q + 1) & 1] = *reinterpret_cast<const f32x4_t*>(sa + (q + 1) * 8);
+                fw[(q + 1) & 1] = *reinterpret_cast<const f32x4_t*>(sw + (q + 1) * 8);
+            }
+#pragma unroll
+            for (int s = 0; s < 4; ++s) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(fw[q & 1][s], fa[q & 1][s], acc, 0, 0, 0);
+        }
+    };
+    static_assert(kChunk == 2 * KS, "a chunk is the two stages");
+    const int chunks = (K + kChunk - 1) / kChunk;  // (a second stage past K is all zeros)
+    fetch(0, 0);
+    fetch(KS, 1);
+    put(0, 0);
+    fetch(2 * KS, 0);
+    lds_barrier();
+    for (int c = 0; c < chunks; ++c) {
+        const int k0 = c * kChunk;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
+        put(k0 + KS, 1);  // (a stage's readers finished before the last barrier)
+        fetch(k0 + 3 * KS, 1);
+        multiply(0);
+        lds_barrier();
+        put(k0 + 2 * KS, 0);
+        fetch(k0 + 4 * KS, 0);
+        multiply(1);
+        lds_barrier();
+#pragma unroll
+        for (int r = 0; r < 16; ++r) tot[r] += acc[r];  // the chunk's chain ends: its sum joins the others'
+    }
+    // w's fragment is the first operand: a lane holds one row, m, and its columns nb + 8 q + {0..3}.
+    // Biases and rows to add to first: a load between two stores would wait for the first.
+    const int m = m0 + wm * 32 + li, nb = n0 + wn * 32 + 4 * g;
+    f32x4_t v[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[q][e] = bias != nullptr ? bias[min(nb + 8 * q + e, N - 1)] : 0.0f;
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[q][e] = finish_f32<EPI, EXACT>(tot[4 * q + e], bias != nullptr, v[q][e]);
+    if (m >= M) return;
+    float* dst = EPI == kEpiResidual ? residual + static_cast<int64_t>(m) * ldr : out + static_cast<int64_t>(m) * ldo;
+    if (vec_out) {  // N is a multiple of 4: four columns are in or out together
+        if constexpr (EPI == kEpiResidual) {
+            f32x4_t r[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) r[q] = *reinterpret_cast<const f32x4_t*>(dst + (nb + 8 * q < N ? nb + 8 * q : 0));
+#pragma unroll
+            for (int q = 0; q < 4; ++q) v[q] += r[q];
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            if (nb + 8 * q < N) *reinterpret_cast<f32x4_t*>(dst + nb + 8 * q) = v[q];
+    } else {
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int n = nb + 8 * q + e;
+                if (n >= N) continue;
+                if constexpr (EPI == kEpiResidual) dst[n] += v[q][e];
+                else dst[n] = v[q][e];
+            }
     }
 }
 
-// The same product for steps of few rows (decoding), in the same order of sums, so a row's
-// result has the same bits whichever of the two kernels computed it. A workgroup of four or
-// eight waves takes NB output features and 16 rows (blockIdx.y: which 16); the chunks of K go round the waves. A wave
-// brings its chunk of the NB rows of `w` and of the rows of `a` through registers into LDS of
-// its own (256 bytes a row and load, the next chunk in flight meanwhile); lane (feature, row
-// group) then runs the chunk's chain for its rows; after each round of chunks one thread
-// an output element adds the round's sums in chunk order. Few features a workgroup where N is
-// small: the weights then stream through enough compute units.
-typedef __attribute__((ext_vector_type(4))) float f32x4_t;
+// Few rows, or too few tiles to go round: a workgroup takes 16 rows and NB output features, its waves the chunks of K in
+// turn, so that a product of few output elements still spreads over the chip. A wave brings its chunk of the rows
+// of `w` and `a` through registers into LDS of its own (256 bytes a row and load, the next chunk in flight
+// meanwhile) and runs the chunk's chains on the matrix core, 16 x 16 x 4 an instruction; after each round of chunks the
+// threads add the round's sums in chunk order. Few features a workgroup where N is small: the weights then stream
+// through enough compute units (features of the block past NB repeat the last one). Reading operands from LDS set the
+// pace when lanes ran the chains themselves (20 to 80 reads of 16 bytes a chunk; here 32 of 4).
+constexpr int kChunkRows = 16;  // rows a workgroup
 
-constexpr int kRowwiseRows = 16;     // rows a workgroup
-constexpr int kRowwiseMaxRows = 64;  // steps of at most this many rows take the row-wise kernel
-constexpr int kTiled128MinTiles = 512;  // tiles of 128 x 128 from this many on: two a compute unit (288 of them, 2,048 x 2,304 x 768: 305 us against 222 in tiles of 64 x 64; 576, 4,096 rows: 349 against 440)
-constexpr int kTiledMinTiles = 512;  // and so do larger ones that would give the tiled kernel fewer tiles than this
-
-template <int NB, int WAVES, int EPI, bool EXACT>
+template <int NB, int WAVES, int EPI, bool EXACT, bool VEC>
 __global__ void __launch_bounds__(64 * WAVES)
-gemm_rowwise_f32_kernel(float* __restrict__ out, int64_t ldo, const float* __restrict__ a, int64_t lda,
-                        const float* __restrict__ w, const float* __restrict__ bias, float* __restrict__ residual,
-                        int64_t ldr, int M_all, int N, int K) {
-    const int row0 = blockIdx.y * kRowwiseRows, M = min(kRowwiseRows, M_all - row0);
+gemm_chunks_f32_kernel(float* __restrict__ out, int64_t ldo, const float* __restrict__ a, int64_t lda,
+                       const float* __restrict__ w, const float* __restrict__ bias, float* __restrict__ residual,
+                       int64_t ldr, int M_all, int N, int K) {
+    const int row0 = blockIdx.y * kChunkRows, M = min(kChunkRows, M_all - row0);
     a += static_cast<int64_t>(row0) * lda;
-    constexpr int LD = kChunk + 4;  // (rows 16 bytes apart in the banks: a lane's 16-byte reads do not collide)
-    constexpr int MG = 64 / NB;                // row groups of lanes
-    constexpr int RPL = kRowwiseRows / MG;     // rows a lane
-    constexpr int W_LOADS = NB / 4, A_LOADS = kRowwiseRows / 4;  // a load covers 4 rows: 16 lanes a row, 16 bytes a lane
-    static_assert(NB % 4 == 0 && 64 % NB == 0 && kRowwiseRows % MG == 0, "lanes are features x row groups");
-    __shared__ float Wt[WAVES][NB][LD];
-    __shared__ float At[WAVES][kRowwiseRows][LD];
-    __shared__ float P[WAVES][kRowwiseRows][NB];
+    constexpr int LD = kChunk + 4;  // (lanes read words 4 banks apart, their neighbours in k beside them: no collisions)
+    constexpr int W_LOADS = NB / 4, A_LOADS = kChunkRows / 4;  // a load covers 4 rows: 16 lanes a row, 16 bytes a lane
+    static_assert(NB % 4 == 0 && NB <= 16 && kChunkRows * NB <= 64 * WAVES, "one block of features, a thread an output element");
+    __shared__ __attribute__((aligned(16))) float Wt[WAVES][NB][LD];
+    __shared__ __attribute__((aligned(16))) float At[WAVES][kChunkRows][LD];
+    __shared__ float P[2][WAVES][kChunkRows][NB];  // rounds take turns, so that one barrier a round is enough
     const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64;
     const int n0 = blockIdx.x * NB;
     const int chunks = (K + kChunk - 1) / kChunk;
     const int lrow = lane / 16, lk = (lane % 16) * 4;  // as a loader
-    const int fn = lane % NB, mg = lane / NB;          // as a summer
+    const int li = lane % 16, g = lane / 16;           // in the matrix core's operands: row (or feature) and k
     f32x4_t wreg[W_LOADS], areg[A_LOADS];
-    auto fetch = [&](int c) {  // chunk c into registers; past K zeros (they add nothing to a chain)
+    auto fetch = [&](int c) {
         const int k = c * kChunk + lk;
-        const bool in = k < K;  // K is a multiple of 4 (the launcher's check): a lane's 4 are in or out together
-        const int kc = in ? k : 0;
 #pragma unroll
-        for (int i = 0; i < W_LOADS; ++i) {
-            const int n = min(n0 + 4 * i + lrow, N - 1);
-            const f32x4_t v = *reinterpret_cast<const f32x4_t*>(w + static_cast<int64_t>(n) * K + kc);
-            wreg[i] = in ? v : f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-        }
+        for (int i = 0; i < W_LOADS; ++i) wreg[i] = load4_f32<VEC>(w + static_cast<int64_t>(min(n0 + 4 * i + lrow, N - 1)) * K, k, K);
 #pragma unroll
-        for (int i = 0; i < A_LOADS; ++i) {
-            if (4 * i < M) {  // (the same for every lane)
-                const int m = min(4 * i + lrow, M - 1);
-                const f32x4_t v = *reinterpret_cast<const f32x4_t*>(a + static_cast<int64_t>(m) * lda + kc);
-                areg[i] = in ? v : f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-            }
-        }
+        for (int i = 0; i < A_LOADS; ++i)
+            if (4 * i < M) areg[i] = load4_f32<VEC>(a + static_cast<int64_t>(min(4 * i + lrow, M - 1)) * lda, k, K);  // (the same for every lane)
     };
     float tot = 0.0f;  // of output element (tid / NB, tid % NB), for tid < 16 * NB
+    const float* wl = &Wt[wave][min(li, NB - 1)][g];
+    const float* al = &At[wave][min(li, (M + 3) / 4 * 4 - 1)][g];  // (rows past M: some row that was written; not stored)
     if (wave < chunks) fetch(wave);
-    for (int c0 = 0; c0 < chunks; c0 += WAVES) {
+    for (int c0 = 0, turn = 0; c0 < chunks; c0 += WAVES, turn ^= 1) {
         const int c = c0 + wave;
         if (c < chunks) {
 #pragma unroll
-            for (int i = 0; i < W_LOADS; ++i) *reinterpret_cast<f32x4_t*>(&Wt[wave][4 * i + lrow][lk]) = wreg[i];
+            for (int i = 0; i < W_LOADS; ++i) *reinterpret_cast<f32x4_t*>(&Wt[wave][4 * i + lrow][lk]) = within_k(wreg[i], c * kChunk + lk, K);
 #pragma unroll
             for (int i = 0; i < A_LOADS; ++i)
-                if (4 * i < M) *reinterpret_cast<f32x4_t*>(&At[wave][4 * i + lrow][lk]) = areg[i];
+                if (4 * i < M) *reinterpret_cast<f32x4_t*>(&At[wave][4 * i + lrow][lk]) = within_k(areg[i], c * kChunk + lk, K);
             if (c + WAVES < chunks) fetch(c + WAVES);
-            float part[RPL];
+            f32x4_t acc{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-            for (int r = 0; r < RPL; ++r) part[r] = 0.0f;
-#pragma unroll 4
-            for (int kk = 0; kk < kChunk; kk += 4) {
-                const f32x4_t wv = *reinterpret_cast<const f32x4_t*>(&Wt[wave][fn][kk]);
+            for (int k = 0; k < kChunk; k += 4) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(wl[k], al[k], acc, 0, 0, 0);
 #pragma unroll
-                for (int r = 0; r < RPL; ++r) {
-                    const f32x4_t av = *reinterpret_cast<const f32x4_t*>(&At[wave][mg + r * MG][kk]);
-                    part[r] = fmaf(av[0], wv[0], part[r]);
-                    part[r] = fmaf(av[1], wv[1], part[r]);
-                    part[r] = fmaf(av[2], wv[2], part[r]);
-                    part[r] = fmaf(av[3], wv[3], part[r]);
-                }
-            }
-#pragma unroll
-            for (int r = 0; r < RPL; ++r) P[wave][mg + r * MG][fn] = part[r];
+            for (int r = 0; r < 4; ++r)  // a lane holds row li and the features 4 g + r
+                if (4 * g + r < NB) P[turn][wave][li][4 * g + r] = acc[r];
         }
-        __syncthreads();
-        if (tid < kRowwiseRows * NB) {
+        lds_barrier();
+        if (tid < kChunkRows * NB) {
             const int live = min(WAVES, chunks - c0);
-            for (int wv = 0; wv < live; ++wv) tot += P[wv][tid / NB][tid % NB];
+            for (int v = 0; v < live; ++v) tot += P[turn][v][tid / NB][tid % NB];
         }
-        __syncthreads();
     }
     const int n = n0 + tid % NB;
-    if (tid >= kRowwiseRows * NB || tid / NB >= M || n >= N) return;
+    if (tid >= kChunkRows * NB || tid / NB >= M || n >= N) return;
     const int m = row0 + tid / NB;
-    float v = tot;
-    if (bias != nullptr) v += bias[n];
-    if constexpr (EPI == kEpiGeluTanh) v = gelu_tanh(v);
-    if constexpr (EPI == kEpiGeluErf) v = EXACT ? gelu_erf_exact(v) : gelu_erf_fast(v);
-    if constexpr (EPI == kEpiResidual) {
-        residual[static_cast<int64_t>(m) * ldr + n] += v;
-    } else {
-        out[static_cast<int64_t>(m) * ldo + n] = v;
-    }
+    const float v = finish_f32<EPI, EXACT>(tot, bias != nullptr, bias != nullptr ? bias[n] : 0.0f);
+    if constexpr (EPI == kEpiResidual) residual[static_cast<int64_t>(m) * ldr + n] += v;
+    else out[static_cast<int64_t>(m) * ldo + n] = v;
 }
 
-// The same once more, one thread an output element, for operands that are not aligned to 16
-// bytes or a K that is no multiple of 4.
-template <int EPI, bool EXACT>
-__global__ void __launch_bounds__(64)
-gemm_rowwise_f32_plain_kernel(float* __restrict__ out, int64_t ldo, const float* __restrict__ a, int64_t lda,
-                              const float* __restrict__ w, const float* __restrict__ bias, float* __restrict__ residual,
-                              int64_t ldr, int N, int K) {
-    const int n = blockIdx.x * 64 + threadIdx.x, m = blockIdx.y;
-    const float* wr = w + static_cast<int64_t>(min(n, N - 1)) * K;
-    const float* ar = a + static_cast<int64_t>(m) * lda;
-    float tot = 0.0f;
-    for (int k0 = 0; k0 < K; k0 += kChunk) {
-        float acc = 0.0f;
-        const int k1 = min(k0 + kChunk, K);
-        for (int k = k0; k < k1; ++k) acc = fmaf(ar[k], wr[k], acc);
-        tot += acc;
-    }
-    if (n >= N) return;
-    float v = tot;
-    if (bias != nullptr) v += bias[n];
-    if constexpr (EPI == kEpiGeluTanh) v = gelu_tanh(v);
-    if constexpr (EPI == kEpiGeluErf) v = EXACT ? gelu_erf_exact(v) : gelu_erf_fast(v);
-    if constexpr (EPI == kEpiResidual) {
-        residual[static_cast<int64_t>(m) * ldr + n] += v;
-    } else {
-        out[static_cast<int64_t>(m) * ldo + n] = v;
-    }
+// Tiles of 64 x 64 from this many on, fewer go to the kernel by chunks, whose steady 48 TFLOP/s over 16 x 16 elements a workgroup
+// beats a round of tiles that leaves compute units idle (512 rows, 3,072 -> 768, 96 tiles: 50 us against 70; 1,222 rows, 240 tiles: 116 against 72)
+constexpr int kTiledMinTiles = 136;
+constexpr int kFewRows = 64;  // steps of at most this many rows never take the tiles: their weights stream (64 rows, 768 -> 3,072: 8 us against 20)
+
+template <int EPI, bool VEC>
+int launch_tiled_f32(float* out, int64_t ldo, const float* a, int64_t lda, const float* w, const float* bias, float* residual, int64_t ldr, int M,
+                     int N, int K, bool vec_out, hipStream_t stream) {
+    gemm_tiled_f32_kernel<EPI, true, VEC><<<((N + kTile - 1) / kTile) * ((M + kTile - 1) / kTile), 256, 0, stream>>>(out, ldo, a, lda, w, bias, residual, ldr, M, N, K, vec_out);
+    return check_launch("gemm_tiled_f32");
+}
+
+template <int NB, int WAVES, int EPI, bool VEC>
+int launch_chunks_f32(float* out, int64_t ldo, const float* a, int64_t lda, const float* w, const float* bias, float* residual, int64_t ldr, int M,
+                      int N, int K, hipStream_t stream) {
+    gemm_chunks_f32_kernel<NB, WAVES, EPI, true, VEC><<<dim3((N + NB - 1) / NB, (M + kChunkRows - 1) / kChunkRows), 64 * WAVES, 0, stream>>>(
+        out, ldo, a, lda, w, bias, residual, ldr, M, N, K);
+    return check_launch("gemm_chunks_f32");
+}
+
+template <int EPI, bool VEC>
+int launch_f32_epi(float* out, int64_t ldo, const float* a, int64_t lda, const float* w, const float* bias, float* residual, int64_t ldr, int M, int N,
+                   int K, hipStream_t stream) {
+    auto al16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
+    const bool vec_out = N % 4 == 0 && (EPI == kEpiResidual ? al16(residual) && ldr % 4 == 0 : al16(out) && ldo % 4 == 0);
+#define LIYAB_ARGS out, ldo, a, lda, w, bias, residual, ldr, M, N, K
+    const int64_t tiles = static_cast<int64_t>((N + 63) / 64) * ((M + 63) / 64);
+    if (M > kFewRows && tiles >= kTiledMinTiles) return launch_tiled_f32<EPI, VEC>(LIYAB_ARGS, vec_out, stream);
+    // Two hundred workgroups of eight waves or more: 4, 8 or 16 features each; four waves once strips of 16 features are more than
+    // one and a half a compute unit (64 rows, 768 -> 3,072: 8.4 us against 12.0; 768 -> 768, 192 of them: 11.1 with eight against 14.8)
+    const int64_t strips = static_cast<int64_t>(N) * ((M + kChunkRows - 1) / kChunkRows);
+    if (strips <= 1024) return launch_chunks_f32<4, 8, EPI, VEC>(LIYAB_ARGS, stream);
+    if (strips <= 2048) return launch_chunks_f32<8, 8, EPI, VEC>(LIYAB_ARGS, stream);
+    if (strips <= 16 * 400) return launch_chunks_f32<16, 8, EPI, VEC>(LIYAB_ARGS, stream);
+    return launch_chunks_f32<16, 4, EPI, VEC>(LIYAB_ARGS, stream);
+#undef LIYAB_ARGS
 }
 
 template <int EPI>
-int launch_rowwise_f32_epi(float* out, int64_t ldo, const float* a, int64_t lda, const float* w, const float* bias,
-                           float* residual, int64_t ldr, int M, int N, int K, hipStream_t stream) {
+int launch_f32(float* out, int64_t ldo, const float* a, int64_t lda, const float* w, const float* bias, float* residual, int64_t ldr, int M, int N,
+               int K, hipStream_t stream) {
     const bool vec = (reinterpret_cast<uintptr_t>(a) & 15) == 0 && (reinterpret_cast<uintptr_t>(w) & 15) == 0 && lda % 4 == 0 && K % 4 == 0;
-    if (!vec) {
-        gemm_rowwise_f32_plain_kernel<EPI, true><<<dim3((N + 63) / 64, M), 64, 0, stream>>>(out, ldo, a, lda, w, bias, residual, ldr, N, K);
-        return check_launch("gemm_rowwise_plain");
-    }
-    // about two hundred workgroups or more: 4 features each up to 1,024 of them, 8 up to 2,560, 16 beyond
-    const int row_blocks = (M + kRowwiseRows - 1) / kRowwiseRows;
-    // (few features and a long K: eight waves share the chunks, twice as many loads in flight)
-    if (N <= 1024 && K >= 2048) gemm_rowwise_f32_kernel<4, 8, EPI, true><<<dim3((N + 3) / 4, row_blocks), 512, 0, stream>>>(out, ldo, a, lda, w, bias, residual, ldr, M, N, K);
-    else if (N <= 1024) gemm_rowwise_f32_kernel<4, 4, EPI, true><<<dim3((N + 3) / 4, row_blocks), 256, 0, stream>>>(out, ldo, a, lda, w, bias, residual, ldr, M, N, K);
-    else if (N <= 2560) gemm_rowwise_f32_kernel<8, 4, EPI, true><<<dim3((N + 7) / 8, row_blocks), 256, 0, stream>>>(out, ldo, a, lda, w, bias, residual, ldr, M, N, K);
-    else gemm_rowwise_f32_kernel<16, 4, EPI, true><<<dim3((N + 15) / 16, row_blocks), 256, 0, stream>>>(out, ldo, a, lda, w, bias, residual, ldr, M, N, K);
-    return check_launch("gemm_rowwise");
-}
-
-int launch_rowwise_f32(float* out, int64_t ldo, const float* a, int64_t lda, const float* w, const float* bias,
-                       float* residual, int64_t ldr, int M, int N, int K, int epi, hipStream_t stream) {
-    switch (epi) {
-        case kEpiNone: return launch_rowwise_f32_epi<kEpiNone>(out, ldo, a, lda, w, bias, residual, ldr, M, N, K, stream);
-        case kEpiGeluTanh: return launch_rowwise_f32_epi<kEpiGeluTanh>(out, ldo, a, lda, w, bias, residual, ldr, M, N, K, stream);
-        case kEpiGeluErf: return launch_rowwise_f32_epi<kEpiGeluErf>(out, ldo, a, lda, w, bias, residual, ldr, M, N, K, stream);
-        case kEpiResidual: return launch_rowwise_f32_epi<kEpiResidual>(out, ldo, a, lda, w, bias, residual, ldr, M, N, K, stream);
-        default: return fail(1, "gemm: unknown epilogue %d", epi);
-    }
+    if (vec) return launch_f32_epi<EPI, true>(out, ldo, a, lda, w, bias, residual, ldr, M, N, K, stream);
+    return launch_f32_epi<EPI, false>(out, ldo, a, lda, w, bias, residual, ldr, M, N, K, stream);
 }
 
 template <typename T, typename OutT, bool EXACT>
@@ -339,22 +379,6 @@ int launch_simple(void* out, int64_t ldo, const void* a, int64_t lda, const void
     auto* o = static_cast<OutT*>(out);
     auto* pa = static_cast<const T*>(a);
     auto* pw = static_cast<const T*>(w);
-    if constexpr (std::is_same<T, float>::value && std::is_same<OutT, float>::value) {
-        // large 32-bit products in tiles of 128 x 128 once those are two a compute unit (45-57 TFLOP/s against 31-37)
-        const dim3 grid2((N + BN2 - 1) / BN2, (M + BM2 - 1) / BM2);
-        if (static_cast<int64_t>(grid2.x) * grid2.y >= kTiled128MinTiles) {
-#define LIYAB_GO2(E) gemm_simple128_f32_kernel<E, EXACT><<<grid2, 256, 0, stream>>>(o, ldo, pa, lda, pw, bias, residual, ldr, M, N, K)
-            switch (epi) {
-                case kEpiNone: LIYAB_GO2(kEpiNone); break;
-                case kEpiGeluTanh: LIYAB_GO2(kEpiGeluTanh); break;
-                case kEpiGeluErf: LIYAB_GO2(kEpiGeluErf); break;
-                case kEpiResidual: LIYAB_GO2(kEpiResidual); break;
-                default: return fail(1, "gemm: unknown epilogue %d", epi);
-            }
-#undef LIYAB_GO2
-            return check_launch("gemm_simple128");
-        }
-    }
 #define LIYAB_GO(E) \
     gemm_simple_kernel<T, OutT, E, EXACT><<<grid, 256, 0, stream>>>(o, ldo, pa, lda, pw, bias, residual, ldr, M, N, K)
     switch (epi) {
@@ -388,16 +412,15 @@ extern "C" int liyab_gemm_simple(void* out, int out_dtype, int64_t ldo, const vo
     if (M == 0) return 0;
     if (dtype == kF32) {
         LIYAB_REQUIRE(epi == kEpiResidual || out_dtype == kF32, "gemm: 32-bit operands give a 32-bit output");
-        // more rows than that take the tiled kernel once its tiles of 64 x 64 are two workgroups for every
-        // compute unit (measured: from there it passes the row-wise kernel's steady 21 TFLOP/s); with fewer tiles
-        // the row-wise kernel's many small workgroups are faster, if its
-        // loads of 16 bytes fit the operands (else it would run one thread an element)
-        const bool vec = (reinterpret_cast<uintptr_t>(a) & 15) == 0 && (reinterpret_cast<uintptr_t>(w) & 15) == 0 && lda % 4 == 0 && K % 4 == 0;
-        const int64_t tiles = static_cast<int64_t>((N + BN - 1) / BN) * ((M + BM - 1) / BM);
-        if (M <= kRowwiseMaxRows || (vec && tiles < kTiledMinTiles))
-            return launch_rowwise_f32(static_cast<float*>(out), ldo, static_cast<const float*>(a), lda, static_cast<const float*>(w),
-                                      bias, residual, ldr, M, N, K, epi, stream);
-        return launch_simple<float, float, true>(out, ldo, a, lda, w, bias, residual, ldr, M, N, K, epi, stream);
+        auto* o = static_cast<float*>(out);
+        auto *pa = static_cast<const float*>(a), *pw = static_cast<const float*>(w);
+        switch (epi) {
+            case kEpiNone: return launch_f32<kEpiNone>(o, ldo, pa, lda, pw, bias, residual, ldr, M, N, K, stream);
+            case kEpiGeluTanh: return launch_f32<kEpiGeluTanh>(o, ldo, pa, lda, pw, bias, residual, ldr, M, N, K, stream);
+            case kEpiGeluErf: return launch_f32<kEpiGeluErf>(o, ldo, pa, lda, pw, bias, residual, ldr, M, N, K, stream);
+            case kEpiResidual: return launch_f32<kEpiResidual>(o, ldo, pa, lda, pw, bias, residual, ldr, M, N, K, stream);
+            default: return fail(1, "gemm: unknown epilogue %d", epi);
+        }
     }
     if (dtype == kBF16) {
         if (out_dtype == kF32) return launch_simple<bf16_t, float, false>(out, ldo, a, lda, w, bias, residual, ldr, M, N, K, epi, stream);

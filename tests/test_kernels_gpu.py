@@ -234,6 +234,31 @@ def test_gemm_float32(ops, M, N, K, epilogue):
         assert torch.equal(many[70:], full)
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 1, 1), (16, 1024, 63), (16, 1025, 65), (17, 1024, 64), (3, 2049, 130), (16, 6400, 128), (16, 6401, 68), (64, 3, 257),
+                                   (65, 4288, 96), (65, 4289, 96), (65, 4352, 100), (129, 4351, 33), (700, 770, 200), (64, 8700, 64)])
+def test_gemm_float32_at_the_edges_of_its_kernels(ops, M, N, K):
+    """Strips of 4, 8 and 16 features, tiles of 64 x 64 (from 136 of them on), remainders in every direction, operands with
+    16-byte loads and without, rows of outputs wider than N. The error of a chain of n multiply-adds is within n 2^-24 times
+    the sum of |a w|: 64 a chunk, the chunks' sums, the bias."""
+    a, w, bias = rnd(M, K), rnd(N, K, seed=1), rnd(N, seed=2)
+    want = a.double() @ w.double().t() + bias.double()
+    bound = (a.double().abs() @ w.double().abs().t() + bias.double().abs()) * ((min(K, 64) + K / 64 + 2) * 2.0 ** -24)
+    out = torch.full((M, N), float("nan"), device=DEV)
+    ops.gemm_simple(a, w, bias, out=out)
+    assert ((out.double() - want).abs() <= bound).all()
+    shifted = torch.empty(M * K + 1, device=DEV)[1:].view(M, K).copy_(a)  # no 16-byte loads
+    wider = torch.full((M, N + 3), float("nan"), device=DEV)
+    ops.gemm_simple(shifted, w, bias, out=wider[:, :N])
+    assert torch.equal(wider[:, :N], out) and wider[:, N:].isnan().all()
+    res = rnd(M, N, seed=3)
+    base = res.clone()
+    ops.gemm_simple(a, w, bias, residual=res, epilogue=ops.EPI_RESIDUAL)
+    assert torch.equal(res, base + out)
+    one = torch.empty(1, N, device=DEV)  # a row alone: the kernel for few rows, in strips of its own
+    ops.gemm_simple(a[M - 1:], w, bias, out=one)
+    assert torch.equal(one[0], out[M - 1])
+
+
 @pytest.mark.parametrize("kernel", ["simple", "mfma128", "mfma64", "mfma128x64", "auto", "skinny1", "skinny4", "skinny16", "skinny4w", "skinny2w", "skinny8m1", "skinny4m2", "skinny2m4",
                                     "dl2", "dl6", "dl8", "dl15", "dl16", "dl17"])
 @pytest.mark.parametrize("epilogue", ["none", "gelu_tanh", "gelu_erf", "residual"])
