@@ -1,0 +1,204 @@
+// out[M,N] = a[M,K] . w[N,K]^T in bfloat16 on the matrix cores for many rows: tiles from 64 x 64 to 256 x 256, operands
+// straight from global memory into a ring of stages in LDS (global_load_lds, 16 bytes a lane), 64 k a stage. K must be a
+// multiple of 64.
+//
+// What bounds it. The matrix cores draw more power than the card has: on random data, nothing but products, 32 x 32 x 16
+// instructions settle at 1.6-1.8 PFLOP/s and 16 x 16 x 32 at 1.9-2.1 (2.4 on zeros), so the blocks are 16 x 16. A compute unit
+// takes operands in at about 113 GB/s, loads alone, when a load covers whole lines of 128 bytes, and at 70 when it covers
+// halves of them (stages of 32 k), so a stage is 64 k; a tile of 256 x 256 then needs 0.6 us a stage for operands and 0.9 for
+// products. A wave that asks for a whole stage at once waits at the load queue before its first product: the loads of the
+// stage ahead go out in two halves, each in front of the products of 32 k. What is left unhidden (a stage's barrier, the
+// first fragments, the outputs) overlaps with another workgroup's products: two workgroups of eight waves a compute unit for
+// the middle tiles, sixteen waves in one for 256 x 256.
+// Measured in prefill steps, us a product, before (32 x 32 x 16 in tiles of 64 x 64, 128 x 128 or 256 x 256, a stage's loads at
+// once) and now: GPT-2 XL's widths, 7,920 rows: 1,600 -> 4,800 164 -> 122, 1,600 -> 6,400 204 -> 157, the two products back
+// to the stream 149 -> 114; 768 wide, 8,001 rows: 768 -> 2,304 51 -> 41, 768 -> 3,072 60 -> 48, the two back 45 -> 34; 2,048
+// rows: 18.4 -> 16.6, 20.2 -> 20.5 and 18.0 -> 16.9; 1,024 wide, some 780 rows: 1,024 -> 3,072 15.7 -> 14.8, -> 4,096 22.0 -> 15.4.
+// (There the operands come from memory, not from L2: three and four stages, which lose in a product repeated alone, win while
+// every tile has a compute unit of its own.) A product of 8,192 cubed runs at 1.2 PFLOP/s, the vendor's library at 1.4.
+// Tried and left: four waves of 128 x 128, eight of 128 x 64, two groups of waves in turn at products and reads (each with
+// 32 x 32 blocks: 173-200 us for 6,400 -> 1,600 alone, 160 here), stages of 32 k four deep (190), fragments read a step ahead in
+// registers of their own or strung between the products by hand (slower than the compiler's order); 128 x 192, 128 x 64, 64 x 128.
+#include "common.h"
+#include "launchers.h"
+#include "gemm_tile.h"
+
+namespace liyab {
+
+typedef __attribute__((address_space(3))) void* lds_void_ptr;
+
+constexpr int TBK = 64;  // k a stage
+
+template <int BM, int BN, int STAGES, int WM, int WN>
+constexpr size_t tile_lds_bytes(size_t out_bytes) {
+    const size_t stages = static_cast<size_t>(STAGES) * (BM + BN) * TBK * 2, staging = staging_bytes<BM, BN, WM, WN, 1>(out_bytes);
+    return stages > staging ? stages : staging;
+}
+
+// WM x WN waves, each with (BM / WM) x (BN / WN) of the tile in blocks of 16 x 16; MIN_WAVES a SIMD: what the registers must leave
+// room for (the workgroups that LDS lets a compute unit hold).
+template <int BM, int BN, int STAGES, typename OutT, int EPI, int WM, int WN, int MIN_WAVES>
+__global__ void __launch_bounds__(64 * WM * WN, MIN_WAVES)
+gemm_mfma_tile_kernel(const bf16_t* __restrict__ a, int64_t lda, const bf16_t* __restrict__ w, int M, int N, int K, EpiParams epi, int vec_ok,
+                      int page_shift, PartsParams parts) {
+    constexpr int WAVES = WM * WN, TM = BM / WM / 16, TN = BN / WN / 16, STAGE = (BM + BN) * TBK;
+    constexpr int A_LOADS = BM / 8 / WAVES, W_LOADS = BN / 8 / WAVES, LOADS = A_LOADS + W_LOADS;  // 1 KiB each: 8 rows of 64 k
+    static_assert(A_LOADS * 8 * WAVES == BM && W_LOADS * 8 * WAVES == BN, "whole loads a wave");
+    static_assert(STAGES >= 2 && STAGES <= 4 && (STAGES - 2) * LOADS <= 63, "the waits below");
+    extern __shared__ __attribute__((aligned(1024))) bf16_t lds[];
+    const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64), wm = wave / WN, wn = wave % WN;
+    int m0, n0;
+    tile_place<BM, BN>(M, N, K, m0, n0);
+
+    int units = K / TBK, first = 0;  // stages of k this workgroup walks, and where it starts
+    if constexpr (EPI == kEpiParts) {
+        first = blockIdx.y * parts.kt_per_part;
+        units = min(units - first, parts.kt_per_part);
+        if (blockIdx.y > 0) epi.bias = nullptr;  // the bias goes to the first plane only
+    }
+    // A load fills 1 KiB of LDS lane after lane: 8 rows of 128 bytes, unpadded. A 16-byte read serves 16 lanes a cycle, here 16
+    // consecutive rows at one piece: even and odd rows start in different halves of the 64 banks, and within a half 8 rows
+    // must land on 8 different pieces, so piece c of a row lies at c ^ ((row / 2) % 8). Rows past M or N: the last valid one
+    // again; what comes of them is never stored.
+    const bf16_t* src[LOADS];
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) {
+        const int row = (i < A_LOADS ? wave * A_LOADS + i : wave * W_LOADS + i - A_LOADS) * 8 + lane / 8;
+        const int c = (lane % 8) ^ ((row >> 1) & 7);
+        src[i] = (i < A_LOADS ? a + static_cast<int64_t>(min(m0 + row, M - 1)) * lda : w + static_cast<int64_t>(min(n0 + row, N - 1)) * K) + first * TBK + c * 8;
+    }
+    bf16_t* const to_a = lds + wave * A_LOADS * 512;
+    bf16_t* const to_w = lds + BM * TBK + wave * W_LOADS * 512;
+    auto issue = [&](int begin, int end, int unit, int stage) {
+#pragma unroll
+        for (int i = 0; i < LOADS; ++i) {
+            if (i < begin || i >= end) continue;
+            const bf16_t* from = src[i] + unit * TBK;
+            bf16_t* to = (i < A_LOADS ? to_a + i * 512 : to_w + (i - A_LOADS) * 512) + stage * STAGE;
+            __builtin_amdgcn_global_load_lds(from, (lds_void_ptr)(to), 16, 0, 0);
+        }
+    };
+
+    f32x4 acc[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    const int li = lane % 16, g = lane / 16, swizzle = (li >> 1) & 7;  // (rows of a block start at multiples of 16)
+    const int row_a = (wm * (BM / WM) + li) * TBK, row_w = BM * TBK + (wn * (BN / WN) + li) * TBK;
+    auto multiply = [&](int stage, int half) {  // 32 k
+        const bf16_t* piece = lds + stage * STAGE + (((4 * half + g) ^ swizzle) * 8);
+        bf16x8 fa[TM], fw[TN];
+#pragma unroll
+        for (int j = 0; j < TN; ++j) fw[j] = *reinterpret_cast<const bf16x8*>(piece + row_w + j * 16 * TBK);
+#pragma unroll
+        for (int i = 0; i < TM; ++i) fa[i] = *reinterpret_cast<const bf16x8*>(piece + row_a + i * 16 * TBK);
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw[j], fa[i], acc[i][j], 0, 0, 0);
+    };
+
+#pragma unroll
+    for (int p = 0; p < STAGES - 1; ++p)
+        if (p < units) issue(0, LOADS, p, p);
+    for (int u = 0, stage = 0, next = STAGES - 1; u < units; ++u) {
+        // unit u must have landed; the loads of the units after it may be in flight (a wave's loads complete in order)
+        const int later = min(units - 1 - u, STAGES - 2);
+        if (STAGES > 3 && later >= 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(STAGES > 3 ? 2 * LOADS : 0) : "memory");
+        else if (STAGES > 2 && later >= 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(STAGES > 2 ? LOADS : 0) : "memory");
+        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        // everyone's loads of unit u are in LDS, everyone is done reading unit u - 1: its stage takes unit u + STAGES - 1
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+        const bool more = u + STAGES - 1 < units;
+        if (more) issue(0, (LOADS + 1) / 2, u + STAGES - 1, next);
+        multiply(stage, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        if (more) issue((LOADS + 1) / 2, LOADS, u + STAGES - 1, next);
+        multiply(stage, 1);
+        __builtin_amdgcn_sched_barrier(0);
+        stage = stage + 1 == STAGES ? 0 : stage + 1;
+        next = next + 1 == STAGES ? 0 : next + 1;
+    }
+    store_tile<BM, BN, OutT, EPI, WM, WN>(acc, lds, epi, parts, m0, n0, M, N, vec_ok, page_shift, wave, wm, wn, lane);
+}
+
+template <int BM, int BN, int STAGES, int WM, int WN, int MIN_WAVES, typename OutT, int EPI>
+int launch_tile_as(const bf16_t* a, int64_t lda, const bf16_t* w, int M, int N, int K, const EpiParams& epi, int kparts, const PartsParams& parts,
+                   hipStream_t stream) {
+    constexpr size_t smem = tile_lds_bytes<BM, BN, STAGES, WM, WN>(sizeof(OutT));
+    static_assert(smem <= 160 * 1024, "a workgroup's LDS");
+    auto kern = gemm_mfma_tile_kernel<BM, BN, STAGES, OutT, EPI, WM, WN, MIN_WAVES>;
+    static bool ready = false;  // once per instantiation, outside any stream capture's first use
+    if (!ready) {
+        hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(smem));
+        ready = true;
+    }
+    int vec_ok, page_shift;
+    store_rules<OutT, EPI>(epi, N, vec_ok, page_shift);
+    if (EPI == kEpiParts && ((reinterpret_cast<uintptr_t>(parts.base) & 15) != 0 || parts.part_stride % 4 != 0 || parts.base_stride % 4 != 0)) vec_ok = 0;
+    const dim3 grid(((N + BN - 1) / BN) * ((M + BM - 1) / BM), kparts);
+    kern<<<grid, 64 * WM * WN, smem, stream>>>(a, lda, w, M, N, K, epi, vec_ok, page_shift, parts);
+    return check_launch("gemm_mfma_tile");
+}
+
+template <int BM, int BN, int STAGES, int WM, int WN, int MIN_WAVES>
+int launch_tile_epi(const bf16_t* a, int64_t lda, const bf16_t* w, int M, int N, int K, const EpiParams& epi, hipStream_t stream) {
+#define LIYAB_TILE(T, E) launch_tile_as<BM, BN, STAGES, WM, WN, MIN_WAVES, T, E>(a, lda, w, M, N, K, epi, 1, PartsParams{}, stream)
+    if (epi.mode == kEpiResidual) return LIYAB_TILE(float, kEpiResidual);
+    if (epi.out_dtype == kF32) return epi.mode == kEpiNone ? LIYAB_TILE(float, kEpiNone) : LIYAB_TILE(float, -1);
+    switch (epi.mode) {
+        case kEpiNone: return LIYAB_TILE(bf16_t, kEpiNone);
+        case kEpiGeluTanh: return LIYAB_TILE(bf16_t, kEpiGeluTanh);
+        case kEpiGeluErf: return LIYAB_TILE(bf16_t, kEpiGeluErf);
+        case kEpiQkvPaged: return LIYAB_TILE(bf16_t, kEpiQkvPaged);
+        default: return LIYAB_TILE(bf16_t, -1);
+    }
+#undef LIYAB_TILE
+}
+
+int choose_gemm_tile(int M, int N, int K) {
+    // The compute units take tiles in rounds. A tile's time a unit of 64 k, measured alone on a compute unit and beside as many
+    // others as fit there, and what a round costs besides (the first operands, the outputs, of which the single workgroup of a 256 x
+    // 256 tile overlaps nothing), in us; a last round that is not full runs at the lower occupancy's time.
+    struct Shape { int tile, bm, bn, fit; float unit[3], round; };
+    constexpr Shape shapes[] = {
+        {15, 256, 256, 1, {1.45f, 0, 0}, 10.0f}, {9, 192, 128, 2, {0.68f, 1.3f, 0}, 5.0f},  {11, 192, 128, 1, {0.62f, 0, 0}, 4.5f},
+        {8, 128, 128, 2, {0.60f, 1.0f, 0}, 4.0f}, {7, 128, 128, 1, {0.45f, 0, 0}, 4.5f},    {6, 64, 64, 2, {0.30f, 0.45f, 0}, 2.0f},
+        {2, 64, 64, 3, {0.30f, 0.45f, 0.62f}, 2.0f}};
+    constexpr int kUnits = 256;  // compute units
+    int best = 0;
+    float best_us = 0.0f;
+    for (const Shape& s : shapes) {
+        const int64_t tiles = static_cast<int64_t>((M + s.bm - 1) / s.bm) * ((N + s.bn - 1) / s.bn);
+        const int64_t slots = static_cast<int64_t>(kUnits) * s.fit, full = tiles / slots, rest = tiles % slots;
+        float us = full * (s.unit[s.fit - 1] * (K / TBK) + s.round);
+        if (rest > 0) us += s.unit[(rest + kUnits - 1) / kUnits - 1] * (K / TBK) + s.round;
+        if (best == 0 || us < best_us) {
+            best = s.tile;
+            best_us = us;
+        }
+    }
+    return best;
+}
+
+int launch_gemm_tile(int tile, const bf16_t* a, int64_t lda, const bf16_t* w, int M, int N, int K, const EpiParams& epi, hipStream_t stream) {
+    switch (tile) {
+        case 2: return launch_tile_epi<64, 64, 3, 2, 2, 3>(a, lda, w, M, N, K, epi, stream);
+        case 6: return launch_tile_epi<64, 64, 4, 2, 2, 2>(a, lda, w, M, N, K, epi, stream);
+        case 7: return launch_tile_epi<128, 128, 3, 4, 2, 2>(a, lda, w, M, N, K, epi, stream);
+        case 8: return launch_tile_epi<128, 128, 2, 4, 2, 4>(a, lda, w, M, N, K, epi, stream);
+        case 9: return launch_tile_epi<192, 128, 2, 4, 2, 4>(a, lda, w, M, N, K, epi, stream);
+        case 11: return launch_tile_epi<192, 128, 3, 4, 2, 2>(a, lda, w, M, N, K, epi, stream);
+        case 15: return launch_tile_epi<256, 256, 2, 4, 4, 4>(a, lda, w, M, N, K, epi, stream);
+        default: return fail(1, "gemm_mfma_dl: unknown tile %d", tile);
+    }
+}
+
+int launch_gemm_tile_parts(const bf16_t* a, int64_t lda, const bf16_t* w, int M, int N, int K, int kparts, const EpiParams& epi, const PartsParams& parts,
+                           hipStream_t stream) {
+    return launch_tile_as<64, 64, 4, 2, 2, 2, float, kEpiParts>(a, lda, w, M, N, K, epi, kparts, parts, stream);
+}
+
+}  // namespace liyab

@@ -260,7 +260,7 @@ def test_gemm_float32_at_the_edges_of_its_kernels(ops, M, N, K):
 
 
 @pytest.mark.parametrize("kernel", ["simple", "mfma128", "mfma64", "mfma128x64", "auto", "skinny1", "skinny4", "skinny16", "skinny4w", "skinny2w", "skinny8m1", "skinny4m2", "skinny2m4",
-                                    "dl2", "dl6", "dl8", "dl15", "dl16", "dl17"])
+                                    "dl2", "dl6", "dl7", "dl8", "dl9", "dl11", "dl15", "dl16", "dl17"])
 @pytest.mark.parametrize("epilogue", ["none", "gelu_tanh", "gelu_erf", "residual"])
 @pytest.mark.parametrize("M,N,K", GEMM_SHAPES + [(300, 264, 1600), (2, 50257 // 16, 64), (8, 130, 3072), (16, 2304, 768), (3, 40, 200), (17, 100, 64), (40, 333, 768), (64, 257, 1600),
                                                  (500, 300, 128), (129, 193, 192), (20, 4800, 1600), (600, 520, 256), (1030, 770, 128), (5, 100, 16384)])
