@@ -93,13 +93,18 @@ attention_decode_kernel(T* __restrict__ out, int64_t out_stride, const T* __rest
                         const int* __restrict__ block_tables, int max_blocks, const int* __restrict__ tok_list,
                         const int* __restrict__ tok_seq, const int* __restrict__ tok_pos, float scale, int window,
                         int n_head, int n_kv_head, int hd, int page_size, int page_shift, int rows_are_requests,
-                        int n_splits, int chunk, float* __restrict__ partials, int num_pages, float softcap = 0.0f,
+                        int n_splits, int chunk, float* __restrict__ partials, int num_pages, int heads_first, float softcap = 0.0f,
                         const float* __restrict__ bias_table = nullptr, int max_dist = 0, const float* __restrict__ sinks = nullptr,
                         int keep_first = 0) {
     constexpr int KPP = 64 / LPK;  // keys per wave and pass
     __shared__ float lds2[2][AD_WAVES][LPK][10];  // the waves' sums, for the first wave to merge; two of them in turn, so that one barrier a split is enough
-    const int t = tok_list != nullptr ? tok_list[blockIdx.x] : blockIdx.x;
-    const int h = blockIdx.y, z = blockIdx.z;
+    // Workgroups go to the 8 XCDs in turn. With heads fastest (the launcher's choice where every query head has keys of its own) a
+    // token's heads spread over all of them, and its neighbours' keys lie beside its own; with tokens fastest, and a number of
+    // tokens that 8 divides, one XCD had all of a token, and the one with the long contexts was waited for (64 tokens of 256 to
+    // 1,015 keys, 25 heads of 64: 57 us a layer, 49 with 636 keys each). Query heads that share keys stay on one XCD and its L2.
+    const int slot = heads_first ? blockIdx.y : blockIdx.x;
+    const int t = tok_list != nullptr ? tok_list[slot] : slot;
+    const int h = heads_first ? blockIdx.x : blockIdx.y, z = blockIdx.z;
     const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64;
     const int c = lane % LPK, kg = lane / LPK;
     const bool active = c * 8 < hd;
@@ -245,7 +250,7 @@ attention_decode_kernel(T* __restrict__ out, int64_t out_stride, const T* __rest
         } else {
             // partials [token slot][head][split][hd + 4]: values, then maximum and sum (and two
             // unused, which keep every split's values 16-byte aligned)
-            float* p = partials + ((static_cast<int64_t>(blockIdx.x) * n_head + h) * n_splits + z) * (hd + 4);
+            float* p = partials + ((static_cast<int64_t>(slot) * n_head + h) * n_splits + z) * (hd + 4);
 #pragma unroll
             for (int e = 0; e < 8; ++e) p[c * 8 + e] = st.acc[e];
             if (c == 0) {
@@ -337,7 +342,8 @@ int launch_attention_decode(void* out, int64_t out_stride, const void* q, int64_
     int page_shift = -1;
     for (int b = 0; b < 31; ++b)
         if ((1 << b) == page_size) page_shift = b;
-    dim3 grid(n, n_head, n_splits);
+    const int heads_first = n_head == n_kv_head && n <= 65535;
+    const dim3 grid = heads_first ? dim3(n_head, n, n_splits) : dim3(n, n_head, n_splits);
     auto* o = static_cast<T*>(out);
     auto* pq = static_cast<const T*>(q);
     auto* pk = static_cast<const T*>(kc);
@@ -347,15 +353,15 @@ int launch_attention_decode(void* out, int64_t out_stride, const void* q, int64_
         if (waves == 4)                                                                                              \
             attention_decode_kernel<T, L, 4, 4, SCORED><<<grid, 256, 0, stream>>>(o, out_stride, pq, q_stride, pk, pv, block_tables, \
                                                                     max_blocks, tok_list, tok_seq, tok_pos, scale,   \
-                                                                    window, n_head, n_kv_head, hd, page_size, page_shift, rows_are_requests, n_splits, chunk, partials, num_pages, softcap, bias_table, max_dist, sinks, keep_first); \
+                                                                    window, n_head, n_kv_head, hd, page_size, page_shift, rows_are_requests, n_splits, chunk, partials, num_pages, heads_first, softcap, bias_table, max_dist, sinks, keep_first); \
         else if (waves == 8)                                                                                         \
             attention_decode_kernel<T, L, 8, 4, SCORED><<<grid, 512, 0, stream>>>(o, out_stride, pq, q_stride, pk, pv, block_tables, \
                                                                     max_blocks, tok_list, tok_seq, tok_pos, scale,   \
-                                                                    window, n_head, n_kv_head, hd, page_size, page_shift, rows_are_requests, n_splits, chunk, partials, num_pages, softcap, bias_table, max_dist, sinks, keep_first); \
+                                                                    window, n_head, n_kv_head, hd, page_size, page_shift, rows_are_requests, n_splits, chunk, partials, num_pages, heads_first, softcap, bias_table, max_dist, sinks, keep_first); \
         else                                                                                                         \
             attention_decode_kernel<T, L, 16, sizeof(T) == 2 ? 8 : 4, SCORED><<<grid, 1024, 0, stream>>>(o, out_stride, pq, q_stride, pk, pv, block_tables, \
                                                                       max_blocks, tok_list, tok_seq, tok_pos, scale, \
-                                                                      window, n_head, n_kv_head, hd, page_size, page_shift, rows_are_requests, n_splits, chunk, partials, num_pages, softcap, bias_table, max_dist, sinks, keep_first); \
+                                                                      window, n_head, n_kv_head, hd, page_size, page_shift, rows_are_requests, n_splits, chunk, partials, num_pages, heads_first, softcap, bias_table, max_dist, sinks, keep_first); \
     } while (0)
     if (hd <= 8) LIYAB_GO(1);
     else if (hd <= 16) LIYAB_GO(2);
