@@ -1087,3 +1087,27 @@ def test_scale_in_place(n):
     want = x * 0.37
     ops.scale_(x, 0.37)
     assert torch.equal(x, want)
+
+
+@pytest.mark.parametrize("n,d,n_sum", [(1, 4, 1), (5, 768, 2), (3, 772, 3), (7, 1024, 1), (2, 1600, 2), (4, 2048, 3), (513, 260, 1), (1025, 64, 2)])
+@pytest.mark.parametrize("centred", [False, True])
+def test_rows_update_by_waves_is_the_one_by_workgroups(ops, n, d, n_sum, centred):
+    """A wave a row where everything is aligned, a workgroup a row where it is not (the gate's columns start at an odd place):
+    the same update to the rounding of two orders of a sum of d squares (d 2^-24 of the norm at most, met by 1e-5)."""
+    x, y = rnd(n, d), rnd(n * n_sum, d, seed=1, scale=2.0) + 0.5
+    w, b, nw = rnd(d, seed=2) + 1.0, rnd(d, seed=3), rnd(d, seed=4) + 1.0
+    wide = rnd(n, d + 4, seed=5)
+    odd = torch.empty(n, d + 5, device=DEV)
+    odd[:, 1:] = wide
+    for cast, nxt in ((None, None), (torch.bfloat16, None), (torch.float32, (nw, 1e-6))):
+        got = []
+        for gate in (wide[:, 4:], odd[:, 5:]):
+            rows = x.clone()
+            out = torch.full((n, d), float("nan"), dtype=cast, device=DEV) if cast else None
+            ops.gated_norm_add(rows, y, w, 1e-5, n_sum=n_sum, gate=gate, cast_out=out, next_norm=nxt, bias=b if centred else None, centred=centred)
+            got.append((rows, out))
+        close(got[0][0], got[1][0], 1e-5, "rows")
+        if cast:
+            close(got[0][1], got[1][1], 1e-5 if cast == torch.float32 else 1e-2, "what the next product reads")
+            if nxt is None:
+                assert torch.equal(got[0][1], got[0][0].to(cast))
