@@ -162,132 +162,134 @@ gated_norm_add_kernel(float* __restrict__ x, T* __restrict__ cast_out, const flo
     }
 }
 
-// The same with a wave a row, NV x 4 values a lane in registers (d a multiple of 4, at most 256 NV, everything aligned to 16 bytes), up
-// to three rows of y a token: everything is asked for before anything is used, 16 bytes a load, absent operands through a pointer to
-// something present instead of a branch (a load under a branch is waited for where the branch ends), and the sums over the row
-// need no barrier. A step of few rows is bound by that one trip to memory; the kernel above makes three or four in turn, its
-// waves meeting at two barriers a sum (4 rows of 768 in a decode step, us: two rows a token and a gate 6.6 -> 4.7, a layer norm 5.4 -> 3.4).
-typedef __attribute__((ext_vector_type(4))) float norm_f32x4;
-template <typename T>
-__device__ __forceinline__ void norm_store4(T* dst, const norm_f32x4& v) {
-    if constexpr (sizeof(T) == 4) {
-        *reinterpret_cast<norm_f32x4*>(dst) = v;
-    } else {
-        uint2 packed;
-        packed.x = static_cast<uint32_t>(float_to_bf16(v[0])) | (static_cast<uint32_t>(float_to_bf16(v[1])) << 16);
-        packed.y = static_cast<uint32_t>(float_to_bf16(v[2])) | (static_cast<uint32_t>(float_to_bf16(v[3])) << 16);
-        *reinterpret_cast<uint2*>(dst) = packed;
-    }
-}
+// The same with a wave a row, up to 256 J values of it in registers (4 J a lane) and up to three rows of y a token: everything is asked
+// for before anything is used, without a branch (a load under one is waited for where it ends), and the sums over the row need
+// no barrier. A step of few rows is bound by that one trip to memory; the kernel above makes three or four in turn, and its waves
+// meet at two barriers a sum (4 rows of 768 in a decode step, us: two rows a token and a gate 6.6 -> RESULT1, a layer norm 5.4 ->
+// RESULT2). A lane holds what lane `lane` of each of the four waves above holds, and the sums are added in their order: the same bits.
+enum : int { kRowOnly = 0, kRowBias = 1, kRowNext = 2 };  // what else a row takes: a bias of its norm, the next norm of the new row
 
-template <typename T, int NV, int NSUM, bool GATE>
+template <typename T, int J, int NSUM, bool GATE, int ALSO>
 __global__ void __launch_bounds__(256)
 gated_norm_add_wave_kernel(float* __restrict__ x, T* __restrict__ cast_out, const float* __restrict__ y, const float* __restrict__ gate, int64_t gate_stride,
                            const float* __restrict__ w, float eps, int normalize, int n, int d, KeepRows keep, const float* __restrict__ next_w,
                            float next_eps, const float* __restrict__ b) {
+    constexpr int W = 4, STRIDE = W * kWave;
     const int lane = threadIdx.x % kWave, t = blockIdx.x * (blockDim.x / kWave) + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     if (t >= n) return;
     float* xr = x + static_cast<int64_t>(t) * d;
     const float* yr = y + static_cast<int64_t>(t) * NSUM * d;
-    const float *wp = w != nullptr ? w : xr, *bp = b != nullptr ? b : xr, *np = next_w != nullptr ? next_w : xr;
-    norm_f32x4 xv[NV], yv[NSUM][NV], gv[GATE ? NV : 1], wv[NV], bv[NV], nv[NV];
-    int at[NV];
+    const float* wp = w != nullptr ? w : xr;
+    float xv[W][J], sv[W][J], yv[NSUM][W][J], gv[GATE ? W : 1][J], wv[W][J], av[ALSO ? W : 1][J];
+    const auto place = [&](int q, int j) { return lane + q * kWave + j * STRIDE; };
+    const auto at = [&](int q, int j) { return min(place(q, j), d - 1); };  // (past the row: its last value, counted as nothing)
 #pragma unroll
-    for (int j = 0; j < NV; ++j) at[j] = min((j * kWave + lane) * 4, d - 4);  // (lanes past the row read its end; their values count as zeros)
+    for (int j = 0; j < J; ++j)
 #pragma unroll
-    for (int j = 0; j < NV; ++j) {
+        for (int q = 0; q < W; ++q) {
 #pragma unroll
-        for (int k = 0; k < NSUM; ++k) yv[k][j] = *reinterpret_cast<const norm_f32x4*>(yr + static_cast<int64_t>(k) * d + at[j]);
-        if constexpr (GATE) gv[j] = *reinterpret_cast<const norm_f32x4*>(gate + static_cast<int64_t>(t) * gate_stride + at[j]);
-    }
+            for (int k = 0; k < NSUM; ++k) yv[k][q][j] = yr[static_cast<int64_t>(k) * d + at(q, j)];
+            if constexpr (GATE) gv[q][j] = gate[static_cast<int64_t>(t) * gate_stride + at(q, j)];
+        }
 #pragma unroll
-    for (int j = 0; j < NV; ++j) {
-        xv[j] = *reinterpret_cast<const norm_f32x4*>(xr + at[j]);
-        wv[j] = *reinterpret_cast<const norm_f32x4*>(wp + at[j]);
-        bv[j] = *reinterpret_cast<const norm_f32x4*>(bp + at[j]);
-        nv[j] = *reinterpret_cast<const norm_f32x4*>(np + at[j]);
-    }
-    const auto inside = [&](int j) { return (j * kWave + lane) * 4 < d; };
-    norm_f32x4 sv[NV];
-    float ss = 0.0f;
+    for (int j = 0; j < J; ++j)
 #pragma unroll
-    for (int j = 0; j < NV; ++j) {
-        sv[j] = yv[0][j];
+        for (int q = 0; q < W; ++q) {
+            xv[q][j] = xr[at(q, j)];
+            wv[q][j] = wp[at(q, j)];
+            if constexpr (ALSO != kRowOnly) av[q][j] = (ALSO == kRowBias ? b : next_w)[at(q, j)];
+        }
+    const auto row_sum = [&](const float (&part)[W]) {
+        float total = 0.0f;
 #pragma unroll
-        for (int k = 1; k < NSUM; ++k) sv[j] += yv[k][j];
+        for (int q = 0; q < W; ++q) total += wave_sum(part[q]);
+        return total;
+    };
+    float ss[W];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            if constexpr (GATE) sv[j][e] *= sigmoidf(gv[j][e]);
-            sv[j][e] = inside(j) ? sv[j][e] : 0.0f;
-            ss += normalize == 2 ? sv[j][e] : sv[j][e] * sv[j][e];
+    for (int q = 0; q < W; ++q) {
+        ss[q] = 0.0f;
+#pragma unroll
+        for (int j = 0; j < J; ++j) {
+            float s = yv[0][q][j];
+#pragma unroll
+            for (int k = 1; k < NSUM; ++k) s += yv[k][q][j];
+            if constexpr (GATE) s *= sigmoidf(gv[q][j]);
+            sv[q][j] = place(q, j) < d ? s : 0.0f;
+            ss[q] += normalize == 2 ? sv[q][j] : sv[q][j] * sv[q][j];
         }
     }
     if (normalize == 2) {
-        const float mean = wave_sum(ss) / static_cast<float>(d);
-        ss = 0.0f;
+        const float mean = row_sum(ss) / static_cast<float>(d);
 #pragma unroll
-        for (int j = 0; j < NV; ++j)
+        for (int q = 0; q < W; ++q) {
+            ss[q] = 0.0f;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                sv[j][e] = inside(j) ? sv[j][e] - mean : 0.0f;
-                ss += sv[j][e] * sv[j][e];
+            for (int j = 0; j < J; ++j) {
+                sv[q][j] -= mean;
+                if (place(q, j) < d) ss[q] += sv[q][j] * sv[q][j];
             }
+        }
     }
-    const float scale = normalize ? 1.0f / sqrtf(wave_sum(ss) / static_cast<float>(d) + eps) : 1.0f;
+    const float scale = normalize ? 1.0f / sqrtf(row_sum(ss) / static_cast<float>(d) + eps) : 1.0f;
     if (keep.state != nullptr && t < *keep.n_real) {
         const int s = keep.tok_seq[t], p = keep.positions[t];
         const int slot = keep.state_slots[s];
         if (p >= keep.context_lens[s] - keep.ring && slot >= 0 && slot < keep.n_slots) {
             float* dst = keep.state + (static_cast<int64_t>(slot) * keep.ring + p % keep.ring) * d;
 #pragma unroll
-            for (int j = 0; j < NV; ++j)
-                if (inside(j)) *reinterpret_cast<norm_f32x4*>(dst + at[j]) = xv[j];
+            for (int j = 0; j < J; ++j)
+#pragma unroll
+                for (int q = 0; q < W; ++q)
+                    if (place(q, j) < d) dst[place(q, j)] = xv[q][j];
         }
     }
-    float ss_new = 0.0f;
+    T* co = cast_out != nullptr ? cast_out + static_cast<int64_t>(t) * d : nullptr;
 #pragma unroll
-    for (int j = 0; j < NV; ++j) {
+    for (int q = 0; q < W; ++q) {
+        ss[q] = 0.0f;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            float v = sv[j][e] * scale;
-            if (w != nullptr) v *= wv[j][e];
-            if (b != nullptr) v += bv[j][e];
-            v += xv[j][e];
-            sv[j][e] = v;
-            ss_new += inside(j) ? v * v : 0.0f;
+        for (int j = 0; j < J; ++j) {
+            float v = sv[q][j] * scale;
+            if (w != nullptr) v *= wv[q][j];
+            if constexpr (ALSO == kRowBias) v += av[q][j];
+            v += xv[q][j];
+            sv[q][j] = v;
+            if (place(q, j) >= d) continue;
+            xr[place(q, j)] = v;
+            if constexpr (ALSO == kRowNext) ss[q] += v * v;
+            else if (co != nullptr) co[place(q, j)] = from_float<T>(v);
         }
-        if (inside(j)) *reinterpret_cast<norm_f32x4*>(xr + at[j]) = sv[j];
     }
-    if (cast_out == nullptr) return;
-    T* co = cast_out + static_cast<int64_t>(t) * d;
-    if (next_w != nullptr) {  // what is written for the next product is the next norm of the new row
-        const float next_scale = 1.0f / sqrtf(wave_sum(ss_new) / static_cast<float>(d) + next_eps);
+    if constexpr (ALSO == kRowNext) {  // what is written for the next product is the next norm of the new row
+        const float next_scale = 1.0f / sqrtf(row_sum(ss) / static_cast<float>(d) + next_eps);
 #pragma unroll
-        for (int j = 0; j < NV; ++j)
+        for (int j = 0; j < J; ++j)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) sv[j][e] = sv[j][e] * next_scale * nv[j][e];
+            for (int q = 0; q < W; ++q)
+                if (place(q, j) < d) co[place(q, j)] = from_float<T>(sv[q][j] * next_scale * av[q][j]);
     }
-#pragma unroll
-    for (int j = 0; j < NV; ++j)
-        if (inside(j)) norm_store4<T>(co + at[j], sv[j]);
 }
 
-template <typename T, int NV, int NSUM>
+template <typename T, int J, int NSUM>
 void launch_gated_norm_add_wave(float* x, T* cast_out, const float* y, const float* gate, int64_t gate_stride, const float* w, float eps, int normalize, int n,
                                 int d, const KeepRows& keep, const float* next_w, float next_eps, const float* b, hipStream_t stream) {
     const int rows = n <= 512 ? 1 : 4;  // rows a workgroup: few of them a wave on a compute unit of its own
-    if (gate != nullptr)
-        gated_norm_add_wave_kernel<T, NV, NSUM, true><<<(n + rows - 1) / rows, kWave * rows, 0, stream>>>(x, cast_out, y, gate, gate_stride, w, eps, normalize, n, d, keep, next_w, next_eps, b);
-    else
-        gated_norm_add_wave_kernel<T, NV, NSUM, false><<<(n + rows - 1) / rows, kWave * rows, 0, stream>>>(x, cast_out, y, gate, gate_stride, w, eps, normalize, n, d, keep, next_w, next_eps, b);
+#define LIYAB_GO(G, A) \
+    gated_norm_add_wave_kernel<T, J, NSUM, G, A><<<(n + rows - 1) / rows, kWave * rows, 0, stream>>>(x, cast_out, y, gate, gate_stride, w, eps, normalize, n, d, keep, next_w, next_eps, b)
+    if (gate != nullptr) LIYAB_GO(true, kRowOnly);
+    else if (b != nullptr) LIYAB_GO(false, kRowBias);
+    else if (next_w != nullptr) LIYAB_GO(false, kRowNext);
+    else LIYAB_GO(false, kRowOnly);
+#undef LIYAB_GO
 }
 
-// Whether the wave kernel took the rows; if not, the one above does.
+// Whether the wave kernel took the rows (of the gate, a bias and the next norm it takes one: what the blocks that exist use); if
+// not, the one above does.
 template <typename T>
 bool gated_norm_add_by_waves(float* x, T* cast_out, const float* y, int n_sum, const float* gate, int64_t gate_stride, const float* w, float eps, int normalize,
                              int n, int d, const KeepRows& keep, const float* next_w, float next_eps, const float* b, hipStream_t stream) {
-    auto al = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
-    if (d % 4 != 0 || d > 2048 || n_sum > 3 || !al(x) || !al(cast_out) || !al(y) || !al(gate) || gate_stride % 4 != 0 || !al(w) || !al(next_w) || !al(b) || !al(keep.state)) return false;
+    if (d > 2048 || n_sum > 3 || (gate != nullptr) + (b != nullptr) + (next_w != nullptr) > 1) return false;
 #define LIYAB_GO(V, S) launch_gated_norm_add_wave<T, V, S>(x, cast_out, y, gate, gate_stride, w, eps, normalize, n, d, keep, next_w, next_eps, b, stream)
 #define LIYAB_SUMS(V) (n_sum == 1 ? LIYAB_GO(V, 1) : n_sum == 2 ? LIYAB_GO(V, 2) : LIYAB_GO(V, 3))
     if (d <= 768) LIYAB_SUMS(3);

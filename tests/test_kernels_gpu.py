@@ -1089,25 +1089,24 @@ def test_scale_in_place(n):
     assert torch.equal(x, want)
 
 
-@pytest.mark.parametrize("n,d,n_sum", [(1, 4, 1), (5, 768, 2), (3, 772, 3), (7, 1024, 1), (2, 1600, 2), (4, 2048, 3), (513, 260, 1), (1025, 64, 2)])
-@pytest.mark.parametrize("centred", [False, True])
-def test_rows_update_by_waves_is_the_one_by_workgroups(ops, n, d, n_sum, centred):
-    """A wave a row where everything is aligned, a workgroup a row where it is not (the gate's columns start at an odd place):
-    the same update to the rounding of two orders of a sum of d squares (d 2^-24 of the norm at most, met by 1e-5)."""
-    x, y = rnd(n, d), rnd(n * n_sum, d, seed=1, scale=2.0) + 0.5
-    w, b, nw = rnd(d, seed=2) + 1.0, rnd(d, seed=3), rnd(d, seed=4) + 1.0
-    wide = rnd(n, d + 4, seed=5)
-    odd = torch.empty(n, d + 5, device=DEV)
-    odd[:, 1:] = wide
-    for cast, nxt in ((None, None), (torch.bfloat16, None), (torch.float32, (nw, 1e-6))):
+@pytest.mark.parametrize("n,d,n_sum", [(1, 3, 1), (5, 768, 2), (3, 769, 3), (7, 1024, 1), (2, 1600, 2), (4, 2048, 3), (513, 260, 1), (1025, 65, 2)])
+@pytest.mark.parametrize("also", ["nothing", "gate", "centred", "next"])
+def test_rows_update_by_waves_is_the_one_by_workgroups(ops, n, d, n_sum, also):
+    """A wave a row for up to three rows of y a token, a workgroup a row for more: with rows of zeros added to make four, the same
+    update (x + 0 is x)."""
+    x, y = rnd(n, d), rnd(n, n_sum, d, seed=1, scale=2.0) + 0.5
+    more = torch.cat([y, torch.zeros(n, 4 - n_sum, d, device=DEV)], dim=1)
+    w, kw = rnd(d, seed=2) + 1.0, {}
+    if also == "gate":
+        kw["gate"] = rnd(n, d + 4, seed=5)[:, 3:3 + d]
+    elif also == "centred":
+        kw.update(bias=rnd(d, seed=3), centred=True)
+    elif also == "next":
+        kw["next_norm"] = (rnd(d, seed=4) + 1.0, 1e-6)
+    for cast in (torch.bfloat16, torch.float32):
         got = []
-        for gate in (wide[:, 4:], odd[:, 5:]):
-            rows = x.clone()
-            out = torch.full((n, d), float("nan"), dtype=cast, device=DEV) if cast else None
-            ops.gated_norm_add(rows, y, w, 1e-5, n_sum=n_sum, gate=gate, cast_out=out, next_norm=nxt, bias=b if centred else None, centred=centred)
-            got.append((rows, out))
-        close(got[0][0], got[1][0], 1e-5, "rows")
-        if cast:
-            close(got[0][1], got[1][1], 1e-5 if cast == torch.float32 else 1e-2, "what the next product reads")
-            if nxt is None:
-                assert torch.equal(got[0][1], got[0][0].to(cast))
+        for rows, k in ((y, n_sum), (more, 4)):
+            into, out = x.clone(), torch.full((n, d), float("nan"), dtype=cast, device=DEV)
+            ops.gated_norm_add(into, rows.reshape(n * k, d), w, 1e-5, n_sum=k, cast_out=out, **kw)
+            got.append((into, out))
+        assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
