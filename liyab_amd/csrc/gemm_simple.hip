@@ -16,6 +16,7 @@
 
 #include "activations.h"
 #include "common.h"
+#include "epilogue.h"
 #include "launchers.h"
 
 namespace liyab {
@@ -129,6 +130,18 @@ __device__ __forceinline__ f32x4_t within_k(f32x4_t v, int k, int K) {
     return v;
 }
 
+// Where element (m, n) of a fused query, key and value product goes: queries to rows of their own, keys and values to their
+// pages (null: a token without a slot, or one outside these caches).
+__device__ __forceinline__ float* qkv_place(const EpiParams& p, int m, int n) {
+    if (n < p.q_dim) return static_cast<float*>(p.out) + static_cast<int64_t>(m) * p.ldo + n;
+    const uint32_t slot = p.slots[m];
+    if (slot >= p.num_slots) return nullptr;
+    const uint32_t page = slot / static_cast<uint32_t>(p.page_size), off = slot - page * static_cast<uint32_t>(p.page_size);
+    const bool is_v = n >= p.q_dim + p.kv_dim;
+    const int c = n - p.q_dim - (is_v ? p.kv_dim : 0), head = c / p.hd;
+    return static_cast<float*>(is_v ? p.vc : p.kc) + ((static_cast<int64_t>(page) * p.n_kv_head + head) * p.page_size + off) * p.hd + (c - head * p.hd);
+}
+
 // Many rows: tiles of 64 x 64 on four waves, a wave 32 x 32. The matrix cores set the pace (a stage of 32 k takes a compute
 // unit 1,024 cycles and 16 KB of operands), so operands go through registers into one of two stages in LDS while the
 // other is multiplied; they are asked for two stages ahead of their products (one stage ahead, a lone workgroup a
@@ -144,7 +157,7 @@ constexpr int kTile = 64;
 template <int EPI, bool EXACT, bool VEC>
 __global__ void __launch_bounds__(256)
 gemm_tiled_f32_kernel(float* __restrict__ out, int64_t ldo, const float* __restrict__ a, int64_t lda, const float* __restrict__ w,
-                      const float* __restrict__ bias, float* __restrict__ residual, int64_t ldr, int M, int N, int K, int vec_out) {
+                      const float* __restrict__ bias, float* __restrict__ residual, int64_t ldr, int M, int N, int K, int vec_out, EpiParams qkv) {
     constexpr int KS = 32, LD = KS + 4;         // k a stage; padded rows: 16 lanes' 16-byte reads fall into different banks
     constexpr int STAGE = 2 * kTile * LD;       // the tile of a, then the tile of w
     __shared__ __attribute__((aligned(16))) float smem[2 * STAGE];
@@ -231,6 +244,23 @@ gemm_tiled_f32_kernel(float* __restrict__ out, int64_t ldo, const float* __restr
 #pragma unroll
         for (int e = 0; e < 4; ++e) v[q][e] = finish_f32<EPI, EXACT>(tot[4 * q + e], bias != nullptr, v[q][e]);
     if (m >= M) return;
+    if constexpr (EPI == kEpiQkvPaged) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int n = nb + 8 * q;
+            if (vec_out) {  // four columns are of one head of one of the three
+                float* place = n < N ? qkv_place(qkv, m, n) : nullptr;
+                if (place != nullptr) *reinterpret_cast<f32x4_t*>(place) = v[q];
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    float* place = n + e < N ? qkv_place(qkv, m, n + e) : nullptr;
+                    if (place != nullptr) *place = v[q][e];
+                }
+            }
+        }
+        return;
+    }
     float* dst = EPI == kEpiResidual ? residual + static_cast<int64_t>(m) * ldr : out + static_cast<int64_t>(m) * ldo;
     if (vec_out) {  // N is a multiple of 4: four columns are in or out together
         if constexpr (EPI == kEpiResidual) {
@@ -269,7 +299,7 @@ template <int NB, int WAVES, int EPI, bool EXACT, bool VEC>
 __global__ void __launch_bounds__(64 * WAVES)
 gemm_chunks_f32_kernel(float* __restrict__ out, int64_t ldo, const float* __restrict__ a, int64_t lda,
                        const float* __restrict__ w, const float* __restrict__ bias, float* __restrict__ residual,
-                       int64_t ldr, int M_all, int N, int K) {
+                       int64_t ldr, int M_all, int N, int K, EpiParams qkv) {
     const int row0 = blockIdx.y * kChunkRows, M = min(kChunkRows, M_all - row0);
     a += static_cast<int64_t>(row0) * lda;
     constexpr int LD = kChunk + 4;  // (lanes read words 4 banks apart, their neighbours in k beside them: no collisions)
@@ -293,6 +323,9 @@ gemm_chunks_f32_kernel(float* __restrict__ out, int64_t ldo, const float* __rest
             if (4 * i < M) areg[i] = load4_f32<VEC>(a + static_cast<int64_t>(min(4 * i + lrow, M - 1)) * lda, k, K);  // (the same for every lane)
     };
     float tot = 0.0f;  // of output element (tid / NB, tid % NB), for tid < 16 * NB
+    float* place = nullptr;  // found while the first operands are on their way
+    if constexpr (EPI == kEpiQkvPaged)
+        if (tid < kChunkRows * NB && tid / NB < M && n0 + tid % NB < N) place = qkv_place(qkv, row0 + tid / NB, n0 + tid % NB);
     const float* wl = &Wt[wave][min(li, NB - 1)][g];
     const float* al = &At[wave][min(li, (M + 3) / 4 * 4 - 1)][g];  // (rows past M: some row that was written; not stored)
     if (wave < chunks) fetch(wave);
@@ -323,6 +356,7 @@ gemm_chunks_f32_kernel(float* __restrict__ out, int64_t ldo, const float* __rest
     const int m = row0 + tid / NB;
     const float v = finish_f32<EPI, EXACT>(tot, bias != nullptr, bias != nullptr ? bias[n] : 0.0f);
     if constexpr (EPI == kEpiResidual) residual[static_cast<int64_t>(m) * ldr + n] += v;
+    else if constexpr (EPI == kEpiQkvPaged) { if (place != nullptr) *place = v; }
     else out[static_cast<int64_t>(m) * ldo + n] = v;
 }
 
@@ -333,43 +367,44 @@ constexpr int kFewRows = 64;  // steps of at most this many rows never take the 
 
 template <int EPI, bool VEC>
 int launch_tiled_f32(float* out, int64_t ldo, const float* a, int64_t lda, const float* w, const float* bias, float* residual, int64_t ldr, int M,
-                     int N, int K, bool vec_out, hipStream_t stream) {
-    gemm_tiled_f32_kernel<EPI, true, VEC><<<((N + kTile - 1) / kTile) * ((M + kTile - 1) / kTile), 256, 0, stream>>>(out, ldo, a, lda, w, bias, residual, ldr, M, N, K, vec_out);
+                     int N, int K, bool vec_out, const EpiParams& qkv, hipStream_t stream) {
+    gemm_tiled_f32_kernel<EPI, true, VEC><<<((N + kTile - 1) / kTile) * ((M + kTile - 1) / kTile), 256, 0, stream>>>(out, ldo, a, lda, w, bias, residual, ldr, M, N, K, vec_out, qkv);
     return check_launch("gemm_tiled_f32");
 }
 
 template <int NB, int WAVES, int EPI, bool VEC>
 int launch_chunks_f32(float* out, int64_t ldo, const float* a, int64_t lda, const float* w, const float* bias, float* residual, int64_t ldr, int M,
-                      int N, int K, hipStream_t stream) {
+                      int N, int K, const EpiParams& qkv, hipStream_t stream) {
     gemm_chunks_f32_kernel<NB, WAVES, EPI, true, VEC><<<dim3((N + NB - 1) / NB, (M + kChunkRows - 1) / kChunkRows), 64 * WAVES, 0, stream>>>(
-        out, ldo, a, lda, w, bias, residual, ldr, M, N, K);
+        out, ldo, a, lda, w, bias, residual, ldr, M, N, K, qkv);
     return check_launch("gemm_chunks_f32");
 }
 
 template <int EPI, bool VEC>
 int launch_f32_epi(float* out, int64_t ldo, const float* a, int64_t lda, const float* w, const float* bias, float* residual, int64_t ldr, int M, int N,
-                   int K, hipStream_t stream) {
+                   int K, const EpiParams& qkv, hipStream_t stream) {
     auto al16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
-    const bool vec_out = N % 4 == 0 && (EPI == kEpiResidual ? al16(residual) && ldr % 4 == 0 : al16(out) && ldo % 4 == 0);
+    bool vec_out = N % 4 == 0 && (EPI == kEpiResidual ? al16(residual) && ldr % 4 == 0 : al16(out) && ldo % 4 == 0);
+    if (EPI == kEpiQkvPaged) vec_out = vec_out && qkv.q_dim % 4 == 0 && qkv.hd % 4 == 0 && al16(qkv.kc) && al16(qkv.vc);
 #define LIYAB_ARGS out, ldo, a, lda, w, bias, residual, ldr, M, N, K
     const int64_t tiles = static_cast<int64_t>((N + 63) / 64) * ((M + 63) / 64);
-    if (M > kFewRows && tiles >= kTiledMinTiles) return launch_tiled_f32<EPI, VEC>(LIYAB_ARGS, vec_out, stream);
+    if (M > kFewRows && tiles >= kTiledMinTiles) return launch_tiled_f32<EPI, VEC>(LIYAB_ARGS, vec_out, qkv, stream);
     // Two hundred workgroups of eight waves or more: 4, 8 or 16 features each; four waves once strips of 16 features are more than
     // one and a half a compute unit (64 rows, 768 -> 3,072: 8.4 us against 12.0; 768 -> 768, 192 of them: 11.1 with eight against 14.8)
     const int64_t strips = static_cast<int64_t>(N) * ((M + kChunkRows - 1) / kChunkRows);
-    if (strips <= 1024) return launch_chunks_f32<4, 8, EPI, VEC>(LIYAB_ARGS, stream);
-    if (strips <= 2048) return launch_chunks_f32<8, 8, EPI, VEC>(LIYAB_ARGS, stream);
-    if (strips <= 16 * 400) return launch_chunks_f32<16, 8, EPI, VEC>(LIYAB_ARGS, stream);
-    return launch_chunks_f32<16, 4, EPI, VEC>(LIYAB_ARGS, stream);
+    if (strips <= 1024) return launch_chunks_f32<4, 8, EPI, VEC>(LIYAB_ARGS, qkv, stream);
+    if (strips <= 2048) return launch_chunks_f32<8, 8, EPI, VEC>(LIYAB_ARGS, qkv, stream);
+    if (strips <= 16 * 400) return launch_chunks_f32<16, 8, EPI, VEC>(LIYAB_ARGS, qkv, stream);
+    return launch_chunks_f32<16, 4, EPI, VEC>(LIYAB_ARGS, qkv, stream);
 #undef LIYAB_ARGS
 }
 
 template <int EPI>
 int launch_f32(float* out, int64_t ldo, const float* a, int64_t lda, const float* w, const float* bias, float* residual, int64_t ldr, int M, int N,
-               int K, hipStream_t stream) {
+               int K, hipStream_t stream, const EpiParams& qkv = EpiParams{}) {
     const bool vec = (reinterpret_cast<uintptr_t>(a) & 15) == 0 && (reinterpret_cast<uintptr_t>(w) & 15) == 0 && lda % 4 == 0 && K % 4 == 0;
-    if (vec) return launch_f32_epi<EPI, true>(out, ldo, a, lda, w, bias, residual, ldr, M, N, K, stream);
-    return launch_f32_epi<EPI, false>(out, ldo, a, lda, w, bias, residual, ldr, M, N, K, stream);
+    if (vec) return launch_f32_epi<EPI, true>(out, ldo, a, lda, w, bias, residual, ldr, M, N, K, qkv, stream);
+    return launch_f32_epi<EPI, false>(out, ldo, a, lda, w, bias, residual, ldr, M, N, K, qkv, stream);
 }
 
 template <typename T, typename OutT, bool EXACT>
@@ -428,4 +463,16 @@ extern "C" int liyab_gemm_simple(void* out, int out_dtype, int64_t ldo, const vo
         return fail(1, "gemm: unknown output dtype %d", out_dtype);
     }
     return fail(1, "gemm: unknown dtype %d", dtype);
+}
+
+// The fused query, key and value product of the 32-bit path: queries to epi->out, keys and values into their pages (epi->mode:
+// the paged one). The bits are liyab_gemm_simple's followed by liyab_kv_write's, without that launch and its trip through memory (4.6 us
+// a layer of a decode step).
+extern "C" int liyab_gemm_f32_qkv(const float* a, int64_t lda, const float* w, int M, int N, int K, const EpiParams* epi, hipStream_t stream) {
+    LIYAB_REQUIRE(a && w && epi, "gemm_f32_qkv: null operand");
+    LIYAB_REQUIRE(M >= 0 && N > 0 && K > 0 && lda >= K, "gemm_f32_qkv: bad sizes M=%d N=%d K=%d lda=%lld", M, N, K, static_cast<long long>(lda));
+    LIYAB_REQUIRE(epi->mode == kEpiQkvPaged && epi->out_dtype == kF32, "gemm_f32_qkv: takes the paged epilogue with 32-bit caches only");
+    if (int rc = check_epilogue(*epi, M, N)) return rc;
+    if (M == 0) return 0;
+    return launch_f32<kEpiQkvPaged>(static_cast<float*>(epi->out), epi->ldo, a, lda, w, epi->bias, nullptr, 0, M, N, K, stream, *epi);
 }

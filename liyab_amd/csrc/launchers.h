@@ -29,6 +29,7 @@ int liyab_gemm_simple(void* out, int out_dtype, int64_t ldo, const void* a, int6
                       float* residual, int64_t ldr, int M, int N, int K, int epi, hipStream_t stream);
 int liyab_gemm_mfma(const void* a, int64_t lda, const void* w, int M, int N, int K, int tile, const liyab::EpiParams* epi_in,
                     hipStream_t stream);
+int liyab_gemm_f32_qkv(const float* a, int64_t lda, const float* w, int M, int N, int K, const liyab::EpiParams* epi, hipStream_t stream);
 int liyab_gemm_mfma_dl(const void* a, int64_t lda, const void* w, int M, int N, int K, int tile, const liyab::EpiParams* epi_in,
                        hipStream_t stream);
 int liyab_gemm_mfma_dl_parts(const void* a, int64_t lda, const void* w, int M, int N, int K, int kparts, int tile, float* parts,

@@ -76,6 +76,7 @@ static const Entry kEntries[] = {
     LIYAB_ENTRY(liyab_layernorm_parts),
     LIYAB_ENTRY(liyab_sum_parts),
     LIYAB_ENTRY(liyab_gemm_simple),
+    LIYAB_ENTRY(liyab_gemm_f32_qkv),
     LIYAB_ENTRY(liyab_gemm_mfma),
     LIYAB_ENTRY(liyab_gemm_mfma_dl),
     LIYAB_ENTRY(liyab_gemm_mfma_dl_parts),

@@ -462,6 +462,18 @@ def gemm_mfma(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], *,
     _lib.call("liyab_gemm_mfma", a.data_ptr(), lda, w.data_ptr(), M, w.shape[0], K, tile, ctypes.byref(e), _stream())
 
 
+def gemm_f32_qkv(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], *, out: torch.Tensor, kv) -> None:
+    """The fused query, key and value product in 32 bits: queries to `out` [M, q_dim], keys and values into their pages;
+    `kv` as `gemm` takes it. The bits of `gemm_simple` followed by `kv_write`."""
+    lda = _rows(a, "a")
+    M, K = a.shape
+    _dev(w, "w")
+    if a.dtype != torch.float32 or w.dtype != torch.float32 or w.dim() != 2 or w.shape[1] != K or not w.is_contiguous() or out.dtype != torch.float32:
+        raise KernelError(f"gemm_f32_qkv: needs float32 a [M, K], contiguous w [N, K] and out, got {tuple(a.shape)} {a.dtype}, {tuple(w.shape)} {w.dtype}, {out.dtype}")
+    e = _epilogue(a, w, bias, out, None, EPI_QKV_PAGED, kv)
+    _lib.call("liyab_gemm_f32_qkv", a.data_ptr(), lda, w.data_ptr(), M, w.shape[0], K, ctypes.byref(e), _stream())
+
+
 def gemm_skinny(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], *, out=None, residual=None,
                 epilogue: int = EPI_NONE, kv=None, ksplit: int = 0, wide: int = -1, mtile: int = 0) -> None:
     """The weight-streaming product for at most 64 bfloat16 rows, K a multiple of 8. ksplit

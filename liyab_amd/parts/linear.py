@@ -56,6 +56,9 @@ def linear(a, w: torch.Tensor, bias: Optional[torch.Tensor], *, out: Optional[to
         return
     if isinstance(a, Normed):
         a = a.tensor()
+    if kv is not None and w.dtype == torch.float32:
+        ops.gemm_f32_qkv(a, w, bias, out=out, kv=kv)
+        return
     ops.gemm(a, w, bias, out=out, residual=residual, epilogue=epilogue, kv=kv)
 
 
@@ -117,4 +120,4 @@ def linear_deferred(a, w: torch.Tensor, bias: Optional[torch.Tensor], ctx, name:
 def paged_qkv_takes(dtype: torch.dtype, k: int) -> bool:
     """Whether the product kernels for this dtype and inner size can write keys and values
     into cache pages from their epilogue."""
-    return dtype == torch.bfloat16 and k % 8 == 0
+    return dtype == torch.float32 or (dtype == torch.bfloat16 and k % 8 == 0)

@@ -1110,3 +1110,24 @@ def test_rows_update_by_waves_is_the_one_by_workgroups(ops, n, d, n_sum, also):
             ops.gated_norm_add(into, rows.reshape(n * k, d), w, 1e-5, n_sum=k, cast_out=out, **kw)
             got.append((into, out))
         assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+
+
+@pytest.mark.parametrize("M,H,Hkv,hd,K,page", [(1, 4, 4, 16, 64, 16), (4, 12, 12, 64, 768, 64), (17, 5, 5, 48, 100, 16), (65, 6, 2, 32, 130, 24), (300, 12, 12, 64, 96, 16), (3, 3, 1, 10, 30, 7)])
+def test_float32_qkv_product_into_the_pages(ops, M, H, Hkv, hd, K, page):
+    """Queries to a dense buffer, keys and values straight into shuffled slots: the bits of the product followed by the
+    scatter, in strips and in tiles, heads that are no multiple of four; slots of no token or outside the caches stay unwritten."""
+    q_dim, kv_dim = H * hd, Hkv * hd
+    a, w, bias = rnd(M, K), rnd(q_dim + 2 * kv_dim, K, seed=1), rnd(q_dim + 2 * kv_dim, seed=2)
+    pages = -(-M // page) + 3
+    slots = torch.randperm(pages * page)[:M].to(torch.int32)
+    if M > 16:
+        slots[3], slots[10] = -1, pages * page
+    slots = slots.to(DEV)
+    full = torch.empty(M, q_dim + 2 * kv_dim, device=DEV)
+    ops.gemm_simple(a, w, bias, out=full)
+    want = [torch.zeros(pages, Hkv, page, hd, device=DEV) for _ in range(2)]
+    ops.kv_write(*want, full, q_dim, q_dim + kv_dim, slots)
+    got = [torch.zeros_like(want[0]) for _ in range(2)]
+    q = torch.full((M, q_dim), float("nan"), device=DEV)
+    ops.gemm_f32_qkv(a, w, bias, out=q, kv=(*got, slots, q_dim))
+    assert torch.equal(q, full[:, :q_dim]) and torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
