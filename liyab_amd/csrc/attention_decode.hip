@@ -98,10 +98,7 @@ attention_decode_kernel(T* __restrict__ out, int64_t out_stride, const T* __rest
                         int keep_first = 0) {
     constexpr int KPP = 64 / LPK;  // keys per wave and pass
     __shared__ float lds2[2][AD_WAVES][LPK][10];  // the waves' sums, for the first wave to merge; two of them in turn, so that one barrier a split is enough
-    // Workgroups go to the 8 XCDs in turn. With heads fastest (the launcher's choice where every query head has keys of its own) a
-    // token's heads spread over all of them, and its neighbours' keys lie beside its own; with tokens fastest, and a number of
-    // tokens that 8 divides, one XCD had all of a token, and the one with the long contexts was waited for (64 tokens of 256 to
-    // 1,015 keys, 25 heads of 64: 57 us a layer, 49 with 636 keys each). Query heads that share keys stay on one XCD and its L2.
+    // (which of the two the grid runs along first: heads_first_pays)
     const int slot = heads_first ? blockIdx.y : blockIdx.x;
     const int t = tok_list != nullptr ? tok_list[slot] : slot;
     const int h = heads_first ? blockIdx.x : blockIdx.y, z = blockIdx.z;
@@ -332,6 +329,27 @@ __global__ void attention_merge_kernel(T* __restrict__ out, int64_t out_stride, 
     out[static_cast<int64_t>(t) * out_stride + static_cast<int64_t>(h) * hd + e] = from_float<T>(o / sum);
 }
 
+// Whether the grid runs along the heads first. Workgroups go to the 8 XCDs in turn, each with 4 MB of L2. With tokens first, and a
+// number of tokens that 8 divides, an XCD has all of a token, and the one with the long contexts is waited for; with heads first a
+// token's heads spread over the XCDs. Measured, us a call, tokens first -> heads first; 64 wide heads, contexts of 256 to 1,015 keys:
+//   one token a request: 64 tokens of 25 heads 58.8 -> 54.6, of 16 heads 36.9 -> 34.7, 128 of 12 heads 53.9 -> 50.8; splits left to the
+//     projection, 1 to 16 tokens, 1-6 % less; up to 16 tokens uncut or merged here: even, scored (8 tokens, a window of 512) 7.4 -> 7.8;
+//   short portions (up to 8 tokens a request, side by side: their common keys stay in an XCD's L2): 8 x 8 tokens of 12 heads
+//     22.5 -> 16.2, 32 x 8 of 20 heads 122 -> 64, of 25 heads even;
+//   whole prompts in fixed chunks (neighbours read the same keys): heads first while the keys and values of the heads that fall
+//     to one XCD, n_head / gcd(n_head, 8) of them, stay in its L2: 300 rows of 12 heads 30.5 -> 28.5 in 32 bits, a bfloat16 prompt of
+//     1,000 118 -> 109; beyond it tokens first: 25 heads in 32 bits, 600 keys (7.7 MB) 504 against 653, 8 x 1,000 keys 2,440 against
+//     4,600; 12 heads of 6,000 keys (9.2 MB) 3,900 against 4,280; at 3.8 to 4.1 MB even. What a request can reach stands for its keys.
+// Query heads that share keys stay on one XCD: tokens first.
+inline bool heads_first_pays(int n, int n_head, int n_kv_head, int hd, size_t elt, int64_t reach, int chunk, bool rows_are_requests, bool leave_splits) {
+    if (n_head != n_kv_head || n > 65535) return false;
+    if (rows_are_requests) return leave_splits || n > 16;
+    if (chunk == 0) return true;
+    int heads = n_head;
+    for (int xcds = 8; xcds > 1 && heads % 2 == 0; xcds /= 2) heads /= 2;
+    return heads * reach * hd * 2 * static_cast<int64_t>(elt) <= (4 << 20);
+}
+
 template <typename T, bool SCORED = false>
 int launch_attention_decode(void* out, int64_t out_stride, const void* q, int64_t q_stride, const void* kc, const void* vc,
                             const int* block_tables, int max_blocks, const int* tok_list, const int* tok_seq,
@@ -342,7 +360,8 @@ int launch_attention_decode(void* out, int64_t out_stride, const void* q, int64_
     int page_shift = -1;
     for (int b = 0; b < 31; ++b)
         if ((1 << b) == page_size) page_shift = b;
-    const int heads_first = n_head == n_kv_head && n <= 65535;
+    const int64_t table = static_cast<int64_t>(max_blocks) * page_size, seen = static_cast<int64_t>(window) + keep_first;
+    const int heads_first = heads_first_pays(n, n_head, n_kv_head, hd, sizeof(T), window > 0 && seen < table ? seen : table, chunk, rows_are_requests, leave_splits);
     const dim3 grid = heads_first ? dim3(n_head, n, n_splits) : dim3(n, n_head, n_splits);
     auto* o = static_cast<T*>(out);
     auto* pq = static_cast<const T*>(q);

@@ -534,6 +534,39 @@ def test_attention_splits_by_position(ops, case_id, dtype, window):
         assert torch.equal(out[rows], outs[0][rows]), f"request {s_} alone"
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_attention_order_of_the_grid(ops, dtype):
+    """The grid runs along the heads or along the tokens first, by what a prompt's heads bring to an XCD's L2 (the width of the
+    block table stands for the keys: five heads of 64 on either side of 4 MB) and by the number of single-token requests (16
+    and 17): the same bits, and right against the plain formula."""
+    H, hd, page = 5, 64, 16
+    scale = 0.7 / math.sqrt(hd)
+    case = paged_case(2, [300, 33], [40, 33], H, H, hd, page, dtype, seed=3)
+    bt = case["bt"]
+    outs = []
+    for columns in (102, 103):
+        columns = columns * 4 // dtype.itemsize  # 4,177,920 bytes of keys and values, 4,218,880
+        case["bt"] = torch.cat([bt, bt.new_zeros(bt.shape[0], columns - bt.shape[1])], dim=1)
+        dev = [case[k].to(DEV) for k in ("q", "kc", "vc", "bt")] + [torch.tensor(case[k], dtype=torch.int32, device=DEV) for k in ("tok_seq", "tok_pos")]
+        out = torch.zeros(case["n"], H * hd, dtype=dtype, device=DEV)
+        ops.attention_decode(out, dev[0][:, :H * hd], *dev[1:], n_head=H, scale=scale, n_splits=1, waves=4, chunk=256)
+        outs.append(out)
+    close(outs[0], attention_reference(case, H, H, hd, scale), 8e-3 if dtype == torch.bfloat16 else 2e-6, "grid order")
+    assert torch.equal(outs[0], outs[1])
+    case = paged_case(17, list(range(20, 20 + 17 * 9, 9)), [1] * 17, H, H, hd, page, dtype, seed=4)
+    dev = [case[k].to(DEV) for k in ("q", "kc", "vc", "bt")] + [torch.tensor(case[k], dtype=torch.int32, device=DEV) for k in ("tok_seq", "tok_pos")]
+    for splits in (1, 3):
+        outs = []
+        for n in (17, 16):
+            out = torch.zeros(n, H * hd, dtype=dtype, device=DEV)
+            partials = torch.empty(n * H * splits * (hd + 4), device=DEV) if splits > 1 else None
+            ops.attention_decode(out, dev[0][:n, :H * hd], *dev[1:4], dev[4][:n], dev[5][:n], n_head=H, scale=scale, n_splits=splits, partials=partials,
+                                 waves=4, rows_are_requests=True)
+            outs.append(out)
+        close(outs[0], attention_reference(case, H, H, hd, scale), 8e-3 if dtype == torch.bfloat16 else 2e-6, "single tokens")
+        assert torch.equal(outs[0][:16], outs[1])
+
+
 @pytest.mark.parametrize("waves", [4, 16])
 @pytest.mark.parametrize("window", [0, 37])
 @pytest.mark.parametrize("splits", [2, 4, 7, 8])
