@@ -272,30 +272,53 @@ gated_norm_add_wave_kernel(float* __restrict__ x, T* __restrict__ cast_out, cons
     }
 }
 
-template <typename T, int J, int NSUM>
-void launch_gated_norm_add_wave(float* x, T* cast_out, const float* y, const float* gate, int64_t gate_stride, const float* w, float eps, int normalize, int n,
-                                int d, const KeepRows& keep, const float* next_w, float next_eps, const float* b, hipStream_t stream) {
-    const int rows = n <= 512 ? 1 : 4;  // rows a workgroup: few of them a wave on a compute unit of its own
-#define LIYAB_GO(G, A) \
-    gated_norm_add_wave_kernel<T, J, NSUM, G, A><<<(n + rows - 1) / rows, kWave * rows, 0, stream>>>(x, cast_out, y, gate, gate_stride, w, eps, normalize, n, d, keep, next_w, next_eps, b)
-    if (gate != nullptr) LIYAB_GO(true, kRowOnly);
-    else if (b != nullptr) LIYAB_GO(false, kRowBias);
-    else if (next_w != nullptr) LIYAB_GO(false, kRowNext);
-    else LIYAB_GO(false, kRowOnly);
-#undef LIYAB_GO
-}
-
 // Whether the wave kernel took the rows (of the gate, a bias and the next norm it takes one: what the blocks that exist use); if
-// not, the one above does.
+// not, the one above does. A place past the row costs what one inside does, which shows where each takes a sigmoid: with a gate J is
+// the least that holds the row (behind the kernels that write y and the gate, us for all of them, by workgroups, by waves with J of 3, 4
+// and 8 only, and now: 4 rows of 256 6.0, 6.3, 5.6; of 1,280 8.2, 9.3, 8.4; 2,048 rows of 1,280 21.1, 21.7, 19.3. Bokulix 1,280 wide, a
+// prompt of 32 and eight decoded tokens, 29.8, 29.1, 28.1 ms). Without one, J of 3, 4 and 8 is enough (behind the kernel that writes y, by
+// workgroups and by waves: 4 rows of 1,280 5.4 and 5.4, with two rows a token 6.7 and 5.7; 2,048 rows of 1,280 13.7 and 12.9; of 2,048 18.6 and
+// 16.6, a layer norm 21.2 and 16.9, three rows a token and the next norm 33.6 and 30.8).
 template <typename T>
 bool gated_norm_add_by_waves(float* x, T* cast_out, const float* y, int n_sum, const float* gate, int64_t gate_stride, const float* w, float eps, int normalize,
                              int n, int d, const KeepRows& keep, const float* next_w, float next_eps, const float* b, hipStream_t stream) {
     if (d > 2048 || n_sum > 3 || (gate != nullptr) + (b != nullptr) + (next_w != nullptr) > 1) return false;
-#define LIYAB_GO(V, S) launch_gated_norm_add_wave<T, V, S>(x, cast_out, y, gate, gate_stride, w, eps, normalize, n, d, keep, next_w, next_eps, b, stream)
-#define LIYAB_SUMS(V) (n_sum == 1 ? LIYAB_GO(V, 1) : n_sum == 2 ? LIYAB_GO(V, 2) : LIYAB_GO(V, 3))
-    if (d <= 768) LIYAB_SUMS(3);
-    else if (d <= 1024) LIYAB_SUMS(4);
-    else LIYAB_SUMS(8);
+    // Rows a workgroup: a few hundred, one (a wave with a compute unit, or a SIMD, of its own: 64 to 300 rows of 768 to 2,048 1-7 % less than
+    // in fours); many, four (780 to 4,096 rows: even, up to 4 % less)
+    const int rows = n <= 512 ? 1 : 4;
+#define LIYAB_GO(J, S, G, A) \
+    gated_norm_add_wave_kernel<T, J, S, G, A><<<(n + rows - 1) / rows, kWave * rows, 0, stream>>>(x, cast_out, y, gate, gate_stride, w, eps, normalize, n, d, keep, next_w, next_eps, b)
+#define LIYAB_SUMS(J, G, A)                 \
+    do {                                    \
+        if (n_sum == 1) LIYAB_GO(J, 1, G, A); \
+        else if (n_sum == 2) LIYAB_GO(J, 2, G, A); \
+        else LIYAB_GO(J, 3, G, A);          \
+    } while (0)
+#define LIYAB_WIDTHS(A)                         \
+    do {                                        \
+        if (d <= 768) LIYAB_SUMS(3, false, A);  \
+        else if (d <= 1024) LIYAB_SUMS(4, false, A); \
+        else LIYAB_SUMS(8, false, A);           \
+    } while (0)
+    if (gate != nullptr) {
+        switch ((d + 255) / 256) {
+            case 1: LIYAB_SUMS(1, true, kRowOnly); break;
+            case 2: LIYAB_SUMS(2, true, kRowOnly); break;
+            case 3: LIYAB_SUMS(3, true, kRowOnly); break;
+            case 4: LIYAB_SUMS(4, true, kRowOnly); break;
+            case 5: LIYAB_SUMS(5, true, kRowOnly); break;
+            case 6: LIYAB_SUMS(6, true, kRowOnly); break;
+            case 7: LIYAB_SUMS(7, true, kRowOnly); break;
+            default: LIYAB_SUMS(8, true, kRowOnly); break;
+        }
+    } else if (b != nullptr) {
+        LIYAB_WIDTHS(kRowBias);
+    } else if (next_w != nullptr) {
+        LIYAB_WIDTHS(kRowNext);
+    } else {
+        LIYAB_WIDTHS(kRowOnly);
+    }
+#undef LIYAB_WIDTHS
 #undef LIYAB_SUMS
 #undef LIYAB_GO
     return true;

@@ -1122,7 +1122,8 @@ def test_scale_in_place(n):
     assert torch.equal(x, want)
 
 
-@pytest.mark.parametrize("n,d,n_sum", [(1, 3, 1), (5, 768, 2), (3, 769, 3), (7, 1024, 1), (2, 1600, 2), (4, 2048, 3), (513, 260, 1), (1025, 65, 2)])
+@pytest.mark.parametrize("n,d,n_sum", [(1, 3, 1), (5, 768, 2), (3, 769, 3), (7, 1024, 1), (2, 1600, 2), (4, 2048, 3), (513, 260, 1), (1025, 65, 2),
+                                     (2, 256, 3), (3, 1280, 1), (600, 1281, 2), (2, 1700, 3)])
 @pytest.mark.parametrize("also", ["nothing", "gate", "centred", "next"])
 def test_rows_update_by_waves_is_the_one_by_workgroups(ops, n, d, n_sum, also):
     """A wave a row for up to three rows of y a token, a workgroup a row for more: with rows of zeros added to make four, the same
