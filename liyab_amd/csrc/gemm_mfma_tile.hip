@@ -165,7 +165,7 @@ int choose_gemm_tile(int M, int N, int K) {
     struct Shape { int tile, bm, bn, fit; float unit[3], round; };
     constexpr Shape shapes[] = {
         {15, 256, 256, 1, {1.45f, 0, 0}, 10.0f}, {9, 192, 128, 2, {0.68f, 1.3f, 0}, 5.0f},  {11, 192, 128, 1, {0.62f, 0, 0}, 4.5f},
-        {8, 128, 128, 2, {0.60f, 1.0f, 0}, 4.0f}, {7, 128, 128, 1, {0.45f, 0, 0}, 4.5f},    {6, 64, 64, 2, {0.30f, 0.45f, 0}, 2.0f},
+        {8, 128, 128, 2, {0.60f, 1.0f, 0}, 4.0f}, {7, 128, 128, 1, {0.50f, 0, 0}, 3.7f},    {6, 64, 64, 2, {0.30f, 0.45f, 0}, 2.0f},
         {2, 64, 64, 3, {0.30f, 0.45f, 0.62f}, 2.0f}};
     constexpr int kUnits = 256;  // compute units
     int best = 0;
@@ -180,6 +180,11 @@ int choose_gemm_tile(int M, int N, int K) {
             best_us = us;
         }
     }
+    // Tiles of 64 x 64 in three stages and in four cost the same here. With a compute unit each, two on every unit, or a long K the fourth
+    // stage is worth its LDS (780 rows, 5,120 -> 1,280 33.4 us against 35.2 in three; 361 rows, 1,280 -> 5,120 14.7 against 14.9); a round
+    // in between with a short K takes three (512 rows: 768 -> 2,304 8.9 against 9.7, 1,024 -> 3,072 10.8 against 11.5).
+    const int64_t small = static_cast<int64_t>((M + 63) / 64) * ((N + 63) / 64);
+    if (best == 6 && K < 1280 && small > kUnits && small < 2 * kUnits) best = 2;
     return best;
 }
 
