@@ -339,15 +339,15 @@ __global__ void attention_merge_kernel(T* __restrict__ out, int64_t out_stride, 
 //   whole prompts in fixed chunks (neighbours read the same keys): heads first while the keys and values of the heads that fall
 //     to one XCD, n_head / gcd(n_head, 8) of them, stay in its L2: 300 rows of 12 heads 30.5 -> 28.5 in 32 bits, a bfloat16 prompt of
 //     1,000 118 -> 109; beyond it tokens first: 25 heads in 32 bits, 600 keys (7.7 MB) 504 against 653, 8 x 1,000 keys 2,440 against
-//     4,600; 12 heads of 6,000 keys (9.2 MB) 3,900 against 4,280; at 3.8 to 4.1 MB even. What a request can reach stands for its keys.
+//     4,600; 12 heads of 6,000 keys (9.2 MB) 3,900 against 4,280; at 3.8 to 4.1 MB even.
 // Query heads that share keys stay on one XCD: tokens first.
-inline bool heads_first_pays(int n, int n_head, int n_kv_head, int hd, size_t elt, int64_t reach, int chunk, bool rows_are_requests, bool leave_splits) {
+inline bool heads_first_pays(int n, int n_head, int n_kv_head, int hd, size_t elt, int64_t keys, int chunk, bool rows_are_requests, bool leave_splits) {
     if (n_head != n_kv_head || n > 65535) return false;
     if (rows_are_requests) return leave_splits || n > 16;
     if (chunk == 0) return true;
     int heads = n_head;
     for (int xcds = 8; xcds > 1 && heads % 2 == 0; xcds /= 2) heads /= 2;
-    return heads * reach * hd * 2 * static_cast<int64_t>(elt) <= (4 << 20);
+    return heads * keys * hd * 2 * static_cast<int64_t>(elt) <= (4 << 20);
 }
 
 template <typename T, bool SCORED = false>
@@ -355,13 +355,15 @@ int launch_attention_decode(void* out, int64_t out_stride, const void* q, int64_
                             const int* block_tables, int max_blocks, const int* tok_list, const int* tok_seq,
                             const int* tok_pos, int n, float scale, int window, int n_head, int n_kv_head, int hd,
                             int page_size, int n_splits, int chunk, int waves, int rows_are_requests, float* partials,
-                            int leave_splits, int num_pages, hipStream_t stream, float softcap = 0.0f, const float* bias_table = nullptr,
+                            int leave_splits, int num_pages, int reach, hipStream_t stream, float softcap = 0.0f, const float* bias_table = nullptr,
                             int max_dist = 0, const float* sinks = nullptr, int keep_first = 0) {
     int page_shift = -1;
     for (int b = 0; b < 31; ++b)
         if ((1 << b) == page_size) page_shift = b;
-    const int64_t table = static_cast<int64_t>(max_blocks) * page_size, seen = static_cast<int64_t>(window) + keep_first;
-    const int heads_first = heads_first_pays(n, n_head, n_kv_head, hd, sizeof(T), window > 0 && seen < table ? seen : table, chunk, rows_are_requests, leave_splits);
+    int64_t keys = static_cast<int64_t>(max_blocks) * page_size;
+    if (reach > 0 && reach < keys) keys = reach;
+    if (window > 0 && static_cast<int64_t>(window) + keep_first < keys) keys = static_cast<int64_t>(window) + keep_first;
+    const int heads_first = heads_first_pays(n, n_head, n_kv_head, hd, sizeof(T), keys, chunk, rows_are_requests, leave_splits);
     const dim3 grid = heads_first ? dim3(n_head, n, n_splits) : dim3(n, n_head, n_splits);
     auto* o = static_cast<T*>(out);
     auto* pq = static_cast<const T*>(q);
@@ -409,6 +411,8 @@ using namespace liyab;
 // split an equal share of the token's keys; > 0 = split z takes keys [z * chunk, (z + 1) * chunk)
 // of the token's (n_splits * chunk must cover the longest context: keys beyond are not read).
 // num_pages: the pages the caches hold; page ids of the block tables are brought into [0, num_pages).
+// reach: the most keys a token of the launch has, rounded up, or 0 for what its block table holds; the order of the grid follows from
+// it and nothing else does.
 static int check_attention_decode(void* out, int64_t out_stride, const void* q, int64_t q_stride, const void* kc, const void* vc, int dtype,
                                   const int* block_tables, int max_blocks, const int* tok_list, const int* tok_seq, const int* tok_pos, int n,
                                   int window, int n_head, int n_kv_head, int hd, int page_size, int n_splits, int chunk, int waves,
@@ -443,7 +447,7 @@ extern "C" int liyab_attention_decode(void* out, int64_t out_stride, const void*
                                       const void* vc, int dtype, const int* block_tables, int max_blocks, const int* tok_list,
                                       const int* tok_seq, const int* tok_pos, int n, float scale, int window,
                                       int n_head, int n_kv_head, int hd, int page_size, int n_splits, int chunk, int waves,
-                                      int rows_are_requests, float* partials, int leave_splits, int num_pages, hipStream_t stream) {
+                                      int rows_are_requests, float* partials, int leave_splits, int num_pages, int reach, hipStream_t stream) {
     if (int rc = check_attention_decode(out, out_stride, q, q_stride, kc, vc, dtype, block_tables, max_blocks, tok_list, tok_seq, tok_pos, n, window,
                                         n_head, n_kv_head, hd, page_size, n_splits, chunk, waves, rows_are_requests, partials, leave_splits, num_pages, 0))
         return rc;
@@ -451,10 +455,10 @@ extern "C" int liyab_attention_decode(void* out, int64_t out_stride, const void*
     if (dtype == kF32)
         return launch_attention_decode<float>(out, out_stride, q, q_stride, kc, vc, block_tables, max_blocks, tok_list, tok_seq,
                                               tok_pos, n, scale, window, n_head, n_kv_head, hd, page_size, n_splits, chunk, waves,
-                                              rows_are_requests, partials, leave_splits, num_pages, stream);
+                                              rows_are_requests, partials, leave_splits, num_pages, reach, stream);
     return launch_attention_decode<bf16_t>(out, out_stride, q, q_stride, kc, vc, block_tables, max_blocks, tok_list, tok_seq,
                                            tok_pos, n, scale, window, n_head, n_kv_head, hd, page_size, n_splits, chunk, waves,
-                                           rows_are_requests, partials, leave_splits, num_pages, stream);
+                                           rows_are_requests, partials, leave_splits, num_pages, reach, stream);
 }
 
 // The same with the scores worked on before the softmax: softcap > 0 caps them, cap * tanh(score / cap); bias_table (float
@@ -464,7 +468,7 @@ extern "C" int liyab_attention_decode_scored(void* out, int64_t out_stride, cons
                                              const void* vc, int dtype, const int* block_tables, int max_blocks, const int* tok_list,
                                              const int* tok_seq, const int* tok_pos, int n, float scale, int window,
                                              int n_head, int n_kv_head, int hd, int page_size, int n_splits, int chunk, int waves,
-                                             int rows_are_requests, float* partials, int leave_splits, int num_pages, float softcap,
+                                             int rows_are_requests, float* partials, int leave_splits, int num_pages, int reach, float softcap,
                                              const float* bias_table, int max_dist, const float* sinks, int keep_first, hipStream_t stream) {
     if (int rc = check_attention_decode(out, out_stride, q, q_stride, kc, vc, dtype, block_tables, max_blocks, tok_list, tok_seq, tok_pos, n, window,
                                         n_head, n_kv_head, hd, page_size, n_splits, chunk, waves, rows_are_requests, partials, leave_splits, num_pages, keep_first))
@@ -475,10 +479,10 @@ extern "C" int liyab_attention_decode_scored(void* out, int64_t out_stride, cons
     if (dtype == kF32)
         return launch_attention_decode<float, true>(out, out_stride, q, q_stride, kc, vc, block_tables, max_blocks, tok_list, tok_seq,
                                                     tok_pos, n, scale, window, n_head, n_kv_head, hd, page_size, n_splits, chunk, waves,
-                                                    rows_are_requests, partials, leave_splits, num_pages, stream, softcap, bias_table, max_dist, sinks, keep_first);
+                                                    rows_are_requests, partials, leave_splits, num_pages, reach, stream, softcap, bias_table, max_dist, sinks, keep_first);
     return launch_attention_decode<bf16_t, true>(out, out_stride, q, q_stride, kc, vc, block_tables, max_blocks, tok_list, tok_seq,
                                                  tok_pos, n, scale, window, n_head, n_kv_head, hd, page_size, n_splits, chunk, waves,
-                                                 rows_are_requests, partials, leave_splits, num_pages, stream, softcap, bias_table, max_dist, sinks, keep_first);
+                                                 rows_are_requests, partials, leave_splits, num_pages, reach, stream, softcap, bias_table, max_dist, sinks, keep_first);
 }
 
 // out[m, h * hd + e] = the splits of (m, h) merged in split order: for splits that

@@ -53,7 +53,8 @@ int liyab_attention_generic(void* out, int64_t out_stride, const void* q, int64_
 int liyab_attention_decode(void* out, int64_t out_stride, const void* q, int64_t q_stride, const void* kc, const void* vc, int dtype,
                            const int* block_tables, int max_blocks, const int* tok_list, const int* tok_seq, const int* tok_pos, int n,
                            float scale, int window, int n_head, int n_kv_head, int hd, int page_size, int n_splits, int chunk,
-                           int waves, int rows_are_requests, float* partials, int leave_splits, int num_pages, hipStream_t stream);
+                           int waves, int rows_are_requests, float* partials, int leave_splits, int num_pages, int reach,
+                           hipStream_t stream);
 int liyab_attention_merge(void* out, int out_dtype, int64_t out_stride, const float* partials, int n, int n_head, int hd, int n_splits,
                           hipStream_t stream);
 int liyab_attention_prefill(void* out, int64_t out_stride, const void* q, int64_t q_stride, const void* kc, const void* vc,
@@ -87,7 +88,7 @@ int liyab_moe_align(const int* ids, int n_entries, int n_experts, int block, int
 int liyab_attention_decode_scored(void* out, int64_t out_stride, const void* q, int64_t q_stride, const void* kc, const void* vc, int dtype,
                                   const int* block_tables, int max_blocks, const int* tok_list, const int* tok_seq, const int* tok_pos, int n,
                                   float scale, int window, int n_head, int n_kv_head, int hd, int page_size, int n_splits, int chunk,
-                                  int waves, int rows_are_requests, float* partials, int leave_splits, int num_pages, float softcap,
+                                  int waves, int rows_are_requests, float* partials, int leave_splits, int num_pages, int reach, float softcap,
                                   const float* bias_table, int max_dist, const float* sinks, int keep_first, hipStream_t stream);
 int liyab_attention_prefill_scored(void* out, int64_t out_stride, const void* q, int64_t q_stride, const void* kc, const void* vc,
                                    const int* block_tables, int max_blocks, const int* work, int n_tiles, int tile, int ksplit, float scale,

@@ -63,7 +63,7 @@ _SIGNATURES = {
     "liyab_attention_generic": [P, c_int64, P, c_int64, P, P, c_int, P, c_int, P, P, c_int, c_float, c_int, c_int,
                                 c_int, c_int, c_int, c_int, P],
     "liyab_attention_decode": [P, c_int64, P, c_int64, P, P, c_int, P, c_int, P, P, P, c_int, c_float, c_int, c_int, c_int,
-                               c_int, c_int, c_int, c_int, c_int, c_int, P, c_int, c_int, P],
+                               c_int, c_int, c_int, c_int, c_int, c_int, P, c_int, c_int, c_int, P],
     "liyab_attention_merge": [P, c_int, c_int64, P, c_int, c_int, c_int, c_int, P],
     "liyab_gemm_att_parts": [P, c_int, c_int, c_int, P, c_int, c_int, c_int, P, c_int64, P, P, c_int, c_int64, P],
     "liyab_gemm_skinny_ln": [P, c_int, c_int64, P, P, c_float, P, c_int, c_int, c_int, c_int, _EPI_PTR, P],
@@ -85,7 +85,7 @@ _SIGNATURES = {
     "liyab_moe_align": [P, c_int, c_int, c_int, P, P, c_int, P],
     "liyab_moe_route_align": [P, c_int64, c_int, c_int, c_int, P, P, c_int, P, P, c_int, c_int, c_int, c_int, P, c_float, c_int, c_int, P],
     "liyab_attention_decode_scored": [P, c_int64, P, c_int64, P, P, c_int, P, c_int, P, P, P, c_int, c_float, c_int, c_int, c_int,
-                                      c_int, c_int, c_int, c_int, c_int, c_int, P, c_int, c_int, c_float, P, c_int, P, c_int, P],
+                                      c_int, c_int, c_int, c_int, c_int, c_int, P, c_int, c_int, c_int, c_float, P, c_int, P, c_int, P],
     "liyab_attention_prefill_scored": [P, c_int64, P, c_int64, P, P, P, c_int, P, c_int, c_int, c_int, c_float, c_int, c_int,
                                        c_int, c_int, c_int, c_int, c_float, P, c_int, P, c_int, P],
     "liyab_gate_rows": [P, c_int, c_int64, P, c_int64, c_int, c_int, c_float, P],

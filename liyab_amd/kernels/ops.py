@@ -798,7 +798,7 @@ def attention_decode(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor, 
                      tok_list: Optional[torch.Tensor] = None, n_tokens: Optional[int] = None, waves: int = 4,
                      rows_are_requests: bool = False, leave_splits: bool = False, chunk: int = 0,
                      num_pages: Optional[int] = None, softcap: float = 0.0, bias_table: Optional[torch.Tensor] = None,
-                     sinks: Optional[torch.Tensor] = None, keep_first: int = 0) -> None:
+                     sinks: Optional[torch.Tensor] = None, keep_first: int = 0, reach: int = 0) -> None:
     """Each token on its own over its request's cache (bfloat16, or float32 throughout), its keys cut into `n_splits`.
     With `tok_list` (int32) only those rows are computed. `rows_are_requests`: row t belongs to
     request t (every request brings one token), which saves the kernel a lookup. With
@@ -808,7 +808,8 @@ def attention_decode(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor, 
     token's keys instead of an equal share (`n_splits * chunk` must cover the longest context): a token's
     sums then follow from its position alone. `softcap` > 0: scores become cap * tanh(score / cap); `bias_table` (float32
     [distances, heads]): + table[min(position - key, distances - 1), head]; `sinks` (float32 [heads]): exp(sinks[head]) joins
-    the softmax's denominator (a learned logit with no key and no value); `keep_first`: with a window, positions below it stay visible."""
+    the softmax's denominator (a learned logit with no key and no value); `keep_first`: with a window, positions below it stay visible.
+    `reach`: the most keys a token has, rounded up (0: what the block table holds); the order of the grid follows from it."""
     if k_cache.dim() != 4 or k_cache.shape != v_cache.shape or not k_cache.is_contiguous() or not v_cache.is_contiguous():
         raise KernelError("attention: caches must be contiguous [pages, kv_heads, page_size, head_dim] of one shape")
     _, hkv, page, hd = k_cache.shape
@@ -837,7 +838,7 @@ def attention_decode(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor, 
     args = (out.data_ptr(), os_, q.data_ptr(), qs, k_cache.data_ptr(), v_cache.data_ptr(),
             dtype_code(q.dtype), block_tables.data_ptr(), block_tables.shape[1], _ptr(tok_list), tok_seq.data_ptr(), tok_pos.data_ptr(),
             n, float(scale), int(window), n_head, hkv, hd, page, n_splits, int(chunk), waves, 1 if rows_are_requests else 0,
-            _ptr(partials), 1 if leave_splits else 0, _pages(k_cache, num_pages))
+            _ptr(partials), 1 if leave_splits else 0, _pages(k_cache, num_pages), int(reach))
     _f32vec(sinks, "sinks", n_head)
     if softcap > 0 or bias_table is not None or sinks is not None or (keep_first > 0 and window > 0):
         if sinks is not None and leave_splits:
@@ -1035,7 +1036,7 @@ def attention(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor, v_cache
         partials = ctx.workspace.get("attn_partials", (n * n_head * splits * (hd + 4),), torch.float32) if splits > 1 else None
         attention_decode(out, q, k_cache, v_cache, block_tables, ctx.tok_seq, ctx.positions, n_head=n_head, scale=scale,
                          window=window, n_splits=splits, partials=partials, waves=4, chunk=chunk,
-                         rows_are_requests=host.max_q_len == 1, **scored)
+                         rows_are_requests=host.max_q_len == 1, reach=plan.context_bucket, **scored)
         return None
     if fast and plan.mode == "decode" and block_tables.shape[1] <= 2048:
         n = out.shape[0]

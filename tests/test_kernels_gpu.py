@@ -544,15 +544,15 @@ def test_attention_order_of_the_grid(ops, dtype):
     case = paged_case(2, [300, 33], [40, 33], H, H, hd, page, dtype, seed=3)
     bt = case["bt"]
     outs = []
-    for columns in (102, 103):
+    for columns, reach in ((102, 0), (103, 0), (103, 512)):
         columns = columns * 4 // dtype.itemsize  # 4,177,920 bytes of keys and values, 4,218,880
         case["bt"] = torch.cat([bt, bt.new_zeros(bt.shape[0], columns - bt.shape[1])], dim=1)
         dev = [case[k].to(DEV) for k in ("q", "kc", "vc", "bt")] + [torch.tensor(case[k], dtype=torch.int32, device=DEV) for k in ("tok_seq", "tok_pos")]
         out = torch.zeros(case["n"], H * hd, dtype=dtype, device=DEV)
-        ops.attention_decode(out, dev[0][:, :H * hd], *dev[1:], n_head=H, scale=scale, n_splits=1, waves=4, chunk=256)
+        ops.attention_decode(out, dev[0][:, :H * hd], *dev[1:], n_head=H, scale=scale, n_splits=1, waves=4, chunk=256, reach=reach)
         outs.append(out)
     close(outs[0], attention_reference(case, H, H, hd, scale), 8e-3 if dtype == torch.bfloat16 else 2e-6, "grid order")
-    assert torch.equal(outs[0], outs[1])
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
     case = paged_case(17, list(range(20, 20 + 17 * 9, 9)), [1] * 17, H, H, hd, page, dtype, seed=4)
     dev = [case[k].to(DEV) for k in ("q", "kc", "vc", "bt")] + [torch.tensor(case[k], dtype=torch.int32, device=DEV) for k in ("tok_seq", "tok_pos")]
     for splits in (1, 3):
