@@ -192,15 +192,15 @@ def gemm_reference(a, w, bias, epilogue, residual=None):
 GEMM_SHAPES = [(1, 64, 64), (7, 200, 96), (33, 777, 144), (130, 50, 320), (64, 1000, 96), (257, 130, 72)]
 
 
-# beside those: each width of the row-wise kernel (4, 8 and 16 features a workgroup), chunks of K
-# with a tail, more chunks than waves, a K that is no multiple of 4 (the one-thread-an-element form)
+# beside those: strips of 16 rows by 4, 8 and 16 features, chunks of K with a tail, more chunks than waves, a K that is no multiple
+# of 4 (element by element), products of many features
 F32_SHAPES = GEMM_SHAPES + [(16, 1500, 100), (9, 2600, 260), (5, 3000, 72), (12, 40, 6), (40, 2561, 132), (3, 1024, 1028),
                             (16, 33, 3076), (20, 70, 50),
-                            # 17 to 64 rows in one workgroup: 16 features a workgroup with 2, 3 and 4 rows a thread,
-                            # 8 with 1 and 2, 4 with a long K
+                            # two to four strips of rows: 16 features a strip on four and eight waves, 4 and 8 with a long K
                             (24, 4100, 200), (45, 4097, 68), (64, 4800, 324), (30, 2050, 1604), (17, 100, 3076),
-                            # large enough for the tiles of 128 x 128 (528 of them), with edges on both sides and a K that ends inside a step of 16
-                            (1100, 7300, 68)]
+                            # tiles of 64 x 64 (from 136 of them on): many of them with edges on both sides; a long K; just 136; a K that
+                            # is no multiple of 4
+                            (1100, 7300, 68), (700, 770, 3072), (65, 4352, 1604), (300, 2304, 770)]
 
 
 @pytest.mark.parametrize("epilogue", ["none", "gelu_tanh", "gelu_erf", "residual"])
@@ -223,11 +223,14 @@ def test_gemm_float32(ops, M, N, K, epilogue):
         full = torch.empty(M, N, device=DEV)
         ops.gemm(a, w, bias, out=full)
         assert torch.equal(one[0], full[M // 2])
-        many = torch.empty(70 + M, N, device=DEV)  # among 70 rows more: the tiled kernel, or the row-wise one again
+        few = torch.empty(min(M, 40), N, device=DEV)  # strips, also of shapes that run in tiles
+        ops.gemm(a[M - len(few):], w, bias, out=few)
+        assert torch.equal(few, full[M - len(few):])
+        many = torch.empty(70 + M, N, device=DEV)  # among 70 rows more: other strips, other tiles, or tiles instead of strips
         rows = torch.cat([rnd(70, K, seed=9), a])
         ops.gemm(rows, w, bias, out=many)
         assert torch.equal(many[70:], full)
-        # from an address that is no multiple of 16 bytes the tiled kernel takes more than 64 rows, however few its tiles
+        # from an address that is no multiple of 16 bytes operands are loaded element by element
         shifted = torch.empty(rows.numel() + 1, device=DEV)[1:].view_as(rows).copy_(rows)
         assert shifted.data_ptr() % 16 != 0
         ops.gemm(shifted, w, bias, out=many)
@@ -257,6 +260,33 @@ def test_gemm_float32_at_the_edges_of_its_kernels(ops, M, N, K):
     one = torch.empty(1, N, device=DEV)  # a row alone: the kernel for few rows, in strips of its own
     ops.gemm_simple(a[M - 1:], w, bias, out=one)
     assert torch.equal(one[0], out[M - 1])
+
+
+@pytest.mark.parametrize("K", [64, 130, 768])
+@pytest.mark.parametrize("M,N", [(20, 70), (700, 770)])
+def test_gemm_float32_is_chains_of_fused_multiply_adds(ops, M, N, K):
+    """Every result has the bits of the chains it stands for, 64 k from zero each, the chunks' sums added in order, computed on the
+    host with the C library's fmaf: for ordinary operands, for products below the normal numbers and for operands below them; in
+    strips (20 x 70) and in tiles (143 of them)."""
+    import ctypes
+
+    fmaf = ctypes.CDLL("libm.so.6").fmaf
+    fmaf.restype, fmaf.argtypes = ctypes.c_float, [ctypes.c_float] * 3
+    rng = np.random.default_rng(K + M)
+    places = [(0, 0), (M - 1, N - 1)] + [(int(rng.integers(M)), int(rng.integers(N))) for _ in range(60)]
+    for scale_a, scale_w in ((1.0, 1.0), (1e-20, 1e-20), (1e-40, 1.0)):
+        a, w = (rng.standard_normal((M, K)) * scale_a).astype(np.float32), (rng.standard_normal((N, K)) * scale_w).astype(np.float32)
+        out = torch.empty(M, N, device=DEV)
+        ops.gemm_simple(torch.from_numpy(a).to(DEV), torch.from_numpy(w).to(DEV), None, out=out)
+        got = out.cpu().numpy()
+        for m, n in places:
+            total = np.float32(0.0)
+            for k0 in range(0, K, 64):
+                chain = 0.0
+                for x, y in zip(a[m, k0:k0 + 64].tolist(), w[n, k0:k0 + 64].tolist()):
+                    chain = fmaf(x, y, chain)
+                total = np.float32(total + np.float32(chain))
+            assert got[m, n].tobytes() == total.tobytes(), (scale_a, scale_w, m, n, got[m, n], total)
 
 
 @pytest.mark.parametrize("kernel", ["simple", "mfma128", "mfma64", "mfma128x64", "auto", "skinny1", "skinny4", "skinny16", "skinny4w", "skinny2w", "skinny8m1", "skinny4m2", "skinny2m4",
@@ -737,7 +767,7 @@ def test_a_page_id_past_the_counted_pages_is_not_followed(ops, kernel, dtype):
         run(counted + 9)
 
 
-@pytest.mark.parametrize("kernel", ["kv_write", "skinny", "dl", "mfma", "folded norm"])
+@pytest.mark.parametrize("kernel", ["kv_write", "skinny", "dl", "dl6", "dl7", "dl9", "dl11", "dl15", "mfma", "folded norm"])
 def test_a_slot_past_the_counted_pages_is_not_written(ops, kernel):
     """Slots in the eight pages the launcher is not told of (and a -1) are skipped; told of all
     pages, the same call writes them."""
@@ -761,8 +791,8 @@ def test_a_slot_past_the_counted_pages_is_not_written(ops, kernel):
             ops.kv_write(kc, vc, full, q_dim, q_dim + kv_dim, slots, num_pages=num_pages)
         elif kernel == "skinny":
             ops.gemm_skinny(a, w, bias, **kw)
-        elif kernel == "dl":
-            ops.gemm_mfma_dl(a, w, bias, tile=2, **kw)
+        elif kernel.startswith("dl"):
+            ops.gemm_mfma_dl(a, w, bias, tile=int(kernel[2:] or 2), **kw)
         elif kernel == "mfma":
             ops.gemm_mfma(a, w, bias, tile=2, **kw)
         else:
@@ -993,9 +1023,27 @@ def test_tiles_of_every_shape_give_a_row_the_same_bits(ops, K):
             assert torch.equal(out, full[108][rows]), f"rows {rows} in tiles {tile}"
 
 
-@pytest.mark.parametrize("kernel", ["skinny", "mfma128", "mfma64", "dl2", "dl8", "dl15", "dl16", "auto"])
+@pytest.mark.parametrize("K", [64, 768, 3072])
+def test_tiles_of_one_sum_give_a_row_the_same_bits(ops, K):
+    """The tiles of many rows take K in one chain of the same steps whatever their shape: the same bits from each, inside the
+    output and at its edges, in 32 bits and in bfloat16."""
+    M, N = 300, 520
+    a, w, bias = rnd(M, K, dtype=torch.bfloat16, seed=K), rnd(N, K, dtype=torch.bfloat16, seed=K + 1, scale=0.2), rnd(N, seed=2)
+    want = gemm_reference(a.float(), w.float(), bias, "none")
+    for dtype, tol in ((torch.float32, 2e-5), (torch.bfloat16, 8e-3)):
+        first = None
+        for tile in (2, 6, 7, 8, 9, 11, 15):
+            out = torch.full((M, N), float("nan"), dtype=dtype, device=DEV)
+            ops.gemm_mfma_dl(a, w, bias, out=out, tile=tile)
+            close(out, want, tol, f"tile {tile}")
+            first = out if first is None else first
+            assert torch.equal(out, first), f"tile {tile} against 2"
+
+
+@pytest.mark.parametrize("kernel", ["skinny", "mfma128", "mfma64", "dl2", "dl6", "dl7", "dl8", "dl9", "dl11", "dl15", "dl16", "dl17", "auto"])
 @pytest.mark.parametrize("M,H,Hkv,hd,K,page", [(5, 3, 3, 16, 64, 4), (40, 4, 2, 32, 128, 16), (200, 5, 5, 48, 192, 8), (130, 2, 1, 64, 64, 64), (700, 6, 3, 64, 128, 16),
-                                               (50, 3, 3, 32, 128, 24), (300, 4, 2, 64, 192, 48)])
+                                               (50, 3, 3, 32, 128, 24), (300, 4, 2, 64, 192, 48),
+                                               (780, 16, 16, 64, 1024, 16)])  # (the size at which `auto` takes tiles of 128 x 128)
 def test_gemm_paged_qkv_epilogue(ops, kernel, M, H, Hkv, hd, K, page):
     """Queries to a dense buffer, keys and values straight into shuffled cache slots, against
     the plain product followed by the scatter kernel."""
@@ -1165,3 +1213,34 @@ def test_float32_qkv_product_into_the_pages(ops, M, H, Hkv, hd, K, page):
     q = torch.full((M, q_dim), float("nan"), device=DEV)
     ops.gemm_f32_qkv(a, w, bias, out=q, kv=(*got, slots, q_dim))
     assert torch.equal(q, full[:, :q_dim]) and torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+
+
+@pytest.mark.parametrize("d", [64, 768, 1300])
+@pytest.mark.parametrize("also", ["nothing", "gate"])
+def test_rows_update_by_waves_keeps_the_rows(ops, d, also):
+    """The rows kept as a convolution's history before the update, by the kernel of a wave a row (two rows of y a token) and by the
+    one of a workgroup a row (four, two of them zeros): the last `ring` rows of each request, of no request without a slot, and
+    none of the rows behind the step's tokens."""
+    from types import SimpleNamespace
+
+    lens, contexts, slots, ring, n_slots, n = [1, 5, 2, 4], [9, 5, 40, 30], [2, 0, -1, 7], 3, 5, 15
+    real = sum(lens)
+    tok_seq = [r for r, q in enumerate(lens) for _ in range(q)] + [0] * (n - real)
+    positions = [contexts[r] - q + i for r, q in enumerate(lens) for i in range(q)] + [8] * (n - real)
+    dev = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)  # noqa: E731
+    ctx = SimpleNamespace(n_tokens=n, n_seqs=len(lens), tok_seq=dev(tok_seq), positions=dev(positions), context_lens=dev(contexts), state_slots=dev(slots),
+                          seq_starts=dev([0, 1, 6, 8, 12]))
+    x, y, w = rnd(n, d), rnd(n, 2, d, seed=1), rnd(d, seed=2) + 1.0
+    gate = rnd(n, d, seed=3) if also == "gate" else None
+    want = torch.full((n_slots, ring, d), 7.0, device=DEV)
+    for t in range(real):
+        r = tok_seq[t]
+        if positions[t] >= contexts[r] - ring and 0 <= slots[r] < n_slots:
+            want[slots[r], positions[t] % ring] = x[t]
+    got = []
+    for rows in (y, torch.cat([y, torch.zeros_like(y)], dim=1)):
+        into, state = x.clone(), torch.full((n_slots, ring, d), 7.0, device=DEV)
+        ops.gated_norm_add(into, rows.reshape(-1, d), w, 1e-5, n_sum=rows.shape[1], gate=gate, keep=(state, ctx))
+        assert torch.equal(state, want)
+        got.append(into)
+    assert torch.equal(got[0], got[1])
