@@ -273,7 +273,7 @@ int launch_dl(const void* a, int64_t lda, const void* w, int M, int N, int K, co
         case kEpiGeluTanh: return launch_dl_as<BM, BN, DSTAGES, bf16_t, kEpiGeluTanh, WM, WN, WK, SETS>(pa, lda, pw, M, N, K, epi, stream);
         case kEpiGeluErf: return launch_dl_as<BM, BN, DSTAGES, bf16_t, kEpiGeluErf, WM, WN, WK, SETS>(pa, lda, pw, M, N, K, epi, stream);
         case kEpiQkvPaged: return launch_dl_as<BM, BN, DSTAGES, bf16_t, kEpiQkvPaged, WM, WN, WK, SETS>(pa, lda, pw, M, N, K, epi, stream);
-        default: return launch_dl_as<BM, BN, DSTAGES, bf16_t, -1, WM, WN, WK, SETS>(pa, lda, pw, M, N, K, epi, stream);
+        default: return fail(1, "gemm: unknown epilogue %d", epi.mode);
     }
 }
 

@@ -153,7 +153,7 @@ int launch_tile_epi(const bf16_t* a, int64_t lda, const bf16_t* w, int M, int N,
         case kEpiGeluTanh: return LIYAB_TILE(bf16_t, kEpiGeluTanh);
         case kEpiGeluErf: return LIYAB_TILE(bf16_t, kEpiGeluErf);
         case kEpiQkvPaged: return LIYAB_TILE(bf16_t, kEpiQkvPaged);
-        default: return LIYAB_TILE(bf16_t, -1);
+        default: return fail(1, "gemm: unknown epilogue %d", epi.mode);
     }
 #undef LIYAB_TILE
 }

@@ -1,7 +1,7 @@
-// out[M,N] = a[M,K] . w[N,K]^T (+ bias) with an epilogue: the plain tiled
-// product. It is the product of the true 32-bit path (32-bit operands, FMA
-// accumulation in 32 bits) and the fallback for bfloat16 shapes the MFMA
-// kernels refuse.
+// out[M,N] = a[M,K] . w[N,K]^T (+ bias) with an epilogue, for 32-bit operands
+// on the matrix cores (fused multiply-adds in 32 bits: strips of 16 rows and
+// tiles of 64 x 64) and for the bfloat16 shapes that the bfloat16 matrix-core
+// kernels refuse, multiplied on the vector units.
 //
 // Both operands are contiguous along K (a row of `w` is one output feature,
 // as the reference lays matrices out: include/liyab/types.h:165-184,
@@ -25,9 +25,10 @@ constexpr int BM = 64, BN = 64, BK = 16;
 constexpr int kChunk = 64;  // k of one chain of multiply-adds
 static_assert(kChunk % BK == 0, "a chunk is whole tiles");
 
-template <typename T, typename OutT, int EPI, bool EXACT>
+// bfloat16 operands of any size and alignment.
+template <typename OutT, int EPI>
 __global__ void __launch_bounds__(256)
-gemm_simple_kernel(OutT* __restrict__ out, int64_t ldo, const T* __restrict__ a, int64_t lda, const T* __restrict__ w,
+gemm_simple_kernel(OutT* __restrict__ out, int64_t ldo, const bf16_t* __restrict__ a, int64_t lda, const bf16_t* __restrict__ w,
                    const float* __restrict__ bias, float* __restrict__ residual, int64_t ldr, int M, int N, int K) {
     __shared__ float As[BK][BM + 4];
     __shared__ float Ws[BK][BN + 4];
@@ -39,13 +40,13 @@ gemm_simple_kernel(OutT* __restrict__ out, int64_t ldo, const T* __restrict__ a,
     for (int k0 = 0; k0 < K; k0 += BK) {
         {
             const int m = m0 + lrow;
-            const T* p = a + static_cast<int64_t>(m) * lda + k0 + lk;
+            const bf16_t* p = a + static_cast<int64_t>(m) * lda + k0 + lk;
 #pragma unroll
-            for (int i = 0; i < 4; ++i) As[lk + i][lrow] = (m < M && k0 + lk + i < K) ? to_float<T>(p[i]) : 0.0f;
+            for (int i = 0; i < 4; ++i) As[lk + i][lrow] = (m < M && k0 + lk + i < K) ? to_float<bf16_t>(p[i]) : 0.0f;
             const int n = n0 + lrow;
-            const T* q = w + static_cast<int64_t>(n) * K + k0 + lk;
+            const bf16_t* q = w + static_cast<int64_t>(n) * K + k0 + lk;
 #pragma unroll
-            for (int i = 0; i < 4; ++i) Ws[lk + i][lrow] = (n < N && k0 + lk + i < K) ? to_float<T>(q[i]) : 0.0f;
+            for (int i = 0; i < 4; ++i) Ws[lk + i][lrow] = (n < N && k0 + lk + i < K) ? to_float<bf16_t>(q[i]) : 0.0f;
         }
         __syncthreads();
 #pragma unroll
@@ -82,7 +83,7 @@ gemm_simple_kernel(OutT* __restrict__ out, int64_t ldo, const T* __restrict__ a,
             float v = tot[i][j];
             if (bias != nullptr) v += bias[n];
             if constexpr (EPI == kEpiGeluTanh) v = gelu_tanh(v);
-            if constexpr (EPI == kEpiGeluErf) v = EXACT ? gelu_erf_exact(v) : gelu_erf_fast(v);
+            if constexpr (EPI == kEpiGeluErf) v = gelu_erf_fast(v);
             if constexpr (EPI == kEpiResidual) {
                 residual[static_cast<int64_t>(m) * ldr + n] += v;
             } else {
@@ -104,12 +105,12 @@ typedef __attribute__((ext_vector_type(4))) float f32x4_t;
 typedef __attribute__((ext_vector_type(2))) float f32x2_t;
 typedef __attribute__((ext_vector_type(16))) float f32x16_t;
 
-// What follows the sum, as in the kernel above.
-template <int EPI, bool EXACT>
+// What follows the sum (the error function in double precision).
+template <int EPI>
 __device__ __forceinline__ float finish_f32(float v, bool has_bias, float bias) {
     if (has_bias) v += bias;
     if constexpr (EPI == kEpiGeluTanh) v = gelu_tanh(v);
-    if constexpr (EPI == kEpiGeluErf) v = EXACT ? gelu_erf_exact(v) : gelu_erf_fast(v);
+    if constexpr (EPI == kEpiGeluErf) v = gelu_erf_exact(v);
     return v;
 }
 
@@ -154,7 +155,7 @@ __device__ __forceinline__ float* qkv_place(const EpiParams& p, int m, int n) {
 // stage's other work strung between its products by hand.
 constexpr int kTile = 64;
 
-template <int EPI, bool EXACT, bool VEC>
+template <int EPI, bool VEC>
 __global__ void __launch_bounds__(256)
 gemm_tiled_f32_kernel(float* __restrict__ out, int64_t ldo, const float* __restrict__ a, int64_t lda, const float* __restrict__ w,
                       const float* __restrict__ bias, float* __restrict__ residual, int64_t ldr, int M, int N, int K, int vec_out, EpiParams qkv) {
@@ -242,7 +243,7 @@ gemm_tiled_f32_kernel(float* __restrict__ out, int64_t ldo, const float* __restr
 #pragma unroll
     for (int q = 0; q < 4; ++q)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[q][e] = finish_f32<EPI, EXACT>(tot[4 * q + e], bias != nullptr, v[q][e]);
+        for (int e = 0; e < 4; ++e) v[q][e] = finish_f32<EPI>(tot[4 * q + e], bias != nullptr, v[q][e]);
     if (m >= M) return;
     if constexpr (EPI == kEpiQkvPaged) {
 #pragma unroll
@@ -295,7 +296,7 @@ gemm_tiled_f32_kernel(float* __restrict__ out, int64_t ldo, const float* __restr
 // pace when lanes ran the chains themselves (20 to 80 reads of 16 bytes a chunk; here 32 of 4).
 constexpr int kChunkRows = 16;  // rows a workgroup
 
-template <int NB, int WAVES, int EPI, bool EXACT, bool VEC>
+template <int NB, int WAVES, int EPI, bool VEC>
 __global__ void __launch_bounds__(64 * WAVES)
 gemm_chunks_f32_kernel(float* __restrict__ out, int64_t ldo, const float* __restrict__ a, int64_t lda,
                        const float* __restrict__ w, const float* __restrict__ bias, float* __restrict__ residual,
@@ -354,7 +355,7 @@ gemm_chunks_f32_kernel(float* __restrict__ out, int64_t ldo, const float* __rest
     const int n = n0 + tid % NB;
     if (tid >= kChunkRows * NB || tid / NB >= M || n >= N) return;
     const int m = row0 + tid / NB;
-    const float v = finish_f32<EPI, EXACT>(tot, bias != nullptr, bias != nullptr ? bias[n] : 0.0f);
+    const float v = finish_f32<EPI>(tot, bias != nullptr, bias != nullptr ? bias[n] : 0.0f);
     if constexpr (EPI == kEpiResidual) residual[static_cast<int64_t>(m) * ldr + n] += v;
     else if constexpr (EPI == kEpiQkvPaged) { if (place != nullptr) *place = v; }
     else out[static_cast<int64_t>(m) * ldo + n] = v;
@@ -368,14 +369,14 @@ constexpr int kFewRows = 64;  // steps of at most this many rows never take the 
 template <int EPI, bool VEC>
 int launch_tiled_f32(float* out, int64_t ldo, const float* a, int64_t lda, const float* w, const float* bias, float* residual, int64_t ldr, int M,
                      int N, int K, bool vec_out, const EpiParams& qkv, hipStream_t stream) {
-    gemm_tiled_f32_kernel<EPI, true, VEC><<<((N + kTile - 1) / kTile) * ((M + kTile - 1) / kTile), 256, 0, stream>>>(out, ldo, a, lda, w, bias, residual, ldr, M, N, K, vec_out, qkv);
+    gemm_tiled_f32_kernel<EPI, VEC><<<((N + kTile - 1) / kTile) * ((M + kTile - 1) / kTile), 256, 0, stream>>>(out, ldo, a, lda, w, bias, residual, ldr, M, N, K, vec_out, qkv);
     return check_launch("gemm_tiled_f32");
 }
 
 template <int NB, int WAVES, int EPI, bool VEC>
 int launch_chunks_f32(float* out, int64_t ldo, const float* a, int64_t lda, const float* w, const float* bias, float* residual, int64_t ldr, int M,
                       int N, int K, const EpiParams& qkv, hipStream_t stream) {
-    gemm_chunks_f32_kernel<NB, WAVES, EPI, true, VEC><<<dim3((N + NB - 1) / NB, (M + kChunkRows - 1) / kChunkRows), 64 * WAVES, 0, stream>>>(
+    gemm_chunks_f32_kernel<NB, WAVES, EPI, VEC><<<dim3((N + NB - 1) / NB, (M + kChunkRows - 1) / kChunkRows), 64 * WAVES, 0, stream>>>(
         out, ldo, a, lda, w, bias, residual, ldr, M, N, K, qkv);
     return check_launch("gemm_chunks_f32");
 }
@@ -407,15 +408,15 @@ int launch_f32(float* out, int64_t ldo, const float* a, int64_t lda, const float
     return launch_f32_epi<EPI, false>(out, ldo, a, lda, w, bias, residual, ldr, M, N, K, qkv, stream);
 }
 
-template <typename T, typename OutT, bool EXACT>
+template <typename OutT>
 int launch_simple(void* out, int64_t ldo, const void* a, int64_t lda, const void* w, const float* bias,
                   float* residual, int64_t ldr, int M, int N, int K, int epi, hipStream_t stream) {
     dim3 grid((N + BN - 1) / BN, (M + BM - 1) / BM);
     auto* o = static_cast<OutT*>(out);
-    auto* pa = static_cast<const T*>(a);
-    auto* pw = static_cast<const T*>(w);
+    auto* pa = static_cast<const bf16_t*>(a);
+    auto* pw = static_cast<const bf16_t*>(w);
 #define LIYAB_GO(E) \
-    gemm_simple_kernel<T, OutT, E, EXACT><<<grid, 256, 0, stream>>>(o, ldo, pa, lda, pw, bias, residual, ldr, M, N, K)
+    gemm_simple_kernel<OutT, E><<<grid, 256, 0, stream>>>(o, ldo, pa, lda, pw, bias, residual, ldr, M, N, K)
     switch (epi) {
         case kEpiNone: LIYAB_GO(kEpiNone); break;
         case kEpiGeluTanh: LIYAB_GO(kEpiGeluTanh); break;
@@ -458,8 +459,8 @@ extern "C" int liyab_gemm_simple(void* out, int out_dtype, int64_t ldo, const vo
         }
     }
     if (dtype == kBF16) {
-        if (out_dtype == kF32) return launch_simple<bf16_t, float, false>(out, ldo, a, lda, w, bias, residual, ldr, M, N, K, epi, stream);
-        if (out_dtype == kBF16) return launch_simple<bf16_t, bf16_t, false>(out, ldo, a, lda, w, bias, residual, ldr, M, N, K, epi, stream);
+        if (out_dtype == kF32) return launch_simple<float>(out, ldo, a, lda, w, bias, residual, ldr, M, N, K, epi, stream);
+        if (out_dtype == kBF16) return launch_simple<bf16_t>(out, ldo, a, lda, w, bias, residual, ldr, M, N, K, epi, stream);
         return fail(1, "gemm: unknown output dtype %d", out_dtype);
     }
     return fail(1, "gemm: unknown dtype %d", dtype);

@@ -90,7 +90,7 @@ __device__ __forceinline__ void store_tile(Sums (&acc)[TM][TN], bf16_t* lds, con
     // operands that are not aligned for it go element by element.
     const bool inside = m0 + BM <= M && n0 + BN <= N, columns_inside = n0 + BN <= N;
     if constexpr (sizeof(OutT) == 2 && EPI >= 0 && EPI != kEpiResidual) {
-        // bfloat16 outputs of interior tiles go through LDS once more, so that they leave as whole
+        // bfloat16 outputs go through LDS once more (at the edges too), so that they leave as whole
         // rows: a wave lays its (BM / WM) x (BN / WN) results out row by row (bias and activation
         // applied), then every lane stores 16 bytes and eight lanes a row of 64 columns: full
         // cache lines, where the accumulators' own layout would write 16 bytes of 32 different

@@ -709,8 +709,8 @@ def skinny_ln_pays(M: int, N: int, K: int) -> bool:
 
 def gemm_mfma_dl(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], *, out=None, residual=None,
                  epilogue: int = EPI_NONE, kv=None, tile: int = 0) -> None:
-    """The matrix-core product with tiles loaded straight into LDS, three stages deep; bfloat16
-    operands, K a multiple of 64."""
+    """The matrix-core product with tiles loaded straight into LDS, two to four stages deep by the tile;
+    bfloat16 operands, K a multiple of 64. tile: csrc/gemm_mfma_dl.hip lists them (0: chosen from the sizes)."""
     lda = _rows(a, "a")
     M, K = a.shape
     _dev(w, "w")
@@ -729,8 +729,8 @@ def mfma_takes(a: torch.Tensor, w: torch.Tensor) -> bool:
 
 def gemm(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], *, out: Optional[torch.Tensor] = None,
          residual: Optional[torch.Tensor] = None, epilogue: int = EPI_NONE, kv=None) -> None:
-    """The product kernel for these operands: matrix cores for bfloat16 shapes they take,
-    the plain tiled kernel for float32 and everything else. `kv` = (k_cache, v_cache, slots,
+    """The product kernel for these operands: the bfloat16 matrix-core kernels for shapes they take, else `gemm_simple`'s (float32 on
+    the matrix cores in 32 bits, other bfloat16 shapes on the vector units). `kv` = (k_cache, v_cache, slots,
     q_dim[, num_pages]) with the paged QKV epilogue (a slot outside the caches' pages is not written)."""
     if _invariant and mfma_takes(a, w):
         # one family of kernels whatever the number of rows: their sum over k has one order for
