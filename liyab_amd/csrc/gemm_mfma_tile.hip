@@ -11,11 +11,12 @@
 // first fragments, the outputs) overlaps with another workgroup's products: two workgroups of eight waves a compute unit for
 // the middle tiles, sixteen waves in one for 256 x 256.
 // Measured in prefill steps, us a product, before (32 x 32 x 16 in tiles of 64 x 64, 128 x 128 or 256 x 256, a stage's loads at
-// once) and now: GPT-2 XL's widths, 7,920 rows: 1,600 -> 4,800 164 -> 122, 1,600 -> 6,400 204 -> 157, the two products back
-// to the stream 149 -> 114; 768 wide, 8,001 rows: 768 -> 2,304 51 -> 41, 768 -> 3,072 60 -> 48, the two back 45 -> 34; 2,048
-// rows: 18.4 -> 16.6, 20.2 -> 20.5 and 18.0 -> 16.9; 1,024 wide, some 780 rows: 1,024 -> 3,072 15.7 -> 14.8, -> 4,096 22.0 -> 15.4.
+// once) and now, on one box in turn: GPT-2 XL's widths, 7,920 rows: 1,600 -> 4,800 159 -> 126, 1,600 -> 6,400 197 -> 161, the two products
+// back to the stream 142 -> 120 on average; 768 wide, 8,001 rows: 768 -> 2,304 48 -> 40, 768 -> 3,072 58 -> 48, the two back 44 -> 33; 2,048
+// rows: 18.5 -> 16.5, 20.2 -> 20.2 and 18.0 -> 16.4; 1,024 wide, some 780 rows: 1,024 -> 3,072 15.6 -> 15.0, -> 4,096 21.9 -> 15.3.
 // (There the operands come from memory, not from L2: three and four stages, which lose in a product repeated alone, win while
-// every tile has a compute unit of its own.) A product of 8,192 cubed runs at 1.2 PFLOP/s, the vendor's library at 1.4.
+// every tile has a compute unit of its own.) Alone and repeated, 8,192 cubed runs at 1.32 PFLOP/s (1.19 before, the vendor's library 1.44),
+// 4,096 x 4,096 x 16,384 at 1.28 (1.15).
 // Tried and left: four waves of 128 x 128, eight of 128 x 64, two groups of waves in turn at products and reads (each with
 // 32 x 32 blocks: 173-200 us for 6,400 -> 1,600 alone, 160 here), stages of 32 k four deep (190), fragments read a step ahead in
 // registers of their own or strung between the products by hand (slower than the compiler's order); 128 x 192, 128 x 64, 64 x 128.
