@@ -11,9 +11,9 @@
 // first fragments, the outputs) overlaps with another workgroup's products: two workgroups of eight waves a compute unit for
 // the middle tiles, sixteen waves in one for 256 x 256.
 // Measured in prefill steps, us a product, before (32 x 32 x 16 in tiles of 64 x 64, 128 x 128 or 256 x 256, a stage's loads at
-// once) and now, on one box in turn: GPT-2 XL's widths, 7,920 rows: 1,600 -> 4,800 159 -> 126, 1,600 -> 6,400 197 -> 161, the two products
-// back to the stream 142 -> 120 on average; 768 wide, 8,001 rows: 768 -> 2,304 48 -> 40, 768 -> 3,072 58 -> 48, the two back 44 -> 33; 2,048
-// rows: 18.5 -> 16.5, 20.2 -> 20.2 and 18.0 -> 16.4; 1,024 wide, some 780 rows: 1,024 -> 3,072 15.6 -> 15.0, -> 4,096 21.9 -> 15.3.
+// once) and now, on one box in turn: GPT-2 XL's widths, 7,920 rows: 1,600 -> 4,800 158 -> 126, 1,600 -> 6,400 198 -> 164, the two products
+// back to the stream 138 -> 115 on average; 768 wide, 8,001 rows: 768 -> 2,304 48 -> 40, 768 -> 3,072 58 -> 49, the two back 44 -> 33; 2,048
+// rows: 18.6 -> 16.3, 20.3 -> 20.1 and 18.0 -> 16.3; 1,024 wide, some 780 rows: 1,024 -> 3,072 15.5 -> 14.8, -> 4,096 21.7 -> 15.3.
 // (There the operands come from memory, not from L2: three and four stages, which lose in a product repeated alone, win while
 // every tile has a compute unit of its own.) Alone and repeated, 8,192 cubed runs at 1.32 PFLOP/s (1.19 before, the vendor's library 1.44),
 // 4,096 x 4,096 x 16,384 at 1.28 (1.15).
