@@ -13,10 +13,18 @@
 // splits) and four waves, which lane adds which key and which sums are merged
 // follow from the token's position alone, as the reference cuts (:2136-2139):
 // the form of the 32-bit path and of the batch-invariant mode.
+// What bounds it: with many pairs the caches' reads (64 tokens of 25 heads over 256 to 1,015 keys, 261 MB: 54.2 -> 51.2 us, where reading
+// the same bytes and doing nothing takes 45.5), so a workgroup of four waves asks for its next trip's keys and values before it
+// absorbs the ones it has; eight and sixteen waves hold as much in flight by their number (24 tokens of 12 heads on eight: 12.7
+// either way, 13.1 with the next trip's loads in flight, whose registers cost a workgroup a compute unit). With few pairs the
+// instructions around the loads: only a split's last trip looks at which keys it has, and the other trips and both forms' loads
+// are free of branches (32 tokens of 16 heads over 100 to 900 keys 20.6 -> 16.7 us, 17 of 12 heads 13.6 -> 10.4, one token in 8 splits 4.7 -> 4.4).
 // The reference cuts a token's keys by its position only (:2136-2139,
 // 2225-2227) to keep bits equal; here the number of splits follows the batch
 // (more splits when few tokens are in flight), which moves results by
 // rounding only. Scores, exponentials and sums are 32-bit.
+#include <type_traits>
+
 #include "common.h"
 #include "launchers.h"
 
@@ -93,10 +101,16 @@ attention_decode_kernel(T* __restrict__ out, int64_t out_stride, const T* __rest
                         const int* __restrict__ block_tables, int max_blocks, const int* __restrict__ tok_list,
                         const int* __restrict__ tok_seq, const int* __restrict__ tok_pos, float scale, int window,
                         int n_head, int n_kv_head, int hd, int page_size, int page_shift, int rows_are_requests,
-                        int n_splits, int chunk, float* __restrict__ partials, int num_pages, int heads_first, float softcap = 0.0f,
+                        int n_splits, int split_shift, int chunk, float* __restrict__ partials, int num_pages, int heads_first, float softcap = 0.0f,
                         const float* __restrict__ bias_table = nullptr, int max_dist = 0, const float* __restrict__ sinks = nullptr,
                         int keep_first = 0) {
     constexpr int KPP = 64 / LPK;  // keys per wave and pass
+    constexpr int TRIP = AD_WAVES * KPP * AD_U;
+    // the next trip's keys are on their way while this one's are absorbed, where the registers hold both (see the head of this file)
+    constexpr bool AHEAD = sizeof(T) == 2 && AD_WAVES <= 4;
+    typedef typename Raw8<T>::type Raw;
+    typedef std::integral_constant<bool, true> Whole;  // every lane has keys throughout the trip
+    typedef std::integral_constant<bool, false> Ragged;
     __shared__ float lds2[2][AD_WAVES][LPK][10];  // the waves' sums, for the first wave to merge; two of them in turn, so that one barrier a split is enough
     // (which of the two the grid runs along first: heads_first_pays)
     const int slot = heads_first ? blockIdx.y : blockIdx.x;
@@ -116,7 +130,8 @@ attention_decode_kernel(T* __restrict__ out, int64_t out_stride, const T* __rest
     for (int i = tid; i < max_blocks; i += 64 * AD_WAVES) sbt[i] = min(max(bt[i], 0), num_pages - 1);
     // (a position past the block table's reach would index the staged ids out of range)
     const int pos = static_cast<int>(min(static_cast<int64_t>(max(tok_pos[t], 0)), static_cast<int64_t>(max_blocks) * page_size - 1));
-    const int hkv = h / (n_head / n_kv_head);
+    const int hkv = n_head == n_kv_head ? h : h / (n_head / n_kv_head);
+    const int64_t page_stride = static_cast<int64_t>(n_kv_head) * page_size * hd;
     // lanes past the head dimension read column 0 and multiply it by a zero query
     const int col = active ? c * 8 : 0;
     float qf[8];
@@ -125,6 +140,7 @@ attention_decode_kernel(T* __restrict__ out, int64_t out_stride, const T* __rest
 #pragma unroll
         for (int e = 0; e < 8; ++e) qf[e] = 0.0f;
     }
+    const int64_t head_off = static_cast<int64_t>(hkv) * page_size * hd + col;
     __syncthreads();
     const int first_seen = window > 0 ? max(0, pos - window + 1) : 0;  // the window's first position
     const int first = SCORED ? first_seen - min(keep_first, first_seen) : first_seen;  // the walk's first place
@@ -140,32 +156,36 @@ attention_decode_kernel(T* __restrict__ out, int64_t out_stride, const T* __rest
     float (&lds)[AD_WAVES][LPK][10] = lds2[zi & 1];
     const int zz = walks_all ? zi : z;
     // split zz: its share of the keys, or keys [zz * chunk, (zz + 1) * chunk) of them (none, for a short context)
-    const int k_begin = first + (chunk > 0 ? zz * chunk : static_cast<int>(static_cast<int64_t>(n_keys) * zz / n_splits));
-    const int k_end = chunk > 0 ? min(pos + 1, k_begin + chunk) : first + static_cast<int>(static_cast<int64_t>(n_keys) * (zz + 1) / n_splits);
+    const auto share = [&](int z0) {  // the keys ahead of split z0: a shift where the splits are a power of two (a 64-bit division is a hundred instructions)
+        const int64_t all = static_cast<int64_t>(n_keys) * z0;
+        return static_cast<int>(split_shift >= 0 ? all >> split_shift : all / n_splits);
+    };
+    const int k_begin = first + (chunk > 0 ? zz * chunk : share(zz));
+    const int k_end = chunk > 0 ? min(pos + 1, k_begin + chunk) : first + share(zz + 1);
     Partial st;
     st.m = -INFINITY;
     st.l = 0.0f;
 #pragma unroll
     for (int e = 0; e < 8; ++e) st.acc[e] = 0.0f;
 
-    const int64_t head_off = static_cast<int64_t>(hkv) * page_size * hd + col;
-    const int64_t page_stride = static_cast<int64_t>(n_kv_head) * page_size * hd;
-    for (int j0 = k_begin + wave * KPP; j0 < k_end; j0 += AD_WAVES * KPP * AD_U) {
-        typename Raw8<T>::type kv[AD_U], vv[AD_U];
-        bool valid[AD_U];
+    // The walk, TRIP keys of the workgroup a trip: lane group kg of wave w takes keys j0 + (u AD_WAVES + w) KPP + kg.
+    const auto fetch = [&](int j0, Raw (&kv)[AD_U], Raw (&vv)[AD_U]) {
 #pragma unroll
         for (int u = 0; u < AD_U; ++u) {
-            const int j = j0 + u * AD_WAVES * KPP + kg;
-            valid[u] = j < k_end;
-            int jc = valid[u] ? j : pos;  // a mapped position; its values are not used
+            // (past the split a mapped position, whose values are not used; no branch around the loads: a load under a branch is
+            // waited for where the branch ends)
+            int jc = j0 + (u * AD_WAVES + wave) * KPP + kg;
+            jc = jc < k_end ? jc : pos;
             if constexpr (SCORED) jc = jc < first_seen ? jc - first : jc;
-            // no branch around the loads: a load under a branch is waited for where the branch ends
             const int lp = page_shift >= 0 ? jc >> page_shift : jc / page_size;
-            const int off = page_shift >= 0 ? jc & (page_size - 1) : jc % page_size;
+            const int off = page_shift >= 0 ? jc & (page_size - 1) : jc - lp * page_size;
             const int64_t at = static_cast<int64_t>(sbt[lp]) * page_stride + head_off + static_cast<int64_t>(off) * hd;
             kv[u] = fetch8(kc + at);
             vv[u] = fetch8(vc + at);
         }
+    };
+    const auto absorb = [&](auto whole, int j0, const Raw (&kv)[AD_U], Raw (&vv)[AD_U]) {
+#pragma clang fp contract(off)  // a whole trip and a ragged one round alike: nothing is fused but what says so
         float s[AD_U];
         float m_new = st.m;
 #pragma unroll
@@ -175,28 +195,29 @@ attention_decode_kernel(T* __restrict__ out, int64_t out_stride, const T* __rest
             float d = 0.0f;
 #pragma unroll
             for (int e = 0; e < 8; ++e) d = fmaf(kf[e], qf[e], d);
-            d = group_sum<LPK>(d);  // over the lanes that share the key
-            s[u] = valid[u] ? d * scale : -INFINITY;
+            s[u] = group_sum<LPK>(d) * scale;  // over the lanes that share the key
+            const int place = j0 + (u * AD_WAVES + wave) * KPP + kg;
             if constexpr (SCORED) {
-                if (valid[u]) {
-                    if (softcap > 0.0f) s[u] = softcap * tanhf(s[u] / softcap);
-                    if (bias_table != nullptr) {
-                        const int place = j0 + u * AD_WAVES * KPP + kg;
-                        s[u] += bias_table[static_cast<int64_t>(min(pos - (place < first_seen ? place - first : place), max_dist)) * n_head + h];
-                    }
+                if (softcap > 0.0f) s[u] = softcap * tanhf(s[u] / softcap);
+                if (bias_table != nullptr) s[u] += bias_table[static_cast<int64_t>(max(0, min(pos - (place < first_seen ? place - first : place), max_dist))) * n_head + h];
+            }
+            if constexpr (!decltype(whole)::value) {
+                if (place >= k_end) {
+                    s[u] = -INFINITY;
+                    vv[u] = Raw{};  // (its weight is 0, and 0 times an infinity would be no number)
                 }
             }
             m_new = fmaxf(m_new, s[u]);
         }
-        if (m_new == -INFINITY) continue;  // this lane group had no key in this trip (and none before)
-        const float corr = st.m == -INFINITY ? 0.0f : exp_for<T>(st.m - m_new);
+        // (a lane group without a key so far: every exponential below is 0)
+        const float ref = m_new == -INFINITY ? 0.0f : m_new;
+        const float corr = exp_for<T>(st.m - ref);
         st.l *= corr;
 #pragma unroll
         for (int e = 0; e < 8; ++e) st.acc[e] *= corr;
 #pragma unroll
         for (int u = 0; u < AD_U; ++u) {
-            if (!valid[u]) continue;
-            const float p = exp_for<T>(s[u] - m_new);
+            const float p = exp_for<T>(s[u] - ref);
             st.l += p;
             float vf[8];
             unpack8(vv[u], vf);
@@ -204,6 +225,42 @@ attention_decode_kernel(T* __restrict__ out, int64_t out_stride, const T* __rest
             for (int e = 0; e < 8; ++e) st.acc[e] = fmaf(p, vf[e], st.acc[e]);
         }
         st.m = m_new;
+    };
+    if (k_begin < k_end) {
+        Raw ka[AD_U], va[AD_U];
+        int j0 = k_begin;
+        if constexpr (AHEAD) {
+            Raw kb[AD_U], vb[AD_U];
+            fetch(j0, ka, va);
+            // (fences for the scheduler, which would sink the loads to their use)
+            for (;;) {
+                if (j0 + TRIP >= k_end) {
+                    absorb(Ragged{}, j0, ka, va);
+                    break;
+                }
+                fetch(j0 + TRIP, kb, vb);
+                __builtin_amdgcn_sched_barrier(0);
+                absorb(Whole{}, j0, ka, va);
+                __builtin_amdgcn_sched_barrier(0);
+                j0 += TRIP;
+                if (j0 + TRIP >= k_end) {
+                    absorb(Ragged{}, j0, kb, vb);
+                    break;
+                }
+                fetch(j0 + TRIP, ka, va);
+                __builtin_amdgcn_sched_barrier(0);
+                absorb(Whole{}, j0, kb, vb);
+                __builtin_amdgcn_sched_barrier(0);
+                j0 += TRIP;
+            }
+        } else {
+            for (; j0 + TRIP < k_end; j0 += TRIP) {
+                fetch(j0, ka, va);
+                absorb(Whole{}, j0, ka, va);
+            }
+            fetch(j0, ka, va);
+            absorb(Ragged{}, j0, ka, va);
+        }
     }
     // lane groups of the wave, in a fixed tree
 #pragma unroll
@@ -357,9 +414,11 @@ int launch_attention_decode(void* out, int64_t out_stride, const void* q, int64_
                             int page_size, int n_splits, int chunk, int waves, int rows_are_requests, float* partials,
                             int leave_splits, int num_pages, int reach, hipStream_t stream, float softcap = 0.0f, const float* bias_table = nullptr,
                             int max_dist = 0, const float* sinks = nullptr, int keep_first = 0) {
-    int page_shift = -1;
-    for (int b = 0; b < 31; ++b)
+    int page_shift = -1, split_shift = -1;
+    for (int b = 0; b < 31; ++b) {
         if ((1 << b) == page_size) page_shift = b;
+        if ((1 << b) == n_splits) split_shift = b;
+    }
     int64_t keys = static_cast<int64_t>(max_blocks) * page_size;
     if (reach > 0 && reach < keys) keys = reach;
     if (window > 0 && static_cast<int64_t>(window) + keep_first < keys) keys = static_cast<int64_t>(window) + keep_first;
@@ -374,15 +433,15 @@ int launch_attention_decode(void* out, int64_t out_stride, const void* q, int64_
         if (waves == 4)                                                                                              \
             attention_decode_kernel<T, L, 4, 4, SCORED><<<grid, 256, 0, stream>>>(o, out_stride, pq, q_stride, pk, pv, block_tables, \
                                                                     max_blocks, tok_list, tok_seq, tok_pos, scale,   \
-                                                                    window, n_head, n_kv_head, hd, page_size, page_shift, rows_are_requests, n_splits, chunk, partials, num_pages, heads_first, softcap, bias_table, max_dist, sinks, keep_first); \
+                                                                    window, n_head, n_kv_head, hd, page_size, page_shift, rows_are_requests, n_splits, split_shift, chunk, partials, num_pages, heads_first, softcap, bias_table, max_dist, sinks, keep_first); \
         else if (waves == 8)                                                                                         \
             attention_decode_kernel<T, L, 8, 4, SCORED><<<grid, 512, 0, stream>>>(o, out_stride, pq, q_stride, pk, pv, block_tables, \
                                                                     max_blocks, tok_list, tok_seq, tok_pos, scale,   \
-                                                                    window, n_head, n_kv_head, hd, page_size, page_shift, rows_are_requests, n_splits, chunk, partials, num_pages, heads_first, softcap, bias_table, max_dist, sinks, keep_first); \
+                                                                    window, n_head, n_kv_head, hd, page_size, page_shift, rows_are_requests, n_splits, split_shift, chunk, partials, num_pages, heads_first, softcap, bias_table, max_dist, sinks, keep_first); \
         else                                                                                                         \
             attention_decode_kernel<T, L, 16, sizeof(T) == 2 ? 8 : 4, SCORED><<<grid, 1024, 0, stream>>>(o, out_stride, pq, q_stride, pk, pv, block_tables, \
                                                                       max_blocks, tok_list, tok_seq, tok_pos, scale, \
-                                                                      window, n_head, n_kv_head, hd, page_size, page_shift, rows_are_requests, n_splits, chunk, partials, num_pages, heads_first, softcap, bias_table, max_dist, sinks, keep_first); \
+                                                                      window, n_head, n_kv_head, hd, page_size, page_shift, rows_are_requests, n_splits, split_shift, chunk, partials, num_pages, heads_first, softcap, bias_table, max_dist, sinks, keep_first); \
     } while (0)
     if (hd <= 8) LIYAB_GO(1);
     else if (hd <= 16) LIYAB_GO(2);
