@@ -22,7 +22,7 @@
 // query's maximum jumps past that, which is rare, instead of at every block.
 // Maximum, exponentials, sums and outputs are 32-bit. A query's result depends
 // on its position and the block grid (multiples of 32 from the window's start),
-// not on the batch or the pages. Head sizes: multiples of 16 up to 128.
+// not on the batch or the pages. Head sizes: multiples of 16 up to 128; those of 64 and 128 go to attention_prefill_direct.hip.
 //
 // A block's work is one chain: fragments from LDS, four products into one accumulator, the
 // maximum across two lanes, sixteen exponentials, fragments of the values, four products; alone
@@ -31,6 +31,7 @@
 // as two streams with a running maximum, sum and output each: nothing in one stream waits for the
 // other, so their chains overlap, and the streams are merged once at the end (in registers, then
 // the KS partial results as before).
+#include "attention_prefill.h"
 #include "common.h"
 #include "launchers.h"
 
@@ -57,7 +58,7 @@ union QFrag {
 constexpr int AP_KEYS = 32;     // keys per block
 constexpr int AP_QUERIES = 128; // queries per tile (4 waves x 32)
 constexpr int kDepth = 6;       // blocks of keys and values in flight in registers
-constexpr int AP_MAX_BLOCKS = 2048;  // page ids of a tile's keys are kept in LDS
+constexpr int AP_MAX_BLOCKS = kPrefillMaxBlocks;
 
 // SCORED: the scores are worked on before the softmax: scale * q . k, capped as cap * tanh(. / cap) when softcap > 0, plus
 // bias_table[min(query position - key position, max_dist), head] when a table is given; the exponentials then take the
@@ -468,6 +469,11 @@ static int run_attention_prefill(void* out, int64_t out_stride, const void* q, i
     int page_shift = -1;
     for (int b = 0; b < 31; ++b)
         if ((1 << b) == page_size) page_shift = b;
+    if (hd == 64 || hd == 128) {
+        const PrefillArgs args{static_cast<bf16_t*>(out), out_stride, static_cast<const bf16_t*>(q), q_stride, static_cast<const bf16_t*>(kc), static_cast<const bf16_t*>(vc),
+                               block_tables, max_blocks, work, scale, window, n_head, n_kv_head, hd, page_size, num_pages, softcap, bias_table, max_dist, sinks, keep_first};
+        return launch_prefill_direct<SCORED>(args, n_tiles, tile, ksplit, page_shift, stream);
+    }
     dim3 grid(n_head, n_tiles);
     auto* o = static_cast<bf16_t*>(out);
     auto* pq = static_cast<const bf16_t*>(q);

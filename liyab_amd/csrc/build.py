@@ -43,6 +43,7 @@ FLAGS = [
 VGPR_MFMA = ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]
 FILE_FLAGS = {
     "attention_prefill.hip": VGPR_MFMA,
+    "attention_prefill_direct.hip": VGPR_MFMA,
     "gemm_simple.hip": VGPR_MFMA,
 }
 

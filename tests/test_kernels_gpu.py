@@ -701,6 +701,44 @@ def test_attention_prefill(ops, case_id, window, tile, ksplit):
     close(out, attention_reference(case, H, Hkv, hd, scale, window), 8e-3, "prefill")
 
 
+@pytest.mark.parametrize("tile,ksplit", [(64, 1), (64, 2), (64, 4), (128, 1), (128, 2)])
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("window,keep", [(0, 0), (100, 0), (100, 20), (70, 130)])
+def test_attention_prefill_by_page_size(ops, window, keep, hd, tile, ksplit):
+    """Contexts that end at and beside the blocks of 64 keys, in pages that a load of keys never crosses (8, 128), that it does (4), and
+    of no power of two (24): the formula, and the same bits from each. What lies between the kept positions and every query's window is
+    given back (no page, or NaN), and must not be read."""
+    if ksplit == 4 and hd > 64:
+        pytest.skip("4 waves a query group are taken up to head size 64")
+    ctx_lens, q_lens, H, Hkv, scale = [63, 128, 193, 300], [63, 65, 1, 131], 2, 1, 0.7 / math.sqrt(hd)
+    outs = []
+    for page in (8, 4, 24, 128):
+        case = paged_case(4, ctx_lens, q_lens, H, Hkv, hd, page, torch.bfloat16, seed=5, shuffle=False)  # (the same values whatever the pages)
+        case["bt"] = torch.where(case["bt"] >= 0, case["kc"].shape[0] - 1 - case["bt"], case["bt"])
+        case["kc"], case["vc"] = case["kc"].flip(0), case["vc"].flip(0)
+        row, work, want = 0, [], torch.zeros(case["n"], H * hd, dtype=torch.float64)
+        for s, (c, n) in enumerate(zip(ctx_lens, q_lens)):
+            for t0 in range(0, n, tile):
+                work += [s, row + t0, c - n + t0, min(tile, n - t0)]
+            for t in range(row, row + n):
+                p = case["tok_pos"][t]
+                seen = [j for j in range(p + 1) if window == 0 or j > p - window or j < keep]
+                for h in range(H):
+                    w = torch.softmax(case["ks"][s][seen, 0].double() @ case["q"][t, h * hd:(h + 1) * hd].double() * scale, dim=0)
+                    want[t, h * hd:(h + 1) * hd] = w @ case["vs"][s][seen, 0].double()
+            for j in range(keep, c - n - window + 1 if window else 0):  # no query sees position j
+                pg = int(case["bt"][s, j // page])
+                case["kc"][pg, :, j % page], case["vc"][pg, :, j % page] = float("nan"), float("nan")
+            row += n
+        out = torch.zeros(case["n"], H * hd, dtype=torch.bfloat16, device=DEV)
+        kw = {k: case[k].to(DEV) for k in ("kc", "vc", "bt")}
+        ops.attention_prefill(out, case["q"].to(DEV)[:, :H * hd], kw["kc"], kw["vc"], kw["bt"], torch.tensor(work, dtype=torch.int32, device=DEV),
+                              len(work) // 4, n_head=H, scale=scale, window=window, tile=tile, ksplit=ksplit, keep_first=keep)
+        close(out, want, 8e-3, f"pages of {page}")
+        outs.append(out)
+    assert all(torch.equal(outs[0], o) for o in outs[1:])
+
+
 def reference_from_pages(case, kc, vc, bt, H, Hkv, hd, page, scale, window=0):
     """The plain formula over whatever pages a block table names (float64)."""
     out = torch.zeros(case["n"], H * hd, dtype=torch.float64)
