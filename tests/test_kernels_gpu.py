@@ -739,6 +739,48 @@ def test_attention_prefill_by_page_size(ops, window, keep, hd, tile, ksplit):
     assert all(torch.equal(outs[0], o) for o in outs[1:])
 
 
+@pytest.mark.parametrize("K", [64, 192, 832, 72])
+@pytest.mark.parametrize("N", [33, 64, 72, 200])
+@pytest.mark.parametrize("form", ["one", "relu2", "two", "clamped", "heads", "gated heads"])
+def test_products_of_listed_rows_and_heads(ops, form, N, K):
+    """Tiles of 64 places with one, some and all of them taken, one in the middle that nobody uses and some at the end; features that fill no
+    tile; K of one stage, of three, of a wide tile's 13, and of no whole stage. Against 32-bit sums of the same bfloat16 operands: the results'
+    rounding to bfloat16 (2^-9) and a sum's order."""
+    E, n = 3, 150
+    if "heads" in form:
+        a, w = rnd(n, E * K, dtype=torch.bfloat16), rnd(E, N, K, seed=1, scale=0.2, dtype=torch.bfloat16)
+        gate = rnd(n, E * N + 3, seed=2)[:, :E * N] if form == "gated heads" else None
+        out = torch.full((n, E * N), float("nan"), dtype=torch.bfloat16, device=DEV)
+        ops.heads_product(out, a, w, gate)
+        want = torch.cat([a[:, h * K:(h + 1) * K].float() @ w[h].float().t() for h in range(E)], dim=1)
+        close(out, want * torch.sigmoid(gate) if gate is not None else want, 4e-3, form)
+        return
+    a = rnd(n, K, dtype=torch.bfloat16)
+    w0, w1 = rnd(E, N, K, seed=1, scale=0.2, dtype=torch.bfloat16), rnd(E, N, K, seed=2, scale=0.2, dtype=torch.bfloat16)
+    expert = torch.tensor([0] * 65 + [1] * 1 + [2] * (2 * n - 66))
+    expert = expert[torch.randperm(2 * n, generator=torch.Generator().manual_seed(3))]
+    tiles = ops.moe_tiles(2 * n, E, 64)
+    rows, group, at = torch.full((tiles, 64), -1, dtype=torch.int32), torch.full((tiles,), -1, dtype=torch.int32), 0
+    for e in range(E):
+        mine = (expert == e).nonzero().flatten().int()
+        for c in mine.split(64):
+            rows[at, :len(c)], group[at], at = c, e, at + 1
+        at += 1 if e == 0 and at + 1 + -(-int((expert > 0).sum()) // 64) < tiles else 0  # a tile nobody uses
+    scale = rnd(2 * n, seed=4)
+    two, clamp = form in ("two", "clamped"), (1.5, 1.7, 1.0) if form == "clamped" else None
+    x = a.float().repeat_interleave(2, 0)
+    u, v = (torch.stack([x[i] @ w[e].float().t() for i, e in enumerate(expert.tolist())]) for w in (w0, w1))
+    if form == "clamped":
+        g = u.clamp(max=1.5)
+        want = g * torch.sigmoid(1.7 * g) * (v.clamp(-1.5, 1.5) + 1.0)
+    else:
+        want = u * torch.sigmoid(u) * v if two else torch.relu(u) ** 2 if form == "relu2" else u
+    for dtype, tol in ((torch.bfloat16, 4e-3), (torch.float32, 1e-5)):
+        out = torch.full((2 * n, N), float("nan"), dtype=dtype, device=DEV)
+        ops.moe_product(out, a, w0, w1 if two else None, rows.to(DEV).flatten(), group.to(DEV), a_div=2, row_scale=scale, act="relu2" if form == "relu2" else "none", clamp=clamp)
+        close(out, want * scale[:, None], tol, form)
+
+
 def reference_from_pages(case, kc, vc, bt, H, Hkv, hd, page, scale, window=0):
     """The plain formula over whatever pages a block table names (float64)."""
     out = torch.zeros(case["n"], H * hd, dtype=torch.float64)
