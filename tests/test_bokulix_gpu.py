@@ -694,3 +694,38 @@ def test_command_line(models):
     turn2 = [json.loads(l) for l in p2.stdout.splitlines() if l.startswith("{")][1]
     assert turn2["tokens"] == turn["tokens"]
     assert set(turn2["phases_ms"]) == {"embed", "latent_attention", "routed_ffn", "lm_head"}
+
+
+@pytest.mark.parametrize("n,E,top", [(1, 2, 2), (4, 8, 2), (16, 64, 8), (17, 33, 3), (64, 64, 8), (16, 64, 16), (17, 8, 2), (4, 65, 3)])
+@pytest.mark.parametrize("block", [16, 64])
+def test_choices_and_lists_of_a_small_step(n, E, top, block):
+    """Each side of the sizes at which a wave chooses for a token and the lists stay in LDS: ids (the lower number among equals, minus
+    infinity and NaN last, a NaN that comes first among what is left chosen), weights, and every entry once in a tile of its expert."""
+    from liyab_amd.kernels import ops
+
+    g = torch.Generator().manual_seed(n + E)
+    z = (torch.randn(n, E + 3, generator=g) * 2).round() / 2  # many equals
+    z[torch.rand(z.shape, generator=g) < 0.1] = float("-inf")
+    z[torch.rand(z.shape, generator=g) < 0.1] = -0.0
+    z[-1, E - 1] = float("nan")
+    ids, w = torch.empty(n, top, dtype=torch.int32, device="cuda:0"), torch.empty(n, top, device="cuda:0")
+    tiles = ops.moe_tiles(n * top, E, block)
+    rows, group = torch.empty(tiles * block, dtype=torch.int32, device="cuda:0"), torch.empty(tiles, dtype=torch.int32, device="cuda:0")
+    ops.moe_route(z.to("cuda:0")[:, :E], top, ids, w, rows, group, block=block)
+    ids, w, rows, group = ids.cpu(), w.cpu(), rows.cpu().view(tiles, block), group.cpu()
+    for t in range(n):
+        left, want = list(range(E)), []
+        for _ in range(top):
+            best = left[0]
+            for e in left[1:]:
+                if z[t, e] > z[t, best]:
+                    best = e
+            want.append(best)
+            left.remove(best)
+        assert ids[t].tolist() == want
+        torch.testing.assert_close(w[t], torch.softmax(z[t, want].double(), 0).float(), rtol=4e-7, atol=1e-30, equal_nan=True)
+    used = int((group >= 0).sum())
+    assert (group[:used] >= 0).all() and (rows[used:] == -1).all() and group[:used].tolist() == sorted(group[:used].tolist())
+    seen = [(int(group[i]), int(r)) for i in range(used) for r in rows[i] if r >= 0]
+    assert sorted(r for _, r in seen) == list(range(n * top)) and all(int(ids.flatten()[r]) == e for e, r in seen)
+    assert all(used_tiles == -(-int((ids == e).sum()) // block) for e in range(E) for used_tiles in [int((group == e).sum())])
