@@ -696,10 +696,10 @@ def test_command_line(models):
     assert set(turn2["phases_ms"]) == {"embed", "latent_attention", "routed_ffn", "lm_head"}
 
 
-@pytest.mark.parametrize("n,E,top", [(1, 2, 2), (4, 8, 2), (16, 64, 8), (17, 33, 3), (64, 64, 8), (16, 64, 16), (17, 8, 2), (4, 65, 3)])
+@pytest.mark.parametrize("n,E,top", [(1, 2, 2), (4, 8, 2), (16, 64, 8), (17, 33, 3), (64, 64, 8), (16, 64, 16), (17, 8, 2), (4, 65, 3), (1030, 8, 2), (1030, 65, 1)])
 @pytest.mark.parametrize("block", [16, 64])
-def test_choices_and_lists_of_a_small_step(n, E, top, block):
-    """Each side of the sizes at which a wave chooses for a token and the lists stay in LDS: ids (the lower number among equals, minus
+def test_choices_and_lists_of_a_step(n, E, top, block):
+    """Each side of the sizes at which a wave chooses for a token and the lists stay in LDS, and of a step in two launches: ids (the lower number among equals, minus
     infinity and NaN last, a NaN that comes first among what is left chosen), weights, and every entry once in a tile of its expert."""
     from liyab_amd.kernels import ops
 
