@@ -916,10 +916,9 @@ def decode_plan(n_tokens: int, n_head: int, context_bucket: int):
     """(splits of the keys, waves per workgroup) for tokens whose attention the kernel finishes
     itself (several splits: plus the merge kernel). `context_bucket`: the most keys a token has,
     rounded up. From measurements at 12 to 32 heads of 64 and 128, 1 to 42 tokens and 300 to
-    8,000 keys (us, attention and merge). Uncut, workgroups of 4 waves, which ask for a trip's keys while they absorb the
-    one before, are the fastest from 200 pairs on and up to 512 keys (4 / 8 / 16 waves, longest of contexts from a quarter of it on:
-    252 pairs at 1,000 keys 11.5 / 12.0 / 12.5, at 2,000 21.0 / 21.8 / 21.2; 312 pairs 15.4 / 16.5 / 20.2; 108 pairs at 300 keys 6.3 / 6.6 /
-    9.1), 8 waves below (108 pairs at 1,000 keys 10.0 / 9.1 / 9.8, at 2,000 16.1 / 13.4 / 13.6), 16 with few pairs of 4,000 keys and more
+    8,000 keys (us, attention and merge). Uncut (4 / 8 / 16 waves, longest of contexts from a quarter of it on): 8 waves
+    (108 pairs at 1,000 keys 10.0 / 9.1 / 9.8, at 2,000 16.1 / 13.4 / 13.6; 252 pairs at 1,000 keys 11.5 / 12.0 / 12.5, at 2,000 21.0 /
+    21.8 / 21.2: 4 waves round otherwise for 4 % there), 4 from 512 pairs on and up to 256 keys, 16 with few pairs of 4,000 keys and more
     (108 pairs at 4,000 29.6 / 30.8 / 27.6, 252 at 8,000 70.0 / 71.5 / 68.1). With fewer pairs than would fill the chip the keys
     are cut across workgroups of 4 waves, into 4, 8 or 16 splits of 128 keys or more, while
     pairs x splits stay within the chip's 256 compute units (32 pairs of 128 dimensions at
@@ -936,9 +935,7 @@ def decode_plan(n_tokens: int, n_head: int, context_bucket: int):
         # (splits of 1,024 keys and more on 8 waves: 12 pairs at 30,000 keys in 16 splits 26.7 us on
         # 4 waves, 22.4 on 8; 32 pairs of 128 dimensions 92.6 and 89.1)
         return splits, (8 if context_bucket // splits >= 1024 else 4)
-    if context_bucket >= 4096 and pairs < 256:
-        return 1, 16
-    return 1, (4 if pairs >= 200 or context_bucket <= 512 else 8)
+    return 1, (16 if context_bucket >= 4096 and pairs < 256 else 8)
 
 
 def decode_split_plan(n_tokens: int, n_head: int, context_bucket: int):
