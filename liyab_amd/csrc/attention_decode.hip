@@ -2,7 +2,7 @@
 // over paged keys and values (bfloat16, or 32-bit for the 32-bit path), with
 // the keys of a token cut into splits so that few tokens still fill the chip.
 //
-// Grid (token, query head, split). A workgroup of 4 or 16 waves walks its split's
+// Grid (token, query head, split). A workgroup of 4, 8 or 16 waves walks its split's
 // keys; LPK lanes share a key (each holds 8 consecutive dimensions, 16
 // bytes), so a wave takes 64 / LPK keys a pass, read straight from the pages
 // through the block table. Each lane group keeps a running maximum, sum and
@@ -13,12 +13,13 @@
 // splits) and four waves, which lane adds which key and which sums are merged
 // follow from the token's position alone, as the reference cuts (:2136-2139):
 // the form of the 32-bit path and of the batch-invariant mode.
-// What bounds it: with many pairs the caches' reads (64 tokens of 25 heads over 256 to 1,015 keys, 261 MB: 54.2 -> 51.2 us, where reading
-// the same bytes and doing nothing takes 45.5), so a workgroup of four waves asks for its next trip's keys and values before it
-// absorbs the ones it has; eight and sixteen waves hold as much in flight by their number (24 tokens of 12 heads on eight: 12.7
-// either way, 13.1 with the next trip's loads in flight, whose registers cost a workgroup a compute unit). With few pairs the
-// instructions around the loads: only a split's last trip looks at which keys it has, and the other trips and both forms' loads
-// are free of branches (32 tokens of 16 heads over 100 to 900 keys 20.6 -> 16.7 us, 17 of 12 heads 13.6 -> 10.4, one token in 8 splits 4.7 -> 4.4).
+// What bounds it: with many pairs the caches' reads (64 tokens of 25 heads over 256 to 1,015 keys, 261 MB: 50.3 us, where reading the same bytes
+// and doing nothing takes 45.5), so four waves ask for the next trip's keys and values before they absorb the ones they have, where that pays
+// (next_trip_ahead_pays); eight and sixteen hold as much in flight by their number (24 tokens of 12 heads on eight: 12.7, 13.1 with the next trip's
+// loads in flight, whose registers cost a workgroup a compute unit). With few pairs the instructions around the loads: only a wave's last trip looks at which
+// keys it has, and the other trips and both forms' loads are free of branches. us, with every key looked at and nothing asked for ahead / now, caches not
+// read before, heads of 64: 64 tokens of 25 heads 51.7 / 50.3, 32 of 16 over 100 to 900 keys 21.5 / 17.2, 17 of 12 over 200 to 1,000 on eight waves 14.5 / 13.1,
+// one of 12 at 1,024 in 8 splits 5.2 / 4.8.
 // The reference cuts a token's keys by its position only (:2136-2139,
 // 2225-2227) to keep bits equal; here the number of splits follows the batch
 // (more splits when few tokens are in flight), which moves results by
@@ -94,7 +95,8 @@ __device__ __forceinline__ void add_sink(float& m, float& l, float (&acc)[N], fl
 // a bias by distance, bias_table[min(position - key, max_dist), head] (bias_table given); `sinks` (one logit a head) join the
 // softmax's denominator where the row's sums are final; with a window, the first `keep_first` positions may stay visible: the
 // walk goes over places first - kept .. position, of which those ahead of `first` are positions 0 .. kept - 1. Without SCORED these arguments are not read, and the kernel is the one it was.
-template <typename T, int LPK, int AD_WAVES, int AD_U, bool SCORED = false>
+// AHEAD: the next trip's keys are on their way while this one's are absorbed (where it pays: next_trip_ahead_pays).
+template <typename T, int LPK, int AD_WAVES, int AD_U, bool SCORED, bool AHEAD>
 __global__ void __launch_bounds__(64 * AD_WAVES)
 attention_decode_kernel(T* __restrict__ out, int64_t out_stride, const T* __restrict__ q, int64_t q_stride,
                         const T* __restrict__ kc, const T* __restrict__ vc,
@@ -106,8 +108,7 @@ attention_decode_kernel(T* __restrict__ out, int64_t out_stride, const T* __rest
                         int keep_first = 0) {
     constexpr int KPP = 64 / LPK;  // keys per wave and pass
     constexpr int TRIP = AD_WAVES * KPP * AD_U;
-    // the next trip's keys are on their way while this one's are absorbed, where the registers hold both (see the head of this file)
-    constexpr bool AHEAD = sizeof(T) == 2 && AD_WAVES <= 4;
+    constexpr bool BY_PASS = SCORED || LPK <= 4;  // a wave leaves out the passes behind its last key too: where one is much arithmetic, or many keys
     typedef typename Raw8<T>::type Raw;
     typedef std::integral_constant<bool, true> Whole;  // every lane has keys throughout the trip
     typedef std::integral_constant<bool, false> Ragged;
@@ -184,12 +185,17 @@ attention_decode_kernel(T* __restrict__ out, int64_t out_stride, const T* __rest
             vv[u] = fetch8(vc + at);
         }
     };
+    // A wave's walk ends with its own last key: a trip is up to 4,096 keys, of which short contexts and windows fill little
+    // (32 tokens of 12 heads of 64 in a window of 256 with 4 kept, 8 waves: 11.5 us with every wave in every trip, 10.0 so).
+    const int own = __builtin_amdgcn_readfirstlane(wave) * KPP;
+    const auto has = [&](int j0, int u) { return j0 + u * AD_WAVES * KPP + own < k_end; };  // pass u of the trip from j0 on has a key of this wave
     const auto absorb = [&](auto whole, int j0, const Raw (&kv)[AD_U], Raw (&vv)[AD_U]) {
 #pragma clang fp contract(off)  // a whole trip and a ragged one round alike: nothing is fused but what says so
         float s[AD_U];
         float m_new = st.m;
 #pragma unroll
         for (int u = 0; u < AD_U; ++u) {
+            if (BY_PASS && !decltype(whole)::value && !has(j0, u)) break;
             float kf[8];
             unpack8(kv[u], kf);
             float d = 0.0f;
@@ -217,6 +223,7 @@ attention_decode_kernel(T* __restrict__ out, int64_t out_stride, const T* __rest
         for (int e = 0; e < 8; ++e) st.acc[e] *= corr;
 #pragma unroll
         for (int u = 0; u < AD_U; ++u) {
+            if (BY_PASS && !decltype(whole)::value && !has(j0, u)) break;
             const float p = exp_for<T>(s[u] - ref);
             st.l += p;
             float vf[8];
@@ -226,7 +233,7 @@ attention_decode_kernel(T* __restrict__ out, int64_t out_stride, const T* __rest
         }
         st.m = m_new;
     };
-    if (k_begin < k_end) {
+    if (has(k_begin, 0)) {
         Raw ka[AD_U], va[AD_U];
         int j0 = k_begin;
         if constexpr (AHEAD) {
@@ -234,7 +241,7 @@ attention_decode_kernel(T* __restrict__ out, int64_t out_stride, const T* __rest
             fetch(j0, ka, va);
             // (fences for the scheduler, which would sink the loads to their use)
             for (;;) {
-                if (j0 + TRIP >= k_end) {
+                if (!has(j0 + TRIP, 0)) {
                     absorb(Ragged{}, j0, ka, va);
                     break;
                 }
@@ -243,7 +250,7 @@ attention_decode_kernel(T* __restrict__ out, int64_t out_stride, const T* __rest
                 absorb(Whole{}, j0, ka, va);
                 __builtin_amdgcn_sched_barrier(0);
                 j0 += TRIP;
-                if (j0 + TRIP >= k_end) {
+                if (!has(j0 + TRIP, 0)) {
                     absorb(Ragged{}, j0, kb, vb);
                     break;
                 }
@@ -254,7 +261,7 @@ attention_decode_kernel(T* __restrict__ out, int64_t out_stride, const T* __rest
                 j0 += TRIP;
             }
         } else {
-            for (; j0 + TRIP < k_end; j0 += TRIP) {
+            for (; has(j0 + TRIP, 0); j0 += TRIP) {
                 fetch(j0, ka, va);
                 absorb(Whole{}, j0, ka, va);
             }
@@ -407,6 +414,14 @@ inline bool heads_first_pays(int n, int n_head, int n_kv_head, int hd, size_t el
     return heads * keys * hd * 2 * static_cast<int64_t>(elt) <= (4 << 20);
 }
 
+// Whether four waves ask for the next trip's keys ahead (bfloat16). The pieces of two trips take 128 to 143 registers, three or four workgroups a
+// compute unit, where one trip takes 63 to 90, five to seven: with small heads or scores to work on, whose arithmetic wants the waves, it pays until those three
+// are placed (us ahead / not, 12 heads over 100 to 1,000 keys, caches not read before. Heads of 16: 64 tokens 9.9 / 10.4, 72 11.8 / 11.0, 130 18.2 / 16.9,
+// 130 with a bias by distance 23.9 / 20.5; of 32: 64 tokens 15.1 / 15.9, 100 21.7 / 21.2, 130 over up to 250 keys 13.3 / 11.6. Heads of 64: 43 tokens with a sink
+// 20.2 / 21.6, 64 26.8 / 26.8, 100 38.8 / 37.4, with a bias 64 32.7 / 33.5, 72 37.9 / 35.4). Heads of 64 and more with plain scores gain at any number (130 tokens
+// 45.6 / 46.6).
+constexpr bool next_trip_ahead_pays(bool scored, int hd, int64_t workgroups) { return (!scored && hd > 32) || workgroups <= 3 * 256; }
+
 template <typename T, bool SCORED = false>
 int launch_attention_decode(void* out, int64_t out_stride, const void* q, int64_t q_stride, const void* kc, const void* vc,
                             const int* block_tables, int max_blocks, const int* tok_list, const int* tok_seq,
@@ -428,20 +443,18 @@ int launch_attention_decode(void* out, int64_t out_stride, const void* q, int64_
     auto* pq = static_cast<const T*>(q);
     auto* pk = static_cast<const T*>(kc);
     auto* pv = static_cast<const T*>(vc);
-#define LIYAB_GO(L)                                                                                                  \
-    do {                                                                                                             \
-        if (waves == 4)                                                                                              \
-            attention_decode_kernel<T, L, 4, 4, SCORED><<<grid, 256, 0, stream>>>(o, out_stride, pq, q_stride, pk, pv, block_tables, \
-                                                                    max_blocks, tok_list, tok_seq, tok_pos, scale,   \
-                                                                    window, n_head, n_kv_head, hd, page_size, page_shift, rows_are_requests, n_splits, split_shift, chunk, partials, num_pages, heads_first, softcap, bias_table, max_dist, sinks, keep_first); \
-        else if (waves == 8)                                                                                         \
-            attention_decode_kernel<T, L, 8, 4, SCORED><<<grid, 512, 0, stream>>>(o, out_stride, pq, q_stride, pk, pv, block_tables, \
-                                                                    max_blocks, tok_list, tok_seq, tok_pos, scale,   \
-                                                                    window, n_head, n_kv_head, hd, page_size, page_shift, rows_are_requests, n_splits, split_shift, chunk, partials, num_pages, heads_first, softcap, bias_table, max_dist, sinks, keep_first); \
-        else                                                                                                         \
-            attention_decode_kernel<T, L, 16, sizeof(T) == 2 ? 8 : 4, SCORED><<<grid, 1024, 0, stream>>>(o, out_stride, pq, q_stride, pk, pv, block_tables, \
-                                                                      max_blocks, tok_list, tok_seq, tok_pos, scale, \
-                                                                      window, n_head, n_kv_head, hd, page_size, page_shift, rows_are_requests, n_splits, split_shift, chunk, partials, num_pages, heads_first, softcap, bias_table, max_dist, sinks, keep_first); \
+    const bool ahead = next_trip_ahead_pays(SCORED, hd, static_cast<int64_t>(n) * n_head * n_splits);
+#define LIYAB_LAUNCH(L, WAVES, U, AHEAD)                                                                                          \
+    attention_decode_kernel<T, L, WAVES, U, SCORED, AHEAD><<<grid, 64 * WAVES, 0, stream>>>(                                      \
+        o, out_stride, pq, q_stride, pk, pv, block_tables, max_blocks, tok_list, tok_seq, tok_pos, scale, window, n_head, n_kv_head, hd, page_size, \
+        page_shift, rows_are_requests, n_splits, split_shift, chunk, partials, num_pages, heads_first, softcap, bias_table, max_dist, sinks, keep_first)
+#define LIYAB_GO(L)                                                                                      \
+    do {                                                                                                 \
+        constexpr bool always = next_trip_ahead_pays(SCORED, 8 * L, INT64_MAX);                          \
+        if (waves == 4 && ahead) LIYAB_LAUNCH(L, 4, 4, sizeof(T) == 2);                                  \
+        else if (waves == 4) LIYAB_LAUNCH(L, 4, 4, sizeof(T) == 2 && always);                            \
+        else if (waves == 8) LIYAB_LAUNCH(L, 8, 4, false);                                               \
+        else LIYAB_LAUNCH(L, 16, sizeof(T) == 2 ? 8 : 4, false);                                         \
     } while (0)
     if (hd <= 8) LIYAB_GO(1);
     else if (hd <= 16) LIYAB_GO(2);
@@ -450,6 +463,7 @@ int launch_attention_decode(void* out, int64_t out_stride, const void* q, int64_
     else if (hd <= 128) LIYAB_GO(16);
     else LIYAB_GO(32);
 #undef LIYAB_GO
+#undef LIYAB_LAUNCH
     if (int rc = check_launch("attention_decode")) return rc;
     if (n_splits > 1 && !leave_splits) {
         attention_merge_kernel<T><<<dim3(n, n_head), ((hd + 63) / 64) * 64, 0, stream>>>(o, out_stride, tok_list, partials, n_head, hd, n_splits, sinks);

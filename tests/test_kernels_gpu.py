@@ -518,6 +518,42 @@ def test_attention_decode(ops, case_id, dtype, splits, waves, window):
         assert torch.equal(part[rows], out[rows]) and (part[1::2] == 0).all()
 
 
+# contexts at and beside one, two and three trips of a workgroup over the keys, where a wave's walk ends: (head size, waves, heads, keys a trip)
+TRIPS = [(64, 4, 2, 128), (64, 8, 2, 256), (64, 16, 2, 1024), (128, 4, 2, 64), (128, 16, 2, 512), (256, 4, 1, 32), (16, 4, 2, 512), (32, 8, 1, 512), (32, 4, 160, 256), (64, 4, 160, 128)]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("scores", ["plain", "kept", "worked on"])
+@pytest.mark.parametrize("hd,waves,H,trip", TRIPS)
+def test_attention_decode_at_the_ends_of_its_trips(ops, hd, waves, H, trip, scores, dtype):
+    """Trips whose keys are all there, the last one's first and last key and the waves that have none in it, with 16 waves a token too, and on both
+    sides of the number of workgroups up to which four waves ask for the next trip's keys ahead."""
+    if dtype == torch.float32 and waves == 16:
+        trip //= 2
+    ctx_lens = [trip - 1, trip, trip + 1, trip + 64 // max(1, hd // 8) + 1] + ([2 * trip, 2 * trip + 1, 3 * trip, 3 * trip + 7] if H <= 2 else [2 * trip + 1])
+    case = paged_case(len(ctx_lens), ctx_lens, [1] * len(ctx_lens), H, H, hd, 16, dtype, seed=hd + waves)
+    scale, window, keep = 0.7 / math.sqrt(hd), trip - 3 if scores == "kept" else 0, 5 if scores == "kept" else 0
+    cap, sinks, table = 0.0, None, None
+    if scores == "worked on":
+        g = torch.Generator().manual_seed(1)
+        cap, sinks, table = 2.0, torch.randn(H, generator=g), torch.randn(trip // 2, H, generator=g)
+    want = torch.zeros(case["n"], H * hd, dtype=torch.float64)
+    for t, p in enumerate(case["tok_pos"]):
+        seen = torch.tensor([j for j in range(p + 1) if window == 0 or j > p - window or j < keep])
+        s = torch.einsum("jhd,hd->hj", case["ks"][t][seen].double(), case["q"][t, :H * hd].double().view(H, hd)) * scale
+        if scores == "worked on":
+            s = cap * torch.tanh(s / cap) + table[(p - seen).clamp(max=len(table) - 1)].double().t()
+            s = torch.cat([s, sinks.double()[:, None]], dim=1)
+        w = torch.softmax(s, dim=1)[:, :len(seen)]
+        want[t] = torch.einsum("hj,jhd->hd", w, case["vs"][t][seen].double()).flatten()
+    dev = lambda x: None if x is None else x.to(DEV)  # noqa: E731
+    out = torch.zeros(case["n"], H * hd, dtype=dtype, device=DEV)
+    ops.attention_decode(out, dev(case["q"])[:, :H * hd], dev(case["kc"]), dev(case["vc"]), dev(case["bt"]), torch.arange(case["n"], dtype=torch.int32, device=DEV),
+                         torch.tensor(case["tok_pos"], dtype=torch.int32, device=DEV), n_head=H, scale=scale, window=window, waves=waves, rows_are_requests=True,
+                         keep_first=keep, softcap=cap, bias_table=dev(table), sinks=dev(sinks))
+    close(out, want, 8e-3 if dtype == torch.bfloat16 else 3e-6, scores)
+
+
 @pytest.mark.parametrize("window", [0, 37, 300])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("case_id", range(len(ATT_CASES)))
