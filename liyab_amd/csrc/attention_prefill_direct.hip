@@ -482,9 +482,11 @@ int launch_direct_pages(const PrefillArgs& p, int n_tiles, int page_shift, hipSt
 
 template <int HD, int QG, int KS, int NS, int STAGES, int MIN_WAVES, bool SCORED>
 int launch_direct_as(const PrefillArgs& p, int n_tiles, int page_shift, hipStream_t stream) {
+    // Two streams and a row a lane to find do not fit the registers of three waves a SIMD (9 spilled, 40 bytes of scratch a lane, read back every step): two
+    // waves (8,001 tokens of 12 heads in pages of 24 178 -> 154 us, of 4 173 -> 145; 2 x 1,024 of 25 heads 27.3 -> 22.9 and 26.8 -> 21.9).
     const bool by_load = page_shift >= 0 && p.page_size * HD >= 512 && !(SCORED && p.window > 0 && p.keep_first > 0);
     return by_load ? launch_direct_pages<HD, QG, KS, NS, STAGES, MIN_WAVES, SCORED, true>(p, n_tiles, page_shift, stream)
-                   : launch_direct_pages<HD, QG, KS, NS, STAGES, MIN_WAVES, SCORED, false>(p, n_tiles, page_shift, stream);
+                   : launch_direct_pages<HD, QG, KS, NS, STAGES, NS == 2 ? 2 : MIN_WAVES, SCORED, false>(p, n_tiles, page_shift, stream);
 }
 
 template <bool SCORED>

@@ -1,0 +1,25 @@
+"""What the compiler says of kernels that are laid out to fit their registers (needs hipcc, no GPU)."""
+
+import os
+import re
+import subprocess
+
+import pytest
+
+from liyab_amd.csrc import build
+
+
+@pytest.mark.parametrize("source", ["attention_prefill_direct.hip"])
+def test_no_kernel_spills(source, tmp_path):
+    """A spilled register goes to memory and back in the walk over the keys, and counts among the loads that its waits count."""
+    hipcc = build.hipcc_path()
+    if hipcc is None:
+        pytest.skip("hipcc was not found")
+    r = subprocess.run([hipcc, *build.FLAGS, *build.FILE_FLAGS.get(source, []), "-I", build.CSRC, "--cuda-device-only", "-Rpass-analysis=kernel-resource-usage", "-c",
+                        os.path.join(build.CSRC, source), "-o", str(tmp_path / "kernels.o")], capture_output=True, text=True, timeout=600)
+    assert r.returncode == 0, r.stderr[-2000:]
+    kernels = re.split(r"Function Name: ", r.stderr)[1:]
+    assert kernels
+    for k in kernels:
+        spilled, scratch = (int(re.search(what + r": (\d+)", k)[1]) for what in ("VGPRs Spill", r"ScratchSize \[bytes/lane\]"))
+        assert spilled == 0 and scratch == 0, f"{k.split()[0]}: {spilled} registers spilled, {scratch} bytes of scratch a lane"
