@@ -817,6 +817,39 @@ def test_products_of_listed_rows_and_heads(ops, form, N, K):
         close(out, want * scale[:, None], tol, form)
 
 
+@pytest.mark.parametrize("K,N", [(64, 130), (192, 200), (832, 200), (832, 70)])
+@pytest.mark.parametrize("form", ["one", "two", "heads"])
+@pytest.mark.parametrize("E", [3, 400])
+def test_products_of_long_lists(ops, form, E, N, K):
+    """Lists and heads of many tiles, whose XCDs take stretches of several tiles, the last one shorter: with a hole inside a stretch, and with more spare tiles
+    at the end than a workgroup looks at. Bounds as above."""
+    n, H = 550 if E == 3 else 1100, 3
+    if form == "heads":
+        a, w = rnd(n, H * K, dtype=torch.bfloat16), rnd(H, N, K, seed=1, scale=0.2, dtype=torch.bfloat16)
+        out = torch.full((n, H * N), float("nan"), dtype=torch.bfloat16, device=DEV)
+        ops.heads_product(out, a, w, None)
+        close(out, torch.cat([a[:, h * K:(h + 1) * K].float() @ w[h].float().t() for h in range(H)], dim=1), 4e-3, form)
+        return
+    a = rnd(n, K, dtype=torch.bfloat16)
+    w0, w1 = rnd(E, N, K, seed=1, scale=0.2, dtype=torch.bfloat16), rnd(E, N, K, seed=2, scale=0.2, dtype=torch.bfloat16)
+    expert = torch.randint(0, 3, (2 * n,), generator=torch.Generator().manual_seed(3)) * (E // 3)
+    tiles = ops.moe_tiles(2 * n, E, 64)
+    rows, group, at = torch.full((tiles, 64), -1, dtype=torch.int32), torch.full((tiles,), -1, dtype=torch.int32), 0
+    for e in sorted(set(expert.tolist())):
+        for c in (expert == e).nonzero().flatten().int().split(64):
+            at += at == 4  # a tile nobody uses
+            rows[at, :len(c)], group[at], at = c, e, at + 1
+    scale = rnd(2 * n, seed=4)
+    x, want = a.float().repeat_interleave(2, 0), torch.empty(2 * n, N, device=DEV)
+    for e in sorted(set(expert.tolist())):
+        mine = (expert == e).nonzero().flatten().to(DEV)
+        u, v = x[mine] @ w0[e].float().t(), x[mine] @ w1[e].float().t()
+        want[mine] = u * torch.sigmoid(u) * v if form == "two" else u
+    out = torch.full((2 * n, N), float("nan"), dtype=torch.bfloat16, device=DEV)
+    ops.moe_product(out, a, w0, w1 if form == "two" else None, rows.to(DEV).flatten(), group.to(DEV), a_div=2, row_scale=scale)
+    close(out, want * scale[:, None], 4e-3, form)
+
+
 def reference_from_pages(case, kc, vc, bt, H, Hkv, hd, page, scale, window=0):
     """The plain formula over whatever pages a block table names (float64)."""
     out = torch.zeros(case["n"], H * hd, dtype=torch.float64)
