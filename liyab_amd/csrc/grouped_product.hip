@@ -615,7 +615,8 @@ extern "C" int liyab_grouped_product(const void* a, int64_t lda, int a_div, int 
         const dim3 skinny(n_tiles, (N + 15) / 16, rows_list ? 1 : n_groups);
         if (w1 != nullptr) grouped_skinny_kernel<2><<<skinny, 256, 0, stream>>>(p);
         else grouped_skinny_kernel<1><<<skinny, 256, 0, stream>>>(p);
-    } else if (matrix && K % 64 == 0 && (w1 == nullptr || gate == nullptr)) {
+    } else if (matrix && K % 64 == 0 && (w1 == nullptr || gate == nullptr) && static_cast<int64_t>(n_tiles) * grid.y * grid.z < (1 << 24)) {
+        // (its tiles lie along one dimension of the grid, which holds less than 2^32 threads: larger grids, of mostly spare tiles, go to the kernel below)
         // Short inner sizes are prologue and epilogue: narrow tiles and more workgroups a compute unit (heads of 128 -> 64 with a gate, 4,000 rows: 18.1 us in
         // tiles of 128 features, half of them outside, 9.5 in 64); long ones a wide tile (3,280 entries, 1,536 -> 768: 22.7 us in three stages, 25.7 in
         // two). Two matrices: two stages, three workgroups a unit (768 -> 2 x 1,536: 35.3 us, 41.5 in three; 600 entries 15.3 and 14.9).

@@ -850,6 +850,17 @@ def test_products_of_long_lists(ops, form, E, N, K):
     close(out, want * scale[:, None], 4e-3, form)
 
 
+def test_products_of_more_tiles_than_a_grid_dimension_holds(ops):
+    """17 million tiles of places and features, all but one column of them spare."""
+    n, tiles, N, K = 4, 1100, 1_000_000, 64
+    a, w = rnd(n, K, dtype=torch.bfloat16), rnd(1, N, K, seed=1, dtype=torch.bfloat16)
+    rows, group = torch.full((tiles * 64,), -1, dtype=torch.int32), torch.full((tiles,), -1, dtype=torch.int32)
+    rows[:n], group[0] = torch.arange(n), 0
+    out = torch.full((n, N), float("nan"), dtype=torch.bfloat16, device=DEV)
+    ops.moe_product(out, a, w, None, rows.to(DEV), group.to(DEV))
+    close(out, a.float() @ w[0].float().t(), 4e-3, "spare tiles")
+
+
 def reference_from_pages(case, kc, vc, bt, H, Hkv, hd, page, scale, window=0):
     """The plain formula over whatever pages a block table names (float64)."""
     out = torch.zeros(case["n"], H * hd, dtype=torch.float64)
