@@ -325,7 +325,11 @@ __device__ __forceinline__ void route_wave_softmax(float zl, int E, int top, int
     }
 }
 
-// Mode 0 for steps of more tokens: a wave a token, four a workgroup (a thread a token: 1,640 tokens, 2 of 8 experts, with their lists 11.8 -> 10.1 us; 5,000, 4 of 64 131 -> 43).
+// Mode 0 for steps of more tokens: a wave a token, four a workgroup, while there are few tokens for what a thread would have to scan one after the other (us with
+// the lists, a thread / a wave a token: 2 of 8 experts 1,640 tokens 11.8 / 10.0, 8,000 26.8 / 26.9, 20,000 55.8 / 59.0; 1 of 2 1,025 6.1 / 6.3, 16,000 30.9 / 34.0;
+// 2 of 2 2,000 11.2 / 11.1, 8,000 30.1 / 31.9; 2 of 16 16,000 50.6 / 50.5; 8 of 64 5,000 386 / 73).
+bool waves_route(int n, int E, int top) { return E > 1 && E <= kWave && n <= int64_t(512) * E * top; }
+
 __global__ void __launch_bounds__(256)
 moe_route_softmax_kernel(const float* __restrict__ logits, int64_t ld, int n, int E, int top, int* __restrict__ ids, float* __restrict__ weights) {
     const int t = blockIdx.x * 4 + threadIdx.x / kWave;
@@ -430,7 +434,7 @@ extern "C" int liyab_moe_route(const float* logits, int64_t ld, int n, int n_exp
     LIYAB_REQUIRE(n_listed >= 1 && n_listed <= n_experts && (extra == 0 || extra == 1) && (mode >= 2 || (n_listed == n_experts && extra == 0)) && ld >= n_experts + extra,
                   "moe_route: %d listed of %d outputs, %d entries for every token do not go with this mode", n_listed, n_experts, extra);
     if (n == 0) return 0;
-    if (mode == 0 && n_experts <= kWave && n_experts > 1) {
+    if (mode == 0 && waves_route(n, n_experts, top)) {
         moe_route_softmax_kernel<<<(n + 3) / 4, 256, 0, stream>>>(logits, ld, n, n_experts, top, ids, weights);
         return check_launch("moe_route");
     }
@@ -467,10 +471,11 @@ extern "C" int liyab_moe_route_align(const float* logits, int64_t ld, int n, int
     if (n == 0) return 0;
     const size_t smem = sizeof(int) * (mode >= 2 ? (1024 / kWave) * static_cast<size_t>(n_experts) + 4 : 2 * static_cast<size_t>(n_experts) + 1);  // (the scores; then the lists' counts)
     const RouteArgs ra{mode, n_groups, keep, correction, scale, n_listed, extra};
-    // More than a token a wave and few experts: a thread a token is faster (64 tokens, 2 of 8 experts 7.2 us against 10.6; 8 of 64 246 against 36).
+    // More than a token a wave and few experts: a thread a token is faster (64 tokens, 2 of 8 experts 7.2 us against 10.6; 8 of 64 246 against 36), and from some
+    // ten tokens on where it has little to scan (16 tokens, 1 of 2 3.3 against 3.7, 1 of 4 3.8 and 4.1, 2 of 4 5.0 and 4.8; 8 tokens, 1 of 2 3.3 and 3.3).
     const int64_t places = static_cast<int64_t>(max_tiles) * block;
     if (mode == 0 && n <= kWaveRouteTokens && n_experts > 1 && n_experts <= kSmallExperts && n * top <= kSmallEntries && places <= kSmallPlaces && max_tiles <= 1024 &&
-        (n <= 1024 / kWave || n_experts * top > 64)) {
+        (n <= 8 || (n <= 1024 / kWave && n_experts * top > 4) || n_experts * top > 64)) {
         moe_route_align_small_kernel<<<1, 1024, static_cast<size_t>(places) * sizeof(int), stream>>>(logits, ld, n, n_experts, top, ids, weights, block, rows_list, tile_group, max_tiles);
         return check_launch("moe_route_align");
     }

@@ -696,17 +696,31 @@ def test_command_line(models):
     assert set(turn2["phases_ms"]) == {"embed", "latent_attention", "routed_ffn", "lm_head"}
 
 
-@pytest.mark.parametrize("n,E,top", [(1, 2, 2), (4, 8, 2), (16, 64, 8), (17, 33, 3), (64, 64, 8), (16, 64, 16), (17, 8, 2), (4, 65, 3), (1030, 8, 2), (1030, 65, 1)])
+def test_choices_of_more_tokens_than_a_grid_of_waves_holds():
+    from liyab_amd.kernels import lib
+
+    n = (1 << 26) + 1
+    z = torch.randn(n, 2, device="cuda:0")
+    ids, w = torch.full((n,), -1, dtype=torch.int32, device="cuda:0"), torch.empty(n, device="cuda:0")
+    lib.call("liyab_moe_route", z.data_ptr(), 2, n, 2, 1, ids.data_ptr(), w.data_ptr(), 0, 1, 1, None, 1.0, 2, 0, torch.cuda.current_stream().cuda_stream)
+    assert torch.equal(ids, (z[:, 1] > z[:, 0]).int()) and bool((w == 1).all())
+
+
+@pytest.mark.parametrize("n,E,top", [(1, 2, 2), (4, 8, 2), (16, 64, 8), (17, 33, 3), (64, 64, 8), (16, 64, 16), (17, 8, 2), (4, 65, 3), (1030, 8, 2), (1030, 65, 1),
+                                     (8, 2, 1), (16, 2, 2), (9, 3, 2), (1025, 2, 1), (2048, 2, 2), (2049, 2, 2)])
 @pytest.mark.parametrize("block", [16, 64])
 def test_choices_and_lists_of_a_step(n, E, top, block):
-    """Each side of the sizes at which a wave chooses for a token and the lists stay in LDS, and of a step in two launches: ids (the lower number among equals, minus
-    infinity and NaN last, a NaN that comes first among what is left chosen), weights, and every entry once in a tile of its expert."""
+    """Each side of the sizes at which a wave chooses for a token and the lists stay in LDS, of a step in two launches, and of the tokens there up to which a wave
+    chooses: ids (the lower number among equals, minus infinity and NaN last, a NaN that comes first among what is left chosen), weights, and every entry once in a
+    tile of its expert."""
     from liyab_amd.kernels import ops
 
     g = torch.Generator().manual_seed(n + E)
     z = (torch.randn(n, E + 3, generator=g) * 2).round() / 2  # many equals
     z[torch.rand(z.shape, generator=g) < 0.1] = float("-inf")
     z[torch.rand(z.shape, generator=g) < 0.1] = -0.0
+    z[1::3, 0] = float("nan")  # first of all, and (below) first of what is left behind the first choice
+    z[2::3, 0], z[2::3, 1] = 5.0, float("nan")
     z[-1, E - 1] = float("nan")
     ids, w = torch.empty(n, top, dtype=torch.int32, device="cuda:0"), torch.empty(n, top, device="cuda:0")
     tiles = ops.moe_tiles(n * top, E, block)
