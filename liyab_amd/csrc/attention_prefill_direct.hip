@@ -6,14 +6,16 @@
 // What bounds it: a wave's 32 queries and 64 keys take 512 cycles of the matrix cores at 64 a head, and some 150 vector instructions (a
 // maximum, a multiply-add, an exponential, a sum and half a conversion a score), which overlap only across the waves of a SIMD. The kernel
 // that keeps a ring of keys in registers needs 312 of them: one wave a SIMD, its chain of products, maximum, exponentials and products laid bare.
-// Without the ring a wave of two streams fits 168, three a SIMD, and with one stream 113 to 180. A load's rows come from one page
+// Without the ring heads of 64 take 166 a wave of two streams and 112 to 123 of one, three and four waves a SIMD; 173 to 176 where a lane finds its own row, 215 to
+// 223 with scores to work on (two waves; one stream 122 to 162), and heads of 128 173 to 230 (two waves). A load's rows come from one page
 // where pages allow it, so that its address is a scalar: a lookup a lane cost 60 vector instructions a step. The sums are in the other
-// kernel's order (blocks of 32 keys, as many streams, the same merges): the same bits, compared over both kernels at 864 combinations of
-// sizes, pages, windows and scores.
-// us a layer, before and now: 1 x 8,001 tokens, 12 heads 172 -> 150 (0.66 PFLOP/s), 8 x 992 of 25 heads 69 -> 46, 2 x 1,024 of 12 heads 19.1 -> 15.9,
-// 4 x 192 behind 256 of 16 heads 11.8 -> 8.5, 8 x 1,000 of 12 heads of 128 82 -> 51; with a sink 4 x 410 of 12 heads 19.7 -> 10.1.
-// Measured and left: one stream of 64 keys (139, 45 and 15.1 us for the first three: other roundings), two stages or four in place of three,
-// an order of the tiles that deals the long ones out from both ends (no faster), two workgroups a compute unit in place of three (151).
+// kernel's order (blocks of 32 keys, as many streams, the same merges): the same bits.
+// us a layer, before and now: 1 x 8,001 tokens, 12 heads 166 -> 143 (0.69 PFLOP/s; in a pass, between the products, 180 -> 150), 8 x 992 of 25 heads 65 -> 44.4 (71 -> 48), 2 x 1,024 of 12 heads 19.2 -> 16.0,
+// 4 x 192 behind 256 of 16 heads 11.7 -> 8.4, 8 x 1,000 of 12 heads of 128 81 -> 52; with a sink 4 x 410 of 12 heads 18.9 -> 10.1.
+// The row table takes a word a page of the block tables' width, so that three workgroups of 128 queries share a compute unit's LDS up to 1,365 pages; with
+// 2,048 there are two (8 x 992 49.6, 1 x 8,001 138).
+// Measured and left: one stream of 64 keys (7, 2 and 5 % faster for the first three: other roundings), two stages or four in place of three,
+// an order of the tiles that deals the long ones out from both ends (no faster).
 #include "attention_prefill.h"
 #include "common.h"
 #include "launchers.h"

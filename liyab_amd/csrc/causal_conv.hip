@@ -25,8 +25,9 @@ __device__ __forceinline__ void conv_store4(bf16_t* dst, const conv_f32x4& v) {
 
 // VEC: four channels a thread; MAXT: the most taps this instance takes (its earlier inputs are loaded together); FOUR: four taps, a channel's
 // weights in one load of 16 bytes, asked for with the inputs. What bounds it is the trips to memory, one after the other: the token's request, its history's
-// place, inputs and weights; a weight loaded under the choice whether its input exists is one more a tap (1,640 rows of 768, four taps, 12.7 -> 4.5 us; 4 rows
-// 4.0 -> 2.8. Other numbers of taps ask for theirs one by one: all of them ahead, as many loads as values, were slower, two taps 8.0 -> 12.4, eight 31 -> 44).
+// place, inputs and weights; a weight loaded under the choice whether its input exists is one more a tap (1,640 rows of 768, four taps, 13.0 -> 4.9 us; 4 rows
+// 4.0 -> 2.8). Other numbers of taps ask for theirs one by one: all of them ahead, as many loads as values, were slower, two taps 8.0 -> 12.4, eight 31 -> 44;
+// two or eight in loads of 8 or 16 bytes were not tried.
 template <typename T, bool VEC, int MAXT, bool FOUR = false>
 __global__ void __launch_bounds__(256)
 causal_conv_kernel(T* __restrict__ out, T* __restrict__ cast_out, const float* __restrict__ x, const float* __restrict__ w, int taps,

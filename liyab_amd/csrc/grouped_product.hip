@@ -214,9 +214,9 @@ grouped_mfma_kernel(GroupedParams p) {
 // What bounds it: the operands, at what a compute unit takes in (24 KiB a stage of 64 k for 1 MFLOP), and with them which L2 they come
 // from. A group's rows stand side by side in the list, so an XCD takes a stretch of the tiles in use: its rows of `a` and a column of
 // weights at a time, for all of its tiles in turn, stay in its L2, where tiles dealt out over the XCDs had every one of them read every expert's weights.
-// The gates' logits and a row's scale and place are asked for before the walk: a load under a choice in the epilogue is waited for there (41 us of
-// which for 35). us before (the kernel above) and now, the same bits: 3,280 entries of 8 experts, 768 -> 2 x 1,536 56 -> 35, 1,536 -> 768 32 -> 23, 768 -> 2 x 768
-// 31 -> 18.5; 10,000 entries 122 -> 97 and 95 -> 47; heads, 1,640 rows of 12, 128 -> 64 with a gate 10.6 -> 7.0, 64 -> 128 8.5 -> 5.6.
+// The gates' logits and a row's scale and place are asked for before the walk: a load under a choice in the epilogue is waited for there (the first
+// of the products below took 41 us so). us before (the kernel above) and now, the same bits: 3,280 entries of 8 experts, 768 -> 2 x 1,536 54 -> 33, 1,536 -> 768
+// 32 -> 21, 768 -> 2 x 768 30 -> 17.2; 10,000 entries 102 -> 83 and 87 -> 45; heads, 1,640 rows of 12, 128 -> 64 with a gate 10.5 -> 6.8, 64 -> 128 8.3 -> 5.5.
 typedef __attribute__((ext_vector_type(4))) float gp_f32x4;
 typedef __attribute__((address_space(3))) void* gp_lds_ptr;
 
@@ -618,7 +618,7 @@ extern "C" int liyab_grouped_product(const void* a, int64_t lda, int a_div, int 
     } else if (matrix && K % 64 == 0 && (w1 == nullptr || gate == nullptr) && static_cast<int64_t>(n_tiles) * grid.y * grid.z < (1 << 24)) {
         // (its tiles lie along one dimension of the grid, which holds less than 2^32 threads: larger grids, of mostly spare tiles, go to the kernel below)
         // Short inner sizes are prologue and epilogue: narrow tiles and more workgroups a compute unit (heads of 128 -> 64 with a gate, 4,000 rows: 18.1 us in
-        // tiles of 128 features, half of them outside, 9.5 in 64); long ones a wide tile (3,280 entries, 1,536 -> 768: 22.7 us in three stages, 25.7 in
+        // tiles of 128 features, half of them outside, 9.1 in 64); long ones a wide tile (3,280 entries, 1,536 -> 768: 22.7 us in three stages, 25.7 in
         // two). Two matrices: two stages, three workgroups a unit (768 -> 2 x 1,536: 35.3 us, 41.5 in three; 600 entries 15.3 and 14.9).
         const int groups = rows_list ? 1 : n_groups;
         if (w1 != nullptr) return launch_grouped_tile<2, 128, 2>(p, n_tiles, groups, stream);

@@ -905,7 +905,9 @@ def attention_prefill(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor,
         _lib.call("liyab_attention_prefill", *args, _stream())
 
 
-PREFILL_KSPLIT4_WORK = 256  # tiles x heads up to which four waves share a tile of 64 queries' keys
+# tiles x heads up to which four waves share a tile of 64 queries' keys (heads of 64, two / four waves: 192 workgroups over 256 keys 7.2 / 7.5 us, 132 over 700
+# 11.4 / 10.5, 400 over 1,000 16.3 / 14.4, 768 17.1 / 20.7)
+PREFILL_KSPLIT4_WORK = 256
 
 
 def prefill_takes(hd: int) -> bool:
@@ -915,16 +917,17 @@ def prefill_takes(hd: int) -> bool:
 def decode_plan(n_tokens: int, n_head: int, context_bucket: int):
     """(splits of the keys, waves per workgroup) for tokens whose attention the kernel finishes
     itself (several splits: plus the merge kernel). `context_bucket`: the most keys a token has,
-    rounded up. From measurements at 12 to 32 heads of 64 and 128, 1 to 42 tokens and 300 to
-    8,000 keys (us, attention and merge). Uncut (4 / 8 / 16 waves, longest of contexts from a quarter of it on): 8 waves
-    (108 pairs at 1,000 keys 10.0 / 9.1 / 9.8, at 2,000 16.1 / 13.4 / 13.6; 252 pairs at 1,000 keys 11.5 / 12.0 / 12.5, at 2,000 21.0 /
-    21.8 / 21.2: 4 waves round otherwise for 4 % there), 4 from 512 pairs on and up to 256 keys, 16 with few pairs of 4,000 keys and more
-    (108 pairs at 4,000 29.6 / 30.8 / 27.6, 252 at 8,000 70.0 / 71.5 / 68.1). With fewer pairs than would fill the chip the keys
+    rounded up. Measured with caches not read before, the contexts from a quarter of the longest on, 12 heads of 64 (us, attention
+    and merge, uncut on 4 / 8 / 16 waves, and in 2 splits of 4): 108 pairs at 300 keys 6.2 / 6.8 / 9.1, 8.0, at 1,000 10.8 / 11.6 / 11.9,
+    10.4, at 2,000 17.4 / 17.8 / 17.0, 14.3, at 4,000 30.9 / 31.5 / 28.5, 21.7; 252 at 1,000 12.8 / 13.9 / 13.7, 14.9, at 8,000 70.9 /
+    73.0 / 71.2, 72.7; 480 at 1,000 19.5 / 20.3 / 25.0, 22.1; 768 27.8 / 30.1 / 37.2, 30.8. So: 4 waves a pair with many pairs and with
+    short contexts. In between the rule is that of the walk before four waves asked for their next trip's keys ahead, when 8 waves won there: they
+    cost 2 to 8 % now, 16 with few pairs of 4,000 keys gain 8, and two splits would gain a fifth to a quarter with a hundred pairs of 2,000 keys and
+    more; other waves and splits add in another order, and the lines have stayed. With fewer pairs than would fill the chip the keys
     are cut across workgroups of 4 waves, into 4, 8 or 16 splits of 128 keys or more, while
     pairs x splits stay within the chip's 256 compute units (32 pairs of 128 dimensions at
-    1,000 / 2,000 / 4,000 keys: 7.5 / 10.6 / 18.4 in 8 splits against 11.8 / 19.1 / 33.1 uncut
-    on 16 waves; 12 pairs of 64: 6.9 / 7.8 / 9.7 against 8.7 / 11.8 / 18.6). Two splits never
-    beat 8 waves uncut."""
+    1,000 / 2,000 / 4,000 keys: 9.5 / 12.3 / 18.3 in 8 splits against 15.8 / 25.9 / 45.3 uncut
+    on 16 waves; 12 pairs of 64: 7.4 / 8.1 / 10.1 against 9.0 / 12.4 / 23.9)."""
     pairs = max(1, n_tokens * n_head)
     if pairs >= 512 or context_bucket <= 256:
         return 1, 4
@@ -932,8 +935,8 @@ def decode_plan(n_tokens: int, n_head: int, context_bucket: int):
     while splits < 16 and pairs * splits * 2 <= 256 and context_bucket // (splits * 2) >= 128:
         splits *= 2
     if splits >= 4:
-        # (splits of 1,024 keys and more on 8 waves: 12 pairs at 30,000 keys in 16 splits 26.7 us on
-        # 4 waves, 22.4 on 8; 32 pairs of 128 dimensions 92.6 and 89.1)
+        # (splits of 1,024 keys and more on 8 waves, from before four asked ahead: 12 pairs at 30,000 keys in 16 splits 26.7 us on
+        # 4 waves and 22.4 on 8 then, 25.6 and 27.0 now; 32 pairs of 128 dimensions 92.6 and 89.1, now 93.6 and 94.7)
         return splits, (8 if context_bucket // splits >= 1024 else 4)
     return 1, (16 if context_bucket >= 4096 and pairs < 256 else 8)
 
@@ -951,9 +954,9 @@ def decode_split_plan(n_tokens: int, n_head: int, context_bucket: int):
     while splits < most and context_bucket // (2 * splits) >= 128:
         splits *= 2
     # very long contexts of one or two requests: 8 splits of 4 waves leave most of the chip idle and
-    # each walks thousands of keys; 16 waves a split walk them four times as fast (us, 12 pairs of 64
-    # at 8,000 / 16,000 / 30,000 keys: 14.5 / 25.1 / 41.2 on 4 waves, 11.7 / 17.0 / 23.6 on 16; from
-    # 48 pairs on 4 waves win)
+    # each walks thousands of keys; 16 waves a split have more of them in flight (us, 12 pairs of 64
+    # at 8,000 / 16,000 / 30,000 keys: 14.5 / 25.1 / 41.2 on 4 waves, 11.7 / 17.0 / 23.6 on 16; since four waves ask for
+    # their next trip's keys ahead, caches not read before, 11.0 / 18.2 / 29.7 and 11.8 / 18.1 / 29.3; from 48 pairs on 4 waves win)
     return splits, (16 if pairs <= 32 and context_bucket // splits >= 1024 else 4)
 
 
@@ -1054,8 +1057,12 @@ def attention(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor, v_cache
         if plan.n_tiles:
             # with fewer workgroups than compute units, two waves share each query group's keys:
             # the longest tile's walk over its keys is then the kernel's critical path, and halves
+            # (heads of 64, us a layer with one / two / four waves a query group: 1 x 700 tokens of 12 heads in tiles of 64 17.1 / 11.4 / 10.5, 2 x 1,000
+            # in tiles of 128 20.1 / 16.6; 3 x 1,000 of 16 20.9 / 19.1, 4 x 1,000 21.4 / 21.9, 8 x 992 of 25 46.7 / 66.7)
             work = plan.n_tiles * n_head
-            # (heads past 96: two waves a query group at every size, 185 against 217 us for 16 x 1,024 tokens of 12 heads of 128)
+            # (heads past 96: two waves a query group at every size, from when heads of 128 kept their keys in registers, one wave a SIMD: 185 against
+            # 217 us for 16 x 1,024 tokens of 12 heads. Straight into LDS one wave a group is the faster past some 500 workgroups, 80 against 101 for
+            # these, 34.5 and 34.0 for 4 x 1,000 of 16, 29.8 and 24.5 for 2 x 1,000 of 12; the line has stayed, since the other form adds in another order)
             ksplit = (4 if plan.tile == 64 and hd <= 64 and work <= PREFILL_KSPLIT4_WORK else 2) if work <= 256 or hd > 96 else 1
             attention_prefill(out, q, k_cache, v_cache, block_tables, plan.work, plan.n_tiles, n_head=n_head,
                               scale=scale, window=window, tile=plan.tile, ksplit=ksplit, **scored)
@@ -1236,7 +1243,7 @@ def heads_product(out: torch.Tensor, a: torch.Tensor, w: torch.Tensor, gate: Opt
         if tuple(gate.shape) != (n, H * N):
             raise KernelError(f"heads_product: the gate must be [{n}, {H * N}]")
     # few rows: tiles of 16 rows x 16 features, so that some hundred workgroups share the heads' matrices (64 rows of 12
-    # heads, 128 -> 64: 10 us in 12 tiles of 64 x 64)
+    # heads, 128 -> 64 with a gate: 3.0 us, 5.5 in tiles of 64 x 64; 128 rows 3.3 and 5.7, 256 3.6 and 5.7: the line is from dearer tiles of 16)
     block = SKINNY_ROWS if (n <= 128 and a.dtype == torch.bfloat16 and K % 8 == 0 and lda % 8 == 0 and a.data_ptr() % 16 == 0
                             and w.data_ptr() % 16 == 0) else GROUPED_ROWS
     _lib.call("liyab_grouped_product", a.data_ptr(), lda, 1, K, w.data_ptr(), None, dtype_code(a.dtype), out.data_ptr(),
@@ -1258,7 +1265,9 @@ def moe_block(n_entries: int, n_experts: int, dtype: torch.dtype, *inner_sizes: 
     rows or fewer on average (the products are then streams of the chosen experts' weights, and tiles of 16
     rows x 16 features make some hundred workgroups pull on them where tiles of 64 x 64 make a few dozen:
     one token of 2 x 1,536 features over 768, 16.4 -> 6 us), 64 beyond; the small tiles are for bfloat16
-    operands whose inner sizes are multiples of 8."""
+    operands whose inner sizes are multiples of 8. The line is from the larger tiles through registers; against those straight into LDS (both products, us
+    in tiles of 16 / 64, 8 experts of 768 <-> 1,536) 8 rows an expert 18.3 / 28.6, 16 27.0 / 28.8, 24 30.5 / 28.8, 32 38.7 / 29.0; 64 experts of 512 <-> 256
+    15.9 / 19.7, 20.8 / 19.5, 28.3 / 19.6, 32.3 / 19.6: they cross at some 16 rows."""
     few = n_entries <= 32 * n_experts and dtype == torch.bfloat16 and all(k % 8 == 0 for k in inner_sizes)
     return SKINNY_ROWS if few else GROUPED_ROWS
 

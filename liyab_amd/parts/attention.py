@@ -20,7 +20,9 @@ from .registry import build_part, register_mixer
 
 ATTN_TILE = 128  # queries of one request that the prefill attention kernel takes together (64 or 128)
 ATTN_TILE_FEW = 64  # the same for steps whose long portions hold few tokens: more, shorter tiles
-ATTN_FEW_TOKENS = 1024  # up to this many tokens in long portions (measured: a step of 256 tokens of one prompt 840 -> 806 us)
+# up to this many tokens in long portions (a step of 256 tokens of one prompt 840 -> 806 us; the kernel alone in tiles of 64 / 128, 12 heads of 64: 4 x 256
+# tokens 7.5 / 8.6, 2 x 1,000 13.7 / 16.6, 4 x 1,000 17.0 / 19.2, 16 x 1,024 50 / 46)
+ATTN_FEW_TOKENS = 1024
 DECODE_Q_LEN = 8  # requests that bring at most this many tokens are attended token by token
 
 
