@@ -414,6 +414,13 @@ inline bool heads_first_pays(int n, int n_head, int n_kv_head, int hd, size_t el
     return heads * keys * hd * 2 * static_cast<int64_t>(elt) <= (4 << 20);
 }
 
+// (made here, so that the merges' code lies ahead of the walks' some 1.5 MB: with it behind them a batch-invariant step of 8 tokens, which merges behind each of 12
+// walks, took 581.8 us, so 578.9, the instructions being the same)
+template __global__ void attention_merge_kernel<float>(float* __restrict__, int64_t, const int* __restrict__, const float* __restrict__, int, int, int,
+                                                       const float* __restrict__);
+template __global__ void attention_merge_kernel<bf16_t>(bf16_t* __restrict__, int64_t, const int* __restrict__, const float* __restrict__, int, int, int,
+                                                        const float* __restrict__);
+
 // Whether four waves ask for the next trip's keys ahead (bfloat16). The pieces of two trips take 128 to 143 registers, three or four workgroups a
 // compute unit, where one trip takes 63 to 90, five to seven: with small heads or scores to work on, whose arithmetic wants the waves, it pays until those three
 // are placed (us ahead / not, 12 heads over 100 to 1,000 keys, caches not read before. Heads of 16: 64 tokens 9.9 / 10.4, 72 11.8 / 11.0, 130 18.2 / 16.9,
