@@ -289,59 +289,177 @@ gemm_tiled_f32_kernel(float* __restrict__ out, int64_t ldo, const float* __restr
 
 // Few rows, or too few tiles to go round: a workgroup takes 16 rows and NB output features, its waves the chunks of K in
 // turn, so that a product of few output elements still spreads over the chip. A wave brings its chunk of the rows
-// of `w` and `a` through registers into LDS of its own (256 bytes a row and load, the next chunk in flight
+// of `w` and `a` through registers into LDS of its own (256 bytes a row and load, the next two chunks in flight
 // meanwhile) and runs the chunk's chains on the matrix core, 16 x 16 x 4 an instruction; after each round of chunks the
 // threads add the round's sums in chunk order. Few features a workgroup where N is small: the weights then stream
 // through enough compute units (features of the block past NB repeat the last one). Reading operands from LDS set the
-// pace when lanes ran the chains themselves (20 to 80 reads of 16 bytes a chunk; here 32 of 4).
+// pace when lanes ran the chains themselves (20 to 80 reads of 16 bytes a chunk; here 32 of 4). What bounds it is a chain: a first trip to
+// memory, a round's products and sums, the epilogue's own reads, so these are asked for first of all.
+// The rows may also be made here (SRC), each workgroup its own 16: the LayerNorm of 32-bit rows, or attention's splits merged, with the
+// operations of layernorm.hip and of attention_decode.hip's merge, so that the bits are those of their own kernels, whose links in
+// a step's chain (3.5 us each) are saved; the weights are on their way meanwhile, and the rows stay in LDS for all chunks.
 constexpr int kChunkRows = 16;  // rows a workgroup
+enum : int { kSrcRows = 0, kSrcNorm = 1, kSrcSplits = 2 };
 
-template <int NB, int WAVES, int EPI, bool VEC>
+// What the rows are made of where they are made here: x [M, K] and its norm, or partials [M][n_head][n_splits][hd + 4].
+struct MadeRows {
+    const float* x;
+    const float* weight;
+    const float* bias;
+    float eps;
+    int n_splits, n_head, hd;
+};
+
+// FORM: pieces of 4 a lane of a row (norm), splits at most (splits); not read for plain rows.
+template <int NB, int WAVES, int EPI, bool VEC, int SRC, int FORM>
 __global__ void __launch_bounds__(64 * WAVES)
 gemm_chunks_f32_kernel(float* __restrict__ out, int64_t ldo, const float* __restrict__ a, int64_t lda,
                        const float* __restrict__ w, const float* __restrict__ bias, float* __restrict__ residual,
-                       int64_t ldr, int M_all, int N, int K, EpiParams qkv) {
+                       int64_t ldr, int M_all, int N, int K, EpiParams qkv, MadeRows made) {
     const int row0 = blockIdx.y * kChunkRows, M = min(kChunkRows, M_all - row0);
     a += static_cast<int64_t>(row0) * lda;
     constexpr int LD = kChunk + 4;  // (lanes read words 4 banks apart, their neighbours in k beside them: no collisions)
-    constexpr int W_LOADS = NB / 4, A_LOADS = kChunkRows / 4;  // a load covers 4 rows: 16 lanes a row, 16 bytes a lane
+    constexpr int W_LOADS = NB / 4, A_LOADS = SRC == kSrcRows ? kChunkRows / 4 : 0;  // a load covers 4 rows: 16 lanes a row, 16 bytes a lane
     static_assert(NB % 4 == 0 && NB <= 16 && kChunkRows * NB <= 64 * WAVES, "one block of features, a thread an output element");
+    static_assert(SRC == kSrcRows || VEC, "rows made here are whole and aligned");
     __shared__ __attribute__((aligned(16))) float Wt[WAVES][NB][LD];
-    __shared__ __attribute__((aligned(16))) float At[WAVES][kChunkRows][LD];
+    __shared__ __attribute__((aligned(16))) float At[SRC == kSrcRows ? WAVES : 1][kChunkRows][LD];
     __shared__ float P[2][WAVES][kChunkRows][NB];  // rounds take turns, so that one barrier a round is enough
+    extern __shared__ __attribute__((aligned(16))) float made_rows[];  // [M][K + 4]
     const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64;
     const int n0 = blockIdx.x * NB;
-    const int chunks = (K + kChunk - 1) / kChunk;
+    const int chunks = (K + kChunk - 1) / kChunk, ldx = K + 4;
     const int lrow = lane / 16, lk = (lane % 16) * 4;  // as a loader
     const int li = lane % 16, g = lane / 16;           // in the matrix core's operands: row (or feature) and k
-    f32x4_t wreg[W_LOADS], areg[A_LOADS];
-    auto fetch = [&](int c) {
+    f32x4_t wreg[2][W_LOADS], areg[2][A_LOADS + 1];
+    auto fetch = [&](int c, int buf) {
         const int k = c * kChunk + lk;
 #pragma unroll
-        for (int i = 0; i < W_LOADS; ++i) wreg[i] = load4_f32<VEC>(w + static_cast<int64_t>(min(n0 + 4 * i + lrow, N - 1)) * K, k, K);
+        for (int i = 0; i < W_LOADS; ++i) wreg[buf][i] = load4_f32<VEC>(w + static_cast<int64_t>(min(n0 + 4 * i + lrow, N - 1)) * K, k, K);
 #pragma unroll
         for (int i = 0; i < A_LOADS; ++i)
-            if (4 * i < M) areg[i] = load4_f32<VEC>(a + static_cast<int64_t>(min(4 * i + lrow, M - 1)) * lda, k, K);  // (the same for every lane)
+            if (4 * i < M) areg[buf][i] = load4_f32<VEC>(a + static_cast<int64_t>(min(4 * i + lrow, M - 1)) * lda, k, K);  // (the same for every lane)
     };
     float tot = 0.0f;  // of output element (tid / NB, tid % NB), for tid < 16 * NB
     float* place = nullptr;  // found while the first operands are on their way
-    if constexpr (EPI == kEpiQkvPaged)
-        if (tid < kChunkRows * NB && tid / NB < M && n0 + tid % NB < N) place = qkv_place(qkv, row0 + tid / NB, n0 + tid % NB);
+    const int n = n0 + tid % NB, m = row0 + tid / NB;
+    const bool mine = tid < kChunkRows * NB && tid / NB < M && n < N;
+    float own_bias = 0.0f, own_res = 0.0f;
+    auto ask = [&]() {  // the weights (and plain rows), then what the epilogue reads
+        if (wave < chunks) fetch(wave, 0);
+        if (wave + WAVES < chunks) fetch(wave + WAVES, 1);
+        if (mine) {
+            if (bias != nullptr) own_bias = bias[n];
+            if constexpr (EPI == kEpiResidual) own_res = residual[static_cast<int64_t>(m) * ldr + n];
+            if constexpr (EPI == kEpiQkvPaged) place = qkv_place(qkv, m, n);
+        }
+    };
+    if constexpr (SRC == kSrcRows) {
+        ask();
+    } else if constexpr (SRC == kSrcNorm) {
+        const int nv = K / 4;
+        const f32x4_t zero = {0.0f, 0.0f, 0.0f, 0.0f}, one = {1.0f, 1.0f, 1.0f, 1.0f};
+        auto norm_row = [&](int r, auto&& between) {
+            f32x4_t v[FORM], gw[FORM], gb[FORM];
+#pragma unroll
+            for (int j = 0; j < FORM; ++j) {
+                const int at = min(lane + kWave * j, nv - 1);  // past the row: its last piece again, unused
+                v[j] = reinterpret_cast<const f32x4_t*>(made.x + static_cast<int64_t>(row0 + r) * K)[at];
+                gw[j] = made.weight != nullptr ? reinterpret_cast<const f32x4_t*>(made.weight)[at] : one;
+                gb[j] = made.bias != nullptr ? reinterpret_cast<const f32x4_t*>(made.bias)[at] : zero;
+            }
+            between();
+            __builtin_amdgcn_sched_barrier(0);  // the row's loads ahead of the weights': a wait for the row is then no wait for these
+            float s = 0.0f;
+#pragma unroll
+            for (int j = 0; j < FORM; ++j)
+                if (lane + kWave * j < nv) s += (v[j][0] + v[j][1]) + (v[j][2] + v[j][3]);
+            const float mean = wave_sum(s) / static_cast<float>(K);
+            float ss = 0.0f;
+#pragma unroll
+            for (int j = 0; j < FORM; ++j)
+                if (lane + kWave * j < nv) {
+                    const f32x4_t dev = v[j] - mean;
+                    ss += (dev[0] * dev[0] + dev[1] * dev[1]) + (dev[2] * dev[2] + dev[3] * dev[3]);
+                }
+            const float scale = 1.0f / sqrtf(wave_sum(ss) / static_cast<float>(K) + made.eps);
+#pragma unroll
+            for (int j = 0; j < FORM; ++j)
+                if (lane + kWave * j < nv) *reinterpret_cast<f32x4_t*>(made_rows + r * ldx + 4 * (lane + kWave * j)) = (v[j] - mean) * scale * gw[j] + gb[j];
+        };
+        if (wave < M) norm_row(wave, ask);
+        else ask();
+        for (int r = wave + WAVES; r < M; r += WAVES) norm_row(r, []() {});
+        lds_barrier();  // the weights may still be on their way
+    } else {
+        // four consecutive k of a token a thread and item
+        constexpr int ITEMS = 2;
+        const int S = made.n_splits, hd4 = made.hd + 4, per = K / 4, items = M * per;
+        struct Item {
+            f32x4_t acc[FORM];
+            f32x2_t ml[FORM];
+            int place;
+        } it[ITEMS];
+        auto get = [&](int first) {
+#pragma unroll
+            for (int i = 0; i < ITEMS; ++i) {
+                const int at = first + i * 64 * WAVES, ac = min(at, items - 1);  // past the end: the last one again, dropped
+                const int r = ac / per, k = (ac - r * per) * 4, head = k / made.hd;
+                const float* p = made.x + (static_cast<int64_t>(row0 + r) * made.n_head + head) * S * hd4;
+                it[i].place = at < items ? r * ldx + k : -1;
+#pragma unroll
+                for (int z = 0; z < FORM; ++z) it[i].ml[z] = *reinterpret_cast<const f32x2_t*>(p + min(z, S - 1) * hd4 + made.hd);
+#pragma unroll
+                for (int z = 0; z < FORM; ++z) it[i].acc[z] = *reinterpret_cast<const f32x4_t*>(p + min(z, S - 1) * hd4 + k - head * made.hd);
+            }
+        };
+        auto merge = [&]() {
+#pragma unroll
+            for (int i = 0; i < ITEMS; ++i) {
+                float mx = -INFINITY;
+#pragma unroll
+                for (int z = 0; z < FORM; ++z)
+                    if (z < S) mx = fmaxf(mx, it[i].ml[z][0]);
+                float sum = 0.0f;
+                f32x4_t o = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                for (int z = 0; z < FORM; ++z) {
+                    if (z >= S || it[i].ml[z][0] == -INFINITY) continue;
+                    const float f = expf(it[i].ml[z][0] - mx);
+                    sum = fmaf(f, it[i].ml[z][1], sum);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) o[e] = fmaf(f, it[i].acc[z][e], o[e]);
+                }
+                if (it[i].place >= 0) *reinterpret_cast<f32x4_t*>(made_rows + it[i].place) = f32x4_t{o[0] / sum, o[1] / sum, o[2] / sum, o[3] / sum};
+            }
+        };
+        get(tid);
+        ask();
+        __builtin_amdgcn_sched_barrier(0);
+        merge();
+        for (int at = tid + ITEMS * 64 * WAVES; at < items; at += ITEMS * 64 * WAVES) {
+            get(at);
+            merge();
+        }
+        lds_barrier();
+    }
     const float* wl = &Wt[wave][min(li, NB - 1)][g];
-    const float* al = &At[wave][min(li, (M + 3) / 4 * 4 - 1)][g];  // (rows past M: some row that was written; not stored)
-    if (wave < chunks) fetch(wave);
-    for (int c0 = 0, turn = 0; c0 < chunks; c0 += WAVES, turn ^= 1) {
+    const float* al = SRC == kSrcRows ? &At[SRC == kSrcRows ? wave : 0][min(li, (M + 3) / 4 * 4 - 1)][g]  // (rows past M: some row that was written; not stored)
+                                      : made_rows + min(li, M - 1) * ldx + g;
+    auto round = [&](int c0, auto buffer) {
+        constexpr int turn = decltype(buffer)::value;
         const int c = c0 + wave;
         if (c < chunks) {
 #pragma unroll
-            for (int i = 0; i < W_LOADS; ++i) *reinterpret_cast<f32x4_t*>(&Wt[wave][4 * i + lrow][lk]) = within_k(wreg[i], c * kChunk + lk, K);
+            for (int i = 0; i < W_LOADS; ++i) *reinterpret_cast<f32x4_t*>(&Wt[wave][4 * i + lrow][lk]) = within_k(wreg[turn][i], c * kChunk + lk, K);
 #pragma unroll
             for (int i = 0; i < A_LOADS; ++i)
-                if (4 * i < M) *reinterpret_cast<f32x4_t*>(&At[wave][4 * i + lrow][lk]) = within_k(areg[i], c * kChunk + lk, K);
-            if (c + WAVES < chunks) fetch(c + WAVES);
+                if (4 * i < M) *reinterpret_cast<f32x4_t*>(&At[wave][4 * i + lrow][lk]) = within_k(areg[turn][i], c * kChunk + lk, K);
+            if (c + 2 * WAVES < chunks) fetch(c + 2 * WAVES, turn);
+            const float* ac = SRC == kSrcRows ? al : al + c * kChunk;
             f32x4_t acc{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-            for (int k = 0; k < kChunk; k += 4) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(wl[k], al[k], acc, 0, 0, 0);
+            for (int k = 0; k < kChunk; k += 4) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(wl[k], ac[k], acc, 0, 0, 0);
 #pragma unroll
             for (int r = 0; r < 4; ++r)  // a lane holds row li and the features 4 g + r
                 if (4 * g + r < NB) P[turn][wave][li][4 * g + r] = acc[r];
@@ -351,12 +469,14 @@ gemm_chunks_f32_kernel(float* __restrict__ out, int64_t ldo, const float* __rest
             const int live = min(WAVES, chunks - c0);
             for (int v = 0; v < live; ++v) tot += P[turn][v][tid / NB][tid % NB];
         }
+    };
+    for (int c0 = 0; c0 < chunks; c0 += 2 * WAVES) {
+        round(c0, std::integral_constant<int, 0>{});
+        if (c0 + WAVES < chunks) round(c0 + WAVES, std::integral_constant<int, 1>{});
     }
-    const int n = n0 + tid % NB;
-    if (tid >= kChunkRows * NB || tid / NB >= M || n >= N) return;
-    const int m = row0 + tid / NB;
-    const float v = finish_f32<EPI>(tot, bias != nullptr, bias != nullptr ? bias[n] : 0.0f);
-    if constexpr (EPI == kEpiResidual) residual[static_cast<int64_t>(m) * ldr + n] += v;
+    if (!mine) return;
+    const float v = finish_f32<EPI>(tot, bias != nullptr, own_bias);
+    if constexpr (EPI == kEpiResidual) residual[static_cast<int64_t>(m) * ldr + n] = own_res + v;
     else if constexpr (EPI == kEpiQkvPaged) { if (place != nullptr) *place = v; }
     else out[static_cast<int64_t>(m) * ldo + n] = v;
 }
@@ -376,9 +496,38 @@ int launch_tiled_f32(float* out, int64_t ldo, const float* a, int64_t lda, const
 template <int NB, int WAVES, int EPI, bool VEC>
 int launch_chunks_f32(float* out, int64_t ldo, const float* a, int64_t lda, const float* w, const float* bias, float* residual, int64_t ldr, int M,
                       int N, int K, const EpiParams& qkv, hipStream_t stream) {
-    gemm_chunks_f32_kernel<NB, WAVES, EPI, VEC><<<dim3((N + NB - 1) / NB, (M + kChunkRows - 1) / kChunkRows), 64 * WAVES, 0, stream>>>(
-        out, ldo, a, lda, w, bias, residual, ldr, M, N, K, qkv);
+    gemm_chunks_f32_kernel<NB, WAVES, EPI, VEC, kSrcRows, 0><<<dim3((N + NB - 1) / NB, (M + kChunkRows - 1) / kChunkRows), 64 * WAVES, 0, stream>>>(
+        out, ldo, a, lda, w, bias, residual, ldr, M, N, K, qkv, MadeRows{});
     return check_launch("gemm_chunks_f32");
+}
+
+template <int NB, int WAVES, int EPI, int SRC, int FORM>
+int launch_made_as(const MadeRows& made, const float* w, int M, int N, int K, const EpiParams& epi, hipStream_t stream) {
+    const size_t rows = static_cast<size_t>(M < kChunkRows ? M : kChunkRows) * (K + 4) * sizeof(float);
+    constexpr size_t fixed = (WAVES * NB + kChunkRows) * (kChunk + 4) * sizeof(float) + 2 * WAVES * kChunkRows * NB * sizeof(float);
+    LIYAB_REQUIRE(rows + fixed <= 160 * 1024, "gemm_made_f32: rows of %d need %zu bytes of LDS", K, rows + fixed);
+    auto kern = gemm_chunks_f32_kernel<NB, WAVES, EPI, true, SRC, FORM>;
+    static bool ready = false;  // once per instantiation, outside any stream capture's first use
+    if (!ready) {
+        hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(160 * 1024 - fixed));
+        ready = true;
+    }
+    kern<<<dim3((N + NB - 1) / NB, (M + kChunkRows - 1) / kChunkRows), 64 * WAVES, rows, stream>>>(
+        static_cast<float*>(epi.out), epi.ldo, nullptr, 0, w, epi.bias, epi.residual, epi.ldr, M, N, K, epi, made);
+    return check_launch("gemm_made_f32");
+}
+template <int EPI, int SRC, int FORM>
+int launch_made(const MadeRows& made, const float* w, int M, int N, int K, const EpiParams& epi, hipStream_t stream) {
+    const int64_t strips = static_cast<int64_t>(N) * ((M + kChunkRows - 1) / kChunkRows);  // (as for plain rows)
+    if (strips <= 1024) return launch_made_as<4, 8, EPI, SRC, FORM>(made, w, M, N, K, epi, stream);
+    if (strips <= 2048) return launch_made_as<8, 8, EPI, SRC, FORM>(made, w, M, N, K, epi, stream);
+    if (strips <= 16 * 400) return launch_made_as<16, 8, EPI, SRC, FORM>(made, w, M, N, K, epi, stream);
+    return launch_made_as<16, 4, EPI, SRC, FORM>(made, w, M, N, K, epi, stream);
+}
+template <int EPI>
+int launch_norm_f32(const MadeRows& made, const float* w, int M, int N, int K, const EpiParams& epi, hipStream_t stream) {
+    if (K <= 768) return launch_made<EPI, kSrcNorm, 3>(made, w, M, N, K, epi, stream);
+    return launch_made<EPI, kSrcNorm, 8>(made, w, M, N, K, epi, stream);
 }
 
 template <int EPI, bool VEC>
@@ -476,4 +625,43 @@ extern "C" int liyab_gemm_f32_qkv(const float* a, int64_t lda, const float* w, i
     if (int rc = check_epilogue(*epi, M, N)) return rc;
     if (M == 0) return 0;
     return launch_f32<kEpiQkvPaged>(static_cast<float*>(epi->out), epi->ldo, a, lda, w, epi->bias, nullptr, 0, M, N, K, stream, *epi);
+}
+
+// The same products over rows that the kernel makes itself (K a multiple of 64, operands 16-byte aligned): LayerNorm(x) of 32-bit rows x [M, K],
+// K <= 2048, every epilogue but the residual one; or attention's splits [M][n_head][n_splits <= 8][hd + 4] merged, K = n_head * hd, the residual
+// epilogue. The bits are those of liyab_layernorm or liyab_attention_merge followed by the product.
+static int check_made(const void* x, const void* w, int M, int N, int K, const EpiParams* epi) {
+    auto al16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
+    LIYAB_REQUIRE(x && w && epi, "gemm_made_f32: null operand");
+    LIYAB_REQUIRE(M >= 0 && N > 0 && K > 0 && K % kChunk == 0, "gemm_made_f32: bad sizes M=%d N=%d K=%d (a multiple of 64)", M, N, K);
+    LIYAB_REQUIRE(al16(x) && al16(w), "gemm_made_f32: operands must be 16-byte aligned");
+    LIYAB_REQUIRE(epi->mode == kEpiResidual || epi->out_dtype == kF32, "gemm_made_f32: 32-bit operands give a 32-bit output");
+    return check_epilogue(*epi, M, N);
+}
+extern "C" int liyab_gemm_f32_ln(const float* x, const float* ln_weight, const float* ln_bias, float eps, const float* w, int M, int N, int K,
+                                 const EpiParams* epi, hipStream_t stream) {
+    if (int rc = check_made(x, w, M, N, K, epi)) return rc;
+    LIYAB_REQUIRE(K <= 2048 && eps >= 0.0f, "gemm_f32_ln: rows of %d (at most 2048), eps %g", K, static_cast<double>(eps));
+    LIYAB_REQUIRE(((reinterpret_cast<uintptr_t>(ln_weight) | reinterpret_cast<uintptr_t>(ln_bias)) & 15) == 0, "gemm_f32_ln: operands must be 16-byte aligned");
+    if (M == 0) return 0;
+    const MadeRows made{x, ln_weight, ln_bias, eps, 0, 0, 0};
+    switch (epi->mode) {
+        case kEpiNone: return launch_norm_f32<kEpiNone>(made, w, M, N, K, *epi, stream);
+        case kEpiGeluTanh: return launch_norm_f32<kEpiGeluTanh>(made, w, M, N, K, *epi, stream);
+        case kEpiGeluErf: return launch_norm_f32<kEpiGeluErf>(made, w, M, N, K, *epi, stream);
+        case kEpiQkvPaged: return launch_norm_f32<kEpiQkvPaged>(made, w, M, N, K, *epi, stream);
+        default: return fail(1, "gemm_f32_ln: epilogue %d is not taken", epi->mode);
+    }
+}
+extern "C" int liyab_gemm_f32_splits(const float* partials, int n_splits, int n_head, int hd, const float* w, int M, int N, const EpiParams* epi,
+                                     hipStream_t stream) {
+    LIYAB_REQUIRE(n_splits >= 1 && n_splits <= 8 && n_head > 0 && hd > 0 && hd % 4 == 0 && static_cast<int64_t>(n_head) * hd <= 8192,
+                  "gemm_f32_splits: %d splits (1 to 8) of %d heads of %d", n_splits, n_head, hd);
+    const int K = n_head * hd;
+    if (int rc = check_made(partials, w, M, N, K, epi)) return rc;
+    LIYAB_REQUIRE(epi->mode == kEpiResidual, "gemm_f32_splits: takes the residual epilogue");
+    if (M == 0) return 0;
+    const MadeRows made{partials, nullptr, nullptr, 0.0f, n_splits, n_head, hd};
+    if (n_splits <= 4) return launch_made<kEpiResidual, kSrcSplits, 4>(made, w, M, N, K, *epi, stream);
+    return launch_made<kEpiResidual, kSrcSplits, 8>(made, w, M, N, K, *epi, stream);
 }

@@ -30,11 +30,20 @@ int liyab_gemm_simple(void* out, int out_dtype, int64_t ldo, const void* a, int6
 int liyab_gemm_mfma(const void* a, int64_t lda, const void* w, int M, int N, int K, int tile, const liyab::EpiParams* epi_in,
                     hipStream_t stream);
 int liyab_gemm_f32_qkv(const float* a, int64_t lda, const float* w, int M, int N, int K, const liyab::EpiParams* epi, hipStream_t stream);
+int liyab_gemm_f32_ln(const float* x, const float* ln_weight, const float* ln_bias, float eps, const float* w, int M, int N, int K,
+                      const liyab::EpiParams* epi, hipStream_t stream);
+int liyab_gemm_f32_splits(const float* partials, int n_splits, int n_head, int hd, const float* w, int M, int N, const liyab::EpiParams* epi,
+                          hipStream_t stream);
 int liyab_gemm_mfma_dl(const void* a, int64_t lda, const void* w, int M, int N, int K, int tile, const liyab::EpiParams* epi_in,
                        hipStream_t stream);
 int liyab_gemm_mfma_dl_parts(const void* a, int64_t lda, const void* w, int M, int N, int K, int kparts, int tile, float* parts,
                              int64_t part_stride, const float* bias, const float* base, int n_base, int64_t base_stride,
                              hipStream_t stream);
+int liyab_gemm_rows(const void* a, int64_t lda, const void* w, int M, int N, int K, int strip, const liyab::EpiParams* epi, hipStream_t stream);
+int liyab_gemm_rows_ln(const float* x, const float* ln_weight, const float* ln_bias, float eps, const void* w, int M, int N, int K, int strip,
+                       const liyab::EpiParams* epi, hipStream_t stream);
+int liyab_gemm_rows_splits(const float* partials, int n_splits, int n_head, int hd, const void* w, int M, int N, int strip,
+                           const liyab::EpiParams* epi, hipStream_t stream);
 int liyab_gemm_skinny(const void* a, int64_t lda, const void* w, int M, int N, int K, int ksplit, int wide, int mtile,
                       const liyab::EpiParams* epi_in, hipStream_t stream);
 int liyab_gemm_skinny_parts(const void* a, int64_t lda, const void* w, int M, int N, int K, int kparts, int ksplit, float* parts,

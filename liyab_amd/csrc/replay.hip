@@ -77,9 +77,14 @@ static const Entry kEntries[] = {
     LIYAB_ENTRY(liyab_sum_parts),
     LIYAB_ENTRY(liyab_gemm_simple),
     LIYAB_ENTRY(liyab_gemm_f32_qkv),
+    LIYAB_ENTRY(liyab_gemm_f32_ln),
+    LIYAB_ENTRY(liyab_gemm_f32_splits),
     LIYAB_ENTRY(liyab_gemm_mfma),
     LIYAB_ENTRY(liyab_gemm_mfma_dl),
     LIYAB_ENTRY(liyab_gemm_mfma_dl_parts),
+    LIYAB_ENTRY(liyab_gemm_rows),
+    LIYAB_ENTRY(liyab_gemm_rows_ln),
+    LIYAB_ENTRY(liyab_gemm_rows_splits),
     LIYAB_ENTRY(liyab_gemm_skinny),
     LIYAB_ENTRY(liyab_gemm_skinny_parts),
     LIYAB_ENTRY(liyab_gemm_att_parts),

@@ -56,9 +56,14 @@ _SIGNATURES = {
     "liyab_gemm_skinny_parts": [P, c_int64, P, c_int, c_int, c_int, c_int, c_int, P, c_int64, P, P, c_int, c_int64, P],
     "liyab_gemm_simple": [P, c_int, c_int64, P, c_int64, P, c_int, P, P, c_int64, c_int, c_int, c_int, c_int, P],
     "liyab_gemm_f32_qkv": [P, c_int64, P, c_int, c_int, c_int, _EPI_PTR, P],
+    "liyab_gemm_f32_ln": [P, P, P, c_float, P, c_int, c_int, c_int, _EPI_PTR, P],
+    "liyab_gemm_f32_splits": [P, c_int, c_int, c_int, P, c_int, c_int, _EPI_PTR, P],
     "liyab_gemm_mfma": [P, c_int64, P, c_int, c_int, c_int, c_int, _EPI_PTR, P],
     "liyab_gemm_mfma_dl": [P, c_int64, P, c_int, c_int, c_int, c_int, _EPI_PTR, P],
     "liyab_gemm_mfma_dl_parts": [P, c_int64, P, c_int, c_int, c_int, c_int, c_int, P, c_int64, P, P, c_int, c_int64, P],
+    "liyab_gemm_rows": [P, c_int64, P, c_int, c_int, c_int, c_int, _EPI_PTR, P],
+    "liyab_gemm_rows_ln": [P, P, P, c_float, P, c_int, c_int, c_int, c_int, _EPI_PTR, P],
+    "liyab_gemm_rows_splits": [P, c_int, c_int, c_int, P, c_int, c_int, c_int, _EPI_PTR, P],
     "liyab_gemm_skinny": [P, c_int64, P, c_int, c_int, c_int, c_int, c_int, c_int, _EPI_PTR, P],
     "liyab_attention_generic": [P, c_int64, P, c_int64, P, P, c_int, P, c_int, P, P, c_int, c_float, c_int, c_int,
                                 c_int, c_int, c_int, c_int, P],

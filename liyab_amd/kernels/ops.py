@@ -474,6 +474,52 @@ def gemm_f32_qkv(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor],
     _lib.call("liyab_gemm_f32_qkv", a.data_ptr(), lda, w.data_ptr(), M, w.shape[0], K, ctypes.byref(e), _stream())
 
 
+def gemm_f32_ln(x: torch.Tensor, ln_weight: Optional[torch.Tensor], ln_bias: Optional[torch.Tensor], eps: float, w: torch.Tensor,
+                bias: Optional[torch.Tensor], *, out=None, epilogue: int = EPI_NONE, kv=None) -> None:
+    """The 32-bit product over LayerNorm(x) of the float32 rows x [M, K], K a multiple of 64 up to 2,048, the norm computed inside the kernel: the bits of
+    `layernorm` followed by `gemm` (`gemm_f32_qkv` with `kv`)."""
+    ptr, n_parts, _, M, K = _planes(x, "gemm_f32_ln")
+    _dev(w, "w")
+    if n_parts != 1 or w.dtype != torch.float32 or w.dim() != 2 or w.shape[1] != K or not w.is_contiguous():
+        raise KernelError(f"gemm_f32_ln: needs rows [M, K] and contiguous float32 w [N, {K}], got {tuple(x.shape)}, {tuple(w.shape)} {w.dtype}")
+    _f32vec(ln_weight, "norm weight", K)
+    _f32vec(ln_bias, "norm bias", K)
+    e = _epilogue(_Rows(M, torch.float32), w, bias, out, None, epilogue, kv)
+    _lib.call("liyab_gemm_f32_ln", ptr, _ptr(ln_weight), _ptr(ln_bias), float(eps), w.data_ptr(), M, w.shape[0], K, ctypes.byref(e), _stream())
+
+
+def f32_norm_pays(M: int, N: int, K: int) -> bool:
+    """Whether the 32-bit path computes a norm inside the product behind it: every workgroup of 16 rows repeats it (us, inside / norm and product: 768 -> 3,072 4 rows
+    6.1 / 7.4, 8 rows 6.3 / 7.8, 16 rows 7.4 / 8.0, 24 rows 11.1 / 11.3; 1,024 -> 3,072 8 rows 8.5 / 8.9, 16 rows 10.0 / 9.5; 1,600 -> 6,400 4 rows 16.9 / 17.5, 8 rows
+    18.6 / 18.3)."""
+    return 0 < M <= 16 and K % 64 == 0 and K <= 2048 and M * K <= 16 * 768
+
+
+def splits_in_product_pay(M: int, splits: int, n_head: int, hd: int) -> bool:
+    """Whether attention's splits by position are merged inside the output projection (`gemm_splits`): every workgroup merges all rows (us, inside / merge and
+    product: bfloat16, 12 heads of 64, 4 splits, 4 rows 4.8 / 5.6, 8 rows 6.4 / 5.7; 25 heads 1 row 6.3 / 7.0, 4 rows 9.6 / 7.3; 32 bits 12 heads, 2 splits, 4 rows
+    5.6 / 6.6, 8 rows 7.0 / 6.8; 8 splits, 1 row 7.2 / 6.9)."""
+    return 1 < splits <= 4 and hd % 4 == 0 and (n_head * hd) % 64 == 0 and 0 < M * n_head * hd <= 4 * 768
+
+
+def gemm_splits(partials: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], *, residual: torch.Tensor) -> None:
+    """residual += merge(partials) . w^T + bias over attention's splits [M, heads, splits, head size + 4], merged inside the product: the bits of
+    `attention_merge` followed by `gemm`, in 32 bits (w float32) or in the batch-invariant mode (w bfloat16)."""
+    if w.dtype != torch.float32:
+        gemm_rows_splits(partials, w, bias, residual=residual)
+        return
+    _dev(partials, "partials")
+    _dev(w, "w")
+    if partials.dtype != torch.float32 or partials.dim() != 4 or not partials.is_contiguous():
+        raise KernelError(f"gemm_splits: partials must be contiguous float32 [M, heads, splits, head size + 4], got {tuple(partials.shape)}")
+    M, H, S, hd4 = partials.shape
+    K = H * (hd4 - 4)
+    if w.dim() != 2 or w.shape[1] != K or not w.is_contiguous():
+        raise KernelError(f"gemm_splits: needs contiguous w [N, {K}], got {tuple(w.shape)}")
+    e = _epilogue(_Rows(M, torch.float32), w, bias, None, residual, EPI_RESIDUAL, None)
+    _lib.call("liyab_gemm_f32_splits", partials.data_ptr(), S, H, hd4 - 4, w.data_ptr(), M, w.shape[0], ctypes.byref(e), _stream())
+
+
 def gemm_skinny(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], *, out=None, residual=None,
                 epilogue: int = EPI_NONE, kv=None, ksplit: int = 0, wide: int = -1, mtile: int = 0) -> None:
     """The weight-streaming product for at most 64 bfloat16 rows, K a multiple of 8. ksplit
@@ -488,6 +534,71 @@ def gemm_skinny(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], 
         raise KernelError(f"gemm_skinny: {M} rows; it takes at most 64")
     e = _epilogue(a, w, bias, out, residual, epilogue, kv)
     _lib.call("liyab_gemm_skinny", a.data_ptr(), lda, w.data_ptr(), M, w.shape[0], K, ksplit, wide, mtile, ctypes.byref(e), _stream())
+
+
+def gemm_rows(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], *, out=None, residual=None, epilogue: int = EPI_NONE,
+              kv=None, strip: int = 0) -> None:
+    """The product of at most 64 bfloat16 rows in the batch-invariant order of sums, K a multiple of 64: the bits of `gemm_mfma_dl`'s tiles 16, 17,
+    102, 106 and 108. strip: output features a workgroup (8, 16 or 32; 0: chosen from N)."""
+    lda = _rows(a, "a")
+    M, K = a.shape
+    _dev(w, "w")
+    if a.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or w.dim() != 2 or w.shape[1] != K or not w.is_contiguous():
+        raise KernelError(f"gemm_rows: needs bfloat16 a [M, K] and contiguous w [N, K], got {tuple(a.shape)} {a.dtype}, {tuple(w.shape)} {w.dtype}")
+    e = _epilogue(a, w, bias, out, residual, epilogue, kv)
+    _lib.call("liyab_gemm_rows", a.data_ptr(), lda, w.data_ptr(), M, w.shape[0], K, strip, ctypes.byref(e), _stream())
+
+
+def rows_takes(M: int, N: int, K: int) -> bool:
+    """Where the batch-invariant mode takes `gemm_rows` for a product of few rows, instead of the small tiles. Alone, cold weights, us, rows / tiles: 8 rows
+    768 -> 768 3.2 / 4.2, -> 3,072 3.6 / 4.6, 3,072 -> 768 5.4 / 8.6, 768 -> 50,257 16.6 / 44, 1,600 -> 6,400 6.3 / 7.4; 16 rows 4,096 -> 4,096 9.8 / 11.7; 32 rows
+    768 -> 3,072 4.3 / 4.8, -> 50,257 30 / 49; 64 rows 768 -> 768 3.5 / 4.7, 6,400 -> 1,600 15.0 / 17.8. A workgroup reads all rows again: up to 16 rows it
+    pays as long as strips of 32 features have a compute unit each (4,096 -> 16,384, 8 rows: 31 / 26), up to 32 rows for fewer features (1,600 -> 6,400 8.7 / 8.1),
+    beyond for fewer still (64 rows, 768 -> 2,304 4.9 / 4.9, -> 3,072 5.0 / 5.0)."""
+    if not 0 < M <= 64 or K % 64 != 0:
+        return False
+    if M <= 16:
+        return N <= 32 * 256 or K <= 2048
+    if M <= 32:
+        return N <= 3072 or (N <= 4096 and K <= 1600) or (N > 8192 and K <= 1024)
+    return N <= 2048
+
+
+def norm_in_rows_pays(M: int, N: int, K: int) -> bool:
+    """Whether the batch-invariant mode computes a norm inside the product behind it (`gemm_rows_ln`) instead of in a kernel of its own: while the rows that every
+    workgroup normalises are few (us, inside / norm and product: 768 -> 3,072 8 rows 4.6 / 6.1, 16 rows 5.7 / 6.2, 24 rows 7.0 / 6.6; 1,024 -> 4,096 8 rows 6.1 / 6.8,
+    16 rows 7.7 / 6.9; 1,600 -> 6,400 8 rows 9.2 / 9.1)."""
+    return 0 < M <= 16 and K % 64 == 0 and K <= 2048 and M * K <= 16 * 768 and N <= 32 * 256
+
+
+def gemm_rows_ln(x: torch.Tensor, ln_weight: Optional[torch.Tensor], ln_bias: Optional[torch.Tensor], eps: float, w: torch.Tensor,
+                 bias: Optional[torch.Tensor], *, out=None, epilogue: int = EPI_NONE, kv=None, strip: int = 0) -> None:
+    """`gemm_rows` over LayerNorm(x) of the float32 rows x [M, K], the norm computed inside the kernel: the bits of `layernorm` and `gemm_rows`."""
+    ptr, n_parts, _, M, K = _planes(x, "gemm_rows_ln")
+    _dev(w, "w")
+    if n_parts != 1 or w.dtype != torch.bfloat16 or w.dim() != 2 or w.shape[1] != K or not w.is_contiguous():
+        raise KernelError(f"gemm_rows_ln: needs rows [M, K] and contiguous bfloat16 w [N, {K}], got {tuple(x.shape)}, {tuple(w.shape)} {w.dtype}")
+    _f32vec(ln_weight, "norm weight", K)
+    _f32vec(ln_bias, "norm bias", K)
+    e = _epilogue(_Rows(M, torch.bfloat16), w, bias, out, None, epilogue, kv)
+    e.exact = 0
+    _lib.call("liyab_gemm_rows_ln", ptr, _ptr(ln_weight), _ptr(ln_bias), float(eps), w.data_ptr(), M, w.shape[0], K, strip, ctypes.byref(e), _stream())
+
+
+def gemm_rows_splits(partials: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], *, residual: torch.Tensor, strip: int = 0) -> None:
+    """residual += merge(partials) . w^T + bias over attention's splits [M, heads, splits, head size + 4], merged inside the kernel: the bits of
+    `attention_merge` and `gemm_rows`."""
+    _dev(partials, "partials")
+    _dev(w, "w")
+    if partials.dtype != torch.float32 or partials.dim() != 4 or not partials.is_contiguous():
+        raise KernelError(f"gemm_rows_splits: partials must be contiguous float32 [M, heads, splits, head size + 4], got {tuple(partials.shape)}")
+    M, H, S, hd4 = partials.shape
+    K = H * (hd4 - 4)
+    if w.dtype != torch.bfloat16 or w.dim() != 2 or w.shape[1] != K or not w.is_contiguous():
+        raise KernelError(f"gemm_rows_splits: needs contiguous bfloat16 w [N, {K}], got {tuple(w.shape)} {w.dtype}")
+    e = _epilogue(_Rows(M, torch.bfloat16), w, bias, None, residual, EPI_RESIDUAL, None)
+    e.exact = 0
+    _lib.call("liyab_gemm_rows_splits", partials.data_ptr(), S, H, hd4 - 4, w.data_ptr(), M, w.shape[0], strip, ctypes.byref(e), _stream())
 
 
 def gemm_skinny_parts(a: torch.Tensor, w: torch.Tensor, planes: torch.Tensor, *, bias: Optional[torch.Tensor] = None,
@@ -736,10 +847,12 @@ def gemm(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], *, out:
         # one family of kernels whatever the number of rows: their sum over k has one order for
         # every tile shape, so a row's bits do not depend on the rows beside it. K a multiple of 64:
         # four sums, unit u of 64 k going to sum u % 4 (16 k an instruction), added in their order;
-        # up to 64 rows four groups of waves walk K side by side, a sum each, in small tiles that
-        # cover the chip; more rows take the large tiles, whose one group keeps the four sums.
+        # up to 64 rows four waves, or groups of them, walk K side by side, a sum each, in strips or small tiles
+        # that cover the chip; more rows take the large tiles, whose one group keeps the four sums.
         M, N, K = a.shape[0], w.shape[0], a.shape[1]
-        if K % 64 == 0:
+        if rows_takes(M, N, K):
+            gemm_rows(a, w, bias, out=out, residual=residual, epilogue=epilogue, kv=kv)
+        elif K % 64 == 0:
             if M <= 64:
                 tile = 17 if M <= 32 or 2 * ((N + 31) // 32) <= compute_units() else 16
             else:
@@ -996,7 +1109,7 @@ def attention(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor, v_cache
     says how the step's tokens are cut, see parts/attention.py; without it every token goes to
     the plain kernel). With `splits_ok`, a step of few tokens may leave `out` unwritten and
     return the splits of each (token, head) pair instead, float32 [tokens, heads, splits, head
-    size + 4], for `gemm_att_parts`. `softcap`, `bias_table`: what is done to the scores before the softmax, `sinks`: a learned
+    size + 4], for `gemm_att_parts` (`gemm_splits` in 32 bits and in the batch-invariant mode). `softcap`, `bias_table`: what is done to the scores before the softmax, `sinks`: a learned
     logit a head in its denominator, `keep_first`: positions that stay visible behind the window (see `attention_decode`); every kernel
     below does the same."""
     hd = k_cache.shape[3]
@@ -1036,11 +1149,12 @@ def attention(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor, v_cache
         # as the merge kernel does), which saves the splits' traffic and leaves the chip as full
         if n * n_head * splits > INVARIANT_SPLIT_WORK:
             splits = 1
-        partials = ctx.workspace.get("attn_partials", (n * n_head * splits * (hd + 4),), torch.float32) if splits > 1 else None
+        leave = splits_ok and splits_in_product_pay(n, splits, n_head, hd)
+        partials = ctx.workspace.get("attn_partials", (n, n_head, splits, hd + 4), torch.float32) if splits > 1 else None
         attention_decode(out, q, k_cache, v_cache, block_tables, ctx.tok_seq, ctx.positions, n_head=n_head, scale=scale,
-                         window=window, n_splits=splits, partials=partials, waves=4, chunk=chunk,
+                         window=window, n_splits=splits, partials=partials, waves=4, chunk=chunk, leave_splits=leave,
                          rows_are_requests=host.max_q_len == 1, reach=plan.context_bucket, **scored)
-        return None
+        return partials if leave else None
     if fast and plan.mode == "decode" and block_tables.shape[1] <= 2048:
         n = out.shape[0]
         splits, waves = decode_split_plan(n, n_head, plan.context_bucket) if splits_ok else (1, 4)

@@ -175,11 +175,15 @@ class Attention:
         att = ws.get("att", (n, self.q_dim), self.dtype)
         # with few tokens attention may leave each (token, head) pair's keys cut into splits, for
         # an output projection that is cut over its inner dimension and merges them as it loads
-        cut = defer and self.dtype == torch.bfloat16 and ops.k_parts(n, self.width, self.q_dim) > 1
+        # (in 32 bits and in the batch-invariant mode: splits by position, for a projection that merges all of them)
+        exact = self.dtype == torch.float32 or ops.is_batch_invariant()
+        cut = defer and (self.out_weight.data_ptr() % 16 == 0 if exact else ops.k_parts(n, self.width, self.q_dim) > 1)
         splits = ops.attention(att, q[:, :self.q_dim] if q.shape[1] != self.q_dim else q, cache.k, cache.v, group.block_tables, ctx,
                                n_head=self.n_head, scale=self.scale, window=self.window, splits_ok=cut)
-        split = linear_deferred(splits if splits is not None else att, self.out_weight, self.out_bias, ctx, "att_parts", residual) if defer else None
-        if split is None:
+        split = linear_deferred(splits if splits is not None else att, self.out_weight, self.out_bias, ctx, "att_parts", residual) if defer and not exact else None
+        if split is None and splits is not None and exact:
+            ops.gemm_splits(splits, self.out_weight, self.out_bias, residual=settled(residual))
+        elif split is None:
             if splits is not None:
                 ops.attention_merge(att, splits)
             linear(att, self.out_weight, self.out_bias, residual=settled(residual))

@@ -37,6 +37,18 @@ def _fuses(a, w: torch.Tensor, residual) -> bool:
             and ops.skinny_ln_pays(a.n_rows, w.shape[0], a.norm.width))
 
 
+def _fuses_exactly(a, w: torch.Tensor, residual) -> bool:
+    """Whether the norm goes into the product where a row's bits may not depend on the step: the kernels that leave the norm's own bits."""
+    if not (isinstance(a, Normed) and getattr(a.norm, "fusable", None) == "layernorm" and residual is None and a.rows is None and a._tensor is None
+            and a.x.dim() == 2 and a.x.dtype == torch.float32 and a.x.is_contiguous()):
+        return False
+    if not all(t is None or t.data_ptr() % 16 == 0 for t in (a.x, a.norm.weight, a.norm.bias, w)):
+        return False
+    if w.dtype == torch.float32:
+        return a.norm.dtype == torch.float32 and ops.f32_norm_pays(a.n_rows, w.shape[0], a.norm.width)
+    return ops.is_batch_invariant() and w.dtype == a.norm.dtype == torch.bfloat16 and ops.norm_in_rows_pays(a.n_rows, w.shape[0], a.norm.width)
+
+
 def linear(a, w: torch.Tensor, bias: Optional[torch.Tensor], *, out: Optional[torch.Tensor] = None,
            residual: Optional[torch.Tensor] = None, activation: str = "none", kv=None) -> None:
     """out = act(a . w^T + bias); with `residual`: residual += a . w^T + bias; with `kv` =
@@ -53,6 +65,9 @@ def linear(a, w: torch.Tensor, bias: Optional[torch.Tensor], *, out: Optional[to
             ops.gemm_skinny_dyt(a.x, n.weight, n.bias, n.alpha, w, bias, out=out, epilogue=epilogue, kv=kv)
         else:
             ops.gemm_skinny_ln(a.x, n.weight, n.bias, n.eps, w, bias, out=out, epilogue=epilogue, kv=kv)
+        return
+    if _fuses_exactly(a, w, residual):
+        (ops.gemm_f32_ln if w.dtype == torch.float32 else ops.gemm_rows_ln)(a.x, a.norm.weight, a.norm.bias, a.norm.eps, w, bias, out=out, epilogue=epilogue, kv=kv)
         return
     if isinstance(a, Normed):
         a = a.tensor()

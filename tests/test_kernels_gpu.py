@@ -1212,6 +1212,74 @@ def test_tiles_of_every_shape_give_a_row_the_same_bits(ops, K):
             assert torch.equal(out, full[108][rows]), f"rows {rows} in tiles {tile}"
 
 
+@pytest.mark.parametrize("K", [64, 192, 768, 832, 1600, 3072])
+def test_rows_give_the_bits_of_the_tiles(ops, K):
+    """The product of few rows leaves the bits of the tiles of four sums (held to the 32-bit reference above): rings of every
+    depth (up to 3, 6 and 12 units a wave, and around them again), every strip, rows and features at the edges of both."""
+    for M in (1, 8, 9, 17, 32, 33, 64):
+        for N in (3, 40, 301):
+            a, w, bias = rnd(M, K, dtype=torch.bfloat16, seed=K), rnd(N, K, dtype=torch.bfloat16, seed=K + 1, scale=0.2), rnd(N, seed=2)
+            want, base = torch.empty(M, N, device=DEV), rnd(M, N, seed=3)
+            ops.gemm_mfma_dl(a, w, bias, out=want, tile=17)
+            added = base.clone()
+            ops.gemm_mfma_dl(a, w, bias, residual=added, epilogue=ops.EPI_RESIDUAL, tile=17)
+            for strip in (0, 8, 16, 32):
+                out, res = torch.full((M, N), float("nan"), device=DEV), base.clone()
+                ops.gemm_rows(a, w, bias, out=out, strip=strip)
+                ops.gemm_rows(a, w, bias, residual=res, epilogue=ops.EPI_RESIDUAL, strip=strip)
+                assert torch.equal(out, want) and torch.equal(res, added), (M, N, strip)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("K", [64, 768, 832, 1024, 1600, 2048])
+def test_a_norm_inside_the_product_leaves_its_own_kernels_bits(ops, dtype, K):
+    """The norm computed inside the product of few rows (the batch-invariant mode's and the 32-bit one) against the norm's kernel and the
+    plain product: the same bits, with and without weight and bias, GELU behind it, keys and values to their pages."""
+    with ops.batch_invariant(dtype == torch.bfloat16):
+        for M in (1, 3, 4, 5, 9, 16, 17, 33):
+            x, lw, lb = rnd(M, K, seed=K, scale=3.0), rnd(K, seed=4), rnd(K, seed=5)
+            w, bias = rnd(3 * 32, K, dtype=dtype, seed=6, scale=0.2), rnd(3 * 32, seed=7)
+            slots = torch.randperm(40)[:M].to(torch.int32).to(DEV)
+            slots[M // 2] = -1
+            for weight, shift in ((lw, lb), (None, None)):
+                normed, want, out = torch.empty(M, K, dtype=dtype, device=DEV), torch.empty(M, 96, dtype=dtype, device=DEV), torch.empty(M, 96, dtype=dtype, device=DEV)
+                fused = ops.gemm_f32_ln if dtype == torch.float32 else ops.gemm_rows_ln
+                ops.layernorm(normed, x, weight, shift, 1e-5)
+                ops.gemm(normed, w, bias, out=want, epilogue=ops.EPI_GELU_TANH)
+                fused(x, weight, shift, 1e-5, w, bias, out=out, epilogue=ops.EPI_GELU_TANH)
+                assert torch.equal(out, want), (M, weight is None)
+                got = []
+                for one in (False, True):
+                    q, kc, vc = (torch.zeros(s, dtype=dtype, device=DEV) for s in ((M, 32), (10, 2, 4, 16), (10, 2, 4, 16)))
+                    kv = dict(out=q, kv=(kc, vc, slots, 32))
+                    if one:
+                        fused(x, weight, shift, 1e-5, w, bias, epilogue=ops.EPI_QKV_PAGED, **kv)
+                    elif dtype == torch.float32:
+                        ops.gemm_f32_qkv(normed, w, bias, **kv)
+                    else:
+                        ops.gemm(normed, w, bias, epilogue=ops.EPI_QKV_PAGED, **kv)
+                    got.append((q, kc, vc))
+                assert all(torch.equal(a, b) for a, b in zip(*got)), (M, weight is None)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("H,hd,S", [(1, 64, 2), (12, 64, 4), (5, 128, 3), (8, 16, 8), (25, 64, 5)])
+def test_splits_merged_inside_the_product_leave_the_merges_bits(ops, dtype, H, hd, S):
+    """Attention's splits merged inside the output projection against the merge's kernel and the plain product, splits without keys among them."""
+    K, N = H * hd, 72
+    with ops.batch_invariant(dtype == torch.bfloat16):
+        for M in (1, 3, 4, 9, 17, 33):
+            p = rnd(M, H, S, hd + 4, seed=M)
+            p[..., hd + 1] = p[..., hd + 1].abs() + 0.5
+            p[::2, :, S - 1, hd], p[::2, :, S - 1, hd + 1] = -float("inf"), 0.0
+            w, bias, base = rnd(N, K, dtype=dtype, seed=1, scale=0.2), rnd(N, seed=2), rnd(M, N, seed=3)
+            att, want, got = torch.empty(M, K, dtype=dtype, device=DEV), base.clone(), base.clone()
+            ops.attention_merge(att, p)
+            ops.gemm(att, w, bias, residual=want, epilogue=ops.EPI_RESIDUAL)
+            ops.gemm_splits(p, w, bias, residual=got)
+            assert torch.equal(got, want), M
+
+
 @pytest.mark.parametrize("K", [64, 768, 3072])
 def test_tiles_of_one_sum_give_a_row_the_same_bits(ops, K):
     """The tiles of many rows take K in one chain of the same steps whatever their shape: the same bits from each, inside the

@@ -178,3 +178,19 @@ def test_padded_sizes_of_steps_with_prompt_portions():
     for n in range(1, 3000):
         unit = 16 if n <= 64 else 64 if n <= 1024 else 128
         assert n <= padded_rows(n) < n + unit and padded_rows(n) % unit == 0 and padded_rows(padded_rows(n)) == padded_rows(n)
+
+
+def test_products_of_few_rows_are_within_what_their_kernels_take(ops):
+    """The rules that send a product of few rows, a norm inside it or attention's splits inside it to their kernels: only sizes these take."""
+    for M in (0, 1, 4, 8, 9, 16, 17, 32, 33, 64, 65, 500):
+        for N in (1, 96, 768, 2048, 2304, 4096, 8192, 50257):
+            for K in (8, 64, 72, 768, 800, 1600, 2048, 2112, 6400):
+                if ops.rows_takes(M, N, K):
+                    assert 0 < M <= 64 and K % 64 == 0
+                for pays in (ops.norm_in_rows_pays, ops.f32_norm_pays):
+                    if pays(M, N, K):
+                        assert 0 < M <= 64 and K % 64 == 0 and K <= 2048 and M * (K + 8) * 2 <= 96 * 1024
+        for splits in (1, 2, 4, 5, 16):
+            for heads, hd in ((1, 8), (12, 64), (3, 36), (25, 64), (64, 128)):
+                if ops.splits_in_product_pay(M, splits, heads, hd):
+                    assert 1 < splits <= 8 and hd % 4 == 0 and heads * hd % 64 == 0 and heads * hd <= 8192 and 0 < M <= 64
