@@ -23,6 +23,9 @@
 #include "launchers.h"
 #include "epilogue.h"
 
+#include <type_traits>
+#include <utility>
+
 namespace liyab {
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
@@ -223,6 +226,219 @@ gemm_skinny_kernel(const bf16_t* __restrict__ a, int64_t lda, const bf16_t* __re
     }
 }
 
+// The same product, bit for bit, for one tile of 16 rows a workgroup, 16 or 32 features and whole units of K (a multiple of 64, and not of 16,384): a
+// wave's units reach it through a ring in LDS of its own, 8 rows of 64 k a load (global_load_lds, whole cache lines), with no barrier: a wave waits
+// for its own loads. What bounds a product of this size is a chain: the first trip to memory, and what stands behind it. Straight into registers a
+// load touched 16 rows' sectors and an operand of 8 rows was read for 16; the waves' sums were read one by one; and waves without a unit of K
+// were launched. The waves, each wave's units and the order of the sums are those of gemm_skinny_kernel. The epilogue is fixed at compile time: a
+// kernel this short waits for its own instructions, cold in every launch of a chain (all epilogues in one, 1,300 instructions and not 500: 768 -> 768
+// 3.8 us and not 3.3). us, cold weights, before / now: 8 rows 768 -> 768 4.5 / 3.3, -> 3,072 5.2 / 4.1, -> 50,257 22.1 / 16.7, 3,072 -> 768 8.0 / 4.9, in
+// four parts 5.3 / 4.3, 1,600 -> 6,400 8.9 / 6.3; 16 rows 768 -> 768 4.8 / 3.4, 1,600 -> 4,800 9.7 / 5.8.
+// MR: rows of the ring, 8 or 16, M rounded up (the matrix operand's other rows repeat the last). NT: tiles of 16 features. R: units of the ring.
+constexpr int kUnit = 64;
+typedef __attribute__((address_space(3))) void* lds_void_ptr;
+__device__ __forceinline__ int ring_swizzle(int row) { return (row >> 1) & 7; }  // 16 rows' reads of one 16-byte piece fall into different banks
+
+// This wave's loads but the last LATER have arrived.
+template <int LATER>
+__device__ __forceinline__ void wait_loads() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt((LATER & 15) | 0x0f70 | ((LATER >> 4) << 14));
+    asm volatile("" ::: "memory");
+}
+template <int... T, typename F>
+__device__ __forceinline__ void in_turn(std::integer_sequence<int, T...>, F&& f) {
+    (f(std::integral_constant<int, T>{}), ...);
+}
+
+// EPI: an epilogue fixed at compile time (none, residual, or kEpiPlanes: planes with rows to add to); -1 reads it from the parameters.
+constexpr int kEpiPlanes = 5;
+template <typename OutT, int MR, int NT, int R, int EPI>
+__global__ void __launch_bounds__(1024)
+gemm_stream_kernel(const bf16_t* __restrict__ a, int64_t lda, const bf16_t* __restrict__ w, int M, int N, int K,
+                   EpiParams epi, BaseSum base, int part_k, int64_t part_stride, int split_shift) {
+    constexpr int NB = 16 * NT, LOADS = (NB + MR) / 8, SLOT = (NB + MR) * kUnit;
+    static_assert((R - 1) * LOADS <= 63, "the counter of loads in flight has six bits");
+    extern __shared__ __attribute__((aligned(1024))) unsigned char stream_lds[];
+    float* const red = reinterpret_cast<float*>(stream_lds);  // [wave][NT][256], once the rings have been read
+    const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64), waves = blockDim.x / 64;
+    const int i = lane % 16, g = lane / 16;
+    const int n0 = blockIdx.x * NB, m0 = blockIdx.y * 16;
+    const int k_begin = blockIdx.z * part_k, k_end = min(K, k_begin + part_k);
+    const int units = (k_end - k_begin) / kUnit, pairs = (units + 1) / 2;
+    // this wave's units: those of pairs wave, wave + ksplit, ... (the last of all may be half a pair); ksplit = 1 << split_shift
+    const int ksplit = 1 << split_shift;
+    const int my_pairs = wave < ksplit ? (pairs - wave + ksplit - 1) >> split_shift : 0;
+    const int mine = 2 * my_pairs - ((units & 1) != 0 && ((pairs - 1) & (ksplit - 1)) == wave ? 1 : 0);
+    if (gridDim.z > 1) epi.out = static_cast<float*>(epi.out) + blockIdx.z * part_stride;
+    if (blockIdx.z > 0) epi.bias = nullptr;  // a cut product's bias goes to its first plane only
+    bf16_t* const ring = reinterpret_cast<bf16_t*>(stream_lds) + wave * R * SLOT;
+
+    const int lrow = lane / 8, lpos = lane % 8;  // this lane's part in a load
+    const bf16_t* from[LOADS];
+#pragma unroll
+    for (int l = 0; l < 2 * NT; ++l) from[l] = w + static_cast<int64_t>(min(n0 + 8 * l + lrow, N - 1)) * K + k_begin + (lpos ^ ring_swizzle(8 * l + lrow)) * 8;
+#pragma unroll
+    for (int l = 2 * NT; l < LOADS; ++l) {
+        const int row = 8 * (l - 2 * NT) + lrow;
+        from[l] = a + static_cast<int64_t>(min(m0 + row, M - 1)) * lda + k_begin + (lpos ^ ring_swizzle(row)) * 8;
+    }
+    auto load = [&](int j, int slot) {  // unit j of this wave's (one past its last: the last of K, not multiplied)
+        const int k = min((((j / 2) << split_shift) + wave) * 2 + j % 2, units - 1) * kUnit;
+#pragma unroll
+        for (int l = 0; l < LOADS; ++l) {
+            const bf16_t* const piece = from[l] + k;
+            bf16_t* const to = ring + slot * SLOT + l * 8 * kUnit;
+            __builtin_amdgcn_global_load_lds(piece, (lds_void_ptr)to, 16, 0, 0);
+        }
+    };
+    // What the epilogue reads for this thread's first output is asked for first of all (counted in order, and the weights are waited for unit by
+    // unit), with no load under a branch: who has nothing to read gets a word of the weights. The first part's share of the rows the product is
+    // added to: up to four planes (a plane past the last is the last one again, dropped).
+    typedef const __attribute__((address_space(1))) float* global_floats;
+    const int e_m = min(m0 + (tid % 256) / 16, M - 1), e_n = min(n0 + 16 * (tid / 256 % NT) + tid % 16, N - 1);
+    const bool based = EPI == kEpiPlanes && blockIdx.z == 0;
+    const auto nothing = (global_floats)(w);
+    auto bias_at = epi.bias != nullptr ? (global_floats)(epi.bias + e_n) : nothing;
+    auto res_at = based                        ? (global_floats)(base.planes + static_cast<int64_t>(e_m) * N + e_n)
+                  : (EPI < 0 ? epi.mode : EPI) == kEpiResidual ? (global_floats)(epi.residual + static_cast<int64_t>(e_m) * epi.ldr + e_n)
+                                             : nothing;
+    const int64_t base_stride = based ? base.stride : 0;
+    const int base_last = based ? base.n - 1 : 0;
+    asm volatile("" : "+v"(bias_at), "+v"(res_at));  // (worked out here, ahead of every load)
+    const float e_bias = *bias_at;
+    float e_res[4];
+#pragma unroll
+    for (int q = 0; q < (EPI == kEpiPlanes ? 4 : 1); ++q) e_res[q] = EPI == kEpiNone ? 0.0f : res_at[min(q, base_last) * base_stride];
+    // (no load may cross to the other side: the waits below count on what is asked for behind them)
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int p = 0; p < R; ++p) load(p, p);
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("" ::: "memory");
+
+    floatx4 acc[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) acc[t] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+    const int arow = min(i, M - 1 - m0);
+    auto multiply = [&](int slot) {
+        const bf16_t* const sw = ring + slot * SLOT + i * kUnit;
+        const bf16_t* const sa = ring + slot * SLOT + (NB + arow) * kUnit;
+        Frag x[NT][2], y[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+#pragma unroll
+            for (int t = 0; t < NT; ++t) x[t][h].u = *reinterpret_cast<const u32x4*>(sw + 16 * t * kUnit + ((4 * h + g) ^ ring_swizzle(i)) * 8);
+            y[h].u = *reinterpret_cast<const u32x4*>(sa + ((4 * h + g) ^ ring_swizzle(arow)) * 8);
+        }
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int t = 0; t < NT; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x[t][h].v, y[h].v, acc[t], 0, 0, 0);
+    };
+    int j0 = 0;
+    for (; j0 + R < mine; j0 += R)
+        in_turn(std::make_integer_sequence<int, R>{}, [&](auto at) {
+            constexpr int t = decltype(at)::value;
+            wait_loads<(R - 1) * LOADS>();
+            multiply(t);
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the place has been read
+            load(j0 + R + t, t);
+        });
+    in_turn(std::make_integer_sequence<int, R>{}, [&](auto at) {
+        constexpr int t = decltype(at)::value;
+        wait_loads<(R - 1 - t) * LOADS>();
+        if (j0 + t < mine) multiply(t);
+    });
+    lds_barrier();  // (the sums take the rings' place)
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) red[(wave * NT + t) * 256 + i * 16 + 4 * g + r] = acc[t][r];
+    lds_barrier();
+    for (int e = tid; e < NT * 256; e += blockDim.x) {
+        const int m = m0 + e % 256 / 16, n = n0 + 16 * (e / 256) + e % 16;
+        if (m >= M || n >= N) continue;
+        float v = 0.0f;
+        for (int q0 = 0; q0 < waves; q0 += 8) {
+            float s[8];
+#pragma unroll
+            for (int q = 0; q < 8; ++q) s[q] = red[min(q0 + q, waves - 1) * NT * 256 + e];
+#pragma unroll
+            for (int q = 0; q < 8; ++q) v += q0 + q < waves ? s[q] : 0.0f;
+        }
+        const bool first = e == tid;
+        const float bias = first ? (epi.bias != nullptr ? e_bias : 0.0f) : epilogue_bias(epi, n);
+        if (based) {
+            // this plane = (sums + bias) + (base planes added up in their order)
+            const float* bp = base.planes + static_cast<int64_t>(m) * N + n;
+            float b = first ? e_res[0] : bp[0];
+#pragma unroll
+            for (int q = 1; q < 4; ++q)
+                if (q < base.n) b += first ? e_res[q] : bp[q * base.stride];
+            for (int q = 4; q < base.n; ++q) b += bp[q * base.stride];
+            static_cast<float*>(epi.out)[static_cast<int64_t>(m) * epi.ldo + n] = (v + bias) + b;
+        } else if (first && (EPI < 0 ? epi.mode : EPI) == kEpiResidual) {
+            epi.residual[static_cast<int64_t>(m) * epi.ldr + n] = e_res[0] + (v + bias);
+        } else {
+            epilogue_store_biased<OutT, EPI == kEpiPlanes ? kEpiNone : EPI>(epi, m, n, v + bias);
+        }
+    }
+}
+
+template <typename OutT, int MR, int NT, int R, int EPI>
+int launch_stream_as(const bf16_t* a, int64_t lda, const bf16_t* w, int M, int N, int K, int ksplit, int waves, const EpiParams& epi, const BaseSum& base,
+                     int kparts, int part_k, int64_t part_stride, hipStream_t stream) {
+    size_t smem = static_cast<size_t>(waves) * R * (16 * NT + MR) * kUnit * sizeof(bf16_t);
+    if (smem < waves * NT * 256 * sizeof(float)) smem = waves * NT * 256 * sizeof(float);
+    LIYAB_REQUIRE(smem <= 160 * 1024, "gemm_skinny: %zu bytes of LDS", smem);
+    auto kern = gemm_stream_kernel<OutT, MR, NT, R, EPI>;
+    static bool ready = false;  // once per instantiation, outside any stream capture's first use
+    if (!ready) {
+        hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+        ready = true;
+    }
+    kern<<<dim3((N + 16 * NT - 1) / (16 * NT), (M + 15) / 16, kparts), 64 * waves, smem, stream>>>(a, lda, w, M, N, K, epi, base, part_k, part_stride, __builtin_ctz(ksplit));
+    return check_launch("gemm_skinny");
+}
+template <typename OutT, int EPI>
+int launch_stream_epi(const void* a, int64_t lda, const void* w, int M, int N, int K, int ksplit, const EpiParams& epi, const BaseSum& base, int kparts,
+                  int64_t part_stride, hipStream_t stream) {
+    const int units = (K / kUnit + kparts - 1) / kparts, pairs = (units + 1) / 2, mine = 2 * ((pairs + ksplit - 1) / ksplit);  // units of a part, units a wave
+    const int rows = M <= 8 ? 8 : 16;
+    int waves = ksplit < pairs ? ksplit : pairs;
+    auto ring = [&](int nt, int r) { return static_cast<size_t>(waves) * r * (16 * nt + rows) * kUnit * 2; };
+    const int64_t strips = static_cast<int64_t>((N + 15) / 16) * ((M + 15) / 16) * kparts;
+    // With a few more strips than compute units a workgroup takes two, where their rings fit (one row, us by one strip / by two, with all epilogues
+    // in one kernel: 1,280 -> 5,120 7.7 / 5.8, 1,600 -> 6,400 8.6 / 7.1; 16 rows 6.5 / 6.1, 7.1 / 7.1); with twice as many it does where a wave has three units
+    // (3,072 -> 8,192 13.3 / 11.9; 1,600 -> 8,192 8.4 / 8.8, 4,096 -> 8,192 16.2 / 17.5, 768 -> 50,257 17.1 / 19.2)
+    const bool wide = strips > 256 && strips <= (K > 1600 && K <= 3072 ? 512 : 448) && ring(2, 2) <= 160 * 1024;
+    const int nt = wide ? 2 : 1;
+    // a thread an output element at least, so that each has what its epilogue reads asked for ahead (waves without a unit of K bring in one again)
+    if (strips <= 256 && waves < 4 * nt && ring(nt, 2) * 4 * nt / waves <= 160 * 1024) waves = 4 * nt;
+    // four units in flight where a wave has more than two and the rings leave a compute unit room for others
+    const bool four = mine > 2 && ring(nt, 4) <= 96 * 1024;
+    auto* pa = static_cast<const bf16_t*>(a);
+    auto* pw = static_cast<const bf16_t*>(w);
+#define LIYAB_STREAM(MR, NT, R) launch_stream_as<OutT, MR, NT, R, EPI>(pa, lda, pw, M, N, K, ksplit, waves, epi, base, kparts, units * kUnit, part_stride, stream)
+    if (rows == 8) {
+        if (wide) return four ? LIYAB_STREAM(8, 2, 4) : LIYAB_STREAM(8, 2, 2);
+        return four ? LIYAB_STREAM(8, 1, 4) : LIYAB_STREAM(8, 1, 2);
+    }
+    if (wide) return four ? LIYAB_STREAM(16, 2, 4) : LIYAB_STREAM(16, 2, 2);
+    return four ? LIYAB_STREAM(16, 1, 4) : LIYAB_STREAM(16, 1, 2);
+#undef LIYAB_STREAM
+}
+int launch_stream(const void* a, int64_t lda, const void* w, int M, int N, int K, int ksplit, const EpiParams& epi, const BaseSum& base, int kparts,
+                  int64_t part_stride, hipStream_t stream) {
+#define LIYAB_STREAM(OUT, EPI) launch_stream_epi<OUT, EPI>(a, lda, w, M, N, K, ksplit, epi, base, kparts, part_stride, stream)
+    if (base.planes != nullptr) return LIYAB_STREAM(float, kEpiPlanes);
+    if (epi.mode == kEpiResidual) return LIYAB_STREAM(float, kEpiResidual);
+    if (epi.out_dtype == kF32) return epi.mode == kEpiNone ? LIYAB_STREAM(float, kEpiNone) : LIYAB_STREAM(float, -1);
+    return epi.mode == kEpiNone ? LIYAB_STREAM(bf16_t, kEpiNone) : LIYAB_STREAM(bf16_t, -1);
+#undef LIYAB_STREAM
+}
 template <int MT, int NT, int MAXW>
 int launch_skinny(const void* a, int64_t lda, const void* w, int M, int N, int K, int ksplit, const EpiParams& epi,
                   const BaseSum& base, int kparts, int64_t part_stride, hipStream_t stream) {
@@ -290,6 +506,10 @@ static int skinny_dispatch(const void* a, int64_t lda, const void* w, int M, int
     }
     LIYAB_REQUIRE(ksplit == 1 || ksplit == 2 || ksplit == 4 || ksplit == 8 || ksplit == 16,
                   "gemm_skinny: ksplit %d is not 1, 2, 4, 8 or 16", ksplit);
+    // (with one or two units of K and more strips than compute units the kernel of registers is as fast, 128 -> 8,192 at one row 3.8 us against 3.9)
+    if (nt == 1 && mt == 1 && K % kUnit == 0 && K % 16384 != 0 && (K > 2 * kUnit || N * ((M + 15) / 16) <= 16 * 256)) {
+        return launch_stream(a, lda, w, M, N, K, ksplit, epi, base, kparts, part_stride, stream);
+    }
     if (nt == 1) {
         if (mt == 1) return launch_skinny<1, 1, 16>(a, lda, w, M, N, K, ksplit, epi, base, kparts, part_stride, stream);
         if (mt == 2) return launch_skinny<2, 1, 16>(a, lda, w, M, N, K, ksplit, epi, base, kparts, part_stride, stream);
