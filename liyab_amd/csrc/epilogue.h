@@ -35,6 +35,16 @@ struct EpiParams {
     uint32_t num_slots;       // pages x page_size of the caches: a slot outside [0, num_slots) is not written
 };
 
+// The paged QKV epilogue: what depends on the row (its slot's place in the pages), for kernels that store several columns of it computed once.
+// Element offset of a slot for head 0, dimension 0; -1 for a token without a slot (-1), or with
+// one past the caches' pages: a wrong word in the slots must not become a store outside them. (Slots fit 32 bits: divided in 64 they are
+// a hundred instructions.)
+__device__ __forceinline__ int64_t qkv_row_base(const EpiParams& p, int slot_word) {
+    const uint32_t slot = slot_word, size = p.page_size, page = slot / size;
+    if (slot >= p.num_slots) return -1;
+    return (static_cast<int64_t>(page) * p.n_kv_head * size + (slot - page * size)) * p.hd;
+}
+
 // `MODE` >= 0 fixes the epilogue at compile time (straight-line code in the kernels' store
 // loops); -1 reads it from the parameters.
 // The bias of column n (0 without one). Kernels that store several rows of a column load it
@@ -63,12 +73,10 @@ __device__ __forceinline__ void epilogue_store_biased(const EpiParams& p, int m,
             if (n >= p.q_dim) {
                 const bool is_v = n >= p.q_dim + p.kv_dim;
                 const int c = n - p.q_dim - (is_v ? p.kv_dim : 0);
-                const int64_t slot = p.slots[m];
-                if (static_cast<uint64_t>(slot) >= p.num_slots) return;  // no slot (-1), or none of these caches
-                const int64_t page = slot / p.page_size;
-                const int off = static_cast<int>(slot % p.page_size);
-                const int64_t dst = ((page * p.n_kv_head + c / p.hd) * p.page_size + off) * p.hd + c % p.hd;
-                static_cast<OutT*>(is_v ? p.vc : p.kc)[dst] = from_float<OutT>(v);
+                const int64_t at = qkv_row_base(p, p.slots[m]);
+                if (at < 0) return;
+                const int head = c / p.hd;
+                static_cast<OutT*>(is_v ? p.vc : p.kc)[at + static_cast<int64_t>(head) * p.page_size * p.hd + (c - head * p.hd)] = from_float<OutT>(v);
                 return;
             }
             break;
@@ -77,15 +85,6 @@ __device__ __forceinline__ void epilogue_store_biased(const EpiParams& p, int m,
     static_cast<OutT*>(p.out)[static_cast<int64_t>(m) * p.ldo + n] = from_float<OutT>(v);
 }
 
-// The paged QKV epilogue for kernels whose lanes hold several rows of one column: what depends
-// on the row (its slot's place in the pages) is computed once per row, ahead of the stores.
-// Element offset of row m's slot for head 0, dimension 0; -1 for a token without a slot (or with
-// one past the caches' pages: a wrong word in the slots must not become a store outside them).
-__device__ __forceinline__ int64_t qkv_row_base(const EpiParams& p, int m) {
-    const int64_t slot = p.slots[m];
-    if (static_cast<uint64_t>(slot) >= p.num_slots) return -1;
-    return (slot / p.page_size) * (static_cast<int64_t>(p.n_kv_head) * p.page_size * p.hd) + (slot % p.page_size) * p.hd;
-}
 // What depends on the column: -1 for a query column, else the offset of (head, dimension)
 // within a page, with bit 62 set for values.
 __device__ __forceinline__ int64_t qkv_col_offset(const EpiParams& p, int n) {

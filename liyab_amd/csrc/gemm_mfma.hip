@@ -118,7 +118,7 @@ gemm_mfma_kernel(const bf16_t* __restrict__ a, int64_t lda, const bf16_t* __rest
             const int mb = m0 + wm * (BM / 2) + i * 32 + 4 * (lane / 32);
             int64_t row_base[16];
 #pragma unroll
-            for (int r = 0; r < 16; ++r) row_base[r] = qkv_row_base(epi, min(mb + 8 * (r / 4) + r % 4, M - 1));
+            for (int r = 0; r < 16; ++r) row_base[r] = qkv_row_base(epi, epi.slots[min(mb + 8 * (r / 4) + r % 4, M - 1)]);
 #pragma unroll
             for (int j = 0; j < TN; ++j) {
                 const int n = n0 + wn * (BN / 2) + j * 32 + li;

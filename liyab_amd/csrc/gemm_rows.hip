@@ -70,7 +70,9 @@ __device__ __forceinline__ void in_turn(std::integer_sequence<int, T...>, F&& f)
 
 // MR: rows of the ring (rows: 8, 16 or 32, M rounded up; otherwise 0). RING: units of the ring, or (norm, splits) sets of three units in
 // registers, 1 or 2. FORM: pieces of 4 a lane of a row (norm), splits merged at most (splits), not read (rows).
-template <typename OutT, int NB, int MR, int SRC, int FORM, int RING>
+// EPI: the epilogue, fixed at compile time (the rarer activations: -1): a kernel this short waits for its own instructions, cold in every launch of a chain
+// (norm and product at 768 -> 3,072, 8 rows: 4.6 us with all epilogues and three forms of the norm in 3,300 instructions, 4.2 with 1,400).
+template <typename OutT, int NB, int MR, int SRC, int FORM, int RING, int EPI>
 __global__ void __launch_bounds__(64 * SUMS)
 gemm_rows_kernel(Source src, const bf16_t* __restrict__ w, int M_all, int N, int K, EpiParams epi) {
     static_assert((SRC == kRows) == (MR > 0) && NB % 8 == 0 && MR % 8 == 0, "whole loads");
@@ -122,8 +124,8 @@ gemm_rows_kernel(Source src, const bf16_t* __restrict__ w, int M_all, int N, int
     typedef const __attribute__((address_space(1))) float* global_floats;
     const auto nothing = (global_floats)(w);
     auto bias_at = epi.bias != nullptr ? (global_floats)(epi.bias + e_n) : nothing;
-    auto word_at = epi.mode == kEpiResidual   ? (global_floats)(epi.residual + static_cast<int64_t>(e_m) * epi.ldr + e_n)
-                   : epi.mode == kEpiQkvPaged ? (global_floats)(epi.slots + e_m)
+    auto word_at = EPI == kEpiResidual   ? (global_floats)(epi.residual + static_cast<int64_t>(e_m) * epi.ldr + e_n)
+                   : EPI == kEpiQkvPaged ? (global_floats)(epi.slots + e_m)
                                               : nothing;
     asm volatile("" : "+v"(bias_at), "+v"(word_at));  // (worked out here, ahead of every load)
     float e_bias;
@@ -156,14 +158,14 @@ gemm_rows_kernel(Source src, const bf16_t* __restrict__ w, int M_all, int N, int
         const floatx4 zero = {0.0f, 0.0f, 0.0f, 0.0f}, one = {1.0f, 1.0f, 1.0f, 1.0f};
         const float* const weight = src.weight != nullptr ? src.weight : src.x;  // (without one: a row's values, read and dropped)
         const float* const bias = src.bias != nullptr ? src.bias : src.x;
-        auto norm_rows = [&](auto count, int m, auto&& between) {
-            constexpr int R = decltype(count)::value;
+        auto norm_rows = [&](int m, auto&& between) {  // rows m and m + 4 (past the last: the last again, not kept)
+            constexpr int R = 2;
             floatx4 v[R][FORM], gw[FORM], gb[FORM];
 #pragma unroll
             for (int j = 0; j < FORM; ++j) {
                 const int at = min(lane + kWave * j, nv - 1);  // past the row: its last piece again, unused
 #pragma unroll
-                for (int r = 0; r < R; ++r) v[r][j] = reinterpret_cast<const floatx4*>(src.x + static_cast<int64_t>(row0 + m + SUMS * r) * K)[at];
+                for (int r = 0; r < R; ++r) v[r][j] = reinterpret_cast<const floatx4*>(src.x + static_cast<int64_t>(row0 + min(m + SUMS * r, M - 1)) * K)[at];
                 gw[j] = reinterpret_cast<const floatx4*>(weight)[at];
                 gb[j] = reinterpret_cast<const floatx4*>(bias)[at];
             }
@@ -197,18 +199,13 @@ gemm_rows_kernel(Source src, const bf16_t* __restrict__ w, int M_all, int N, int
                 for (int r = 0; r < R; ++r) {
                     const floatx4 y = (v[r][j] - mean[r]) * scale[r] * gw[j] + gb[j];
                     const float four[4] = {y[0], y[1], y[2], y[3]};
-                    if (lane + kWave * j < nv) store4<bf16_t>(xs + (m + SUMS * r) * ldx + 4 * (lane + kWave * j), four);
+                    if (lane + kWave * j < nv && m + SUMS * r < M) store4<bf16_t>(xs + (m + SUMS * r) * ldx + 4 * (lane + kWave * j), four);
                 }
             }
         };
-        auto nothing = []() {};
-        if (wave + SUMS < M) norm_rows(std::integral_constant<int, 2>{}, wave, ask);
-        else if (wave < M) norm_rows(std::integral_constant<int, 1>{}, wave, ask);
+        if (wave < M) norm_rows(wave, ask);
         else ask();
-        for (int m = wave + 2 * SUMS; m < M; m += 2 * SUMS) {
-            if (m + SUMS < M) norm_rows(std::integral_constant<int, 2>{}, m, nothing);
-            else norm_rows(std::integral_constant<int, 1>{}, m, nothing);
-        }
+        for (int m = wave + 2 * SUMS; m < M; m += 2 * SUMS) norm_rows(m, []() {});
         lds_barrier();  // the weights may still be on their way
     } else {
         // four consecutive k of a token a thread and item, merged over the splits; ITEMS items' loads in flight together
@@ -336,33 +333,34 @@ gemm_rows_kernel(Source src, const bf16_t* __restrict__ w, int M_all, int N, int
         float v = red[j * (ROWS + 1) + m];
 #pragma unroll
         for (int q = 1; q < SUMS; ++q) v += red[(q * NB + j) * (ROWS + 1) + m];
-        if (e != tid) {
-            epilogue_store<OutT>(epi, row0 + m, n, v);
-            continue;
-        }
-        v += epi.bias != nullptr ? e_bias : 0.0f;
-        if (epi.mode == kEpiResidual) {
-            epi.residual[static_cast<int64_t>(e_m) * epi.ldr + n] = e_word + v;
-        } else if (epi.mode == kEpiQkvPaged && n >= epi.q_dim) {
-            const uint32_t at = __float_as_uint(e_word), page = at / static_cast<uint32_t>(epi.page_size), off = at - page * static_cast<uint32_t>(epi.page_size);
-            if (at >= epi.num_slots) continue;  // no slot (-1), or none of these caches
-            const bool is_v = n >= epi.q_dim + epi.kv_dim;
-            const int c = n - epi.q_dim - (is_v ? epi.kv_dim : 0), head = c / epi.hd;
-            OutT* const pages = static_cast<OutT*>(is_v ? epi.vc : epi.kc);
-            pages[((static_cast<int64_t>(page) * epi.n_kv_head + head) * epi.page_size + off) * epi.hd + c - head * epi.hd] = from_float<OutT>(v);
-        } else if (epi.mode == kEpiQkvPaged) {
-            static_cast<OutT*>(epi.out)[static_cast<int64_t>(e_m) * epi.ldo + n] = from_float<OutT>(v);
+        // (a thread's later outputs read what they need here)
+        const bool first = e == tid;
+        const float bias = first ? e_bias : epi.bias != nullptr ? epi.bias[n] : 0.0f;
+        if (epi.bias != nullptr) v += bias;
+        if constexpr (EPI == kEpiResidual) {
+            float* const at = epi.residual + static_cast<int64_t>(row0 + m) * epi.ldr + n;
+            *at = (first ? e_word : *at) + v;
+        } else if constexpr (EPI == kEpiQkvPaged) {
+            if (n < epi.q_dim) {
+                static_cast<OutT*>(epi.out)[static_cast<int64_t>(row0 + m) * epi.ldo + n] = from_float<OutT>(v);
+            } else {
+                const int64_t at = qkv_row_base(epi, first ? __float_as_int(e_word) : epi.slots[row0 + m]);
+                if (at < 0) continue;
+                const bool is_v = n >= epi.q_dim + epi.kv_dim;
+                const int c = n - epi.q_dim - (is_v ? epi.kv_dim : 0), head = c / epi.hd;
+                static_cast<OutT*>(is_v ? epi.vc : epi.kc)[at + static_cast<int64_t>(head) * epi.page_size * epi.hd + (c - head * epi.hd)] = from_float<OutT>(v);
+            }
         } else {
-            epilogue_store_biased<OutT, -1>(epi, e_m, n, v);
+            epilogue_store_biased<OutT, EPI>(epi, row0 + m, n, v);
         }
     }
 }
 
-template <typename OutT, int NB, int MR, int SRC, int FORM, int RING>
+template <typename OutT, int NB, int MR, int SRC, int FORM, int RING, int EPI>
 int launch_as(const Source& src, const bf16_t* w, int M, int N, int K, const EpiParams& epi, hipStream_t stream) {
     const size_t smem = ring_bytes<NB, MR, RING>() + (SRC == kRows ? 0 : static_cast<size_t>(M < ROWS ? M : ROWS) * (K + 8) * 2);
     LIYAB_REQUIRE(smem <= 160 * 1024, "gemm_rows: %d rows of %d need %zu bytes of LDS", M, K, smem);
-    auto kern = gemm_rows_kernel<OutT, NB, MR, SRC, FORM, RING>;
+    auto kern = gemm_rows_kernel<OutT, NB, MR, SRC, FORM, RING, EPI>;
     static bool ready = false;  // once per instantiation, outside any stream capture's first use
     if (!ready) {
         hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
@@ -373,35 +371,35 @@ int launch_as(const Source& src, const bf16_t* w, int M, int N, int K, const Epi
 }
 
 // The units a wave has in flight: all of them up to 768 k; beyond, as many as the LDS holds of 6 and 12, or six in registers.
-template <typename OutT, int NB, int MR, int SRC, int FORM>
+template <typename OutT, int NB, int MR, int SRC, int FORM, int EPI>
 int launch_ring(const Source& src, const bf16_t* w, int M, int N, int K, const EpiParams& epi, hipStream_t stream) {
     const int units = (K / UNIT + SUMS - 1) / SUMS;  // a wave's
     if constexpr (SRC == kRows) {
         constexpr int most = 288 / (NB + MR);
         if constexpr (most >= 12)
-            if (units > 6) return launch_as<OutT, NB, MR, SRC, FORM, 12>(src, w, M, N, K, epi, stream);
+            if (units > 6) return launch_as<OutT, NB, MR, SRC, FORM, 12, EPI>(src, w, M, N, K, epi, stream);
         if constexpr (most >= 6)
-            if (units > 3) return launch_as<OutT, NB, MR, SRC, FORM, 6>(src, w, M, N, K, epi, stream);
-        return launch_as<OutT, NB, MR, SRC, FORM, 3>(src, w, M, N, K, epi, stream);
+            if (units > 3) return launch_as<OutT, NB, MR, SRC, FORM, 6, EPI>(src, w, M, N, K, epi, stream);
+        return launch_as<OutT, NB, MR, SRC, FORM, 3, EPI>(src, w, M, N, K, epi, stream);
     } else {
-        return units > 3 ? launch_as<OutT, NB, MR, SRC, FORM, 2>(src, w, M, N, K, epi, stream) : launch_as<OutT, NB, MR, SRC, FORM, 1>(src, w, M, N, K, epi, stream);
+        return units > 3 ? launch_as<OutT, NB, MR, SRC, FORM, 2, EPI>(src, w, M, N, K, epi, stream) : launch_as<OutT, NB, MR, SRC, FORM, 1, EPI>(src, w, M, N, K, epi, stream);
     }
 }
-template <typename OutT, int NB, int SRC>
+template <typename OutT, int NB, int SRC, int EPI>
 int launch_form(const Source& src, const bf16_t* w, int M, int N, int K, const EpiParams& epi, hipStream_t stream) {
     if constexpr (SRC == kRows) {
-        if (M <= 8) return launch_ring<OutT, NB, 8, SRC, 0>(src, w, M, N, K, epi, stream);
-        if (M <= 16) return launch_ring<OutT, NB, 16, SRC, 0>(src, w, M, N, K, epi, stream);
-        return launch_ring<OutT, NB, 32, SRC, 0>(src, w, M, N, K, epi, stream);
+        if (M <= 8) return launch_ring<OutT, NB, 8, SRC, 0, EPI>(src, w, M, N, K, epi, stream);
+        if (M <= 16) return launch_ring<OutT, NB, 16, SRC, 0, EPI>(src, w, M, N, K, epi, stream);
+        return launch_ring<OutT, NB, 32, SRC, 0, EPI>(src, w, M, N, K, epi, stream);
     } else if constexpr (SRC == kNorm) {
-        if (K <= 768) return launch_ring<OutT, NB, 0, SRC, 3>(src, w, M, N, K, epi, stream);
-        return K <= 1024 ? launch_ring<OutT, NB, 0, SRC, 4>(src, w, M, N, K, epi, stream) : launch_ring<OutT, NB, 0, SRC, 8>(src, w, M, N, K, epi, stream);
+        if (K <= 768) return launch_ring<OutT, NB, 0, SRC, 3, EPI>(src, w, M, N, K, epi, stream);
+        return K <= 1024 ? launch_ring<OutT, NB, 0, SRC, 4, EPI>(src, w, M, N, K, epi, stream) : launch_ring<OutT, NB, 0, SRC, 8, EPI>(src, w, M, N, K, epi, stream);
     } else {
-        return src.n_splits <= 4 ? launch_ring<OutT, NB, 0, SRC, 4>(src, w, M, N, K, epi, stream) : launch_ring<OutT, NB, 0, SRC, 8>(src, w, M, N, K, epi, stream);
+        return src.n_splits <= 4 ? launch_ring<OutT, NB, 0, SRC, 4, EPI>(src, w, M, N, K, epi, stream) : launch_ring<OutT, NB, 0, SRC, 8, EPI>(src, w, M, N, K, epi, stream);
     }
 }
 
-template <typename OutT, int SRC>
+template <typename OutT, int SRC, int EPI>
 int launch_strip(const Source& src, const bf16_t* w, int M, int N, int K, int strip, const EpiParams& epi, hipStream_t stream) {
     if (strip == 0) {
         // the narrowest strips that still have a compute unit each (128 combinations of K and N up to 8,192, 1 to 64 rows: within 3 % of the best of the
@@ -413,11 +411,31 @@ int launch_strip(const Source& src, const bf16_t* w, int M, int N, int K, int st
         if (SRC == kRows && N > 32 * 256 && K <= 1280) strip = 16;
     }
     switch (strip) {
-        case 8: return launch_form<OutT, 8, SRC>(src, w, M, N, K, epi, stream);
-        case 16: return launch_form<OutT, 16, SRC>(src, w, M, N, K, epi, stream);
-        case 32: return launch_form<OutT, 32, SRC>(src, w, M, N, K, epi, stream);
+        case 8: return launch_form<OutT, 8, SRC, EPI>(src, w, M, N, K, epi, stream);
+        case 16: return launch_form<OutT, 16, SRC, EPI>(src, w, M, N, K, epi, stream);
+        case 32: return launch_form<OutT, 32, SRC, EPI>(src, w, M, N, K, epi, stream);
         default: return fail(1, "gemm_rows: strips of %d features (8, 16 or 32)", strip);
     }
+}
+
+template <int SRC>
+int launch_epi(const Source& src, const bf16_t* w, int M, int N, int K, int strip, const EpiParams& epi, hipStream_t stream) {
+#define LIYAB_ROWS(OUT, EPI) launch_strip<OUT, SRC, EPI>(src, w, M, N, K, strip, epi, stream)
+    if constexpr (SRC != kNorm)
+        if (epi.mode == kEpiResidual) return LIYAB_ROWS(float, kEpiResidual);
+    if constexpr (SRC != kSplits) {
+        if (epi.out_dtype == kF32) {
+            LIYAB_REQUIRE(epi.mode != kEpiQkvPaged, "gemm_rows: bfloat16 rows go to bfloat16 pages");
+            if (SRC == kRows && epi.mode == kEpiNone) return LIYAB_ROWS(float, kEpiNone);
+            if (epi.mode <= kEpiGeluErf) return LIYAB_ROWS(float, -1);
+        } else {
+            if (epi.mode == kEpiGeluTanh) return LIYAB_ROWS(bf16_t, kEpiGeluTanh);
+            if (epi.mode == kEpiQkvPaged) return LIYAB_ROWS(bf16_t, kEpiQkvPaged);
+            if (epi.mode <= kEpiGeluErf) return LIYAB_ROWS(bf16_t, -1);
+        }
+    }
+#undef LIYAB_ROWS
+    return fail(1, "gemm_rows: epilogue %d is not taken", epi.mode);
 }
 
 static bool al16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
@@ -443,9 +461,7 @@ extern "C" int liyab_gemm_rows(const void* a, int64_t lda, const void* w, int M,
     Source src{};
     src.a = static_cast<const bf16_t*>(a);
     src.lda = lda;
-    auto* pw = static_cast<const bf16_t*>(w);
-    if (epi->mode == kEpiResidual || epi->out_dtype == kF32) return launch_strip<float, kRows>(src, pw, M, N, K, strip, *epi, stream);
-    return launch_strip<bf16_t, kRows>(src, pw, M, N, K, strip, *epi, stream);
+    return launch_epi<kRows>(src, static_cast<const bf16_t*>(w), M, N, K, strip, *epi, stream);
 }
 
 // The same over LayerNorm(x) of 32-bit rows x [M, K], K <= 2048.
@@ -462,9 +478,7 @@ extern "C" int liyab_gemm_rows_ln(const float* x, const float* ln_weight, const 
     src.weight = ln_weight;
     src.bias = ln_bias;
     src.eps = eps;
-    auto* pw = static_cast<const bf16_t*>(w);
-    if (epi->out_dtype == kF32) return launch_strip<float, kNorm>(src, pw, M, N, K, strip, *epi, stream);
-    return launch_strip<bf16_t, kNorm>(src, pw, M, N, K, strip, *epi, stream);
+    return launch_epi<kNorm>(src, static_cast<const bf16_t*>(w), M, N, K, strip, *epi, stream);
 }
 
 // residual += merge(partials) . w^T + bias over attention's splits [M][n_head][n_splits <= 8][hd + 4] (liyab_attention_decode with
@@ -482,5 +496,5 @@ extern "C" int liyab_gemm_rows_splits(const float* partials, int n_splits, int n
     src.n_splits = n_splits;
     src.n_head = n_head;
     src.hd = hd;
-    return launch_strip<float, kSplits>(src, static_cast<const bf16_t*>(w), M, N, n_head * hd, strip, *epi, stream);
+    return launch_epi<kSplits>(src, static_cast<const bf16_t*>(w), M, N, n_head * hd, strip, *epi, stream);
 }

@@ -46,7 +46,10 @@ struct NormParams {
     const float* alpha;   // null: LayerNorm. Else the Dynamic Tanh norm, tanh(alpha[0] x) * weight + bias (no statistics)
 };
 
-template <typename OutT, int MAXV, int MT, int NT>
+// EPI, DYT: the epilogue (-1: read from the parameters) and the norm, fixed at compile time: a kernel this short waits for its own instructions, cold in
+// every launch of a chain (a decode step of one request, 24 of its 66 kernels these: 327 us with both norms and all epilogues in one kernel, which divided slots
+// in 64 bits and asked for the norm's weight and bias under branches, 318 so; of eight 423 and 414).
+template <typename OutT, int MAXV, int MT, int NT, int EPI, bool DYT>
 __global__ void __launch_bounds__(64 * LN_WAVES)
 gemm_skinny_ln_kernel(NormParams ln, const bf16_t* __restrict__ w, int M, int N, int K, EpiParams epi) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
@@ -83,14 +86,19 @@ gemm_skinny_ln_kernel(NormParams ln, const bf16_t* __restrict__ w, int M, int N,
         }
     };
     Frag wc[2][NT][2];
-    // this thread's first output: tile tid / 256 = (row tile, feature tile)
-    const int e_m = 16 * ((tid / 256) / NT) + (tid % 256) / 16, e_n = n0 + 16 * ((tid / 256) % NT) + tid % 16;
-    const bool e_mine = tid < TILES * 256 && e_m < M && e_n < N;
+    // this thread's first output: tile tid / 256 = (row tile, feature tile), and what its epilogue reads, its bias and its row's slot. No load under a
+    // branch, which would be waited for where the branch ends: who has nothing to read gets a word of the weights.
+    const int e_m = min(16 * ((tid / 256 % TILES) / NT) + (tid % 256) / 16, M - 1), e_n = min(n0 + 16 * ((tid / 256) % NT) + tid % 16, N - 1);
+    const float* const bias_at = epi.bias != nullptr ? epi.bias + e_n : reinterpret_cast<const float*>(w);
+    const int* const slot_at = EPI == kEpiQkvPaged ? epi.slots + e_m : reinterpret_cast<const int*>(w);
     float e_bias = 0.0f;
+    int e_slot = 0;
 
     // -- the norm: a wave per row, the row in registers ---------------------------------
     const int nv = K / 4;
     const floatx4 fzero = {0.0f, 0.0f, 0.0f, 0.0f}, fone = {1.0f, 1.0f, 1.0f, 1.0f};
+    const float* const norm_weight = ln.weight != nullptr ? ln.weight : ln.planes;  // (without one: a row's values, read and dropped)
+    const float* const norm_bias = ln.bias != nullptr ? ln.bias : ln.planes;
     // `between` runs once the row's first loads are asked for and before anything waits for them
     auto norm_row = [&](int m, bool keep, auto&& between) {
         const float* row0 = ln.planes + static_cast<int64_t>(m) * K;
@@ -101,8 +109,8 @@ gemm_skinny_ln_kernel(NormParams ln, const bf16_t* __restrict__ w, int M, int N,
         for (int j = 0; j < MAXV; ++j) {
             const int at = min(lane + kWave * j, nv - 1);  // past the row: its last piece again, unused
             v[j] = reinterpret_cast<const floatx4*>(row0)[at];
-            gw[j] = ln.weight != nullptr ? reinterpret_cast<const floatx4*>(ln.weight)[at] : fone;
-            gb[j] = ln.bias != nullptr ? reinterpret_cast<const floatx4*>(ln.bias)[at] : fzero;
+            gw[j] = reinterpret_cast<const floatx4*>(norm_weight)[at];
+            gb[j] = reinterpret_cast<const floatx4*>(norm_bias)[at];
         }
         // further planes, PB together (a plane past the last is the last one again, read and dropped)
         constexpr int PB = MAXV <= 4 ? 3 : 1;  // what the registers hold
@@ -126,7 +134,12 @@ gemm_skinny_ln_kernel(NormParams ln, const bf16_t* __restrict__ w, int M, int N,
                 for (int j = 0; j < MAXV; ++j)
                     if (q0 + u < ln.n_planes) v[j] += plane[u][j];
         }
-        if (ln.alpha != nullptr) {
+#pragma unroll
+        for (int j = 0; j < MAXV; ++j) {
+            gw[j] = ln.weight != nullptr ? gw[j] : fone;
+            gb[j] = ln.bias != nullptr ? gb[j] : fzero;
+        }
+        if constexpr (DYT) {
             // tanh(z) = 1 - 2 / (1 + e^(2z)): one hardware exponential and one reciprocal a value
             const float a2 = 2.0f * 1.4426950408889634f * ln.alpha[0];
 #pragma unroll
@@ -172,7 +185,8 @@ gemm_skinny_ln_kernel(NormParams ln, const bf16_t* __restrict__ w, int M, int N,
     // which come from further away and arrive while the norm is computed.
     auto ask_weights = [&]() {
         load_w(wave * 2, wc);
-        e_bias = (e_mine && epi.bias != nullptr) ? epi.bias[e_n] : 0.0f;
+        e_bias = *bias_at;
+        if constexpr (EPI == kEpiQkvPaged) e_slot = *slot_at;
     };
     // (a wave past the last row asks for its weights only: a compute unit takes 64 bytes a cycle from
     // its cache, and eight waves that each ask for a row in four planes and the norm's two vectors
@@ -238,17 +252,30 @@ gemm_skinny_ln_kernel(NormParams ln, const bf16_t* __restrict__ w, int M, int N,
 #pragma unroll
         for (int q = 0; q < LN_WAVES; ++q) v += red[q * TILES * 256 + e];
         if (m >= M || n >= N) continue;
-        if (e == tid) epilogue_store_biased<OutT>(epi, m, n, v + e_bias);
-        else epilogue_store<OutT>(epi, m, n, v);
+        const bool first = e == tid;
+        if (epi.bias != nullptr) v += first ? e_bias : epi.bias[n];
+        if constexpr (EPI == kEpiQkvPaged) {
+            if (n >= epi.q_dim) {
+                const int64_t at = qkv_row_base(epi, first ? e_slot : epi.slots[m]);
+                if (at < 0) continue;
+                const bool is_v = n >= epi.q_dim + epi.kv_dim;
+                const int c = n - epi.q_dim - (is_v ? epi.kv_dim : 0), head = c / epi.hd;
+                static_cast<OutT*>(is_v ? epi.vc : epi.kc)[at + static_cast<int64_t>(head) * epi.page_size * epi.hd + (c - head * epi.hd)] = from_float<OutT>(v);
+            } else {
+                static_cast<OutT*>(epi.out)[static_cast<int64_t>(m) * epi.ldo + n] = from_float<OutT>(v);
+            }
+        } else {
+            epilogue_store_biased<OutT, EPI>(epi, m, n, v);
+        }
     }
 }
 
-template <typename OutT, int MAXV, int MT, int NT>
+template <typename OutT, int MAXV, int MT, int NT, int EPI, bool DYT>
 int launch_kernel(const NormParams& ln, const void* w, int M, int N, int K, const EpiParams& epi, hipStream_t stream) {
     const dim3 grid((N + 16 * NT - 1) / (16 * NT));
     const size_t smem = ((static_cast<size_t>(M) * (K + 8) * 2 + 15) / 16) * 16 + LN_WAVES * MT * NT * 256 * sizeof(float);
     LIYAB_REQUIRE(smem <= 160 * 1024, "gemm_skinny_ln: %d rows of %d need %zu bytes of LDS", M, K, smem);
-    auto kern = gemm_skinny_ln_kernel<OutT, MAXV, MT, NT>;
+    auto kern = gemm_skinny_ln_kernel<OutT, MAXV, MT, NT, EPI, DYT>;
     static bool ready = false;
     if (!ready) {
         hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
@@ -261,15 +288,20 @@ int launch_kernel(const NormParams& ln, const void* w, int M, int N, int K, cons
 // A workgroup keeps a row in registers and so fills a compute unit: with more strips of 16
 // output features than compute units a workgroup takes two strips, or the workgroups would run
 // in two rounds (one tile of rows only: with more rows the sums across waves fill the LDS).
-template <typename OutT, int MAXV>
+template <typename OutT, int MAXV, int EPI, bool DYT>
 int launch_rows(const NormParams& ln, const void* w, int M, int N, int K, int wide, const EpiParams& epi, hipStream_t stream) {
-    if (M <= 16) return wide ? launch_kernel<OutT, MAXV, 1, 2>(ln, w, M, N, K, epi, stream) : launch_kernel<OutT, MAXV, 1, 1>(ln, w, M, N, K, epi, stream);
-    return launch_kernel<OutT, MAXV, 2, 1>(ln, w, M, N, K, epi, stream);
+    if (M <= 16) return wide ? launch_kernel<OutT, MAXV, 1, 2, EPI, DYT>(ln, w, M, N, K, epi, stream) : launch_kernel<OutT, MAXV, 1, 1, EPI, DYT>(ln, w, M, N, K, epi, stream);
+    return launch_kernel<OutT, MAXV, 2, 1, EPI, DYT>(ln, w, M, N, K, epi, stream);
 }
 template <int MAXV>
 int launch_ln(const NormParams& ln, const void* w, int M, int N, int K, int wide, const EpiParams& epi, hipStream_t stream) {
-    if (epi.out_dtype == kF32) return launch_rows<float, MAXV>(ln, w, M, N, K, wide, epi, stream);
-    return launch_rows<bf16_t, MAXV>(ln, w, M, N, K, wide, epi, stream);
+#define LIYAB_LN(OUT, EPI, DYT) launch_rows<OUT, MAXV, EPI, DYT>(ln, w, M, N, K, wide, epi, stream)
+    const bool f32 = epi.out_dtype == kF32;
+    if (ln.alpha != nullptr) return f32 ? LIYAB_LN(float, -1, true) : LIYAB_LN(bf16_t, -1, true);
+    if (f32) return LIYAB_LN(float, -1, false);
+    if (epi.mode == kEpiQkvPaged) return LIYAB_LN(bf16_t, kEpiQkvPaged, false);
+    return epi.mode == kEpiGeluTanh ? LIYAB_LN(bf16_t, kEpiGeluTanh, false) : LIYAB_LN(bf16_t, -1, false);
+#undef LIYAB_LN
 }
 
 }  // namespace ln_fold
