@@ -1501,3 +1501,10 @@ def test_rows_update_by_waves_keeps_the_rows(ops, d, also):
         assert torch.equal(state, want)
         got.append(into)
     assert torch.equal(got[0], got[1])
+
+
+@pytest.mark.parametrize("V", [330, 600, 4093, 4100, 9000, 20000])
+def test_sampler_at_few_ids_a_thread(ops, V):
+    """The same rules where the floor for the k-th largest is found among the threads' largest keys and among those of four neighbours (from 512 such
+    values on), with ties at the boundary inside and outside the pool."""
+    test_sampler_against_the_plain_sampler(ops, V)
