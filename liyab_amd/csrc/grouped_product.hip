@@ -20,6 +20,9 @@
 #include "common.h"
 #include "launchers.h"
 
+#include <type_traits>
+#include <utility>
+
 namespace liyab {
 
 constexpr int kGroupedRows = 64;  // rows a tile; liyab_moe_align lays its lists out in these,
@@ -581,6 +584,174 @@ grouped_plain_kernel(GroupedParams p) {
     }
 }
 
+// The same product, bit for bit, for whole units of K (a multiple of 64): what bounds it is its chain of trips to memory, the lists, then the
+// weights of the expert that they name, unit after unit. The tile's group, its rows and what the epilogue reads are asked for together, and a wave's
+// units come into a ring in LDS of its own (8 rows of 64 k a load, whole cache lines), R of them in flight, waited for one by one without a barrier.
+// us, cold weights, before / now: of 8 experts, 768 -> 2 x 1,536, 2 entries 6.7 / 6.3, 16 entries 11.7 / 9.5, 120 entries 16.7 / 13.4; 1,536 -> 768 16 entries
+// 8.5 / 7.4, 120 12.3 / 8.7; of 16 experts, 1,600 -> 2 x 3,200, 16 entries 62 / 45; 4 rows of 12 heads, 64 -> 128 3.5 / 3.35, 128 -> 64 with a gate 3.7 / 3.55;
+// 128 rows, 256 -> 512 10.4 / 7.3.
+typedef __attribute__((address_space(3))) void* gp_lds_ptr;
+__device__ __forceinline__ int gp_ring_swizzle(int row) { return (row >> 1) & 7; }  // 16 rows' reads of one 16-byte piece fall into different banks
+template <int LATER>
+__device__ __forceinline__ void gp_wait_loads() {  // this wave's loads but the last LATER have arrived
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt((LATER & 15) | 0x0f70 | ((LATER >> 4) << 14));
+    asm volatile("" ::: "memory");
+}
+template <int... T, typename F>
+__device__ __forceinline__ void gp_in_turn(std::integer_sequence<int, T...>, F&& f) {
+    (f(std::integral_constant<int, T>{}), ...);
+}
+
+// LISTED: rows by a router's lists; FACTORS: a row's scale or a gate on the output.
+template <int NW, int R, bool LISTED, bool FACTORS>
+__global__ void __launch_bounds__(256)
+grouped_stream_kernel(GroupedParams p) {
+    constexpr int ROWS = 16 * (1 + NW), LOADS = ROWS / 8, SLOT = ROWS * 64;
+    static_assert((R - 1) * LOADS <= 63, "the counter of loads in flight has six bits");
+    constexpr size_t RING = static_cast<size_t>(4) * R * SLOT * 2, SUMS = 4 * NW * 256 * 4;
+    __shared__ __attribute__((aligned(1024))) unsigned char lds[RING > SUMS ? RING : SUMS];
+    float* const red = reinterpret_cast<float*>(lds);
+    const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
+    const int i = lane % 16, q = lane / 16, lrow = lane / 8, lpos = lane % 8;
+    const int tile = blockIdx.x, N = p.N, K = p.K, n0 = blockIdx.y * 16;
+    bf16_t* const ring = reinterpret_cast<bf16_t*>(lds) + wave * R * SLOT;
+    // the rows this lane brings in (places lrow and lrow + 8) and the one it stores (place tid / 16), together with the tile's group
+    int g, id[2], e_id;
+    if constexpr (LISTED) {
+        const int* const places = p.rows_list + tile * kSkinnyRows;
+        const int group = p.tile_group[tile];
+        id[0] = places[lrow];
+        id[1] = places[lrow + 8];
+        e_id = places[tid / 16];
+        g = __builtin_amdgcn_readfirstlane(group);
+        if (g < 0) return;
+    } else {
+        const int m0 = tile * kSkinnyRows;
+        g = blockIdx.z;
+        id[0] = m0 + lrow < p.M ? m0 + lrow : -1;
+        id[1] = m0 + lrow + 8 < p.M ? m0 + lrow + 8 : -1;
+        e_id = m0 + tid / 16 < p.M ? m0 + tid / 16 : -1;
+    }
+    // an empty place reads the first row, a feature past N the last one: computed, never stored
+    const bf16_t* from[LOADS];
+#pragma unroll
+    for (int l = 0; l < 2; ++l) {
+        const int piece = (lpos ^ gp_ring_swizzle(8 * l + lrow)) * 8;
+        const int row = LISTED ? (id[l] >= 0 ? id[l] / p.a_div : 0) : max(id[l], 0);
+        from[l] = static_cast<const bf16_t*>(p.a) + static_cast<int64_t>(row) * p.lda + static_cast<int64_t>(g) * p.a_group_cols + piece;
+        const int64_t wrow = (static_cast<int64_t>(g) * N + min(n0 + 8 * l + lrow, N - 1)) * K + piece;
+        from[2 + l] = static_cast<const bf16_t*>(p.w0) + wrow;
+        if constexpr (NW == 2) from[4 + l] = static_cast<const bf16_t*>(p.w1) + wrow;
+    }
+    const int units = K / 64, mine = (units - wave + 3) / 4;  // this wave's units: wave, wave + 4, ...
+    auto load = [&](int j, int slot) {  // (one past the last: the last of K again, not multiplied)
+        const int k = min(wave + 4 * j, units - 1) * 64;
+#pragma unroll
+        for (int l = 0; l < LOADS; ++l) {
+            const bf16_t* const piece = from[l] + k;
+            bf16_t* const to = ring + slot * SLOT + l * 8 * 64;
+            __builtin_amdgcn_global_load_lds(piece, (gp_lds_ptr)to, 16, 0, 0);
+        }
+    };
+    // what the epilogue reads, ahead of the weights; no load under a branch: who has nothing to read gets a word of the weights
+    const int n = n0 + tid % 16;
+    float e_scale = 1.0f, e_gate = 0.0f;
+    uint32_t e_gate_word = 0;
+    if constexpr (FACTORS) {
+        const int row = max(e_id, 0);
+        const int64_t ga = static_cast<int64_t>(row) * p.gate_stride + static_cast<int64_t>(g) * N + min(n, N - 1);
+        const float* const scale_at = p.row_scale != nullptr ? p.row_scale + row : static_cast<const float*>(p.w0);
+        const bf16_t* const gate16_at = p.gate != nullptr && p.gate_dtype == kBF16 ? static_cast<const bf16_t*>(p.gate) + ga : static_cast<const bf16_t*>(p.w0);
+        const float* const gate32_at = p.gate != nullptr && p.gate_dtype == kF32 ? static_cast<const float*>(p.gate) + ga : static_cast<const float*>(p.w0);
+        e_scale = *scale_at;
+        e_gate_word = *gate16_at;
+        e_gate = *gate32_at;
+    }
+    // (no load may cross to the other side: the waits below count on what is asked for behind them)
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int t = 0; t < R; ++t) load(t, t);
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("" ::: "memory");
+
+    gp_floatx4 acc[NW];
+#pragma unroll
+    for (int u = 0; u < NW; ++u) acc[u] = gp_floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+    auto multiply = [&](int slot) {
+        const bf16_t* const at = ring + slot * SLOT + i * 64;
+        GpFrag x[2], w[NW][2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int piece = ((4 * h + q) ^ gp_ring_swizzle(i)) * 8;
+            x[h].u = *reinterpret_cast<const gp_u32x4*>(at + piece);
+#pragma unroll
+            for (int u = 0; u < NW; ++u) w[u][h].u = *reinterpret_cast<const gp_u32x4*>(at + 16 * (1 + u) * 64 + piece);
+        }
+#pragma unroll
+        for (int u = 0; u < NW; ++u) {
+            acc[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[u][0].v, x[0].v, acc[u], 0, 0, 0);
+            acc[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[u][1].v, x[1].v, acc[u], 0, 0, 0);
+        }
+    };
+    int j0 = 0;
+    for (; j0 + R < mine; j0 += R)
+        gp_in_turn(std::make_integer_sequence<int, R>{}, [&](auto at) {
+            constexpr int t = decltype(at)::value;
+            gp_wait_loads<(R - 1) * LOADS>();
+            multiply(t);
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the place has been read
+            load(j0 + R + t, t);
+        });
+    gp_in_turn(std::make_integer_sequence<int, R>{}, [&](auto at) {
+        constexpr int t = decltype(at)::value;
+        gp_wait_loads<(R - 1 - t) * LOADS>();
+        if (j0 + t < mine) multiply(t);
+    });
+    lds_barrier();  // (the sums take the rings' place)
+#pragma unroll
+    for (int u = 0; u < NW; ++u)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) red[(wave * NW + u) * 256 + i * 16 + 4 * q + r] = acc[u][r];
+    lds_barrier();
+    float v[2] = {0.0f, 0.0f};
+#pragma unroll
+    for (int u = 0; u < NW; ++u)
+#pragma unroll
+        for (int wv = 0; wv < 4; ++wv) v[u] += red[(wv * NW + u) * 256 + tid];
+    if (e_id < 0 || n >= N) return;
+    float value = grouped_act<NW>(p, v[0], v[1]);
+    if constexpr (FACTORS) {
+        if (p.row_scale != nullptr) value *= e_scale;
+        if (p.gate != nullptr) value *= gp_sigmoid(p.gate_dtype == kF32 ? e_gate : bf16_to_float(static_cast<bf16_t>(e_gate_word)));
+    }
+    const int64_t at = grouped_place(p, e_id, g) + n;
+    if (p.out_dtype == kF32) static_cast<float*>(p.out)[at] = value;
+    else static_cast<bf16_t*>(p.out)[at] = float_to_bf16(value);
+}
+
+template <int NW>
+int launch_grouped_stream(const GroupedParams& p, const dim3& grid, hipStream_t stream) {
+    const int mine = (p.K / 64 + 3) / 4;  // units a wave
+    const bool factors = p.row_scale != nullptr || p.gate != nullptr;
+#define LIYAB_STREAM(R)                                                                                                        \
+    do {                                                                                                                       \
+        if (p.rows_list != nullptr && factors) grouped_stream_kernel<NW, R, true, true><<<grid, 256, 0, stream>>>(p);          \
+        else if (p.rows_list != nullptr) grouped_stream_kernel<NW, R, true, false><<<grid, 256, 0, stream>>>(p);               \
+        else if (factors) grouped_stream_kernel<NW, R, false, true><<<grid, 256, 0, stream>>>(p);                              \
+        else grouped_stream_kernel<NW, R, false, false><<<grid, 256, 0, stream>>>(p);                                          \
+    } while (0)
+    // Three units in flight, two where a unit has both halves' weights: 48 KiB of LDS, so that three workgroups share a compute unit (six units, 96 KiB and one
+    // workgroup: 16 entries of 16 experts, 3,200 -> 1,600, 33 us, three 24, two 25; 2 entries of 8, 1,536 -> 768 5.4, 5.4, 5.9. Both halves, three and two: 1,600 ->
+    // 2 x 3,200 49 and 45, 768 -> 2 x 768 7.0 and 7.2).
+    if (mine <= 1) LIYAB_STREAM(1);
+    else if (NW == 2 || mine <= 2) LIYAB_STREAM(2);
+    else LIYAB_STREAM(3);
+#undef LIYAB_STREAM
+    return check_launch("grouped_product");
+}
+
 }  // namespace liyab
 
 using namespace liyab;
@@ -613,6 +784,7 @@ extern "C" int liyab_grouped_product(const void* a, int64_t lda, int a_div, int 
     LIYAB_REQUIRE(block == kGroupedRows || matrix, "grouped_product: tiles of %d rows are for bfloat16 operands in 16-byte pieces", kSkinnyRows);
     if (block == kSkinnyRows) {
         const dim3 skinny(n_tiles, (N + 15) / 16, rows_list ? 1 : n_groups);
+        if (K % 64 == 0) return w1 != nullptr ? launch_grouped_stream<2>(p, skinny, stream) : launch_grouped_stream<1>(p, skinny, stream);
         if (w1 != nullptr) grouped_skinny_kernel<2><<<skinny, 256, 0, stream>>>(p);
         else grouped_skinny_kernel<1><<<skinny, 256, 0, stream>>>(p);
     } else if (matrix && K % 64 == 0 && (w1 == nullptr || gate == nullptr) && static_cast<int64_t>(n_tiles) * grid.y * grid.z < (1 << 24)) {

@@ -1508,3 +1508,35 @@ def test_sampler_at_few_ids_a_thread(ops, V):
     """The same rules where the floor for the k-th largest is found among the threads' largest keys and among those of four neighbours (from 512 such
     values on), with ties at the boundary inside and outside the pool."""
     test_sampler_against_the_plain_sampler(ops, V)
+
+@pytest.mark.parametrize("form", ["one", "relu2", "two", "clamped", "heads", "gated heads"])
+@pytest.mark.parametrize("K", [64, 192, 256, 448, 832, 1600])
+def test_products_of_whole_units_leave_the_bits_of_the_others(ops, form, K):
+    """Tiles of 16 places: the kernel for whole units of 64 k against the one for any K (held to the 32-bit reference above), which gets eight zeros more
+    a row: units a wave of none, one, and around the ring; rows and features at the edges of a tile, empty places, an unused tile."""
+    pad = lambda t: torch.nn.functional.pad(t, (0, 8)).contiguous()  # noqa: E731
+    for n, N in ((1, 3), (5, 40), (33, 16), (17, 130)):
+        if "heads" in form:
+            H = 3
+            a, w = rnd(n, H, K, dtype=torch.bfloat16), rnd(H, N, K, seed=1, scale=0.2, dtype=torch.bfloat16)
+            for gate in ((rnd(n, H * N, seed=2), rnd(n, H * N, seed=2, dtype=torch.bfloat16)) if form == "gated heads" else (None,)):
+                got, want = (torch.full((n, H * N), float("nan"), device=DEV) for _ in range(2))
+                ops.heads_product(got, a.reshape(n, H * K), w, gate)
+                ops.heads_product(want, pad(a).reshape(n, H * (K + 8)), pad(w), gate)
+                assert torch.equal(got, want), (n, N)
+            continue
+        E, two = 5, form in ("two", "clamped")
+        a, w0, w1 = rnd(n, K, dtype=torch.bfloat16), rnd(E, N, K, seed=1, scale=0.2, dtype=torch.bfloat16), rnd(E, N, K, seed=2, scale=0.2, dtype=torch.bfloat16)
+        expert = torch.randint(0, E - 1, (2 * n,), generator=torch.Generator().manual_seed(3))
+        tiles = ops.moe_tiles(2 * n, E, 16) + 1
+        rows, group, at = torch.full((tiles, 16), -1, dtype=torch.int32), torch.full((tiles,), -1, dtype=torch.int32), 0
+        for e in sorted(set(expert.tolist())):
+            for c in (expert == e).nonzero().flatten().int().split(16):
+                at += at == 1  # a tile nobody uses
+                rows[at, :len(c)], group[at], at = c, e, at + 1
+        for scale in (None, rnd(2 * n, seed=4)):
+            got, want = (torch.full((2 * n, N), float("nan"), device=DEV) for _ in range(2))
+            for out, x, u, v in ((got, a, w0, w1), (want, pad(a), pad(w0), pad(w1))):
+                ops.moe_product(out, x, u, v if two else None, rows.to(DEV).flatten(), group.to(DEV), a_div=2, row_scale=scale, block=16,
+                                act="relu2" if form == "relu2" else "none", clamp=(0.7, 1.702, 1.0) if form == "clamped" else None)
+            assert torch.equal(got, want), (n, N)
