@@ -251,19 +251,23 @@ __device__ __forceinline__ void in_turn(std::integer_sequence<int, T...>, F&& f)
     (f(std::integral_constant<int, T>{}), ...);
 }
 
-// EPI: an epilogue fixed at compile time (none, residual, or kEpiPlanes: planes with rows to add to); -1 reads it from the parameters.
-constexpr int kEpiPlanes = 5;
+// EPI: an epilogue fixed at compile time: none, residual, kEpiPlanes (planes with rows to add to), or a gated feed-forward's first product, kEpiGlu* (w = the
+// gate's N rows, then the other half's: a workgroup takes 16 features of both, and their 32-bit sums meet in act(gate) * other, as in
+// elementwise_norms.hip's kernel, whose link in the chain and trip through memory go); -1 reads it from the parameters.
+constexpr int kEpiPlanes = 5, kEpiGluSilu = 6, kEpiGluGelu = 7;
 template <typename OutT, int MR, int NT, int R, int EPI>
 __global__ void __launch_bounds__(1024)
 gemm_stream_kernel(const bf16_t* __restrict__ a, int64_t lda, const bf16_t* __restrict__ w, int M, int N, int K,
                    EpiParams epi, BaseSum base, int part_k, int64_t part_stride, int split_shift) {
+    constexpr bool GLU = EPI == kEpiGluSilu || EPI == kEpiGluGelu;
+    static_assert(!GLU || NT == 2, "one tile of the gate's features and one of the other half's");
     constexpr int NB = 16 * NT, LOADS = (NB + MR) / 8, SLOT = (NB + MR) * kUnit;
     static_assert((R - 1) * LOADS <= 63, "the counter of loads in flight has six bits");
     extern __shared__ __attribute__((aligned(1024))) unsigned char stream_lds[];
     float* const red = reinterpret_cast<float*>(stream_lds);  // [wave][NT][256], once the rings have been read
     const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64), waves = blockDim.x / 64;
     const int i = lane % 16, g = lane / 16;
-    const int n0 = blockIdx.x * NB, m0 = blockIdx.y * 16;
+    const int n0 = blockIdx.x * (GLU ? 16 : NB), m0 = blockIdx.y * 16;
     const int k_begin = blockIdx.z * part_k, k_end = min(K, k_begin + part_k);
     const int units = (k_end - k_begin) / kUnit, pairs = (units + 1) / 2;
     // this wave's units: those of pairs wave, wave + ksplit, ... (the last of all may be half a pair); ksplit = 1 << split_shift
@@ -277,7 +281,10 @@ gemm_stream_kernel(const bf16_t* __restrict__ a, int64_t lda, const bf16_t* __re
     const int lrow = lane / 8, lpos = lane % 8;  // this lane's part in a load
     const bf16_t* from[LOADS];
 #pragma unroll
-    for (int l = 0; l < 2 * NT; ++l) from[l] = w + static_cast<int64_t>(min(n0 + 8 * l + lrow, N - 1)) * K + k_begin + (lpos ^ ring_swizzle(8 * l + lrow)) * 8;
+    for (int l = 0; l < 2 * NT; ++l) {
+        const int row = GLU && l >= 2 ? N + min(n0 + 8 * (l - 2) + lrow, N - 1) : min(n0 + 8 * l + lrow, N - 1);
+        from[l] = w + static_cast<int64_t>(row) * K + k_begin + (lpos ^ ring_swizzle(8 * l + lrow)) * 8;
+    }
 #pragma unroll
     for (int l = 2 * NT; l < LOADS; ++l) {
         const int row = 8 * (l - 2 * NT) + lrow;
@@ -306,10 +313,10 @@ gemm_stream_kernel(const bf16_t* __restrict__ a, int64_t lda, const bf16_t* __re
     const int64_t base_stride = based ? base.stride : 0;
     const int base_last = based ? base.n - 1 : 0;
     asm volatile("" : "+v"(bias_at), "+v"(res_at));  // (worked out here, ahead of every load)
-    const float e_bias = *bias_at;
+    const float e_bias = GLU ? 0.0f : *bias_at;
     float e_res[4];
 #pragma unroll
-    for (int q = 0; q < (EPI == kEpiPlanes ? 4 : 1); ++q) e_res[q] = EPI == kEpiNone ? 0.0f : res_at[min(q, base_last) * base_stride];
+    for (int q = 0; q < (EPI == kEpiPlanes ? 4 : 1); ++q) e_res[q] = EPI == kEpiNone || GLU ? 0.0f : res_at[min(q, base_last) * base_stride];
     // (no load may cross to the other side: the waits below count on what is asked for behind them)
     asm volatile("" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
@@ -357,6 +364,19 @@ gemm_stream_kernel(const bf16_t* __restrict__ a, int64_t lda, const bf16_t* __re
 #pragma unroll
         for (int r = 0; r < 4; ++r) red[(wave * NT + t) * 256 + i * 16 + 4 * g + r] = acc[t][r];
     lds_barrier();
+    if constexpr (GLU) {
+        for (int e = tid; e < 256; e += blockDim.x) {
+            const int m = m0 + e / 16, n = n0 + e % 16;
+            if (m >= M || n >= N) continue;
+            float v[2] = {0.0f, 0.0f};
+            for (int q = 0; q < waves; ++q)
+#pragma unroll
+                for (int t = 0; t < 2; ++t) v[t] += red[(q * 2 + t) * 256 + e];
+            const float act = EPI == kEpiGluSilu ? v[0] * (1.0f / (1.0f + expf(-v[0]))) : gelu_tanh_fast(v[0]);
+            static_cast<OutT*>(epi.out)[static_cast<int64_t>(m) * epi.ldo + n] = from_float<OutT>(act * v[1]);
+        }
+        return;
+    }
     for (int e = tid; e < NT * 256; e += blockDim.x) {
         const int m = m0 + e % 256 / 16, n = n0 + 16 * (e / 256) + e % 16;
         if (m >= M || n >= N) continue;
@@ -399,7 +419,8 @@ int launch_stream_as(const bf16_t* a, int64_t lda, const bf16_t* w, int M, int N
         hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
         ready = true;
     }
-    kern<<<dim3((N + 16 * NT - 1) / (16 * NT), (M + 15) / 16, kparts), 64 * waves, smem, stream>>>(a, lda, w, M, N, K, epi, base, part_k, part_stride, __builtin_ctz(ksplit));
+    constexpr int wide = EPI >= kEpiGluSilu ? 16 : 16 * NT;  // output features a workgroup
+    kern<<<dim3((N + wide - 1) / wide, (M + 15) / 16, kparts), 64 * waves, smem, stream>>>(a, lda, w, M, N, K, epi, base, part_k, part_stride, __builtin_ctz(ksplit));
     return check_launch("gemm_skinny");
 }
 template <typename OutT, int EPI>
@@ -470,6 +491,16 @@ int launch_skinny(const void* a, int64_t lda, const void* w, int M, int N, int K
     return check_launch("gemm_skinny");
 }
 
+// Waves that share K: until each has one trip's worth of it (everything is then asked for at once),
+// or they cover the chip several times over.
+static int choose_ksplit(int tiles, int units, int per_trip) {
+    int ksplit = 1;
+    // (with so many output features that one wave a workgroup covers the chip, two or four
+    // still pay while a wave keeps more than 8 units: 18.3 against 20.0 us for 768 -> 50,257)
+    while (ksplit < 16 && units > ksplit * per_trip && (tiles * ksplit < 2048 || units / ksplit > 8)) ksplit *= 2;
+    return ksplit;
+}
+
 static int skinny_dispatch(const void* a, int64_t lda, const void* w, int M, int N, int K, int ksplit, int wide, int mtile,
                            const EpiParams& epi, const BaseSum& base, hipStream_t stream, int kparts = 1,
                            int64_t part_stride = 0) {
@@ -495,14 +526,8 @@ static int skinny_dispatch(const void* a, int64_t lda, const void* w, int M, int
     if (wide < 0) wide = (mt > 1 && static_cast<long>(N) * M > (1L << 20)) ? 1 : 0;
     const int nt = wide ? 4 : 1;
     if (ksplit == 0) {
-        // waves until each has one trip's worth of K (everything is then asked for at once),
-        // or they cover the chip several times over
         const int tiles = ((N + 16 * nt - 1) / (16 * nt)) * ((M + 16 * mt - 1) / (16 * mt)) * kparts;
-        const int units = ((K + 63) / 64 + kparts - 1) / kparts, per_trip = mt * nt == 1 ? 2 : 1;
-        ksplit = 1;
-        // (with so many output features that one wave a workgroup covers the chip, two or four
-        // still pay while a wave keeps more than 8 units: 18.3 against 20.0 us for 768 -> 50,257)
-        while (ksplit < 16 && units > ksplit * per_trip && (tiles * ksplit < 2048 || units / ksplit > 8)) ksplit *= 2;
+        ksplit = choose_ksplit(tiles, ((K + 63) / 64 + kparts - 1) / kparts, mt * nt == 1 ? 2 : 1);
     }
     LIYAB_REQUIRE(ksplit == 1 || ksplit == 2 || ksplit == 4 || ksplit == 8 || ksplit == 16,
                   "gemm_skinny: ksplit %d is not 1, 2, 4, 8 or 16", ksplit);
@@ -581,4 +606,29 @@ extern "C" int liyab_gemm_skinny_parts(const void* a, int64_t lda, const void* w
     // cut over K: 16 rows a workgroup (the parts cover the chip); whole: as the plain product chooses
     return skinny_dispatch(a, lda, w, M, N, K, ksplit, 0, kparts > 1 ? 1 : 0, epi, BaseSum{base, n_base, base_stride}, stream, kparts,
                            part_stride);
+}
+
+// A gated feed-forward's first product and its activation: out[m, n] = act(a[m] . w[n]) * (a[m] . w[ff + n]), a [M <= 16, K] and w [2 ff, K] bfloat16, out
+// [M, ff] bfloat16, K a multiple of 64 and not of 16,384; act 0: silu, 1: the tanh form of gelu. The bits of liyab_gemm_skinny to 32-bit rows followed by
+// liyab_glu. (8 rows, cold weights, us in two kernels and in one: 768 -> 2 x 2,048 6.8 and 5.0, 1,024 -> 2 x 2,720 7.5 and 5.5, 4,096 -> 2 x 8,064 30.0 and 26.8.)
+extern "C" int liyab_gemm_skinny_glu(const void* a, int64_t lda, const void* w, int M, int ff, int K, int act, void* out, int64_t ldo, hipStream_t stream) {
+    LIYAB_REQUIRE(a && w && out, "gemm_skinny_glu: null operand");
+    LIYAB_REQUIRE(M >= 0 && M <= 16 && ff > 0 && K > 0 && K % kUnit == 0 && K % 16384 != 0, "gemm_skinny_glu: bad sizes M=%d (at most 16) ff=%d K=%d", M, ff, K);
+    LIYAB_REQUIRE(lda % 8 == 0 && lda >= K && ldo >= ff, "gemm_skinny_glu: bad row strides %lld, %lld", static_cast<long long>(lda), static_cast<long long>(ldo));
+    LIYAB_REQUIRE((reinterpret_cast<uintptr_t>(a) & 15) == 0 && (reinterpret_cast<uintptr_t>(w) & 15) == 0, "gemm_skinny_glu: operands must be 16-byte aligned");
+    LIYAB_REQUIRE(act == 0 || act == 1, "gemm_skinny_glu: unknown activation %d", act);
+    if (M == 0) return 0;
+    EpiParams epi{};
+    epi.out_dtype = kBF16;
+    epi.out = out;
+    epi.ldo = ldo;
+    // (the waves that the product alone would have: the order of its sums)
+    const int units = K / kUnit, ksplit = choose_ksplit((2 * ff + 15) / 16, units, 2), pairs = (units + 1) / 2, live = ksplit < pairs ? ksplit : pairs;
+    const int rows = M <= 8 ? 8 : 16, waves = live < 4 ? 4 : live;
+    auto* pa = static_cast<const bf16_t*>(a);
+    auto* pw = static_cast<const bf16_t*>(w);
+#define LIYAB_GLU(MR, EPI) launch_stream_as<bf16_t, MR, 2, 2, EPI>(pa, lda, pw, M, ff, K, ksplit, waves, epi, BaseSum{nullptr, 0, 0}, 1, K, 0, stream)
+    if (rows == 8) return act == 0 ? LIYAB_GLU(8, kEpiGluSilu) : LIYAB_GLU(8, kEpiGluGelu);
+    return act == 0 ? LIYAB_GLU(16, kEpiGluSilu) : LIYAB_GLU(16, kEpiGluGelu);
+#undef LIYAB_GLU
 }

@@ -46,6 +46,7 @@ int liyab_gemm_rows_splits(const float* partials, int n_splits, int n_head, int 
                            const liyab::EpiParams* epi, hipStream_t stream);
 int liyab_gemm_skinny(const void* a, int64_t lda, const void* w, int M, int N, int K, int ksplit, int wide, int mtile,
                       const liyab::EpiParams* epi_in, hipStream_t stream);
+int liyab_gemm_skinny_glu(const void* a, int64_t lda, const void* w, int M, int ff, int K, int act, void* out, int64_t ldo, hipStream_t stream);
 int liyab_gemm_skinny_parts(const void* a, int64_t lda, const void* w, int M, int N, int K, int kparts, int ksplit, float* parts,
                             int64_t part_stride, const float* bias, const float* base, int n_base, int64_t base_stride,
                             hipStream_t stream);

@@ -86,6 +86,7 @@ static const Entry kEntries[] = {
     LIYAB_ENTRY(liyab_gemm_rows_ln),
     LIYAB_ENTRY(liyab_gemm_rows_splits),
     LIYAB_ENTRY(liyab_gemm_skinny),
+    LIYAB_ENTRY(liyab_gemm_skinny_glu),
     LIYAB_ENTRY(liyab_gemm_skinny_parts),
     LIYAB_ENTRY(liyab_gemm_att_parts),
     LIYAB_ENTRY(liyab_gemm_skinny_ln),

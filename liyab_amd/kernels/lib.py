@@ -53,6 +53,7 @@ _SIGNATURES = {
     "liyab_layernorm": [P, c_int, P, P, P, P, c_int, c_int, c_float, P],
     "liyab_layernorm_parts": [P, c_int, P, c_int, c_int64, c_int, P, P, P, c_int, c_int, c_float, P],
     "liyab_sum_parts": [P, c_int, c_int, P, c_int, c_int64, P],
+    "liyab_gemm_skinny_glu": [P, c_int64, P, c_int, c_int, c_int, c_int, P, c_int64, P],
     "liyab_gemm_skinny_parts": [P, c_int64, P, c_int, c_int, c_int, c_int, c_int, P, c_int64, P, P, c_int, c_int64, P],
     "liyab_gemm_simple": [P, c_int, c_int64, P, c_int64, P, c_int, P, P, c_int64, c_int, c_int, c_int, c_int, P],
     "liyab_gemm_f32_qkv": [P, c_int64, P, c_int, c_int, c_int, _EPI_PTR, P],

@@ -551,7 +551,7 @@ def gemm_rows(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], *,
 
 def rows_takes(M: int, N: int, K: int) -> bool:
     """Where the batch-invariant mode takes `gemm_rows` for a product of few rows, instead of the small tiles. Alone, cold weights, us, rows / tiles: 8 rows
-    768 -> 768 3.2 / 4.2, -> 3,072 3.6 / 4.6, 3,072 -> 768 5.4 / 8.6, 768 -> 50,257 16.6 / 44, 1,600 -> 6,400 6.3 / 7.4; 16 rows 4,096 -> 4,096 9.8 / 11.7; 32 rows
+    768 -> 768 3.0 / 4.2, -> 3,072 3.4 / 4.6, 3,072 -> 768 5.1 / 8.7, 768 -> 50,257 16.5 / 44, 1,600 -> 6,400 6.3 / 7.4; 16 rows 4,096 -> 4,096 9.8 / 11.7; 32 rows
     768 -> 3,072 4.3 / 4.8, -> 50,257 30 / 49; 64 rows 768 -> 768 3.5 / 4.7, 6,400 -> 1,600 15.0 / 17.8. A workgroup reads all rows again: up to 16 rows it
     pays as long as strips of 32 features have a compute unit each (4,096 -> 16,384, 8 rows: 31 / 26), up to 32 rows for fewer features (1,600 -> 6,400 8.7 / 8.1),
     beyond for fewer still (64 rows, 768 -> 2,304 4.9 / 4.9, -> 3,072 5.0 / 5.0)."""
@@ -566,7 +566,7 @@ def rows_takes(M: int, N: int, K: int) -> bool:
 
 def norm_in_rows_pays(M: int, N: int, K: int) -> bool:
     """Whether the batch-invariant mode computes a norm inside the product behind it (`gemm_rows_ln`) instead of in a kernel of its own: while the rows that every
-    workgroup normalises are few (us, inside / norm and product: 768 -> 3,072 8 rows 4.6 / 6.1, 16 rows 5.7 / 6.2, 24 rows 7.0 / 6.6; 1,024 -> 4,096 8 rows 6.1 / 6.8,
+    workgroup normalises are few (us, inside / norm and product: 768 -> 3,072 8 rows 4.3 / 6.0, 16 rows 5.4 / 6.0, 24 rows 6.6 / 6.6; 1,024 -> 4,096 8 rows 6.1 / 6.8,
     16 rows 7.7 / 6.9; 1,600 -> 6,400 8 rows 9.2 / 9.1)."""
     return 0 < M <= 16 and K % 64 == 0 and K <= 2048 and M * K <= 16 * 768 and N <= 32 * 256
 
@@ -599,6 +599,26 @@ def gemm_rows_splits(partials: torch.Tensor, w: torch.Tensor, bias: Optional[tor
     e = _epilogue(_Rows(M, torch.bfloat16), w, bias, None, residual, EPI_RESIDUAL, None)
     e.exact = 0
     _lib.call("liyab_gemm_rows_splits", partials.data_ptr(), S, H, hd4 - 4, w.data_ptr(), M, w.shape[0], strip, ctypes.byref(e), _stream())
+
+
+def glu_in_product_takes(a, w: torch.Tensor) -> bool:
+    """Whether `gemm_glu` takes these operands and leaves the bits of `gemm` and `glu`: where `gemm` would take the streaming kernel in strips of 16 features."""
+    return (isinstance(a, torch.Tensor) and not _invariant and w.dtype == torch.bfloat16 and mfma_takes(a, w) and 0 < a.shape[0] <= 8 and w.shape[0] < 16384
+            and a.shape[1] % 64 == 0 and a.shape[1] % 16384 != 0 and 128 < a.shape[1] <= 8192)
+
+
+def gemm_glu(out: torch.Tensor, a: torch.Tensor, w: torch.Tensor, activation: str) -> None:
+    """out = act(a . G^T) * (a . U^T) for w = [G | U] as rows, bfloat16 [2 * ff, K], and few rows (`glu_in_product_takes`): a gated feed-forward's first product
+    and its activation in one kernel, the bits of `gemm` to 32-bit rows followed by `glu`."""
+    lda, ldo = _rows(a, "a"), _rows(out, "out")
+    M, K = a.shape
+    _dev(w, "w")
+    if a.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or w.dim() != 2 or w.shape[1] != K or w.shape[0] % 2 or not w.is_contiguous():
+        raise KernelError(f"gemm_glu: needs bfloat16 a [M, K] and contiguous w [2 * ff, K], got {tuple(a.shape)} {a.dtype}, {tuple(w.shape)} {w.dtype}")
+    ff = w.shape[0] // 2
+    if out.dtype != torch.bfloat16 or tuple(out.shape) != (M, ff):
+        raise KernelError(f"gemm_glu: out must be bfloat16 [{M}, {ff}], got {tuple(out.shape)} {out.dtype}")
+    _lib.call("liyab_gemm_skinny_glu", a.data_ptr(), lda, w.data_ptr(), M, ff, K, GLU_ACTIVATIONS[activation], out.data_ptr(), ldo, _stream())
 
 
 def gemm_skinny_parts(a: torch.Tensor, w: torch.Tensor, planes: torch.Tensor, *, bias: Optional[torch.Tensor] = None,

@@ -116,7 +116,14 @@ class GatedFFN:
         self.down_weight = store.fetch(t["down"], (self.width, self.inner), "matrix")
 
     def begin(self, h, ctx: StepContext) -> torch.Tensor:
-        """The first product, [gate | up] of h in 32 bits: everything of the feed-forward that reads its input."""
+        """The first product, [gate | up] of h in 32 bits: everything of the feed-forward that reads its input. In steps of few rows the
+        activation is taken in the product's epilogue: what is handed on are the inner rows then."""
+        from ..kernels import ops
+
+        if self.dtype == torch.bfloat16 and ops.glu_in_product_takes(h, self.in_weight):
+            inner = ctx.workspace.get("ffn_inner", (h.shape[0], self.inner), self.dtype)
+            ops.gemm_glu(inner, h, self.in_weight, self.activation)
+            return inner
         gu = ctx.workspace.get("glu_in", (h.shape[0], 2 * self.inner), torch.float32)
         linear(h, self.in_weight, None, out=gu)
         return gu
@@ -124,8 +131,10 @@ class GatedFFN:
     def finish(self, gu: torch.Tensor, ctx: StepContext, residual: Optional[torch.Tensor], out: Optional[torch.Tensor] = None):
         from ..kernels import ops
 
-        inner = ctx.workspace.get("ffn_inner", (gu.shape[0], self.inner), self.dtype)
-        ops.glu(inner, gu, self.activation)
+        inner = gu
+        if gu.shape[1] != self.inner:
+            inner = ctx.workspace.get("ffn_inner", (gu.shape[0], self.inner), self.dtype)
+            ops.glu(inner, gu, self.activation)
         if out is not None:
             linear(inner, self.down_weight, None, out=out)
         else:

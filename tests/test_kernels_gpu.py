@@ -1540,3 +1540,17 @@ def test_products_of_whole_units_leave_the_bits_of_the_others(ops, form, K):
                 ops.moe_product(out, x, u, v if two else None, rows.to(DEV).flatten(), group.to(DEV), a_div=2, row_scale=scale, block=16,
                                 act="relu2" if form == "relu2" else "none", clamp=(0.7, 1.702, 1.0) if form == "clamped" else None)
             assert torch.equal(got, want), (n, N)
+
+@pytest.mark.parametrize("activation", ["silu", "gelu_tanh"])
+@pytest.mark.parametrize("K,ff", [(192, 1), (192, 24), (768, 2048), (832, 17), (1600, 100), (2048, 5504), (8192, 40)])
+def test_an_activation_inside_its_product_leaves_its_own_kernels_bits(ops, K, ff, activation):
+    """A gated feed-forward's first product with the activation in its epilogue against the product to 32-bit rows and the
+    activation's kernel: the same bits, at the edges of a strip of features and of the waves that share K."""
+    for M in (1, 3, 8):
+        a, w = rnd(M, K + 8, dtype=torch.bfloat16, seed=K)[:, :K], rnd(2 * ff, K, dtype=torch.bfloat16, seed=K + 1, scale=0.2)
+        assert ops.glu_in_product_takes(a, w)
+        both, want, got = torch.empty(M, 2 * ff, device=DEV), torch.empty(M, ff, dtype=torch.bfloat16, device=DEV), torch.zeros(M, ff, dtype=torch.bfloat16, device=DEV)
+        ops.gemm(a, w, None, out=both)
+        ops.glu(want, both, activation)
+        ops.gemm_glu(got, a, w, activation)
+        assert torch.equal(got, want), M
