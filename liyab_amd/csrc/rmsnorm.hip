@@ -272,6 +272,92 @@ gated_norm_add_wave_kernel(float* __restrict__ x, T* __restrict__ cast_out, cons
     }
 }
 
+// The same with four waves a row, for up to some 1,500 rows: wave q holds what the kernel above holds as its q-th quarter, so that a row's loads, sigmoids and
+// sums go side by side on four SIMDs, and the sums meet through LDS in the same order: the same bits. What a step of few rows waits for beside memory is one
+// wave's sixty loads of 256 bytes and four sums in turn. us, 4 rows of 768 in a chain, before / now: 3.1 / 2.5, a layer norm
+// 3.3 / 2.7, a gate 3.7 / 2.6, with two rows a token 3.8 / 2.6, the next norm too 3.5 / 2.9; 512 rows 3.4 / 2.9, a gate 4.1 / 3.1.
+template <typename T, int J, int NSUM, bool GATE, int ALSO>
+__global__ void __launch_bounds__(256)
+gated_norm_add_quarters_kernel(float* __restrict__ x, T* __restrict__ cast_out, const float* __restrict__ y, const float* __restrict__ gate, int64_t gate_stride,
+                               const float* __restrict__ w, float eps, int normalize, int n, int d, KeepRows keep, const float* __restrict__ next_w,
+                               float next_eps, const float* __restrict__ b) {
+    constexpr int W = 4, STRIDE = W * kWave;
+    __shared__ float meet[3][W];  // the quarters' sums: the mean's, the mean square's, the next norm's
+    const int lane = threadIdx.x % kWave, q = threadIdx.x / kWave, t = blockIdx.x;
+    float* xr = x + static_cast<int64_t>(t) * d;
+    const float* yr = y + static_cast<int64_t>(t) * NSUM * d;
+    const float* wp = w != nullptr ? w : xr;
+    float xv[J], sv[J], yv[NSUM][J], gv[J], wv[J], av[J];
+    const auto place = [&](int j) { return static_cast<int>(threadIdx.x) + j * STRIDE; };
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+        const int at = min(place(j), d - 1);  // (past the row: its last value, counted as nothing)
+#pragma unroll
+        for (int k = 0; k < NSUM; ++k) yv[k][j] = yr[static_cast<int64_t>(k) * d + at];
+        if constexpr (GATE) gv[j] = gate[static_cast<int64_t>(t) * gate_stride + at];
+        xv[j] = xr[at];
+        wv[j] = wp[at];
+        if constexpr (ALSO != kRowOnly) av[j] = (ALSO == kRowBias ? b : next_w)[at];
+    }
+    // where the old row is kept: looked up while the row is on its way
+    float* kept = nullptr;
+    if (keep.state != nullptr && t < *keep.n_real) {
+        const int s = keep.tok_seq[t], p = keep.positions[t];
+        const int slot = keep.state_slots[s];
+        if (p >= keep.context_lens[s] - keep.ring && slot >= 0 && slot < keep.n_slots) kept = keep.state + (static_cast<int64_t>(slot) * keep.ring + p % keep.ring) * d;
+    }
+    const auto row_sum = [&](float part, int which) {
+        part = wave_sum(part);
+        if (lane == 0) meet[which][q] = part;
+        lds_barrier();
+        float total = 0.0f;
+#pragma unroll
+        for (int i = 0; i < W; ++i) total += meet[which][i];
+        return total;
+    };
+    float ss = 0.0f;
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+        float s = yv[0][j];
+#pragma unroll
+        for (int k = 1; k < NSUM; ++k) s += yv[k][j];
+        if constexpr (GATE) s *= sigmoidf(gv[j]);
+        sv[j] = place(j) < d ? s : 0.0f;
+        ss += normalize == 2 ? sv[j] : sv[j] * sv[j];
+    }
+    if (normalize == 2) {
+        const float mean = row_sum(ss, 0) / static_cast<float>(d);
+        ss = 0.0f;
+#pragma unroll
+        for (int j = 0; j < J; ++j) {
+            sv[j] -= mean;
+            if (place(j) < d) ss += sv[j] * sv[j];
+        }
+    }
+    const float scale = normalize ? 1.0f / sqrtf(row_sum(ss, 1) / static_cast<float>(d) + eps) : 1.0f;
+    T* co = cast_out != nullptr ? cast_out + static_cast<int64_t>(t) * d : nullptr;
+    ss = 0.0f;
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+        float v = sv[j] * scale;
+        if (w != nullptr) v *= wv[j];
+        if constexpr (ALSO == kRowBias) v += av[j];
+        v += xv[j];
+        sv[j] = v;
+        if (place(j) >= d) continue;
+        if (kept != nullptr) kept[place(j)] = xv[j];
+        xr[place(j)] = v;
+        if constexpr (ALSO == kRowNext) ss += v * v;
+        else if (co != nullptr) co[place(j)] = from_float<T>(v);
+    }
+    if constexpr (ALSO == kRowNext) {  // what is written for the next product is the next norm of the new row
+        const float next_scale = 1.0f / sqrtf(row_sum(ss, 2) / static_cast<float>(d) + next_eps);
+#pragma unroll
+        for (int j = 0; j < J; ++j)
+            if (place(j) < d) co[place(j)] = from_float<T>(sv[j] * next_scale * av[j]);
+    }
+}
+
 // Whether the wave kernel took the rows (of the gate, a bias and the next norm it takes one: what the blocks that exist use); if
 // not, the one above does. A place past the row costs what one inside does, which shows where each takes a sigmoid: with a gate J is
 // the least that holds the row (behind the kernels that write y and the gate, us for all of them, by workgroups, by waves with J of 3, 4
@@ -279,15 +365,20 @@ gated_norm_add_wave_kernel(float* __restrict__ x, T* __restrict__ cast_out, cons
 // prompt of 32 and eight decoded tokens, 29.8, 29.1, 28.1 ms). Without one, J of 3, 4 and 8 is enough (behind the kernel that writes y, by
 // workgroups and by waves: 4 rows of 1,280 5.4 and 5.4, with two rows a token 6.7 and 5.7; 2,048 rows of 1,280 13.7 and 12.9; of 2,048 18.6 and
 // 16.6, a layer norm 21.2 and 16.9, three rows a token and the next norm 33.6 and 30.8).
+// Rows up to which four waves share one: while they do not fill the chip (512 rows of 320 to 2,048 0.73 with a gate and 0.79 to 0.80 of a wave a row, 1,500 0.82
+// and 0.86 to 0.88; 2,048 rows of 320 1.03 and 1.00, of 2,048 0.84 and 0.92; 4,096 even).
+constexpr int kQuarterRows = 1536;
 template <typename T>
 bool gated_norm_add_by_waves(float* x, T* cast_out, const float* y, int n_sum, const float* gate, int64_t gate_stride, const float* w, float eps, int normalize,
                              int n, int d, const KeepRows& keep, const float* next_w, float next_eps, const float* b, hipStream_t stream) {
     if (d > 2048 || n_sum > 3 || (gate != nullptr) + (b != nullptr) + (next_w != nullptr) > 1) return false;
-    // Rows a workgroup: a few hundred, one (a wave with a compute unit, or a SIMD, of its own: 64 to 300 rows of 768 to 2,048 1-7 % less than
-    // in fours); many, four (780 to 4,096 rows: even, up to 4 % less)
-    const int rows = n <= 512 ? 1 : 4;
-#define LIYAB_GO(J, S, G, A) \
-    gated_norm_add_wave_kernel<T, J, S, G, A><<<(n + rows - 1) / rows, kWave * rows, 0, stream>>>(x, cast_out, y, gate, gate_stride, w, eps, normalize, n, d, keep, next_w, next_eps, b)
+#define LIYAB_ROWS(KERNEL, THREADS, ROWS, J, S, G, A) \
+    KERNEL<T, J, S, G, A><<<(n + ROWS - 1) / ROWS, THREADS, 0, stream>>>(x, cast_out, y, gate, gate_stride, w, eps, normalize, n, d, keep, next_w, next_eps, b)
+#define LIYAB_GO(J, S, G, A)                                                                            \
+    do {                                                                                                \
+        if (n <= kQuarterRows) LIYAB_ROWS(gated_norm_add_quarters_kernel, 4 * kWave, 1, J, S, G, A);    \
+        else LIYAB_ROWS(gated_norm_add_wave_kernel, 4 * kWave, 4, J, S, G, A);                          \
+    } while (0)
 #define LIYAB_SUMS(J, G, A)                 \
     do {                                    \
         if (n_sum == 1) LIYAB_GO(J, 1, G, A); \
@@ -318,6 +409,7 @@ bool gated_norm_add_by_waves(float* x, T* cast_out, const float* y, int n_sum, c
     } else {
         LIYAB_WIDTHS(kRowOnly);
     }
+#undef LIYAB_ROWS
 #undef LIYAB_WIDTHS
 #undef LIYAB_SUMS
 #undef LIYAB_GO

@@ -1554,3 +1554,18 @@ def test_an_activation_inside_its_product_leaves_its_own_kernels_bits(ops, K, ff
         ops.glu(want, both, activation)
         ops.gemm_glu(got, a, w, activation)
         assert torch.equal(got, want), M
+
+@pytest.mark.parametrize("form", ["one", "centred", "gate", "next"])
+def test_rows_update_shares_a_row_among_four_waves_with_the_same_bits(ops, form):
+    """Up to 1,536 rows a row belongs to four waves, beyond to one: what a row becomes does not depend on how many there are."""
+    for d in (64, 256, 260, 768, 1021, 2048):
+        x, y, w, b, gate = rnd(1537, d), rnd(1537 * 3, d, seed=1), rnd(d, seed=2), rnd(d, seed=3), rnd(1537, d + 3, seed=4)[:, :d]
+        for k in (1, 2, 3):
+            got = []
+            for n in (1537, 1536, 3):
+                into, cast = x[:n].clone(), torch.empty(n, d, dtype=torch.bfloat16, device=DEV)
+                ops.gated_norm_add(into, y[:n * k], w, 1e-5, n_sum=k, cast_out=cast, gate=gate[:n] if form == "gate" else None,
+                                   **({"bias": b, "centred": True} if form == "centred" else {"next_norm": (b, 1e-5)} if form == "next" else {}))
+                got.append((into, cast))
+            for into, cast in got[1:]:
+                assert torch.equal(into, got[0][0][:len(into)]) and torch.equal(cast, got[0][1][:len(into)]), (d, k, len(into))
