@@ -582,6 +582,26 @@ def test_the_streams_update_alone(out_dtype, S, d, n_sum):
     assert tt.rel_err(f64(out), normed(f64(x)[[3, 0, 3]], np.ones(S), f64(w))) < tol and torch.equal(xd.cpu(), x)
 
 
+@pytest.mark.parametrize("S", [1, 2, 3, 4])
+def test_the_streams_update_of_few_rows_a_token_has_the_same_bits(S):
+    """Up to four rows a token and 1,024 entries have a kernel of their own: against the general one, which gets a fifth row of zeros."""
+    from liyab_amd.kernels import ops
+
+    n = 5
+    for d in (64, 256, 260, 1024):
+        x = torch.randn(n, S, d, device=DEV)
+        mix, add, take, w = torch.randn(S, S, device=DEV), torch.randn(S, device=DEV), torch.randn(S, device=DEV), torch.randn(d, device=DEV)
+        for k in (1, 2, 4):
+            y = torch.randn(n, k, d, device=DEV)
+            for norm in ((take, w, 1e-5), (None, None, 1e-5), None):
+                got = []
+                for rows in (y, torch.cat([y, torch.zeros(n, 5 - k, d, device=DEV)], dim=1)):
+                    into, out = x.clone(), torch.empty(n, d, dtype=torch.bfloat16, device=DEV)
+                    ops.streams_update(into, y=rows.reshape(-1, d), n_sum=rows.shape[1], mix=mix, add=add, next_norm=norm, out=out if norm is not None else None)
+                    got.append((into, out if norm is not None else into))
+                assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1]), (d, k)
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_connections_that_single_a_stream_out(dtype, tmp_path):
     """A sublayer that reads the second stream alone and gives to the first alone, and a mix that moves each stream to the next: a
