@@ -142,6 +142,48 @@ layernorm_wave_kernel(T* __restrict__ out, const float* __restrict__ x, const fl
         if (lane + kWave * j < nv) store_row4<T>(o + 4 * (lane + kWave * j), (v[j] - mean) * scale * gw[j] + gb[j]);
 }
 
+// The same with W waves a row, wave j with what the kernel above holds as its j-th piece: a row's loads and sums go side by side on W SIMDs, all planes' loads
+// in flight together, and the pieces' sums meet through LDS in that kernel's order, lane by lane: the same bits. For rows that do not fill the chip, where a
+// step waits for one trip to memory and one wave's instructions.
+template <typename T, int W, bool PARTS>
+__global__ void __launch_bounds__(W * kWave)
+layernorm_pieces_kernel(T* __restrict__ out, const float* __restrict__ x, const float* __restrict__ w, const float* __restrict__ b,
+                        const int* __restrict__ rows, int d, float eps, PartSums ps) {
+    constexpr int PB = 4;  // planes asked for together beside the first
+    __shared__ float meet[2][W][kWave];
+    const int lane = threadIdx.x % kWave, piece = threadIdx.x / kWave, r = blockIdx.x, nv = d / 4;
+    const int64_t src = rows != nullptr ? rows[r] : r;
+    const int i = min(static_cast<int>(threadIdx.x), nv - 1);  // past the row: its last piece again, unused
+    const bool inside = threadIdx.x < nv;
+    const f32x4* const row0 = reinterpret_cast<const f32x4*>(x + src * d) + i;
+    const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f}, one = {1.0f, 1.0f, 1.0f, 1.0f};
+    f32x4 v = *row0, plane[PB];
+    if constexpr (PARTS) {
+#pragma unroll
+        for (int u = 0; u < PB; ++u) plane[u] = row0[min(1 + u, ps.n_parts - 1) * (ps.stride / 4)];
+    }
+    const f32x4 gw = w != nullptr ? reinterpret_cast<const f32x4*>(w)[i] : one;
+    const f32x4 gb = b != nullptr ? reinterpret_cast<const f32x4*>(b)[i] : zero;
+    if constexpr (PARTS) {
+#pragma unroll
+        for (int u = 0; u < PB; ++u)
+            if (1 + u < ps.n_parts) v += plane[u];
+        for (int q = 1 + PB; q < ps.n_parts; ++q) v += row0[q * (ps.stride / 4)];
+    }
+    const auto row_sum = [&](float part, int which) {
+        meet[which][piece][lane] = inside ? part : 0.0f;
+        lds_barrier();
+        float s = 0.0f;
+#pragma unroll
+        for (int j = 0; j < W; ++j) s += meet[which][j][lane];
+        return wave_sum(s);
+    };
+    const float mean = row_sum((v[0] + v[1]) + (v[2] + v[3]), 0) / static_cast<float>(d);
+    const f32x4 dev = v - mean;
+    const float scale = 1.0f / sqrtf(row_sum((dev[0] * dev[0] + dev[1] * dev[1]) + (dev[2] * dev[2] + dev[3] * dev[3]), 1) / static_cast<float>(d) + eps);
+    if (inside) store_row4<T>(out + static_cast<int64_t>(r) * d + 4 * threadIdx.x, (v - mean) * scale * gw + gb);
+}
+
 // The same for wider rows (d a multiple of 4, at most THREADS * 4 * MAXV): a workgroup a row,
 // the row in its threads' registers, sums across the waves through LDS.
 template <typename T, int THREADS, int MAXV, bool PARTS>
@@ -215,9 +257,36 @@ __global__ void __launch_bounds__(256) sum_parts_kernel(float* out, const float*
     out[i] = v;
 }
 
+// Whether a row's pieces go to waves of their own: while the rows do not fill the chip and a wave would have several pieces or planes to read (us, a wave a row /
+// a wave a piece: 64 rows of 1,600 3.05 / 2.70, in five planes 3.81 / 2.94, of 768 in five 3.04 / 2.61; 256 rows of 2,048 3.18 / 2.87; 512 of 768 2.67 / 2.71, in
+// four planes 3.01 / 2.93; 800 rows in five planes of 1,024 3.88 / 3.44, of 1,600 4.84 / 4.61; 1,024 of 2,048 8.8 / 9.4; 64 rows of 512 2.40 / 2.40).
+static bool pieces_pay(int n, int d, int n_parts) {
+    if (n_parts > 4) return n <= 512 || (n <= 1024 && static_cast<int64_t>(n) * d <= 1300000);
+    return n <= 256 ? d > 512 || n_parts > 1 : n <= 512 && n_parts > 1 && d > 512;
+}
 template <typename T, int MAXV>
 void launch_wave(T* out, const float* x, const float* w, const float* b, const int* rows, int n, int d, float eps,
                  const PartSums& ps, hipStream_t stream) {
+    if constexpr (MAXV > 1) {
+        if (pieces_pay(n, d, ps.n_parts)) {
+            switch ((d / 4 + kWave - 1) / kWave) {
+#define LIYAB_PIECES(W)                                                                                                                       \
+    case W:                                                                                                                                   \
+        if (ps.n_parts > 1) layernorm_pieces_kernel<T, W, true><<<n, W * kWave, 0, stream>>>(out, x, w, b, rows, d, eps, ps);                 \
+        else layernorm_pieces_kernel<T, W, false><<<n, W * kWave, 0, stream>>>(out, x, w, b, rows, d, eps, ps);                               \
+        return
+                LIYAB_PIECES(2);
+                LIYAB_PIECES(3);
+                LIYAB_PIECES(4);
+                LIYAB_PIECES(5);
+                LIYAB_PIECES(6);
+                LIYAB_PIECES(7);
+                LIYAB_PIECES(8);
+#undef LIYAB_PIECES
+                default: break;
+            }
+        }
+    }
     const int waves = n <= 512 ? 1 : 4;  // rows a workgroup
     const int grid = (n + waves - 1) / waves;
     if (ps.n_parts > 1) layernorm_wave_kernel<T, MAXV, true><<<grid, kWave * waves, 0, stream>>>(out, x, w, b, rows, n, d, eps, ps);

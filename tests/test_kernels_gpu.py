@@ -1509,6 +1509,7 @@ def test_sampler_at_few_ids_a_thread(ops, V):
     values on), with ties at the boundary inside and outside the pool."""
     test_sampler_against_the_plain_sampler(ops, V)
 
+
 @pytest.mark.parametrize("form", ["one", "relu2", "two", "clamped", "heads", "gated heads"])
 @pytest.mark.parametrize("K", [64, 192, 256, 448, 832, 1600])
 def test_products_of_whole_units_leave_the_bits_of_the_others(ops, form, K):
@@ -1541,6 +1542,7 @@ def test_products_of_whole_units_leave_the_bits_of_the_others(ops, form, K):
                                 act="relu2" if form == "relu2" else "none", clamp=(0.7, 1.702, 1.0) if form == "clamped" else None)
             assert torch.equal(got, want), (n, N)
 
+
 @pytest.mark.parametrize("activation", ["silu", "gelu_tanh"])
 @pytest.mark.parametrize("K,ff", [(192, 1), (192, 24), (768, 2048), (832, 17), (1600, 100), (2048, 5504), (8192, 40)])
 def test_an_activation_inside_its_product_leaves_its_own_kernels_bits(ops, K, ff, activation):
@@ -1554,6 +1556,7 @@ def test_an_activation_inside_its_product_leaves_its_own_kernels_bits(ops, K, ff
         ops.glu(want, both, activation)
         ops.gemm_glu(got, a, w, activation)
         assert torch.equal(got, want), M
+
 
 @pytest.mark.parametrize("form", ["one", "centred", "gate", "next"])
 def test_rows_update_shares_a_row_among_four_waves_with_the_same_bits(ops, form):
@@ -1569,3 +1572,24 @@ def test_rows_update_shares_a_row_among_four_waves_with_the_same_bits(ops, form)
                 got.append((into, cast))
             for into, cast in got[1:]:
                 assert torch.equal(into, got[0][0][:len(into)]) and torch.equal(cast, got[0][1][:len(into)]), (d, k, len(into))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("d", [260, 516, 768, 1028, 1600, 2048])
+def test_norm_of_few_rows_shares_a_row_among_waves_with_the_same_bits(ops, d, dtype):
+    """Where the rows are few, each piece of 256 entries has a wave of its own; among many a row has one: the same bits, rows in planes too."""
+    n, w, b = 1100, rnd(d, seed=1), rnd(d, seed=2)
+    for planes in (1, 2, 5, 8):
+        x = rnd(planes, n, d, seed=3)
+        picked = torch.tensor([3, 0, 1099], dtype=torch.int32, device=DEV)
+        for weights in ((w, b), (w, None)):
+            many, few, gathered = (torch.empty(rows, d, dtype=dtype, device=DEV) for rows in (n, 5, 3))
+            if planes == 1:
+                ops.layernorm(many, x[0], *weights, 1e-5)
+                ops.layernorm(few, x[0, :5], *weights, 1e-5)
+                ops.layernorm(gathered, x[0], *weights, 1e-5, rows=picked)
+            else:
+                ops.layernorm(many, x, *weights, 1e-5)
+                ops.layernorm(few, x[:, :5].contiguous(), *weights, 1e-5)
+                ops.layernorm(gathered, x, *weights, 1e-5, rows=picked)
+            assert torch.equal(few, many[:5]) and torch.equal(gathered, many[picked.long()]), planes
