@@ -320,6 +320,105 @@ qk_prepare_rows_kernel(const float* __restrict__ src, int64_t ld, int q_off, int
     }
 }
 
+// The same for rows whose queries, keys and values are at most 256 J entries each (dk, dv of any width): 256 threads for each of the three, everything asked for
+// together and held, a head's pairs met through LDS, a slot's page found by one division in 32 bits. (The kernel above has 256 threads for all, reads the rows
+// again behind the sums, the weights with them, and divides in 64 bits an entry.) The same operations, the same bits.
+// us, 4 rows: 12 heads of 64 5.7 -> 3.9, 12 over 4 4.6 -> 3.8, 16 over 4 of 128 6.8 -> 4.5, 8 of 256 10.5 -> 5.1.
+template <typename T, int J>
+__global__ void __launch_bounds__(3 * AS_THREADS)
+qk_prepare_held_rows_kernel(const float* __restrict__ src, int64_t ld, int q_off, int k_off, int v_off, int H, int G, int dk, int dv, int dk_out,
+                            int dv_out, T* __restrict__ q_out, T* __restrict__ kc, T* __restrict__ vc, const int* __restrict__ slots, int page_size,
+                            int num_pages, const float* __restrict__ q_norm, const float* __restrict__ k_norm, float eps,
+                            const double* __restrict__ freqs, int rot_dims, const int* __restrict__ positions, int rot_halves) {
+    __shared__ float2 turn[QR_MAX_PAIRS];
+    __shared__ float red[3][AS_THREADS / kWave], rows[3][J * AS_THREADS];  // the rows of queries and keys behind their norms, the values
+    const int t = blockIdx.x, tid = threadIdx.x % AS_THREADS, part = __builtin_amdgcn_readfirstlane(threadIdx.x / AS_THREADS), n_turned = rot_dims / 2;
+    const bool keys = kc != nullptr;
+    // (without keys: the queries again, dropped)
+    const int n = !keys || part == 0 ? H * dk : part == 1 ? G * dk : G * dv, n_w = !keys || part != 1 ? H * dk : G * dk;
+    const float* const row = src + static_cast<int64_t>(t) * ld + (!keys || part == 0 ? q_off : part == 1 ? k_off : v_off);
+    const float* const weight = !keys || part != 1 ? q_norm : k_norm;
+    const int* const slot_at = keys ? slots : positions;
+    float x[J], w[J];
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+        x[j] = row[min(tid + j * AS_THREADS, n - 1)];
+        w[j] = weight[min(tid + j * AS_THREADS, n_w - 1)];
+    }
+    const int p = positions[t], slot = slot_at[t];
+    settle_loads(x);
+    settle_loads(w);
+    float sum = 0.0f;
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+        const float v = tid + j * AS_THREADS < n ? x[j] : 0.0f;
+        sum = fmaf(v, v, sum);
+    }
+    if (part == 2)
+        for (int i = tid; i < n_turned; i += AS_THREADS) {
+            const float angle = turn_angle(p, freqs[i]);
+            turn[i] = float2{cosf(angle), sinf(angle)};
+        }
+    sum = wave_sum(sum);
+    if (tid % kWave == 0) red[part][tid / kWave] = sum;
+    const bool stored = keys && slot >= 0 && slot < static_cast<int64_t>(num_pages) * page_size;
+    const uint32_t page = stored ? static_cast<uint32_t>(slot) / static_cast<uint32_t>(page_size) : 0u;
+    const int64_t in_page = slot - static_cast<int64_t>(page) * page_size, page_heads = static_cast<int64_t>(page) * G;
+    lds_barrier();
+    sum = 0.0f;
+#pragma unroll
+    for (int i = 0; i < AS_THREADS / kWave; ++i) sum += red[part][i];
+    const float factor = 1.0f / sqrtf(sum / static_cast<float>((part == 0 ? H : G) * dk) + eps);
+#pragma unroll
+    for (int j = 0; j < J; ++j) rows[part][tid + j * AS_THREADS] = part == 2 ? x[j] : x[j] * factor * w[j];
+    lds_barrier();
+    if (part > 0 && !stored) return;
+    if (part < 2) {
+        const uint32_t per = (dk_out + 1) / 2, items = (part == 0 ? H : G) * per;
+        for (uint32_t item = tid; item < items; item += AS_THREADS) {
+            const int head = item / per, u = item - head * per;
+            int e0 = 2 * u, e1 = e0 + 1;
+            if (rot_halves && u < n_turned) {
+                e0 = u;
+                e1 = u + n_turned;
+            }
+            const float* const from = rows[part] + head * dk;
+            float a = e0 < dk ? from[e0] : 0.0f, b = e1 < dk ? from[e1] : 0.0f;
+            if (u < n_turned) {
+                const float2 cs = turn[u];
+                const float ra = a * cs.x - b * cs.y, rb = b * cs.x + a * cs.y;
+                a = ra;
+                b = rb;
+            }
+            T* const dst = part == 0 ? q_out + (static_cast<int64_t>(t) * H + head) * dk_out : kc + ((page_heads + head) * page_size + in_page) * dk_out;
+            dst[e0] = from_float<T>(a);
+            if (e1 < dk_out) dst[e1] = from_float<T>(b);
+        }
+        return;
+    }
+    for (uint32_t item = tid; item < static_cast<uint32_t>(G * dv_out); item += AS_THREADS) {
+        const int head = item / static_cast<uint32_t>(dv_out), i = item - head * dv_out;
+        vc[((page_heads + head) * page_size + in_page) * dv_out + i] = from_float<T>(i < dv ? rows[2][head * dv + i] : 0.0f);
+    }
+}
+
+template <typename T>
+void launch_prepare_rows(const float* src, int64_t ld, int q_off, int k_off, int v_off, int H, int G, int dk, int dv, int dk_out, int dv_out, T* q_out, T* kc,
+                         T* vc, const int* slots, int page_size, int num_pages, const float* q_norm, const float* k_norm, float eps, const double* freqs,
+                         int rot_dims, const int* positions, int rot_halves, int n, hipStream_t stream) {
+#define LIYAB_ROWS(THREADS, ...)                                                                                                                                     \
+    __VA_ARGS__<<<n, THREADS, 0, stream>>>(src, ld, q_off, k_off, v_off, H, G, dk, dv, dk_out, dv_out, q_out, kc, vc, slots, page_size, num_pages, q_norm, k_norm, \
+                                              eps, freqs, rot_dims, positions, rot_halves)
+    const int widest = kc != nullptr ? max(H * dk, max(G * dk, G * dv)) : H * dk;
+    // while the rows are few: each then has a compute unit, or half of one, to itself (us, 256 threads a row / 768: 12 heads of 64 4 rows 5.7 / 3.9, 300 6.4 / 5.3,
+    // 2,000 13.1 / 15.9; 12 over 4 4.6 / 3.8, 5.0 / 4.9, 8.8 / 13.9; 6 over 2 of 40 3.6 / 3.5, 4.1 / 4.5)
+    if (n > 128) LIYAB_ROWS(AS_THREADS, qk_prepare_rows_kernel<T>);
+    else if (widest <= 3 * AS_THREADS) LIYAB_ROWS(3 * AS_THREADS, qk_prepare_held_rows_kernel<T, 3>);
+    else if (widest <= 8 * AS_THREADS) LIYAB_ROWS(3 * AS_THREADS, qk_prepare_held_rows_kernel<T, 8>);
+    else LIYAB_ROWS(AS_THREADS, qk_prepare_rows_kernel<T>);
+#undef LIYAB_ROWS
+}
+
 template <typename T>
 __global__ void __launch_bounds__(AS_THREADS)
 attention_scored_kernel(T* __restrict__ out, int64_t out_stride, const T* __restrict__ q, int64_t q_stride, const T* __restrict__ kc,
@@ -471,14 +570,12 @@ extern "C" int liyab_qk_prepare_rows(const float* src, int64_t ld, int q_off, in
                   "qk_prepare_rows: the keys' or values' columns pass the source's rows");
     LIYAB_REQUIRE(rot_dims >= 0 && rot_dims <= dk && rot_dims % 2 == 0 && (rot_dims == 0 || freqs != nullptr), "qk_prepare_rows: %d turned entries of heads of %d", rot_dims, dk);
     if (n == 0) return 0;
-    if (dtype == kF32)
-        qk_prepare_rows_kernel<float><<<n, AS_THREADS, 0, stream>>>(src, ld, q_off, k_off, v_off, H, G, dk, dv, dk_out, dv_out, static_cast<float*>(q_out),
-                                                                    static_cast<float*>(kc), static_cast<float*>(vc), slots, page_size, num_pages, q_norm,
-                                                                    k_norm, eps, freqs, rot_dims, positions, rot_halves);
-    else if (dtype == kBF16)
-        qk_prepare_rows_kernel<bf16_t><<<n, AS_THREADS, 0, stream>>>(src, ld, q_off, k_off, v_off, H, G, dk, dv, dk_out, dv_out, static_cast<bf16_t*>(q_out),
-                                                                     static_cast<bf16_t*>(kc), static_cast<bf16_t*>(vc), slots, page_size, num_pages, q_norm,
-                                                                     k_norm, eps, freqs, rot_dims, positions, rot_halves);
+    const auto launch = [&](auto* q, auto* k, auto* v) {
+        launch_prepare_rows(src, ld, q_off, k_off, v_off, H, G, dk, dv, dk_out, dv_out, q, k, v, slots, page_size, num_pages, q_norm, k_norm, eps, freqs, rot_dims, positions, rot_halves, n,
+                            stream);
+    };
+    if (dtype == kF32) launch(static_cast<float*>(q_out), static_cast<float*>(kc), static_cast<float*>(vc));
+    else if (dtype == kBF16) launch(static_cast<bf16_t*>(q_out), static_cast<bf16_t*>(kc), static_cast<bf16_t*>(vc));
     else return fail(1, "qk_prepare_rows: unknown dtype %d", dtype);
     return check_launch("qk_prepare_rows");
 }

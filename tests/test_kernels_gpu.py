@@ -1593,3 +1593,32 @@ def test_norm_of_few_rows_shares_a_row_among_waves_with_the_same_bits(ops, d, dt
                 ops.layernorm(few, x[:, :5].contiguous(), *weights, 1e-5)
                 ops.layernorm(gathered, x, *weights, 1e-5, rows=picked)
             assert torch.equal(few, many[:5]) and torch.equal(gathered, many[picked.long()]), planes
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("H,G,dk,dv", [(12, 12, 64, 64), (6, 2, 40, 40), (5, 1, 30, 33), (8, 8, 256, 256), (32, 8, 128, 64)])
+def test_prepared_rows_do_not_depend_on_how_many_there_are(ops, H, G, dk, dv, dtype):
+    """Queries, keys and values of up to 128 rows have 256 threads each and stay in registers, those of more (and of wider rows) do not: the same bits;
+    turned as neighbours and as halves, rows wider than the heads, slots outside the pages, queries alone."""
+    n, page = 131, 16
+    src, q_norm, k_norm = rnd(n, (H + G) * dk + G * dv), rnd(H * dk, seed=1), rnd(G * dk, seed=2)
+    slots = torch.randperm(20 * page, generator=torch.Generator().manual_seed(3))[:n].int()
+    slots[1], slots[2] = -1, 20 * page + 2
+    slots, positions = slots.to(DEV), torch.arange(n, dtype=torch.int32, device=DEV) * 37
+    for rot, halves in ((0, False), (dk // 2 * 2, False), (dk // 4 * 2, True)):
+        freqs = torch.rand(max(rot // 2, 1), dtype=torch.float64, generator=torch.Generator().manual_seed(4)).to(DEV) if rot else None
+        for wide in (0, 7):
+            for keys in (True, False):
+                got = []
+                for rows in (n, 3):
+                    q = torch.full((rows, H * (dk + wide)), 7.0, dtype=dtype, device=DEV)
+                    kc, vc = (torch.full((20, G, page, w + wide), 7.0, dtype=dtype, device=DEV) for w in (dk, dv))
+                    ops.qk_prepare_rows(src[:rows], q, kc if keys else None, vc if keys else None, slots[:rows], positions[:rows], q_off=0, k_off=H * dk, v_off=(H + G) * dk,
+                                        n_head=H, n_kv_head=G, head_dim=dk, value_dim=dv, q_norm=q_norm, k_norm=k_norm if keys else None, eps=1e-5, freqs=freqs, rot_dims=rot,
+                                        rot_halves=halves)
+                    got.append((q, kc, vc))
+                assert torch.equal(got[1][0], got[0][0][:3])
+                for few, many in zip(got[1][1:], got[0][1:]):
+                    at = slots[:1].long()
+                    rows_of = lambda c: c.transpose(1, 2).flatten(0, 1)  # noqa: E731
+                    assert torch.equal(rows_of(few)[at], rows_of(many)[at]) and (rows_of(few) != 7.0).any(dim=2).any(dim=1).sum().item() == (1 if keys else 0)
