@@ -345,16 +345,20 @@ selective_single_kernel(SelectiveArgs a, const T* __restrict__ wt, const float* 
     const float x = to_float<T>(static_cast<const T*>(a.x)[t * a.C + cc]);
     // this wave's quarter of the states: the first four are asked for before anything is computed
     const int nq = (a.N + 3) / 4, n0 = wave * nq, n1 = min(a.N, n0 + nq);
-    float S[4], A2[4];
+    float S[4], A2[4], B[4], C[4];
     auto states = [&](int i0) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            const int64_t at = static_cast<int64_t>(min(i0 + j, a.N - 1)) * a.C + cc;
+            const int i = min(i0 + j, a.N - 1);
+            const int64_t at = static_cast<int64_t>(i) * a.C + cc;
             A2[j] = a.a2[at];
             S[j] = base[at];
+            B[j] = row[rank + i];
+            C[j] = row[rank + a.N + i];
         }
     };
     states(n0);
+    const float own_bias = bias[cc], skip = a.skip[cc];
     const float z = a.z[t * a.ldz + cc], raw = a.places > 0 ? a.raw[t * a.ldr + cc] : 0.0f;
     // this wave's quarter of the rank; weights [rank, C], a row's channels side by side
     const int kq = (rank + 3) / 4, k1 = min(rank, (wave + 1) * kq);
@@ -373,7 +377,7 @@ selective_single_kernel(SelectiveArgs a, const T* __restrict__ wt, const float* 
     }
     part[wave][lane] = acc;
     __syncthreads();
-    if (wave == 0) steps[lane] = ss_softplus((part[0][lane] + part[1][lane]) + (part[2][lane] + part[3][lane]) + bias[cc]);
+    if (wave == 0) steps[lane] = ss_softplus((part[0][lane] + part[1][lane]) + (part[2][lane] + part[3][lane]) + own_bias);
     __syncthreads();
     const float dt = steps[lane], dx = dt * x;
     float y = 0.0f;
@@ -383,8 +387,8 @@ selective_single_kernel(SelectiveArgs a, const T* __restrict__ wt, const float* 
         for (int j = 0; j < 4; ++j) {
             const int i = i0 + j;
             if (i < n1) {
-                const float v = fmaf(ss_exp2(dt * A2[j]), from_slot ? S[j] : 0.0f, dx * row[rank + i]);
-                y = fmaf(v, row[rank + a.N + i], y);
+                const float v = fmaf(ss_exp2(dt * A2[j]), from_slot ? S[j] : 0.0f, dx * B[j]);
+                y = fmaf(v, C[j], y);
                 if (c_ok && slot_ok) base[static_cast<int64_t>(i) * a.C + c] = v;
             }
         }
@@ -393,7 +397,7 @@ selective_single_kernel(SelectiveArgs a, const T* __restrict__ wt, const float* 
     __syncthreads();
     if (wave == 0 && c_ok) {
         const float sum = (part[0][lane] + part[1][lane]) + (part[2][lane] + part[3][lane]);
-        static_cast<T*>(a.out)[t * a.C + c] = from_float<T>(fmaf(a.skip[c], x, sum) * ss_silu(z));
+        static_cast<T*>(a.out)[t * a.C + c] = from_float<T>(fmaf(skip, x, sum) * ss_silu(z));
         if (slot_ok && a.places > 0) base[static_cast<int64_t>(a.N) * a.C + static_cast<int64_t>(pos % a.places) * a.C + c] = raw;
     }
 }
