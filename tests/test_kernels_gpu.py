@@ -1622,3 +1622,32 @@ def test_prepared_rows_do_not_depend_on_how_many_there_are(ops, H, G, dk, dv, dt
                     at = slots[:1].long()
                     rows_of = lambda c: c.transpose(1, 2).flatten(0, 1)  # noqa: E731
                     assert torch.equal(rows_of(few)[at], rows_of(many)[at]) and (rows_of(few) != 7.0).any(dim=2).any(dim=1).sum().item() == (1 if keys else 0)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("C", [5, 256, 770])
+@pytest.mark.parametrize("taps", [2, 3, 4])
+def test_a_short_convolution_with_its_inputs_ahead_has_the_general_kernels_bits(ops, taps, C, dtype):
+    """Two to four taps against six, the first ones zeros (the kernel that walks the taps): tokens whose inputs lie in the step, in the ring, in
+    both, before position 0, and of a request without a slot."""
+    from types import SimpleNamespace
+
+    lens, contexts, slots = [1, 1, 4, 2, 1], [0, 9, 2, 1, 7], [2, 0, 4, 1, -1]
+    n = sum(lens)
+    seq = [r for r, q in enumerate(lens) for _ in range(q)]
+    dev = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)  # noqa: E731
+    ctx = SimpleNamespace(n_tokens=n, n_seqs=len(lens), max_q=max(lens), tok_seq=dev(seq), positions=dev([contexts[r] + i for r, q in enumerate(lens) for i in range(q)]),
+                          seq_starts=dev([sum(lens[:r]) for r in range(len(lens) + 1)]), state_slots=dev(slots), context_lens=dev([c + q for c, q in zip(contexts, lens)]))
+    x, weight, before = rnd(n, C), rnd(C, taps, seed=1), rnd(len(lens), 10, C, seed=2)
+    for bias in (rnd(C, seed=3), None):
+        got = []
+        for t, w in ((taps, weight), (6, torch.cat([torch.zeros(C, 6 - taps, device=DEV), weight], dim=1).contiguous())):
+            state = torch.full((5, (t - 1) * C), 7.0, device=DEV)
+            for r, slot in enumerate(slots):
+                for at in range(max(0, contexts[r] - (t - 1)), contexts[r]):
+                    if slot >= 0:
+                        state[slot, at % (t - 1) * C:(at % (t - 1) + 1) * C] = before[r, at]
+            out = torch.empty(n, C, dtype=dtype, device=DEV)
+            ops.conv_act(out, x, w, bias, state, 0, ctx)
+            got.append(out)
+        assert torch.equal(*got)
