@@ -10,7 +10,8 @@
 // instruction reads 64 contiguous bytes of each of 16 rows (whole sectors;
 // a lane reading 32 contiguous bytes in two instructions touched every
 // sector twice). Weights are
-// read once, straight from global memory into registers, 16 bytes a lane,
+// read, where K is whole units of 64 by way of a ring in LDS of each wave's own
+// (gemm_stream_kernel), otherwise straight from global memory into registers, 16 bytes a lane,
 // one trip ahead of the multiplies; the tokens' rows come from L2 (every
 // workgroup reads all of them: few, wide tiles of N would starve most CUs).
 // K must be a multiple of 8. The order of the sum depends on the output feature, K and the
@@ -258,7 +259,7 @@ constexpr int kEpiPlanes = 5, kEpiGluSilu = 6, kEpiGluGelu = 7;
 template <typename OutT, int MR, int NT, int R, int EPI>
 __global__ void __launch_bounds__(1024)
 gemm_stream_kernel(const bf16_t* __restrict__ a, int64_t lda, const bf16_t* __restrict__ w, int M, int N, int K,
-                   EpiParams epi, BaseSum base, int part_k, int64_t part_stride, int split_shift) {
+                   EpiParams epi, BaseSum base, int part_k, int64_t part_stride, int split_shift, int trip_shift) {
     constexpr bool GLU = EPI == kEpiGluSilu || EPI == kEpiGluGelu;
     static_assert(!GLU || NT == 2, "one tile of the gate's features and one of the other half's");
     constexpr int NB = 16 * NT, LOADS = (NB + MR) / 8, SLOT = (NB + MR) * kUnit;
@@ -269,11 +270,11 @@ gemm_stream_kernel(const bf16_t* __restrict__ a, int64_t lda, const bf16_t* __re
     const int i = lane % 16, g = lane / 16;
     const int n0 = blockIdx.x * (GLU ? 16 : NB), m0 = blockIdx.y * 16;
     const int k_begin = blockIdx.z * part_k, k_end = min(K, k_begin + part_k);
-    const int units = (k_end - k_begin) / kUnit, pairs = (units + 1) / 2;
-    // this wave's units: those of pairs wave, wave + ksplit, ... (the last of all may be half a pair); ksplit = 1 << split_shift
-    const int ksplit = 1 << split_shift;
-    const int my_pairs = wave < ksplit ? (pairs - wave + ksplit - 1) >> split_shift : 0;
-    const int mine = 2 * my_pairs - ((units & 1) != 0 && ((pairs - 1) & (ksplit - 1)) == wave ? 1 : 0);
+    // this wave's units: those of trips wave, wave + ksplit, ..., of one or two units each (the last of all may be half a pair); ksplit = 1 << split_shift
+    const int per_trip = 1 << trip_shift, ksplit = 1 << split_shift;
+    const int units = (k_end - k_begin) / kUnit, trips = (units + per_trip - 1) >> trip_shift;
+    const int my_trips = wave < ksplit ? (trips - wave + ksplit - 1) >> split_shift : 0;
+    const int mine = (my_trips << trip_shift) - ((units & (per_trip - 1)) != 0 && ((trips - 1) & (ksplit - 1)) == wave ? 1 : 0);
     if (gridDim.z > 1) epi.out = static_cast<float*>(epi.out) + blockIdx.z * part_stride;
     if (blockIdx.z > 0) epi.bias = nullptr;  // a cut product's bias goes to its first plane only
     bf16_t* const ring = reinterpret_cast<bf16_t*>(stream_lds) + wave * R * SLOT;
@@ -291,7 +292,7 @@ gemm_stream_kernel(const bf16_t* __restrict__ a, int64_t lda, const bf16_t* __re
         from[l] = a + static_cast<int64_t>(min(m0 + row, M - 1)) * lda + k_begin + (lpos ^ ring_swizzle(row)) * 8;
     }
     auto load = [&](int j, int slot) {  // unit j of this wave's (one past its last: the last of K, not multiplied)
-        const int k = min((((j / 2) << split_shift) + wave) * 2 + j % 2, units - 1) * kUnit;
+        const int k = min(((((j >> trip_shift) << split_shift) + wave) << trip_shift) + (j & (per_trip - 1)), units - 1) * kUnit;
 #pragma unroll
         for (int l = 0; l < LOADS; ++l) {
             const bf16_t* const piece = from[l] + k;
@@ -409,7 +410,7 @@ gemm_stream_kernel(const bf16_t* __restrict__ a, int64_t lda, const bf16_t* __re
 
 template <typename OutT, int MR, int NT, int R, int EPI>
 int launch_stream_as(const bf16_t* a, int64_t lda, const bf16_t* w, int M, int N, int K, int ksplit, int waves, const EpiParams& epi, const BaseSum& base,
-                     int kparts, int part_k, int64_t part_stride, hipStream_t stream) {
+                     int kparts, int part_k, int64_t part_stride, int trip_shift, hipStream_t stream) {
     size_t smem = static_cast<size_t>(waves) * R * (16 * NT + MR) * kUnit * sizeof(bf16_t);
     if (smem < waves * NT * 256 * sizeof(float)) smem = waves * NT * 256 * sizeof(float);
     LIYAB_REQUIRE(smem <= 160 * 1024, "gemm_skinny: %zu bytes of LDS", smem);
@@ -420,21 +421,22 @@ int launch_stream_as(const bf16_t* a, int64_t lda, const bf16_t* w, int M, int N
         ready = true;
     }
     constexpr int wide = EPI >= kEpiGluSilu ? 16 : 16 * NT;  // output features a workgroup
-    kern<<<dim3((N + wide - 1) / wide, (M + 15) / 16, kparts), 64 * waves, smem, stream>>>(a, lda, w, M, N, K, epi, base, part_k, part_stride, __builtin_ctz(ksplit));
+    kern<<<dim3((N + wide - 1) / wide, (M + 15) / 16, kparts), 64 * waves, smem, stream>>>(a, lda, w, M, N, K, epi, base, part_k, part_stride, __builtin_ctz(ksplit), trip_shift);
     return check_launch("gemm_skinny");
 }
 template <typename OutT, int EPI>
 int launch_stream_epi(const void* a, int64_t lda, const void* w, int M, int N, int K, int ksplit, const EpiParams& epi, const BaseSum& base, int kparts,
-                  int64_t part_stride, hipStream_t stream) {
-    const int units = (K / kUnit + kparts - 1) / kparts, pairs = (units + 1) / 2, mine = 2 * ((pairs + ksplit - 1) / ksplit);  // units of a part, units a wave
+                  int64_t part_stride, int trip_shift, hipStream_t stream) {
+    const int per_trip = 1 << trip_shift, units = (K / kUnit + kparts - 1) / kparts;
+    const int trips = (units + per_trip - 1) / per_trip, mine = per_trip * ((trips + ksplit - 1) / ksplit);  // units of a part, units a wave
     const int rows = M <= 8 ? 8 : 16;
-    int waves = ksplit < pairs ? ksplit : pairs;
+    int waves = ksplit < trips ? ksplit : trips;
     auto ring = [&](int nt, int r) { return static_cast<size_t>(waves) * r * (16 * nt + rows) * kUnit * 2; };
     const int64_t strips = static_cast<int64_t>((N + 15) / 16) * ((M + 15) / 16) * kparts;
     // With a few more strips than compute units a workgroup takes two, where their rings fit (one row, us by one strip / by two, with all epilogues
     // in one kernel: 1,280 -> 5,120 7.7 / 5.8, 1,600 -> 6,400 8.6 / 7.1; 16 rows 6.5 / 6.1, 7.1 / 7.1); with twice as many it does where a wave has three units
     // (3,072 -> 8,192 13.3 / 11.9; 1,600 -> 8,192 8.4 / 8.8, 4,096 -> 8,192 16.2 / 17.5, 768 -> 50,257 17.1 / 19.2)
-    const bool wide = strips > 256 && strips <= (K > 1600 && K <= 3072 ? 512 : 448) && ring(2, 2) <= 160 * 1024;
+    const bool wide = trip_shift == 1 && strips > 256 && strips <= (K > 1600 && K <= 3072 ? 512 : 448) && ring(2, 2) <= 160 * 1024;
     const int nt = wide ? 2 : 1;
     // a thread an output element at least, so that each has what its epilogue reads asked for ahead (waves without a unit of K bring in one again)
     if (strips <= 256 && waves < 4 * nt && ring(nt, 2) * 4 * nt / waves <= 160 * 1024) waves = 4 * nt;
@@ -442,7 +444,10 @@ int launch_stream_epi(const void* a, int64_t lda, const void* w, int M, int N, i
     const bool four = mine > 2 && ring(nt, 4) <= 96 * 1024;
     auto* pa = static_cast<const bf16_t*>(a);
     auto* pw = static_cast<const bf16_t*>(w);
-#define LIYAB_STREAM(MR, NT, R) launch_stream_as<OutT, MR, NT, R, EPI>(pa, lda, pw, M, N, K, ksplit, waves, epi, base, kparts, units * kUnit, part_stride, stream)
+#define LIYAB_STREAM(MR, NT, R) launch_stream_as<OutT, MR, NT, R, EPI>(pa, lda, pw, M, N, K, ksplit, waves, epi, base, kparts, units * kUnit, part_stride, trip_shift, stream)
+    // more workgroups than compute units, of a wave a unit or two: one unit in flight, so that two of them share a compute unit (48 rows, us, two in flight and
+    // one: 768 -> 2,304 6.5 and 5.0, -> 3,072 8.6 and 6.0, 1,600 -> 1,600 7.4 and 6.2)
+    if (trip_shift == 0 && strips > 256 && mine <= 2 && ring(1, 2) > 80 * 1024) return LIYAB_STREAM(16, 1, 1);
     if (rows == 8) {
         if (wide) return four ? LIYAB_STREAM(8, 2, 4) : LIYAB_STREAM(8, 2, 2);
         return four ? LIYAB_STREAM(8, 1, 4) : LIYAB_STREAM(8, 1, 2);
@@ -452,8 +457,8 @@ int launch_stream_epi(const void* a, int64_t lda, const void* w, int M, int N, i
 #undef LIYAB_STREAM
 }
 int launch_stream(const void* a, int64_t lda, const void* w, int M, int N, int K, int ksplit, const EpiParams& epi, const BaseSum& base, int kparts,
-                  int64_t part_stride, hipStream_t stream) {
-#define LIYAB_STREAM(OUT, EPI) launch_stream_epi<OUT, EPI>(a, lda, w, M, N, K, ksplit, epi, base, kparts, part_stride, stream)
+                  int64_t part_stride, int trip_shift, hipStream_t stream) {
+#define LIYAB_STREAM(OUT, EPI) launch_stream_epi<OUT, EPI>(a, lda, w, M, N, K, ksplit, epi, base, kparts, part_stride, trip_shift, stream)
     if (base.planes != nullptr) return LIYAB_STREAM(float, kEpiPlanes);
     if (epi.mode == kEpiResidual) return LIYAB_STREAM(float, kEpiResidual);
     if (epi.out_dtype == kF32) return epi.mode == kEpiNone ? LIYAB_STREAM(float, kEpiNone) : LIYAB_STREAM(float, -1);
@@ -533,8 +538,12 @@ static int skinny_dispatch(const void* a, int64_t lda, const void* w, int M, int
                   "gemm_skinny: ksplit %d is not 1, 2, 4, 8 or 16", ksplit);
     // (with one or two units of K and more strips than compute units the kernel of registers is as fast, 128 -> 8,192 at one row 3.8 us against 3.9)
     if (nt == 1 && mt == 1 && K % kUnit == 0 && K % 16384 != 0 && (K > 2 * kUnit || N * ((M + 15) / 16) <= 16 * 256)) {
-        return launch_stream(a, lda, w, M, N, K, ksplit, epi, base, kparts, part_stride, stream);
+        return launch_stream(a, lda, w, M, N, K, ksplit, epi, base, kparts, part_stride, 1, stream);
     }
+    // More rows than 16: blocks of 16, each reading the weights again (from L2 but for the first), with the waves and the order of sums of the tiles of rows
+    // chosen above. (us, cold weights, registers / rings: 24 rows 768 -> 768 4.9 / 3.4, -> 3,072 6.3 / 5.0, 3,072 -> 768 9.0 / 5.5, 6,400 -> 1,600 15.1 / 10.1; 64 rows
+    // 768 -> 768 5.0 / 3.6, -> 2,304 8.3 / 5.9, 1,600 -> 1,600 8.0 / 6.4, -> 4,800 17.8 / 12.0, 2,048 -> 8,192 24.6 / 20.8.)
+    if (nt == 1 && mt > 1 && K % kUnit == 0 && K % 16384 != 0) return launch_stream(a, lda, w, M, N, K, ksplit, epi, base, kparts, part_stride, 0, stream);
     if (nt == 1) {
         if (mt == 1) return launch_skinny<1, 1, 16>(a, lda, w, M, N, K, ksplit, epi, base, kparts, part_stride, stream);
         if (mt == 2) return launch_skinny<2, 1, 16>(a, lda, w, M, N, K, ksplit, epi, base, kparts, part_stride, stream);
@@ -627,7 +636,7 @@ extern "C" int liyab_gemm_skinny_glu(const void* a, int64_t lda, const void* w, 
     const int rows = M <= 8 ? 8 : 16, waves = live < 4 ? 4 : live;
     auto* pa = static_cast<const bf16_t*>(a);
     auto* pw = static_cast<const bf16_t*>(w);
-#define LIYAB_GLU(MR, EPI) launch_stream_as<bf16_t, MR, 2, 2, EPI>(pa, lda, pw, M, ff, K, ksplit, waves, epi, BaseSum{nullptr, 0, 0}, 1, K, 0, stream)
+#define LIYAB_GLU(MR, EPI) launch_stream_as<bf16_t, MR, 2, 2, EPI>(pa, lda, pw, M, ff, K, ksplit, waves, epi, BaseSum{nullptr, 0, 0}, 1, K, 0, 1, stream)
     if (rows == 8) return act == 0 ? LIYAB_GLU(8, kEpiGluSilu) : LIYAB_GLU(8, kEpiGluGelu);
     return act == 0 ? LIYAB_GLU(16, kEpiGluSilu) : LIYAB_GLU(16, kEpiGluGelu);
 #undef LIYAB_GLU

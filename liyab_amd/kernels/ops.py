@@ -715,8 +715,9 @@ def k_parts(M: int, N: int, K: int) -> int:
     """Into how many parts of K the weight-streaming product is best cut (1: not at all). With
     few output features a product fills a fraction of the chip's compute units, and a long K
     then streams through those few; cut over K it covers the chip. Measured at 8 rows, whole
-    and in parts (us): 3,072 -> 768 7.2 and 4.5 (four parts), 768 -> 768 4.6 and 3.4 (four),
-    6,400 -> 1,600 13.4 and 8.5 (two), 1,600 -> 1,600 5.4 and 4.6 (two)."""
+    and in parts (us): 3,072 -> 768 5.1 and 4.2 (four parts), 768 -> 768 3.3 and 3.4 (four: with the kernel that held
+    its operands in registers 4.5 and 3.7; the parts stay, whose sums another cut would round otherwise),
+    6,400 -> 1,600 7.5 and 6.8 (two), 1,600 -> 1,600 4.5 and 4.3 (two)."""
     if M > 32 or K % 8 != 0 or _invariant:
         return 1
     groups, units = (N + 15) // 16 * ((M + 15) // 16), (K + 63) // 64  # workgroups uncut; units of 64 k
@@ -737,8 +738,8 @@ def tiled_k_parts(M: int, N: int, K: int) -> int:
     Several tiles of rows, few output features and a long K (a prompt's portion through the feed-forward's second product: 128 x 768 x 3,072 is
     24 tiles of 64 x 64, each walking the whole of K in 18.7 us): cut until the tiles cover the
     chip. One tile of rows (33 to 64): the 64 x 32 tiles are few and each walks the whole of K;
-    cut over K they cover the chip: alone, at 64 rows, 3,072 -> 768 takes 8.2 us whole (the streaming kernel) and 4.9 in 8 parts, 6,400 ->
-    1,600 19.8 and 8.2. In a decode step the next readers pay for the planes, though: inner
+    cut over K they cover the chip: alone, at 64 rows, 3,072 -> 768 takes 5.7 us whole (the streaming kernel) and 4.9 in 8 parts, 6,400 ->
+    1,600 16.3 and 8.2. In a decode step the next readers pay for the planes, though: inner
     dimensions from 3,072 gain, in 4 parts (ms a step at 64 rows, whole and cut: GPT-2 small's
     sizes 0.806 and 0.797, medium's 1.767 and 1.715; XL's 5.19 and 4.90)."""
     if K % 64 != 0 or M <= 16 or _invariant:
@@ -834,7 +835,7 @@ def skinny_ln_pays(M: int, N: int, K: int) -> bool:
     product. The folded kernel keeps a row in registers, so one workgroup fills a compute unit:
     with more workgroups (16 or 32 output features each) than compute units they run in two
     rounds, which costs more than the norm's kernel (GPT-2 XL's 1,600 -> 4,800 at 8 rows in
-    strips of 16: 15.2 us folded against 9 + 4.5)."""
+    strips of 16: 9.5 us folded against 8.8 for both)."""
     return not _invariant and skinny_ln_takes(M, K) and (N + (31 if M <= 16 else 15)) // (32 if M <= 16 else 16) <= compute_units()
 
 
@@ -892,7 +893,8 @@ def gemm(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], *, out:
               and (M + 63) // 64 * ((N + 31) // 32) <= compute_units()):
             # one tile of 33 to 64 rows and many output features: 64 x 32 tiles share the tokens'
             # rows through LDS where the streaming kernel's workgroups each read them again (40
-            # rows: 5.2 against 6.4 us for 768 -> 2,304, 8.0 against 10.4 for 1,600 -> 4,800; the
+            # rows: 5.2 against 6.4 us for 768 -> 2,304, 8.0 against 10.4 for 1,600 -> 4,800, before the streaming
+            # kernel's rings: 5.0 and 10.1 at 48 rows since, 5.9 and 12.0 at 64; the lines stay, for the two add in different orders; the
             # products back to the model's width, with fewer tiles, stay with the streaming kernel);
             # the largest matrices already from 17 rows (32 rows, weights cold from HBM: 8.9
             # against 12.5 us for 1,600 -> 4,800, but 6.6 against 6.1 for 1,024 -> 3,072); more

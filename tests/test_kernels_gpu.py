@@ -1651,3 +1651,23 @@ def test_a_short_convolution_with_its_inputs_ahead_has_the_general_kernels_bits(
             ops.conv_act(out, x, w, bias, state, 0, ctx)
             got.append(out)
         assert torch.equal(*got)
+
+
+@pytest.mark.parametrize("K", [64, 192, 832, 1600, 3072])
+def test_streamed_products_of_17_rows_and_more_leave_the_bits_of_the_others(ops, K):
+    """17 to 64 rows: the kernel whose operands come through rings in LDS (whole units of 64 k) against the one that holds them in registers, which gets
+    eight zeros more a row; blocks of rows and strips of features at their edges, sums, the residual stream and parts of K."""
+    pad = lambda t: torch.nn.functional.pad(t, (0, 8)).contiguous()  # noqa: E731
+    for M in (17, 32, 33, 64):
+        for N in (3, 40, 768, 2310):
+            a, w, bias = rnd(M, K, dtype=torch.bfloat16, seed=K), rnd(N, K, dtype=torch.bfloat16, seed=K + 1, scale=0.2), rnd(N, seed=2)
+            got = []
+            for x, y in ((a, w), (pad(a), pad(w))):
+                out, half, added = torch.empty(M, N, device=DEV), torch.empty(M, N, dtype=torch.bfloat16, device=DEV), rnd(M, N, seed=3)
+                ops.gemm_skinny(x, y, bias, out=out)
+                ops.gemm_skinny(x, y, None, out=half)
+                ops.gemm_skinny(x, y, bias, residual=added, epilogue=ops.EPI_RESIDUAL)
+                planes = torch.empty(1, M, N, device=DEV)
+                ops.gemm_skinny_parts(x, y, planes, bias=bias, base=rnd(2, M, N, seed=4))
+                got.append((out, half, added, planes))
+            assert all(torch.equal(p, q) for p, q in zip(*got)), (M, N)
