@@ -400,9 +400,13 @@ sample_registers_kernel(int* __restrict__ out, const float* __restrict__ logits,
             for (int e = 0; e < 4; ++e) keys[4 * g + e] = v[e];
         }
     }
-    // (a wave whose ids all lie inside the row, most waves, does not look at each)
+    // Up to 72 ids a thread: a wave whose ids all lie inside the row, most waves, does not look at each; the place of the largest key is looked for afterwards, only
+    // by a thread that holds the wave's largest; and four neighbours' largest keys count as one. With 128 ids the registers hold little beside the row (that
+    // form spilled 48 of them, 44 with cuts): one loop finds the largest key and its place, and each thread's counts for itself (8 rows of 60,000, us, spilling and
+    // not: no cuts 39.5 and 36.0, top-k 40 with top-p 0.95 30.5 and 26.8, the largest alone 14.7 and 11.3).
+    constexpr bool kRoomy = EPT < 128;
     const int first_id = __builtin_amdgcn_readfirstlane(span0);
-    if (chunk == EPT && first_id >= 0 && first_id + kWave * EPT <= V) {
+    if (kRoomy && chunk == EPT && first_id >= 0 && first_id + kWave * EPT <= V) {
 #pragma unroll
         for (int j = 0; j < EPT; ++j) keys[j] = ordered_key(__uint_as_float(again(keys[j])));
     } else {
@@ -412,12 +416,16 @@ sample_registers_kernel(int* __restrict__ out, const float* __restrict__ logits,
             keys[j] = (j < chunk && id_of(j) >= 0 && id_of(j) < V) ? ordered_key(__uint_as_float(raw)) : 0u;
         }
     }
-    // the largest key and its lowest id (only a thread that holds the wave's largest key looks for the place)
+    // the largest key and its lowest id
     uint32_t kmax = 0;
+    int imax = 0x7fffffff;
 #pragma unroll
-    for (int j = 0; j < EPT; ++j) kmax = max(kmax, keys[j]);
+    for (int j = 0; j < EPT; ++j) {
+        if constexpr (kRoomy) kmax = max(kmax, keys[j]);
+        else if (keys[j] > kmax) { kmax = keys[j]; imax = id_of(j); }
+    }
     // the largest of four neighbours' keys, where there are enough such groups to find a floor among
-    const bool by_four = (V + shift) / chunk >= 8 * kWaveCandidates;
+    const bool by_four = kRoomy && (V + shift) / chunk >= 8 * kWaveCandidates;
     if constexpr (!PLAIN) {
         uint32_t group = kmax;
         if (by_four) {
@@ -428,8 +436,7 @@ sample_registers_kernel(int* __restrict__ out, const float* __restrict__ logits,
             thread_max[tid] = group;
         }
     }
-    int imax = 0x7fffffff;
-    {
+    if constexpr (kRoomy) {
         const uint32_t wave_largest = wave_max_key(kmax);
         if (kmax == wave_largest && kmax != 0u) {
 #pragma unroll
