@@ -97,6 +97,10 @@ gemm_skinny_ln_kernel(NormParams ln, const bf16_t* __restrict__ w, int M, int N,
     // -- the norm: a wave per row, the row in registers ---------------------------------
     const int nv = K / 4;
     const floatx4 fzero = {0.0f, 0.0f, 0.0f, 0.0f}, fone = {1.0f, 1.0f, 1.0f, 1.0f};
+    // Where a wave has a row or two of up to 1,024 they are read in any case and chosen behind the planes' sums. Past 1,024 there are no registers for vectors
+    // that may be dropped (2 to 10 spilled), and past 16 rows a wave has several rows in turn: chosen at the load there (us, late / at the load: 8 rows 1,600 ->
+    // 4,800 10.5 / 9.3, 16 rows 2,048 -> 6,144 16.1 / 13.9, 1,280 -> 3,840 9.9 / 9.4; 24 rows 768 -> 2,304 8.4 / 7.7, 1,024 -> 3,072 9.9 / 8.8).
+    constexpr bool CHOSEN_LATE = MAXV < 8 && MT == 1;
     const float* const norm_weight = ln.weight != nullptr ? ln.weight : ln.planes;  // (without one: a row's values, read and dropped)
     const float* const norm_bias = ln.bias != nullptr ? ln.bias : ln.planes;
     // `between` runs once the row's first loads are asked for and before anything waits for them
@@ -109,8 +113,13 @@ gemm_skinny_ln_kernel(NormParams ln, const bf16_t* __restrict__ w, int M, int N,
         for (int j = 0; j < MAXV; ++j) {
             const int at = min(lane + kWave * j, nv - 1);  // past the row: its last piece again, unused
             v[j] = reinterpret_cast<const floatx4*>(row0)[at];
-            gw[j] = reinterpret_cast<const floatx4*>(norm_weight)[at];
-            gb[j] = reinterpret_cast<const floatx4*>(norm_bias)[at];
+            if constexpr (CHOSEN_LATE) {
+                gw[j] = reinterpret_cast<const floatx4*>(norm_weight)[at];
+                gb[j] = reinterpret_cast<const floatx4*>(norm_bias)[at];
+            } else {
+                gw[j] = ln.weight != nullptr ? reinterpret_cast<const floatx4*>(ln.weight)[at] : fone;
+                gb[j] = ln.bias != nullptr ? reinterpret_cast<const floatx4*>(ln.bias)[at] : fzero;
+            }
         }
         // further planes, PB together (a plane past the last is the last one again, read and dropped)
         constexpr int PB = MAXV <= 4 ? 3 : 1;  // what the registers hold
@@ -134,10 +143,12 @@ gemm_skinny_ln_kernel(NormParams ln, const bf16_t* __restrict__ w, int M, int N,
                 for (int j = 0; j < MAXV; ++j)
                     if (q0 + u < ln.n_planes) v[j] += plane[u][j];
         }
+        if constexpr (CHOSEN_LATE) {
 #pragma unroll
-        for (int j = 0; j < MAXV; ++j) {
-            gw[j] = ln.weight != nullptr ? gw[j] : fone;
-            gb[j] = ln.bias != nullptr ? gb[j] : fzero;
+            for (int j = 0; j < MAXV; ++j) {
+                gw[j] = ln.weight != nullptr ? gw[j] : fone;
+                gb[j] = ln.bias != nullptr ? gb[j] : fzero;
+            }
         }
         if constexpr (DYT) {
             // tanh(z) = 1 - 2 / (1 + e^(2z)): one hardware exponential and one reciprocal a value
