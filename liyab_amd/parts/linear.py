@@ -26,8 +26,10 @@ from .norms import Normed
 # together, where the stream is whole (the feed-forward's first product): 721 against 713, 48 rows 656
 # against 652. That form was taken out again.)
 # Since the streaming product's rings the two kernels are as fast from 13 rows on (us a decode step, folded and not: small's sizes 12 rows 441 / 452, 13
-# 463 / 459, 16 474 / 464, medium's 12 899 / 904, 13 953 / 900, 16 967 / 907): up to 16 rows of up to 1,024 they take over, where both leave the same bits; rows
-# past 16 (24: 549 / 528, 1,151 / 1,078) and wider ones stay folded, whose products add in another order.
+# 463 / 459, 16 474 / 464, medium's 12 899 / 904, 13 953 / 900, 16 967 / 907): up to 16 rows of 513 to 1,024, a multiple of 64, they take over. Both leave the same
+# bits, but for 8,177 to 8,192 features, where four waves share K and not the folded kernel's eight (another order of the same sum). Narrower rows and those
+# without rings stay folded (16 rows, us, folded / not: 576 -> 2,304 6.3 / 6.0; 512 -> 1,536 5.6 / 5.9, 128 -> 384 4.4 / 5.3, 200 -> 600 4.2 / 5.7, 72 -> 1,024 4.3 /
+# 6.1), rows past 16 (24: 549 / 528, 1,151 / 1,078) and wider ones too, whose products add in another order.
 FOLD_NORM = True
 FOLD_NORM_ROWS = 24
 TILED_PARTS = True  # products of 33 to 64 rows that are added to the stream: tiled and cut over K (ops.tiled_k_parts)
@@ -37,7 +39,7 @@ def _fuses(a, w: torch.Tensor, residual) -> bool:
     return (FOLD_NORM and isinstance(a, Normed) and getattr(a.norm, "fusable", None) in ("layernorm", "dyt") and residual is None
             and a.rows is None and a._tensor is None and w.dtype == torch.bfloat16 and a.x.dtype == torch.float32
             and a.x.is_contiguous() and a.n_rows <= FOLD_NORM_ROWS
-            and not (12 < a.n_rows <= 16 and a.norm.width <= 1024 and a.norm.fusable == "layernorm")
+            and not (12 < a.n_rows <= 16 and 512 < a.norm.width <= 1024 and a.norm.width % 64 == 0 and a.norm.fusable == "layernorm")
             and ops.skinny_ln_pays(a.n_rows, w.shape[0], a.norm.width))
 
 

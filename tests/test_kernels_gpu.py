@@ -1671,3 +1671,41 @@ def test_streamed_products_of_17_rows_and_more_leave_the_bits_of_the_others(ops,
                 ops.gemm_skinny_parts(x, y, planes, bias=bias, base=rnd(2, M, N, seed=4))
                 got.append((out, half, added, planes))
             assert all(torch.equal(p, q) for p, q in zip(*got)), (M, N)
+
+
+@pytest.mark.parametrize("K", [64, 512, 576, 768, 832, 1000, 1024])
+def test_steps_of_13_to_16_rows_keep_the_folded_norms_bits(ops, K, monkeypatch):
+    """A norm and the product behind it as the parts run them, against the kernel that folds them: the same bits on either side of the rows (13 to 16) and widths
+    (513 to 1,024) that take the norm's own kernel instead, in planes too. From 8,177 features on four waves share K and not eight: another order of the same
+    sum, no further from the 64-bit product."""
+    from types import SimpleNamespace
+
+    from liyab_amd.parts import linear as lin
+    from liyab_amd.parts.norms import LayerNorm, Normed
+
+    taken = []
+    for name in ("gemm_skinny_ln", "layernorm"):
+        monkeypatch.setattr(ops, name, (lambda f, n: lambda *a, **k: (taken.append(n), f(*a, **k))[1])(getattr(ops, name), name))
+    norm = LayerNorm.__new__(LayerNorm)
+    norm.width, norm.eps, norm.dtype, norm.weight, norm.bias = K, 1e-5, torch.bfloat16, rnd(K, seed=1) + 1.0, rnd(K, seed=2)
+    for M in (12, 13, 16, 17):
+        for N in (16, 300, 8176, 8177, 8192):
+            if not ops.skinny_ln_pays(M, N, K):
+                continue
+            w, bias = rnd(N, K, dtype=torch.bfloat16, seed=3, scale=0.2), rnd(N, seed=4)
+            for planes in (1, 4):
+                x = rnd(planes, M, K, seed=5) if planes > 1 else rnd(M, K, seed=5)
+                ctx = SimpleNamespace(workspace=SimpleNamespace(get=lambda name, shape, dtype: torch.empty(shape, dtype=dtype, device=DEV)))
+                got, want = torch.empty(M, N, device=DEV), torch.empty(M, N, device=DEV)
+                taken.clear()
+                lin.linear(Normed(norm, x, ctx), w, bias, out=got)
+                own_kernel = 12 < M <= 16 and 512 < K <= 1024 and K % 64 == 0
+                assert taken == (["layernorm"] if own_kernel else ["gemm_skinny_ln"]), (M, N)
+                ops.gemm_skinny_ln(x, norm.weight, norm.bias, 1e-5, w, bias, out=want)
+                if N <= 8176 or not own_kernel:
+                    assert torch.equal(got, want), (M, N, planes)
+                    continue
+                rows = torch.nn.functional.layer_norm(x.sum(0) if planes > 1 else x, (K,), norm.weight, norm.bias, 1e-5).bfloat16()
+                exact = rows.double() @ w.double().T + bias.double()
+                err = lambda t: ((t.double() - exact).norm() / exact.norm()).item()  # noqa: E731
+                assert err(got) <= 1.1 * err(want) + 1e-7, (M, N, planes, err(got), err(want))
