@@ -617,12 +617,12 @@ extern "C" int liyab_gemm_skinny_parts(const void* a, int64_t lda, const void* w
                            part_stride);
 }
 
-// A gated feed-forward's first product and its activation: out[m, n] = act(a[m] . w[n]) * (a[m] . w[ff + n]), a [M <= 16, K] and w [2 ff, K] bfloat16, out
-// [M, ff] bfloat16, K a multiple of 64 and not of 16,384; act 0: silu, 1: the tanh form of gelu. The bits of liyab_gemm_skinny to 32-bit rows followed by
+// A gated feed-forward's first product and its activation: out[m, n] = act(a[m] . w[n]) * (a[m] . w[ff + n]), a [M <= 8, K] and w [2 ff, K] bfloat16, out
+// [M, ff] bfloat16, K a multiple of 64 and not of 16,384 (rings of 8 rows: 16 waves of them are the LDS a workgroup may have); act 0: silu, 1: the tanh form of gelu. The bits of liyab_gemm_skinny to 32-bit rows followed by
 // liyab_glu. (8 rows, cold weights, us in two kernels and in one: 768 -> 2 x 2,048 6.8 and 5.0, 1,024 -> 2 x 2,720 7.5 and 5.5, 4,096 -> 2 x 8,064 30.0 and 26.8.)
 extern "C" int liyab_gemm_skinny_glu(const void* a, int64_t lda, const void* w, int M, int ff, int K, int act, void* out, int64_t ldo, hipStream_t stream) {
     LIYAB_REQUIRE(a && w && out, "gemm_skinny_glu: null operand");
-    LIYAB_REQUIRE(M >= 0 && M <= 16 && ff > 0 && K > 0 && K % kUnit == 0 && K % 16384 != 0, "gemm_skinny_glu: bad sizes M=%d (at most 16) ff=%d K=%d", M, ff, K);
+    LIYAB_REQUIRE(M >= 0 && M <= 8 && ff > 0 && K > 0 && K % kUnit == 0 && K % 16384 != 0, "gemm_skinny_glu: bad sizes M=%d (at most 8) ff=%d K=%d", M, ff, K);
     LIYAB_REQUIRE(lda % 8 == 0 && lda >= K && ldo >= ff, "gemm_skinny_glu: bad row strides %lld, %lld", static_cast<long long>(lda), static_cast<long long>(ldo));
     LIYAB_REQUIRE((reinterpret_cast<uintptr_t>(a) & 15) == 0 && (reinterpret_cast<uintptr_t>(w) & 15) == 0, "gemm_skinny_glu: operands must be 16-byte aligned");
     LIYAB_REQUIRE(act == 0 || act == 1, "gemm_skinny_glu: unknown activation %d", act);
@@ -633,11 +633,10 @@ extern "C" int liyab_gemm_skinny_glu(const void* a, int64_t lda, const void* w, 
     epi.ldo = ldo;
     // (the waves that the product alone would have: the order of its sums)
     const int units = K / kUnit, ksplit = choose_ksplit((2 * ff + 15) / 16, units, 2), pairs = (units + 1) / 2, live = ksplit < pairs ? ksplit : pairs;
-    const int rows = M <= 8 ? 8 : 16, waves = live < 4 ? 4 : live;
+    const int waves = live < 4 ? 4 : live;
     auto* pa = static_cast<const bf16_t*>(a);
     auto* pw = static_cast<const bf16_t*>(w);
-#define LIYAB_GLU(MR, EPI) launch_stream_as<bf16_t, MR, 2, 2, EPI>(pa, lda, pw, M, ff, K, ksplit, waves, epi, BaseSum{nullptr, 0, 0}, 1, K, 0, 1, stream)
-    if (rows == 8) return act == 0 ? LIYAB_GLU(8, kEpiGluSilu) : LIYAB_GLU(8, kEpiGluGelu);
-    return act == 0 ? LIYAB_GLU(16, kEpiGluSilu) : LIYAB_GLU(16, kEpiGluGelu);
+#define LIYAB_GLU(EPI) launch_stream_as<bf16_t, 8, 2, 2, EPI>(pa, lda, pw, M, ff, K, ksplit, waves, epi, BaseSum{nullptr, 0, 0}, 1, K, 0, 1, stream)
+    return act == 0 ? LIYAB_GLU(kEpiGluSilu) : LIYAB_GLU(kEpiGluGelu);
 #undef LIYAB_GLU
 }

@@ -1558,6 +1558,20 @@ def test_an_activation_inside_its_product_leaves_its_own_kernels_bits(ops, K, ff
         assert torch.equal(got, want), M
 
 
+@pytest.mark.parametrize("K", [64, 192, 1728, 2048])
+def test_an_activation_inside_its_product_takes_eight_rows_at_most(ops, K):
+    """What the entry says of itself at every K: nine rows are refused by their number (16 waves' rings of 16 rows would pass a workgroup's LDS), eight run."""
+    a, w = rnd(9, K, dtype=torch.bfloat16, seed=1), rnd(2 * 24, K, dtype=torch.bfloat16, seed=2, scale=0.2)
+    out = torch.zeros(9, 24, dtype=torch.bfloat16, device=DEV)
+    assert not ops.glu_in_product_takes(a, w)
+    with pytest.raises(ops.KernelError, match="at most 8"):
+        ops.gemm_glu(out, a, w, "silu")
+    ops.gemm_glu(out[:8], a[:8], w, "silu")
+    y = a[:8].double() @ w.double().T
+    want = torch.nn.functional.silu(y[:, :24]) * y[:, 24:]
+    assert (out[:8].double() - want).norm() <= 1e-2 * want.norm() and not out[8].any()
+
+
 @pytest.mark.parametrize("form", ["one", "centred", "gate", "next"])
 def test_rows_update_shares_a_row_among_four_waves_with_the_same_bits(ops, form):
     """Up to 1,536 rows a row belongs to four waves, beyond to one: what a row becomes does not depend on how many there are."""
