@@ -745,9 +745,14 @@ int launch_grouped_stream(const GroupedParams& p, const dim3& grid, hipStream_t 
     // Three units in flight, two where a unit has both halves' weights: 48 KiB of LDS, so that three workgroups share a compute unit (six units, 96 KiB and one
     // workgroup: 16 entries of 16 experts, 3,200 -> 1,600, 33 us, three 24, two 25; 2 entries of 8, 1,536 -> 768 5.4, 5.4, 5.9. Both halves, three and two: 1,600 ->
     // 2 x 3,200 49 and 45, 768 -> 2 x 768 7.0 and 7.2).
-    if (mine <= 1) LIYAB_STREAM(1);
-    else if (NW == 2 || mine <= 2) LIYAB_STREAM(2);
-    else LIYAB_STREAM(3);
+    if (mine <= 1) {
+        LIYAB_STREAM(1);
+    } else if constexpr (NW == 2) {
+        LIYAB_STREAM(2);
+    } else {
+        if (mine <= 2) LIYAB_STREAM(2);
+        else LIYAB_STREAM(3);
+    }
 #undef LIYAB_STREAM
     return check_launch("grouped_product");
 }
