@@ -482,7 +482,7 @@ extern "C" int liyab_gemm_rows_ln(const float* x, const float* ln_weight, const 
 }
 
 // residual += merge(partials) . w^T + bias over attention's splits [M][n_head][n_splits <= 8][hd + 4] (liyab_attention_decode with
-// leave_splits), K = n_head * hd.
+// leave_splits), K = n_head * hd. The rows lie in LDS, up to 32 a workgroup: 32 of up to 2,240 fit whatever the strip, 8 of 8,192; what does not is refused.
 extern "C" int liyab_gemm_rows_splits(const float* partials, int n_splits, int n_head, int hd, const void* w, int M, int N, int strip,
                                       const EpiParams* epi, hipStream_t stream) {
     LIYAB_REQUIRE(partials != nullptr, "gemm_rows_splits: null operand");

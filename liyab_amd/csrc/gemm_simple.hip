@@ -629,7 +629,8 @@ extern "C" int liyab_gemm_f32_qkv(const float* a, int64_t lda, const float* w, i
 
 // The same products over rows that the kernel makes itself (K a multiple of 64, operands 16-byte aligned): LayerNorm(x) of 32-bit rows x [M, K],
 // K <= 2048, every epilogue but the residual one; or attention's splits [M][n_head][n_splits <= 8][hd + 4] merged, K = n_head * hd, the residual
-// epilogue. The bits are those of liyab_layernorm or liyab_attention_merge followed by the product.
+// epilogue. As many rows as a workgroup's LDS holds beside its chunks (16 of up to 1,664 whatever N; of 2,048 up to 13): more is refused. The bits are those of
+// liyab_layernorm or liyab_attention_merge followed by the product.
 static int check_made(const void* x, const void* w, int M, int N, int K, const EpiParams* epi) {
     auto al16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
     LIYAB_REQUIRE(x && w && epi, "gemm_made_f32: null operand");

@@ -477,7 +477,8 @@ def gemm_f32_qkv(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor],
 def gemm_f32_ln(x: torch.Tensor, ln_weight: Optional[torch.Tensor], ln_bias: Optional[torch.Tensor], eps: float, w: torch.Tensor,
                 bias: Optional[torch.Tensor], *, out=None, epilogue: int = EPI_NONE, kv=None) -> None:
     """The 32-bit product over LayerNorm(x) of the float32 rows x [M, K], K a multiple of 64 up to 2,048, the norm computed inside the kernel: the bits of
-    `layernorm` followed by `gemm` (`gemm_f32_qkv` with `kv`)."""
+    `layernorm` followed by `gemm` (`gemm_f32_qkv` with `kv`). 16 rows at a time lie in LDS beside the weights: past 1,664 a row not in every product of 16 (an error
+    then; `f32_norm_pays` asks for less)."""
     ptr, n_parts, _, M, K = _planes(x, "gemm_f32_ln")
     _dev(w, "w")
     if n_parts != 1 or w.dtype != torch.float32 or w.dim() != 2 or w.shape[1] != K or not w.is_contiguous():
@@ -504,7 +505,8 @@ def splits_in_product_pay(M: int, splits: int, n_head: int, hd: int) -> bool:
 
 def gemm_splits(partials: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], *, residual: torch.Tensor) -> None:
     """residual += merge(partials) . w^T + bias over attention's splits [M, heads, splits, head size + 4], merged inside the product: the bits of
-    `attention_merge` followed by `gemm`, in 32 bits (w float32) or in the batch-invariant mode (w bfloat16)."""
+    `attention_merge` followed by `gemm`, in 32 bits (w float32) or in the batch-invariant mode (w bfloat16). Up to 8 splits, and as many rows as LDS holds (an error
+    beyond; `splits_in_product_pay` asks for less)."""
     if w.dtype != torch.float32:
         gemm_rows_splits(partials, w, bias, residual=residual)
         return

@@ -1280,6 +1280,36 @@ def test_splits_merged_inside_the_product_leave_the_merges_bits(ops, dtype, H, h
             assert torch.equal(got, want), M
 
 
+def test_rows_made_inside_a_product_are_as_many_as_lds_holds(ops):
+    """16 rows of 1,664, or 13 of 2,048, beside a workgroup's weights in 32 bits; 8 of 8,192 as merged splits in bfloat16, 4 in 32 bits: they run. More are refused, not run past it."""
+    for M, K, runs in ((16, 1664, True), (13, 2048, True), (14, 2048, False), (16, 2048, False)):
+        x, w = rnd(M, K, seed=1), rnd(2064, K, seed=2, scale=0.2)
+        rows, want, got = torch.empty(M, K, device=DEV), torch.empty(M, 2064, device=DEV), torch.zeros(M, 2064, device=DEV)
+        if not runs:
+            with pytest.raises(ops.KernelError, match="LDS"):
+                ops.gemm_f32_ln(x, None, None, 1e-5, w, None, out=got)
+            assert not got.any()
+            continue
+        ops.layernorm(rows, x, None, None, 1e-5)
+        ops.gemm(rows, w, None, out=want)
+        ops.gemm_f32_ln(x, None, None, 1e-5, w, None, out=got)
+        assert torch.equal(got, want), (M, K)
+    for M, H, dtype, runs in ((8, 64, torch.bfloat16, True), (32, 64, torch.bfloat16, False), (4, 64, torch.float32, True), (16, 64, torch.float32, False)):
+        p, w, base = rnd(M, H, 2, 132, seed=3), rnd(40, H * 128, dtype=dtype, seed=4, scale=0.2), rnd(M, 40, seed=5)
+        p[..., 129] = p[..., 129].abs() + 0.5
+        att, want, got = torch.empty(M, H * 128, dtype=dtype, device=DEV), base.clone(), base.clone()
+        with ops.batch_invariant(dtype == torch.bfloat16):
+            if not runs:
+                with pytest.raises(ops.KernelError, match="LDS"):
+                    ops.gemm_splits(p, w, None, residual=got)
+                assert torch.equal(got, base)
+                continue
+            ops.attention_merge(att, p)
+            ops.gemm(att, w, None, residual=want, epilogue=ops.EPI_RESIDUAL)
+            ops.gemm_splits(p, w, None, residual=got)
+            assert torch.equal(got, want), (M, H, dtype)
+
+
 @pytest.mark.parametrize("K", [64, 768, 3072])
 def test_tiles_of_one_sum_give_a_row_the_same_bits(ops, K):
     """The tiles of many rows take K in one chain of the same steps whatever their shape: the same bits from each, inside the
