@@ -1717,6 +1717,41 @@ def test_streamed_products_of_17_rows_and_more_leave_the_bits_of_the_others(ops,
             assert all(torch.equal(p, q) for p, q in zip(*got)), (M, N)
 
 
+@pytest.mark.parametrize("ksplit", [1, 4, 16])
+@pytest.mark.parametrize("K", [64, 192, 832, 1600])
+def test_streamed_products_of_up_to_16_rows_leave_the_bits_of_the_others(ops, K, ksplit):
+    """As above for 1 to 16 rows, both kernels on the same waves: one strip of 16 features a workgroup and two (5,000 features), rings of two units and of four, every
+    epilogue, K in one part and in two."""
+    pad = lambda t: torch.nn.functional.pad(t, (0, 8)).contiguous()  # noqa: E731
+    for M in (1, 8, 9, 16):
+        for N in (48, 768, 5000):  # whole heads of 16 below, for the pages
+            a, w, bias, base = rnd(M, K, dtype=torch.bfloat16, seed=K), rnd(N, K, dtype=torch.bfloat16, seed=K + 1, scale=0.2), rnd(N, seed=2), rnd(5, M, N, seed=4)
+            slots = torch.randperm(40)[:M].to(torch.int32).to(DEV)
+            slots[M // 2] = -1
+            got = []
+            for x, y in ((a, w), (pad(a), pad(w))):
+                out, half, added = torch.empty(M, N, device=DEV), torch.empty(M, N, dtype=torch.bfloat16, device=DEV), rnd(M, N, seed=3)
+                gelu, erf = torch.empty(M, N, device=DEV), torch.empty(M, N, dtype=torch.bfloat16, device=DEV)
+                ops.gemm_skinny(x, y, bias, out=out, ksplit=ksplit)
+                ops.gemm_skinny(x, y, None, out=half, ksplit=ksplit)
+                ops.gemm_skinny(x, y, bias, out=gelu, epilogue=ops.EPI_GELU_TANH, ksplit=ksplit)
+                ops.gemm_skinny(x, y, bias, out=erf, epilogue=ops.EPI_GELU_ERF, ksplit=ksplit)
+                ops.gemm_skinny(x, y, bias, residual=added, epilogue=ops.EPI_RESIDUAL, ksplit=ksplit)
+                one, two = torch.empty(1, M, N, device=DEV), torch.empty(2, M, N, device=DEV)
+                ops.gemm_skinny_parts(x, y, one, bias=bias, base=base, ksplit=ksplit)
+                if K > 64:  # (an odd number of units: the eight zeros leave the parts' border where it is)
+                    ops.gemm_skinny_parts(x, y, two, bias=bias, base=base[:2], ksplit=ksplit)
+                else:
+                    two.zero_()
+                outs = [out, half, gelu, erf, added, one, two]
+                if N == 768:
+                    q, kc, vc = (torch.zeros(s, dtype=torch.bfloat16, device=DEV) for s in ((M, 256), (10, 16, 4, 16), (10, 16, 4, 16)))
+                    ops.gemm_skinny(x, y, bias, out=q, epilogue=ops.EPI_QKV_PAGED, kv=(kc, vc, slots, 256), ksplit=ksplit)
+                    outs += [q, kc, vc]
+                got.append(outs)
+            assert all(torch.equal(p, q) for p, q in zip(*got)), (M, N, [torch.equal(p, q) for p, q in zip(*got)])
+
+
 @pytest.mark.parametrize("K", [64, 512, 576, 768, 832, 1000, 1024])
 def test_steps_of_13_to_16_rows_keep_the_folded_norms_bits(ops, K, monkeypatch):
     """A norm and the product behind it as the parts run them, against the kernel that folds them: the same bits on either side of the rows (13 to 16) and widths

@@ -602,6 +602,47 @@ def test_the_streams_update_of_few_rows_a_token_has_the_same_bits(S):
                 assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1]), (d, k)
 
 
+@pytest.mark.parametrize("out_dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("S", [1, 2, 3, 4])
+def test_identity_entries_and_entering_rows_have_the_general_kernels_bits(S, out_dtype):
+    """The kernel for few rows a token against the general one: identity entries among its rows (the rows that were routed lie where the next ones go, and what an
+    identity entry's row of y holds is not read), rows that enter with a sum behind them (a fifth row of zeros for the general kernel), rows that only enter and rows
+    that are only gathered (2,049 of them)."""
+    from liyab_amd.kernels import ops
+
+    n, eps = 5, 1e-5
+    rng = np.random.default_rng(S)
+    cut = lambda *shape: rand(rng, *shape).to(DEV)  # noqa: E731
+    for d in (64, 260, 768, 1024):
+        x, e, h = cut(n, S, d), cut(n, d), cut(n, d).to(out_dtype)
+        mix, add, take, w = cut(S, S), cut(S), cut(S), cut(d)
+        for k in (1, 2, 3, 4):
+            for n_ids in sorted({1, k - 1, k} - {0}):
+                ids = torch.from_numpy(rng.integers(-1, 2, (n, n_ids)).astype(np.int32)).to(DEV)
+                ids[0], ids[n - 1] = -1, 0
+                weights, y = cut(n, n_ids), cut(n, k, d)
+                y[:, :n_ids][ids < 0] = float("nan")
+                for enter in (None, e):
+                    got = []
+                    for rows in (y, torch.cat([y, torch.zeros(n, 5 - k, d, device=DEV)], dim=1)):
+                        into, out = x.clone(), h.clone()
+                        entries = ops.IdentityEntries(ids, weights, n_ids, out)
+                        ops.streams_update(into, enter=enter, y=rows.reshape(-1, d), n_sum=rows.shape[1], identity=entries, mix=mix, add=add, next_norm=(take, w, eps), out=out)
+                        got.append((into, out))
+                    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1]) and bool(got[0][1].isfinite().all()), (d, k, n_ids)
+    d, many = 256, 2049
+    x, e, w = cut(n, S, d), cut(many, d), cut(d)
+    big, out, few = torch.empty(many, S, d, device=DEV), torch.empty(many, d, dtype=out_dtype, device=DEV), torch.empty(n, d, dtype=out_dtype, device=DEV)
+    ops.streams_update(big, enter=e, next_norm=(None, w, eps), out=out)
+    into = x.clone()
+    ops.streams_update(into, enter=e[:n].contiguous(), next_norm=(None, w, eps), out=few)
+    assert torch.equal(into, big[:n]) and torch.equal(few, out[:n])
+    picked = torch.from_numpy(rng.integers(0, n, many).astype(np.int32)).to(DEV)
+    ops.streams_update(x, next_norm=(None, w, eps), out=out, rows=picked)
+    ops.streams_update(x, next_norm=(None, w, eps), out=few, rows=picked[:n].contiguous())
+    assert torch.equal(few, out[:n])
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_connections_that_single_a_stream_out(dtype, tmp_path):
     """A sublayer that reads the second stream alone and gives to the first alone, and a mix that moves each stream to the next: a
