@@ -14,9 +14,7 @@
 #include "common.h"
 #include "launchers.h"
 #include "epilogue.h"
-
-#include <type_traits>
-#include <utility>
+#include "ring.h"
 
 namespace liyab {
 namespace by_rows {
@@ -34,7 +32,6 @@ union Frag {
 
 enum : int { kRows = 0, kNorm = 1, kSplits = 2 };
 constexpr int SUMS = 4, ROWS = 32, UNIT = 64;  // sums, and waves; rows a workgroup; k of a unit
-typedef __attribute__((address_space(3))) void* lds_void_ptr;
 
 struct Source {
     const bf16_t* a;  // rows: [M, lda]
@@ -51,21 +48,6 @@ template <int NB, int MR, int RING>
 constexpr size_t ring_bytes() {
     constexpr size_t ring = MR > 0 ? static_cast<size_t>(SUMS) * RING * (NB + MR) * UNIT * 2 : 0, sums = static_cast<size_t>(SUMS) * NB * (ROWS + 1) * 4;
     return ring > sums ? ring : sums;
-}
-// Where the 16-byte pieces of a ring's row sit, so that 16 lanes' reads of 16 rows at one piece fall into different banks.
-__device__ __forceinline__ int swizzle(int row) { return (row >> 1) & 7; }
-
-// This wave's loads but the last LATER have arrived.
-template <int LATER>
-__device__ __forceinline__ void wait_loads() {
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_waitcnt((LATER & 15) | 0x0f70 | ((LATER >> 4) << 14));
-    asm volatile("" ::: "memory");
-}
-
-template <int... T, typename F>
-__device__ __forceinline__ void in_turn(std::integer_sequence<int, T...>, F&& f) {
-    (f(std::integral_constant<int, T>{}), ...);
 }
 
 // MR: rows of the ring (rows: 8, 16 or 32, M rounded up; otherwise 0). RING: units of the ring, or (norm, splits) sets of three units in
@@ -92,10 +74,10 @@ gemm_rows_kernel(Source src, const bf16_t* __restrict__ w, int M_all, int N, int
     const int lrow = lane / 8, lpos = lane % 8;
     const bf16_t* from[LOADS];
 #pragma unroll
-    for (int i = 0; i < W_LOADS; ++i) from[i] = w + static_cast<int64_t>(min(n0 + 8 * i + lrow, N - 1)) * K + (lpos ^ swizzle(8 * i + lrow)) * 8;
+    for (int i = 0; i < W_LOADS; ++i) from[i] = w + static_cast<int64_t>(min(n0 + 8 * i + lrow, N - 1)) * K + (lpos ^ ring_swizzle(8 * i + lrow)) * 8;
 #pragma unroll
     for (int i = 0; i < A_LOADS; ++i)
-        from[W_LOADS + i] = src.a + static_cast<int64_t>(row0 + min(8 * i + lrow, M - 1)) * src.lda + (lpos ^ swizzle(8 * i + lrow)) * 8;
+        from[W_LOADS + i] = src.a + static_cast<int64_t>(row0 + min(8 * i + lrow, M - 1)) * src.lda + (lpos ^ ring_swizzle(8 * i + lrow)) * 8;
     // unit i of this wave's into place `slot` (one past the end of K: the last one again, not multiplied)
     auto load = [&](int i, int slot) {
         const int k = min(wave + SUMS * i, units - 1) * UNIT;
@@ -271,8 +253,8 @@ gemm_rows_kernel(Source src, const bf16_t* __restrict__ w, int M_all, int N, int
             Frag x[4], y[4];
 #pragma unroll
             for (int s = 0; s < 4; ++s) {
-                x[s].u = *reinterpret_cast<const u32x4*>(sw + ((2 * s + g) ^ swizzle(wrow)) * 8);
-                y[s].u = *reinterpret_cast<const u32x4*>(sa + ((2 * s + g) ^ swizzle(arow)) * 8);
+                x[s].u = *reinterpret_cast<const u32x4*>(sw + ((2 * s + g) ^ ring_swizzle(wrow)) * 8);
+                y[s].u = *reinterpret_cast<const u32x4*>(sa + ((2 * s + g) ^ ring_swizzle(arow)) * 8);
             }
 #pragma unroll
             for (int s = 0; s < 4; ++s) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x[s].v, y[s].v, acc, 0, 0, 0);

@@ -23,9 +23,7 @@
 #include "common.h"
 #include "launchers.h"
 #include "epilogue.h"
-
-#include <type_traits>
-#include <utility>
+#include "ring.h"
 
 namespace liyab {
 
@@ -237,20 +235,6 @@ gemm_skinny_kernel(const bf16_t* __restrict__ a, int64_t lda, const bf16_t* __re
 // four parts 5.3 / 4.3, 1,600 -> 6,400 8.9 / 6.3; 16 rows 768 -> 768 4.8 / 3.4, 1,600 -> 4,800 9.7 / 5.8.
 // MR: rows of the ring, 8 or 16, M rounded up (the matrix operand's other rows repeat the last). NT: tiles of 16 features. R: units of the ring.
 constexpr int kUnit = 64;
-typedef __attribute__((address_space(3))) void* lds_void_ptr;
-__device__ __forceinline__ int ring_swizzle(int row) { return (row >> 1) & 7; }  // 16 rows' reads of one 16-byte piece fall into different banks
-
-// This wave's loads but the last LATER have arrived.
-template <int LATER>
-__device__ __forceinline__ void wait_loads() {
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_waitcnt((LATER & 15) | 0x0f70 | ((LATER >> 4) << 14));
-    asm volatile("" ::: "memory");
-}
-template <int... T, typename F>
-__device__ __forceinline__ void in_turn(std::integer_sequence<int, T...>, F&& f) {
-    (f(std::integral_constant<int, T>{}), ...);
-}
 
 // EPI: an epilogue fixed at compile time: none, residual, kEpiPlanes (planes with rows to add to), or a gated feed-forward's first product, kEpiGlu* (w = the
 // gate's N rows, then the other half's: a workgroup takes 16 features of both, and their 32-bit sums meet in act(gate) * other, as in

@@ -19,9 +19,7 @@
 // Every output element is a sum over k in one order whatever rows share its tile.
 #include "common.h"
 #include "launchers.h"
-
-#include <type_traits>
-#include <utility>
+#include "ring.h"
 
 namespace liyab {
 
@@ -221,7 +219,6 @@ grouped_mfma_kernel(GroupedParams p) {
 // of the products below took 41 us so). us before (the kernel above) and now, the same bits: 3,280 entries of 8 experts, 768 -> 2 x 1,536 54 -> 33, 1,536 -> 768
 // 32 -> 21, 768 -> 2 x 768 30 -> 17.2; 10,000 entries 102 -> 83 and 87 -> 45; heads, 1,640 rows of 12, 128 -> 64 with a gate 10.5 -> 6.8, 64 -> 128 8.3 -> 5.5.
 typedef __attribute__((ext_vector_type(4))) float gp_f32x4;
-typedef __attribute__((address_space(3))) void* gp_lds_ptr;
 
 // WR: rows of weights a tile, WR / NW features of each matrix.
 template <int NW, int WR, int STAGES>
@@ -313,7 +310,7 @@ grouped_tile_kernel(GroupedParams p, int n_tiles, int n_groups, int vec_ok, int 
             if (i < begin || i >= end) continue;
             bf16_t* to = ring + stage * STAGE + (i < A_LOADS ? wave * A_LOADS + i : 8 + wave * W_LOADS + i - A_LOADS) * 512;
             const bf16_t* from = src[i] + unit * GPK;
-            __builtin_amdgcn_global_load_lds(from, (gp_lds_ptr)(to), 16, 0, 0);
+            __builtin_amdgcn_global_load_lds(from, (lds_void_ptr)(to), 16, 0, 0);
         }
     };
     // a wave's 32 rows by 64 rows of weights, 32 features of each matrix where there are two: acc[i][j]
@@ -590,19 +587,6 @@ grouped_plain_kernel(GroupedParams p) {
 // us, cold weights, before / now: of 8 experts, 768 -> 2 x 1,536, 2 entries 6.7 / 6.3, 16 entries 11.7 / 9.5, 120 entries 16.7 / 13.4; 1,536 -> 768 16 entries
 // 8.5 / 7.4, 120 12.3 / 8.7; of 16 experts, 1,600 -> 2 x 3,200, 16 entries 62 / 45; 4 rows of 12 heads, 64 -> 128 3.5 / 3.35, 128 -> 64 with a gate 3.7 / 3.55;
 // 128 rows, 256 -> 512 10.4 / 7.3.
-typedef __attribute__((address_space(3))) void* gp_lds_ptr;
-__device__ __forceinline__ int gp_ring_swizzle(int row) { return (row >> 1) & 7; }  // 16 rows' reads of one 16-byte piece fall into different banks
-template <int LATER>
-__device__ __forceinline__ void gp_wait_loads() {  // this wave's loads but the last LATER have arrived
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_waitcnt((LATER & 15) | 0x0f70 | ((LATER >> 4) << 14));
-    asm volatile("" ::: "memory");
-}
-template <int... T, typename F>
-__device__ __forceinline__ void gp_in_turn(std::integer_sequence<int, T...>, F&& f) {
-    (f(std::integral_constant<int, T>{}), ...);
-}
-
 // LISTED: rows by a router's lists; FACTORS: a row's scale or a gate on the output.
 template <int NW, int R, bool LISTED, bool FACTORS>
 __global__ void __launch_bounds__(256)
@@ -637,7 +621,7 @@ grouped_stream_kernel(GroupedParams p) {
     const bf16_t* from[LOADS];
 #pragma unroll
     for (int l = 0; l < 2; ++l) {
-        const int piece = (lpos ^ gp_ring_swizzle(8 * l + lrow)) * 8;
+        const int piece = (lpos ^ ring_swizzle(8 * l + lrow)) * 8;
         const int row = LISTED ? (id[l] >= 0 ? id[l] / p.a_div : 0) : max(id[l], 0);
         from[l] = static_cast<const bf16_t*>(p.a) + static_cast<int64_t>(row) * p.lda + static_cast<int64_t>(g) * p.a_group_cols + piece;
         const int64_t wrow = (static_cast<int64_t>(g) * N + min(n0 + 8 * l + lrow, N - 1)) * K + piece;
@@ -651,7 +635,7 @@ grouped_stream_kernel(GroupedParams p) {
         for (int l = 0; l < LOADS; ++l) {
             const bf16_t* const piece = from[l] + k;
             bf16_t* const to = ring + slot * SLOT + l * 8 * 64;
-            __builtin_amdgcn_global_load_lds(piece, (gp_lds_ptr)to, 16, 0, 0);
+            __builtin_amdgcn_global_load_lds(piece, (lds_void_ptr)to, 16, 0, 0);
         }
     };
     // what the epilogue reads, ahead of the weights; no load under a branch: who has nothing to read gets a word of the weights
@@ -684,7 +668,7 @@ grouped_stream_kernel(GroupedParams p) {
         GpFrag x[2], w[NW][2];
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-            const int piece = ((4 * h + q) ^ gp_ring_swizzle(i)) * 8;
+            const int piece = ((4 * h + q) ^ ring_swizzle(i)) * 8;
             x[h].u = *reinterpret_cast<const gp_u32x4*>(at + piece);
 #pragma unroll
             for (int u = 0; u < NW; ++u) w[u][h].u = *reinterpret_cast<const gp_u32x4*>(at + 16 * (1 + u) * 64 + piece);
@@ -697,16 +681,16 @@ grouped_stream_kernel(GroupedParams p) {
     };
     int j0 = 0;
     for (; j0 + R < mine; j0 += R)
-        gp_in_turn(std::make_integer_sequence<int, R>{}, [&](auto at) {
+        in_turn(std::make_integer_sequence<int, R>{}, [&](auto at) {
             constexpr int t = decltype(at)::value;
-            gp_wait_loads<(R - 1) * LOADS>();
+            wait_loads<(R - 1) * LOADS>();
             multiply(t);
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the place has been read
             load(j0 + R + t, t);
         });
-    gp_in_turn(std::make_integer_sequence<int, R>{}, [&](auto at) {
+    in_turn(std::make_integer_sequence<int, R>{}, [&](auto at) {
         constexpr int t = decltype(at)::value;
-        gp_wait_loads<(R - 1 - t) * LOADS>();
+        wait_loads<(R - 1 - t) * LOADS>();
         if (j0 + t < mine) multiply(t);
     });
     lds_barrier();  // (the sums take the rings' place)
