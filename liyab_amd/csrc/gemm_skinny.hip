@@ -417,10 +417,12 @@ int launch_stream_epi(const void* a, int64_t lda, const void* w, int M, int N, i
     int waves = ksplit < trips ? ksplit : trips;
     auto ring = [&](int nt, int r) { return static_cast<size_t>(waves) * r * (16 * nt + rows) * kUnit * 2; };
     const int64_t strips = static_cast<int64_t>((N + 15) / 16) * ((M + 15) / 16) * kparts;
-    // With a few more strips than compute units a workgroup takes two, where their rings fit (one row, us by one strip / by two, with all epilogues
-    // in one kernel: 1,280 -> 5,120 7.7 / 5.8, 1,600 -> 6,400 8.6 / 7.1; 16 rows 6.5 / 6.1, 7.1 / 7.1); with twice as many it does where a wave has three units
-    // (3,072 -> 8,192 13.3 / 11.9; 1,600 -> 8,192 8.4 / 8.8, 4,096 -> 8,192 16.2 / 17.5, 768 -> 50,257 17.1 / 19.2)
-    const bool wide = trip_shift == 1 && strips > 256 && strips <= (K > 1600 && K <= 3072 ? 512 : 448) && ring(2, 2) <= 160 * 1024;
+    // With a few more strips than compute units a workgroup takes two, where their rings fit: one strip's rings of eight waves, four units in flight, leave a compute unit
+    // no room for another workgroup, and the strips past 256 would wait for a second round (8 rows, us by one strip / by two: 1,280 -> 5,120 7.3 / 5.7, 1,600 -> 6,144 8.1 /
+    // 6.6, 3,072 -> 7,168 12.4 / 10.4; 16 rows 6.6 / 6.0, 7.5 / 6.9, 11.7 / 10.8; up to 1,024 even). With up to twice as many it does where eight waves still share K (1,920 ->
+    // 7,680 9.6 / 8.4, 2,304 -> 8,192 11.1 / 9.8, 3,072 -> 8,192 13.1 / 11.7), not with four, whose rings share a unit (8,177 features on, up to 2,240 long: 1,664 -> 8,192
+    // 7.5 / 8.0, 2,048 -> 8,192 9.1 / 9.8). Beyond, the bytes are the bound (1,600 -> 10,240 9.3 / 10.5, 4,096 -> 7,168 14.4 / 14.7, -> 8,192 15.4 / 16.8)
+    const bool wide = trip_shift == 1 && strips > 256 && strips <= (K > 1600 && K <= 3072 && ksplit > 4 ? 512 : 448) && ring(2, 2) <= 160 * 1024;
     const int nt = wide ? 2 : 1;
     // a thread an output element at least, so that each has what its epilogue reads asked for ahead (waves without a unit of K bring in one again)
     if (strips <= 256 && waves < 4 * nt && ring(nt, 2) * 4 * nt / waves <= 160 * 1024) waves = 4 * nt;
