@@ -410,9 +410,10 @@ void launch_prepare_rows(const float* src, int64_t ld, int q_off, int k_off, int
     __VA_ARGS__<<<n, THREADS, 0, stream>>>(src, ld, q_off, k_off, v_off, H, G, dk, dv, dk_out, dv_out, q_out, kc, vc, slots, page_size, num_pages, q_norm, k_norm, \
                                               eps, freqs, rot_dims, positions, rot_halves)
     const int widest = kc != nullptr ? max(H * dk, max(G * dk, G * dv)) : H * dk;
-    // while the rows are few: each then has a compute unit, or half of one, to itself (us, 256 threads a row / 768: 12 heads of 64 4 rows 5.7 / 3.9, 300 6.4 / 5.3,
-    // 2,000 13.1 / 15.9; 12 over 4 4.6 / 3.8, 5.0 / 4.9, 8.8 / 13.9; 6 over 2 of 40 3.6 / 3.5, 4.1 / 4.5)
-    if (n > 128) LIYAB_ROWS(AS_THREADS, qk_prepare_rows_kernel<T>);
+    // up to 256 rows: each then has a compute unit to itself (us, 256 threads a row / 768, at 256, 257 and 300 rows: 12 heads of 64 5.6 / 3.9, 5.7 / 4.6, 6.1 / 4.9; 12 over 4
+    // 4.4 / 3.6, 4.4 / 4.2, 4.7 / 4.5; 6 over 2 of 40 3.6 / 3.5, 3.6 / 3.9, 3.9 / 4.2; at 1,000 rows 7.7 / 8.3, 5.7 / 7.5, 4.3 / 6.7; rows wider than 768 gain beyond the
+    // line too, 25 heads of 64 at 300 rows 10.2 / 6.5)
+    if (n > 256) LIYAB_ROWS(AS_THREADS, qk_prepare_rows_kernel<T>);
     else if (widest <= 3 * AS_THREADS) LIYAB_ROWS(3 * AS_THREADS, qk_prepare_held_rows_kernel<T, 3>);
     else if (widest <= 8 * AS_THREADS) LIYAB_ROWS(3 * AS_THREADS, qk_prepare_held_rows_kernel<T, 8>);
     else LIYAB_ROWS(AS_THREADS, qk_prepare_rows_kernel<T>);

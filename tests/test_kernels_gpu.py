@@ -1642,9 +1642,9 @@ def test_norm_of_few_rows_shares_a_row_among_waves_with_the_same_bits(ops, d, dt
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("H,G,dk,dv", [(12, 12, 64, 64), (6, 2, 40, 40), (5, 1, 30, 33), (8, 8, 256, 256), (32, 8, 128, 64)])
 def test_prepared_rows_do_not_depend_on_how_many_there_are(ops, H, G, dk, dv, dtype):
-    """Queries, keys and values of up to 128 rows have 256 threads each and stay in registers, those of more (and of wider rows) do not: the same bits;
+    """Queries, keys and values of up to 256 rows have 256 threads each and stay in registers, those of more (and of wider rows) do not: the same bits;
     turned as neighbours and as halves, rows wider than the heads, slots outside the pages, queries alone."""
-    n, page = 131, 16
+    n, page = 259, 16
     src, q_norm, k_norm = rnd(n, (H + G) * dk + G * dv), rnd(H * dk, seed=1), rnd(G * dk, seed=2)
     slots = torch.randperm(20 * page, generator=torch.Generator().manual_seed(3))[:n].int()
     slots[1], slots[2] = -1, 20 * page + 2
