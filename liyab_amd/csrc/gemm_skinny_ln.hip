@@ -48,7 +48,7 @@ struct NormParams {
 
 // EPI, DYT: the epilogue (-1: read from the parameters) and the norm, fixed at compile time: a kernel this short waits for its own instructions, cold in
 // every launch of a chain (a decode step of one request, 24 of its 66 kernels these: 327 us with both norms and all epilogues in one kernel, which divided slots
-// in 64 bits and asked for the norm's weight and bias under branches, 318 so; of eight 423 and 414).
+// in 64 bits, 314 so; of eight 423 and 410).
 template <typename OutT, int MAXV, int MT, int NT, int EPI, bool DYT>
 __global__ void __launch_bounds__(64 * LN_WAVES)
 gemm_skinny_ln_kernel(NormParams ln, const bf16_t* __restrict__ w, int M, int N, int K, EpiParams epi) {
@@ -86,9 +86,12 @@ gemm_skinny_ln_kernel(NormParams ln, const bf16_t* __restrict__ w, int M, int N,
         }
     };
     Frag wc[2][NT][2];
-    // this thread's first output: tile tid / 256 = (row tile, feature tile), and what its epilogue reads, its bias and its row's slot. No load under a
-    // branch, which would be waited for where the branch ends: who has nothing to read gets a word of the weights.
+    // this thread's first output: tile tid / 256 = (row tile, feature tile), and what its epilogue reads, its bias and its row's slot. In one tile of rows no load
+    // is under a branch, which would be waited for where the branch ends: who has nothing to read gets a word of the weights. In two, where a wave has
+    // several rows in turn, who has no output does not ask for its bias (us, asked for by all / by those who have one: 24 rows in four planes
+    // 768 -> 3,072 8.6 / 8.2, 1,024 -> 4,096 10.4 / 9.3; 8 rows 5.7 / 6.2, 6.3 / 6.5).
     const int e_m = min(16 * ((tid / 256 % TILES) / NT) + (tid % 256) / 16, M - 1), e_n = min(n0 + 16 * ((tid / 256) % NT) + tid % 16, N - 1);
+    const bool e_mine = MT == 1 || (16 * ((tid / 256) / NT) + (tid % 256) / 16 < M && n0 + 16 * ((tid / 256) % NT) + tid % 16 < N);
     const float* const bias_at = epi.bias != nullptr ? epi.bias + e_n : reinterpret_cast<const float*>(w);
     const int* const slot_at = EPI == kEpiQkvPaged ? epi.slots + e_m : reinterpret_cast<const int*>(w);
     float e_bias = 0.0f;
@@ -97,12 +100,6 @@ gemm_skinny_ln_kernel(NormParams ln, const bf16_t* __restrict__ w, int M, int N,
     // -- the norm: a wave per row, the row in registers ---------------------------------
     const int nv = K / 4;
     const floatx4 fzero = {0.0f, 0.0f, 0.0f, 0.0f}, fone = {1.0f, 1.0f, 1.0f, 1.0f};
-    // Where a wave has a row or two of up to 1,024 they are read in any case and chosen behind the planes' sums. Past 1,024 there are no registers for vectors
-    // that may be dropped (2 to 10 spilled), and past 16 rows a wave has several rows in turn: chosen at the load there (us, late / at the load: 8 rows 1,600 ->
-    // 4,800 10.5 / 9.3, 16 rows 2,048 -> 6,144 16.1 / 13.9, 1,280 -> 3,840 9.9 / 9.4; 24 rows 768 -> 2,304 8.4 / 7.7, 1,024 -> 3,072 9.9 / 8.8).
-    constexpr bool CHOSEN_LATE = MAXV < 8 && MT == 1;
-    const float* const norm_weight = ln.weight != nullptr ? ln.weight : ln.planes;  // (without one: a row's values, read and dropped)
-    const float* const norm_bias = ln.bias != nullptr ? ln.bias : ln.planes;
     // `between` runs once the row's first loads are asked for and before anything waits for them
     auto norm_row = [&](int m, bool keep, auto&& between) {
         const float* row0 = ln.planes + static_cast<int64_t>(m) * K;
@@ -113,13 +110,10 @@ gemm_skinny_ln_kernel(NormParams ln, const bf16_t* __restrict__ w, int M, int N,
         for (int j = 0; j < MAXV; ++j) {
             const int at = min(lane + kWave * j, nv - 1);  // past the row: its last piece again, unused
             v[j] = reinterpret_cast<const floatx4*>(row0)[at];
-            if constexpr (CHOSEN_LATE) {
-                gw[j] = reinterpret_cast<const floatx4*>(norm_weight)[at];
-                gb[j] = reinterpret_cast<const floatx4*>(norm_bias)[at];
-            } else {
-                gw[j] = ln.weight != nullptr ? reinterpret_cast<const floatx4*>(ln.weight)[at] : fone;
-                gb[j] = ln.bias != nullptr ? reinterpret_cast<const floatx4*>(ln.bias)[at] : fzero;
-            }
+            // (chosen here; read in any case and chosen behind the planes' sums they hold up the sums and, past 1,024, spill. us, late / here: 768 -> 2,304 1 row 4.8 / 4.5, 8 rows
+            // in five planes 6.8 / 6.5, 1,024 -> 3,072 7.6 / 7.3, 1,600 -> 4,800 8 rows 10.5 / 9.3; the one form that loses is 1,024 -> 4,096 at 4 rows, 5.1 / 5.3)
+            gw[j] = ln.weight != nullptr ? reinterpret_cast<const floatx4*>(ln.weight)[at] : fone;
+            gb[j] = ln.bias != nullptr ? reinterpret_cast<const floatx4*>(ln.bias)[at] : fzero;
         }
         // further planes, PB together (a plane past the last is the last one again, read and dropped)
         constexpr int PB = MAXV <= 4 ? 3 : 1;  // what the registers hold
@@ -142,13 +136,6 @@ gemm_skinny_ln_kernel(NormParams ln, const bf16_t* __restrict__ w, int M, int N,
 #pragma unroll
                 for (int j = 0; j < MAXV; ++j)
                     if (q0 + u < ln.n_planes) v[j] += plane[u][j];
-        }
-        if constexpr (CHOSEN_LATE) {
-#pragma unroll
-            for (int j = 0; j < MAXV; ++j) {
-                gw[j] = ln.weight != nullptr ? gw[j] : fone;
-                gb[j] = ln.bias != nullptr ? gb[j] : fzero;
-            }
         }
         if constexpr (DYT) {
             // tanh(z) = 1 - 2 / (1 + e^(2z)): one hardware exponential and one reciprocal a value
@@ -196,7 +183,7 @@ gemm_skinny_ln_kernel(NormParams ln, const bf16_t* __restrict__ w, int M, int N,
     // which come from further away and arrive while the norm is computed.
     auto ask_weights = [&]() {
         load_w(wave * 2, wc);
-        e_bias = *bias_at;
+        if (e_mine) e_bias = *bias_at;
         if constexpr (EPI == kEpiQkvPaged) e_slot = *slot_at;
     };
     // (a wave past the last row asks for its weights only: a compute unit takes 64 bytes a cycle from

@@ -25,11 +25,11 @@ from .norms import Normed
 # with a workgroup normalising 32 of them for 32 output features, a wave asking for its four rows
 # together, where the stream is whole (the feed-forward's first product): 721 against 713, 48 rows 656
 # against 652. That form was taken out again.)
-# Since the streaming product's rings the two kernels are as fast from 13 rows on (us a decode step, folded and not: small's sizes 12 rows 441 / 452, 13
-# 463 / 459, 16 474 / 464, medium's 12 899 / 904, 13 953 / 900, 16 967 / 907): up to 16 rows of 513 to 1,024, a multiple of 64, they take over. Both leave the same
+# Since the streaming product's rings the two kernels are as fast from 13 rows on or nearly so (us a decode step, folded and not: small's sizes 12 rows 441 / 461, 13
+# 460 / 463, 16 471 / 472, medium's 12 906 / 917, 13 950 / 912, 16 982 / 930): up to 16 rows of 513 to 1,024, a multiple of 64, they take over. Both leave the same
 # bits, but for 8,177 to 8,192 features, where four waves share K and not the folded kernel's eight (another order of the same sum). Narrower rows and those
 # without rings stay folded (16 rows, us, folded / not: 576 -> 2,304 6.3 / 6.0; 512 -> 1,536 5.6 / 5.9, 128 -> 384 4.4 / 5.3, 200 -> 600 4.2 / 5.7, 72 -> 1,024 4.3 /
-# 6.1), rows past 16 (24: 549 / 528, 1,151 / 1,078) and wider ones too, whose products add in another order.
+# 6.1), rows past 16 (17: 469 / 483, 1,040 / 1,068; 24: 540 / 534, 1,124 / 1,103) and wider ones too, whose products add in another order.
 FOLD_NORM = True
 FOLD_NORM_ROWS = 24
 TILED_PARTS = True  # products of 33 to 64 rows that are added to the stream: tiled and cut over K (ops.tiled_k_parts)
