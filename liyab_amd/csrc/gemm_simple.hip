@@ -289,7 +289,7 @@ gemm_tiled_f32_kernel(float* __restrict__ out, int64_t ldo, const float* __restr
 
 // Few rows, or too few tiles to go round: a workgroup takes 16 rows and NB output features, its waves the chunks of K in
 // turn, so that a product of few output elements still spreads over the chip. A wave brings its chunk of the rows
-// of `w` and `a` through registers into LDS of its own (256 bytes a row and load, the next two chunks in flight
+// of `w` and `a` through registers into LDS of its own (256 bytes a row and load, the next chunk in flight
 // meanwhile) and runs the chunk's chains on the matrix core, 16 x 16 x 4 an instruction; after each round of chunks the
 // threads add the round's sums in chunk order. Few features a workgroup where N is small: the weights then stream
 // through enough compute units (features of the block past NB repeat the last one). Reading operands from LDS set the
@@ -331,14 +331,14 @@ gemm_chunks_f32_kernel(float* __restrict__ out, int64_t ldo, const float* __rest
     const int chunks = (K + kChunk - 1) / kChunk, ldx = K + 4;
     const int lrow = lane / 16, lk = (lane % 16) * 4;  // as a loader
     const int li = lane % 16, g = lane / 16;           // in the matrix core's operands: row (or feature) and k
-    f32x4_t wreg[2][W_LOADS], areg[2][A_LOADS + 1];
-    auto fetch = [&](int c, int buf) {
+    f32x4_t wreg[W_LOADS], areg[A_LOADS + 1];
+    auto fetch = [&](int c) {
         const int k = c * kChunk + lk;
 #pragma unroll
-        for (int i = 0; i < W_LOADS; ++i) wreg[buf][i] = load4_f32<VEC>(w + static_cast<int64_t>(min(n0 + 4 * i + lrow, N - 1)) * K, k, K);
+        for (int i = 0; i < W_LOADS; ++i) wreg[i] = load4_f32<VEC>(w + static_cast<int64_t>(min(n0 + 4 * i + lrow, N - 1)) * K, k, K);
 #pragma unroll
         for (int i = 0; i < A_LOADS; ++i)
-            if (4 * i < M) areg[buf][i] = load4_f32<VEC>(a + static_cast<int64_t>(min(4 * i + lrow, M - 1)) * lda, k, K);  // (the same for every lane)
+            if (4 * i < M) areg[i] = load4_f32<VEC>(a + static_cast<int64_t>(min(4 * i + lrow, M - 1)) * lda, k, K);  // (the same for every lane)
     };
     float tot = 0.0f;  // of output element (tid / NB, tid % NB), for tid < 16 * NB
     float* place = nullptr;  // found while the first operands are on their way
@@ -346,8 +346,7 @@ gemm_chunks_f32_kernel(float* __restrict__ out, int64_t ldo, const float* __rest
     const bool mine = tid < kChunkRows * NB && tid / NB < M && n < N;
     float own_bias = 0.0f, own_res = 0.0f;
     auto ask = [&]() {  // the weights (and plain rows), then what the epilogue reads
-        if (wave < chunks) fetch(wave, 0);
-        if (wave + WAVES < chunks) fetch(wave + WAVES, 1);
+        if (wave < chunks) fetch(wave);
         if (mine) {
             if (bias != nullptr) own_bias = bias[n];
             if constexpr (EPI == kEpiResidual) own_res = residual[static_cast<int64_t>(m) * ldr + n];
@@ -446,16 +445,15 @@ gemm_chunks_f32_kernel(float* __restrict__ out, int64_t ldo, const float* __rest
     const float* wl = &Wt[wave][min(li, NB - 1)][g];
     const float* al = SRC == kSrcRows ? &At[SRC == kSrcRows ? wave : 0][min(li, (M + 3) / 4 * 4 - 1)][g]  // (rows past M: some row that was written; not stored)
                                       : made_rows + min(li, M - 1) * ldx + g;
-    auto round = [&](int c0, auto buffer) {
-        constexpr int turn = decltype(buffer)::value;
+    for (int c0 = 0, turn = 0; c0 < chunks; c0 += WAVES, turn ^= 1) {
         const int c = c0 + wave;
         if (c < chunks) {
 #pragma unroll
-            for (int i = 0; i < W_LOADS; ++i) *reinterpret_cast<f32x4_t*>(&Wt[wave][4 * i + lrow][lk]) = within_k(wreg[turn][i], c * kChunk + lk, K);
+            for (int i = 0; i < W_LOADS; ++i) *reinterpret_cast<f32x4_t*>(&Wt[wave][4 * i + lrow][lk]) = within_k(wreg[i], c * kChunk + lk, K);
 #pragma unroll
             for (int i = 0; i < A_LOADS; ++i)
-                if (4 * i < M) *reinterpret_cast<f32x4_t*>(&At[wave][4 * i + lrow][lk]) = within_k(areg[turn][i], c * kChunk + lk, K);
-            if (c + 2 * WAVES < chunks) fetch(c + 2 * WAVES, turn);
+                if (4 * i < M) *reinterpret_cast<f32x4_t*>(&At[wave][4 * i + lrow][lk]) = within_k(areg[i], c * kChunk + lk, K);
+            if (c + WAVES < chunks) fetch(c + WAVES);
             const float* ac = SRC == kSrcRows ? al : al + c * kChunk;
             f32x4_t acc{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
@@ -469,10 +467,6 @@ gemm_chunks_f32_kernel(float* __restrict__ out, int64_t ldo, const float* __rest
             const int live = min(WAVES, chunks - c0);
             for (int v = 0; v < live; ++v) tot += P[turn][v][tid / NB][tid % NB];
         }
-    };
-    for (int c0 = 0; c0 < chunks; c0 += 2 * WAVES) {
-        round(c0, std::integral_constant<int, 0>{});
-        if (c0 + WAVES < chunks) round(c0 + WAVES, std::integral_constant<int, 1>{});
     }
     if (!mine) return;
     const float v = finish_f32<EPI>(tot, bias != nullptr, own_bias);
