@@ -386,11 +386,12 @@ int launch_strip(const Source& src, const bf16_t* w, int M, int N, int K, int st
     if (strip == 0) {
         // the narrowest strips that still have a compute unit each (128 combinations of K and N up to 8,192, 1 to 64 rows: within 3 % of the best of the
         // three on average); a vocabulary's worth of features in strips of 16 while K is short (8 rows, 768 -> 50,257: 15.3 us against 15.7 in strips
-        // of 32, 1,024 -> 50,257 23.7 against 25.7; 1,600 -> 16,384 19.2 against 12.2). A norm is repeated by every workgroup: wider ones
+        // of 32, 1,024 -> 50,257 23.7 against 25.7; 1,600 -> 16,384 19.2 against 12.2), past 768 k only up to 8 rows: with the rings of 16 rows or more a workgroup
+        // of 16 features fills a compute unit (16 rows, 1,024 -> 50,257 37.1 against 30.8, 1,280 -> 16,384 15.2 against 12.2; 768 -> 50,257 17.5 against 18.5). A norm is repeated by every workgroup: wider ones
         // there (1,024 -> 4,096, 8 rows: 6.1 us in strips of 32, 6.4 in strips of 16)
         const int tiles = (M + ROWS - 1) / ROWS, most = SRC == kNorm ? 192 : 256;
         strip = SRC != kNorm && (N + 7) / 8 * tiles <= most ? 8 : (N + 15) / 16 * tiles <= most ? 16 : 32;
-        if (SRC == kRows && N > 32 * 256 && K <= 1280) strip = 16;
+        if (SRC == kRows && N > 32 * 256 && K <= (M <= 8 ? 1280 : 768)) strip = 16;
     }
     switch (strip) {
         case 8: return launch_form<OutT, 8, SRC, EPI>(src, w, M, N, K, epi, stream);
