@@ -336,8 +336,12 @@ extern "C" int liyab_streams_update(float* x, const float* enter, const float* y
     const auto aligned = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
     const bool vec = d % 4 == 0 && aligned(x) && aligned(enter) && aligned(y) && aligned(w) && aligned(out);
     // (thousands of rows of which a wave or less holds one: the general kernel's are shorter where nothing is left to wait for, 4,096 of 256 5.9 us against 6.2;
-    // of 768 with two rows a token 9.8 against 9.1)
-    if (vec && d <= 4 * ST_THREADS && (y == nullptr || n_sum <= 4) && (n <= 2048 || d > 256)) {
+    // of 768 with two rows a token 9.8 against 9.1. Where rows only enter or are only read, or identity experts' rows are loaded whether one is there or not, there is
+    // less to gain by loads ahead and more to run: up to some 500 rows only; us, general / this one, two streams of 768, identity experts at 300, 1,000 and 2,048 rows
+    // 3.2 / 3.0, 4.3 / 4.4, 6.1 / 6.5; entering 2.8 / 2.6, 3.8 / 3.9, 5.2 / 5.7.
+    // One row a token for one or two streams: up to 1,024 rows, 1,000 of two streams of 768 4.0 / 4.0, 2,048 5.7 / 6.0)
+    const bool few = n_ids > 0 || y == nullptr ? n <= 512 : n_sum == 1 && S <= 2 ? n <= 1024 : n <= 2048 || d > 256;
+    if (vec && d <= 4 * ST_THREADS && (y == nullptr || n_sum <= 4) && few) {
         const bool ids_in = n_ids > 0;
         const bool done = out_dtype == kF32 ? (ids_in ? launch_streams_row<float, true>(a, n, S, stream) : launch_streams_row<float, false>(a, n, S, stream))
                                             : (ids_in ? launch_streams_row<bf16_t, true>(a, n, S, stream) : launch_streams_row<bf16_t, false>(a, n, S, stream));
