@@ -259,10 +259,11 @@ __global__ void __launch_bounds__(256) sum_parts_kernel(float* out, const float*
 
 // Whether a row's pieces go to waves of their own: while the rows do not fill the chip and a wave would have several pieces or planes to read (us, a wave a row /
 // a wave a piece: 64 rows of 1,600 3.05 / 2.70, in five planes 3.81 / 2.94, of 768 in five 3.04 / 2.61; 256 rows of 2,048 3.18 / 2.87; 512 of 768 2.67 / 2.71, in
-// four planes 3.01 / 2.93; 800 rows in five planes of 1,024 3.88 / 3.44, of 1,600 4.84 / 4.61; 1,024 of 2,048 8.8 / 9.4; 64 rows of 512 2.40 / 2.40).
+// four planes 3.01 / 2.93; 800 rows in five planes of 1,024 3.88 / 3.44, of 1,600 4.84 / 4.61; 1,024 of 2,048 8.8 / 9.4; 64 rows of 512 2.40 / 2.40;
+// 512 rows in two planes of 1,280 3.17 / 3.15, of 1,600 3.30 / 3.48).
 static bool pieces_pay(int n, int d, int n_parts) {
     if (n_parts > 4) return n <= 512 || (n <= 1024 && static_cast<int64_t>(n) * d <= 1300000);
-    return n <= 256 ? d > 512 || n_parts > 1 : n <= 512 && n_parts > 1 && d > 512;
+    return n <= 256 ? d > 512 || n_parts > 1 : n <= 512 && n_parts > 1 && d > 512 && (n_parts > 2 || d < 1600);
 }
 template <typename T, int MAXV>
 void launch_wave(T* out, const float* x, const float* w, const float* b, const int* rows, int n, int d, float eps,
