@@ -241,7 +241,7 @@ constexpr int kUnit = 64;
 // elementwise_norms.hip's kernel, whose link in the chain and trip through memory go); -1 reads it from the parameters.
 constexpr int kEpiPlanes = 5, kEpiGluSilu = 6, kEpiGluGelu = 7;
 template <typename OutT, int MR, int NT, int R, int EPI>
-__global__ void __launch_bounds__(1024)
+__global__ void __launch_bounds__(1024, R == 1 ? 8 : 4)  // one unit in flight: two workgroups of 16 waves a compute unit
 gemm_stream_kernel(const bf16_t* __restrict__ a, int64_t lda, const bf16_t* __restrict__ w, int M, int N, int K,
                    EpiParams epi, BaseSum base, int part_k, int64_t part_stride, int split_shift, int trip_shift) {
     constexpr bool GLU = EPI == kEpiGluSilu || EPI == kEpiGluGelu;
@@ -433,7 +433,16 @@ int launch_stream_epi(const void* a, int64_t lda, const void* w, int M, int N, i
 #define LIYAB_STREAM(MR, NT, R) launch_stream_as<OutT, MR, NT, R, EPI>(pa, lda, pw, M, N, K, ksplit, waves, epi, base, kparts, units * kUnit, part_stride, trip_shift, stream)
     // more workgroups than compute units, of a wave a unit or two: one unit in flight, so that two of them share a compute unit (48 rows, us, two in flight and
     // one: 768 -> 2,304 6.5 and 5.0, -> 3,072 8.6 and 6.0, 1,600 -> 1,600 7.4 and 6.2)
-    if (trip_shift == 0 && strips > 256 && mine <= 2 && ring(1, 2) > 80 * 1024) return LIYAB_STREAM(16, 1, 1);
+    if (trip_shift == 0 && strips > 256 && mine <= 2 && ring(1, 2) > 80 * 1024) {
+        // (two of 16 waves share one as long as a wave has 64 registers, which a kernel that reads its epilogue from the parameters passes by 12: each has a kernel of its own. us, 17
+        // and 24 rows, 1,280 -> 3,840 with GELU, one kernel / its own 7.2 / 6.2, 7.1 / 6.2)
+#define LIYAB_FIXED(E) launch_stream_as<OutT, 16, 1, 1, E>(pa, lda, pw, M, N, K, ksplit, waves, epi, base, kparts, units * kUnit, part_stride, trip_shift, stream)
+        if constexpr (EPI >= 0) return LIYAB_FIXED(EPI);
+        else if (epi.mode == kEpiGeluTanh) return LIYAB_FIXED(kEpiGeluTanh);
+        else if (epi.mode == kEpiGeluErf) return LIYAB_FIXED(kEpiGeluErf);
+        else return LIYAB_FIXED(kEpiQkvPaged);
+#undef LIYAB_FIXED
+    }
     if (rows == 8) {
         if (wide) return four ? LIYAB_STREAM(8, 2, 4) : LIYAB_STREAM(8, 2, 2);
         return four ? LIYAB_STREAM(8, 1, 4) : LIYAB_STREAM(8, 1, 2);
