@@ -289,7 +289,7 @@ gemm_tiled_f32_kernel(float* __restrict__ out, int64_t ldo, const float* __restr
 
 // Few rows, or too few tiles to go round: a workgroup takes 16 rows and NB output features, its waves the chunks of K in
 // turn, so that a product of few output elements still spreads over the chip. A wave brings its chunk of the rows
-// of `w` and `a` through registers into LDS of its own (256 bytes a row and load, the next chunk in flight
+// of `w` and `a` through registers into LDS of its own (256 bytes a row and load, the next one or two chunks in flight
 // meanwhile) and runs the chunk's chains on the matrix core, 16 x 16 x 4 an instruction; after each round of chunks the
 // threads add the round's sums in chunk order. Few features a workgroup where N is small: the weights then stream
 // through enough compute units (features of the block past NB repeat the last one). Reading operands from LDS set the
@@ -311,7 +311,10 @@ struct MadeRows {
 };
 
 // FORM: pieces of 4 a lane of a row (norm), splits at most (splits); not read for plain rows.
-template <int NB, int WAVES, int EPI, bool VEC, int SRC, int FORM>
+// DEPTH: chunks in flight beside the one that is multiplied. Two for one block of 16 rows, whose weights come from HBM one trip after the other; one for more rows, where the registers of two
+// (104 a lane, 70 with one) and their code cost more than they hide (us, two / one: 33 rows 768 -> 3,072 9.4 / 7.9, 1,024 -> 4,096 12.3 / 10.9, 100 rows
+// 15.3 / 13.9; a decode step of small's sizes, ms, 1 request 0.475 / 0.479, 8 0.540 / 0.539, 24 0.847 / 0.822, 64 1.209 / 1.172).
+template <int NB, int WAVES, int EPI, bool VEC, int SRC, int FORM, int DEPTH>
 __global__ void __launch_bounds__(64 * WAVES)
 gemm_chunks_f32_kernel(float* __restrict__ out, int64_t ldo, const float* __restrict__ a, int64_t lda,
                        const float* __restrict__ w, const float* __restrict__ bias, float* __restrict__ residual,
@@ -331,14 +334,14 @@ gemm_chunks_f32_kernel(float* __restrict__ out, int64_t ldo, const float* __rest
     const int chunks = (K + kChunk - 1) / kChunk, ldx = K + 4;
     const int lrow = lane / 16, lk = (lane % 16) * 4;  // as a loader
     const int li = lane % 16, g = lane / 16;           // in the matrix core's operands: row (or feature) and k
-    f32x4_t wreg[W_LOADS], areg[A_LOADS + 1];
-    auto fetch = [&](int c) {
+    f32x4_t wreg[DEPTH][W_LOADS], areg[DEPTH][A_LOADS + 1];
+    auto fetch = [&](int c, int buf) {
         const int k = c * kChunk + lk;
 #pragma unroll
-        for (int i = 0; i < W_LOADS; ++i) wreg[i] = load4_f32<VEC>(w + static_cast<int64_t>(min(n0 + 4 * i + lrow, N - 1)) * K, k, K);
+        for (int i = 0; i < W_LOADS; ++i) wreg[buf][i] = load4_f32<VEC>(w + static_cast<int64_t>(min(n0 + 4 * i + lrow, N - 1)) * K, k, K);
 #pragma unroll
         for (int i = 0; i < A_LOADS; ++i)
-            if (4 * i < M) areg[i] = load4_f32<VEC>(a + static_cast<int64_t>(min(4 * i + lrow, M - 1)) * lda, k, K);  // (the same for every lane)
+            if (4 * i < M) areg[buf][i] = load4_f32<VEC>(a + static_cast<int64_t>(min(4 * i + lrow, M - 1)) * lda, k, K);  // (the same for every lane)
     };
     float tot = 0.0f;  // of output element (tid / NB, tid % NB), for tid < 16 * NB
     float* place = nullptr;  // found while the first operands are on their way
@@ -346,7 +349,9 @@ gemm_chunks_f32_kernel(float* __restrict__ out, int64_t ldo, const float* __rest
     const bool mine = tid < kChunkRows * NB && tid / NB < M && n < N;
     float own_bias = 0.0f, own_res = 0.0f;
     auto ask = [&]() {  // the weights (and plain rows), then what the epilogue reads
-        if (wave < chunks) fetch(wave);
+        if (wave < chunks) fetch(wave, 0);
+        if constexpr (DEPTH == 2)
+            if (wave + WAVES < chunks) fetch(wave + WAVES, 1);
         if (mine) {
             if (bias != nullptr) own_bias = bias[n];
             if constexpr (EPI == kEpiResidual) own_res = residual[static_cast<int64_t>(m) * ldr + n];
@@ -445,15 +450,16 @@ gemm_chunks_f32_kernel(float* __restrict__ out, int64_t ldo, const float* __rest
     const float* wl = &Wt[wave][min(li, NB - 1)][g];
     const float* al = SRC == kSrcRows ? &At[SRC == kSrcRows ? wave : 0][min(li, (M + 3) / 4 * 4 - 1)][g]  // (rows past M: some row that was written; not stored)
                                       : made_rows + min(li, M - 1) * ldx + g;
-    for (int c0 = 0, turn = 0; c0 < chunks; c0 += WAVES, turn ^= 1) {
+    auto round = [&](int c0, int turn, auto buffer) {
+        constexpr int buf = decltype(buffer)::value;
         const int c = c0 + wave;
         if (c < chunks) {
 #pragma unroll
-            for (int i = 0; i < W_LOADS; ++i) *reinterpret_cast<f32x4_t*>(&Wt[wave][4 * i + lrow][lk]) = within_k(wreg[i], c * kChunk + lk, K);
+            for (int i = 0; i < W_LOADS; ++i) *reinterpret_cast<f32x4_t*>(&Wt[wave][4 * i + lrow][lk]) = within_k(wreg[buf][i], c * kChunk + lk, K);
 #pragma unroll
             for (int i = 0; i < A_LOADS; ++i)
-                if (4 * i < M) *reinterpret_cast<f32x4_t*>(&At[wave][4 * i + lrow][lk]) = within_k(areg[i], c * kChunk + lk, K);
-            if (c + WAVES < chunks) fetch(c + WAVES);
+                if (4 * i < M) *reinterpret_cast<f32x4_t*>(&At[wave][4 * i + lrow][lk]) = within_k(areg[buf][i], c * kChunk + lk, K);
+            if (c + DEPTH * WAVES < chunks) fetch(c + DEPTH * WAVES, buf);
             const float* ac = SRC == kSrcRows ? al : al + c * kChunk;
             f32x4_t acc{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
@@ -467,6 +473,14 @@ gemm_chunks_f32_kernel(float* __restrict__ out, int64_t ldo, const float* __rest
             const int live = min(WAVES, chunks - c0);
             for (int v = 0; v < live; ++v) tot += P[turn][v][tid / NB][tid % NB];
         }
+    };
+    if constexpr (DEPTH == 2) {
+        for (int c0 = 0; c0 < chunks; c0 += 2 * WAVES) {
+            round(c0, 0, std::integral_constant<int, 0>{});
+            if (c0 + WAVES < chunks) round(c0 + WAVES, 1, std::integral_constant<int, 1>{});
+        }
+    } else {
+        for (int c0 = 0, turn = 0; c0 < chunks; c0 += WAVES, turn ^= 1) round(c0, turn, std::integral_constant<int, 0>{});
     }
     if (!mine) return;
     const float v = finish_f32<EPI>(tot, bias != nullptr, own_bias);
@@ -490,8 +504,9 @@ int launch_tiled_f32(float* out, int64_t ldo, const float* a, int64_t lda, const
 template <int NB, int WAVES, int EPI, bool VEC>
 int launch_chunks_f32(float* out, int64_t ldo, const float* a, int64_t lda, const float* w, const float* bias, float* residual, int64_t ldr, int M,
                       int N, int K, const EpiParams& qkv, hipStream_t stream) {
-    gemm_chunks_f32_kernel<NB, WAVES, EPI, VEC, kSrcRows, 0><<<dim3((N + NB - 1) / NB, (M + kChunkRows - 1) / kChunkRows), 64 * WAVES, 0, stream>>>(
-        out, ldo, a, lda, w, bias, residual, ldr, M, N, K, qkv, MadeRows{});
+    const dim3 grid((N + NB - 1) / NB, (M + kChunkRows - 1) / kChunkRows);
+    const auto kern = M <= kChunkRows ? gemm_chunks_f32_kernel<NB, WAVES, EPI, VEC, kSrcRows, 0, 2> : gemm_chunks_f32_kernel<NB, WAVES, EPI, VEC, kSrcRows, 0, 1>;
+    kern<<<grid, 64 * WAVES, 0, stream>>>(out, ldo, a, lda, w, bias, residual, ldr, M, N, K, qkv, MadeRows{});
     return check_launch("gemm_chunks_f32");
 }
 
@@ -500,7 +515,7 @@ int launch_made_as(const MadeRows& made, const float* w, int M, int N, int K, co
     const size_t rows = static_cast<size_t>(M < kChunkRows ? M : kChunkRows) * (K + 4) * sizeof(float);
     constexpr size_t fixed = (WAVES * NB + kChunkRows) * (kChunk + 4) * sizeof(float) + 2 * WAVES * kChunkRows * NB * sizeof(float);
     LIYAB_REQUIRE(rows + fixed <= 160 * 1024, "gemm_made_f32: rows of %d need %zu bytes of LDS", K, rows + fixed);
-    auto kern = gemm_chunks_f32_kernel<NB, WAVES, EPI, true, SRC, FORM>;
+    auto kern = gemm_chunks_f32_kernel<NB, WAVES, EPI, true, SRC, FORM, 2>;
     static bool ready = false;  // once per instantiation, outside any stream capture's first use
     if (!ready) {
         hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(160 * 1024 - fixed));
