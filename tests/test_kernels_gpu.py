@@ -1752,6 +1752,32 @@ def test_streamed_products_of_up_to_16_rows_leave_the_bits_of_the_others(ops, K,
             assert all(torch.equal(p, q) for p, q in zip(*got)), (M, N, [torch.equal(p, q) for p, q in zip(*got)])
 
 
+@pytest.mark.parametrize("K", [768, 1280])
+@pytest.mark.parametrize("M", [17, 32])
+def test_streamed_products_with_one_unit_in_flight_keep_every_epilogues_bits(ops, M, K):
+    """More than 256 blocks of 16 rows and 16 features, of a wave a unit or two: each epilogue has a kernel of its own there; against the kernel that holds its operands
+    in registers, which gets eight zeros more a row."""
+    pad = lambda t: torch.nn.functional.pad(t, (0, 8)).contiguous()  # noqa: E731
+    N = 3 * 704
+    a, w, bias = rnd(M, K, dtype=torch.bfloat16, seed=K), rnd(N, K, dtype=torch.bfloat16, seed=K + 1, scale=0.2), rnd(N, seed=2)
+    slots = torch.randperm(60)[:M].to(torch.int32).to(DEV)
+    slots[M // 2] = -1
+    got = []
+    for x, y in ((a, w), (pad(a), pad(w))):
+        outs = []
+        for dtype in (torch.float32, torch.bfloat16):
+            for epilogue in (ops.EPI_NONE, ops.EPI_GELU_TANH, ops.EPI_GELU_ERF):
+                out = torch.empty(M, N, dtype=dtype, device=DEV)
+                ops.gemm_skinny(x, y, bias, out=out, epilogue=epilogue, ksplit=16)
+                outs.append(out)
+        added = rnd(M, N, seed=3)
+        ops.gemm_skinny(x, y, bias, residual=added, epilogue=ops.EPI_RESIDUAL, ksplit=16)
+        q, kc, vc = (torch.zeros(s, dtype=torch.bfloat16, device=DEV) for s in ((M, 704), (15, 44, 4, 16), (15, 44, 4, 16)))
+        ops.gemm_skinny(x, y, bias, out=q, epilogue=ops.EPI_QKV_PAGED, kv=(kc, vc, slots, 704), ksplit=16)
+        got.append(outs + [added, q, kc, vc])
+    assert all(torch.equal(p, q) for p, q in zip(*got)), [torch.equal(p, q) for p, q in zip(*got)]
+
+
 @pytest.mark.parametrize("K", [64, 512, 576, 768, 832, 1000, 1024])
 def test_steps_of_13_to_16_rows_keep_the_folded_norms_bits(ops, K, monkeypatch):
     """A norm and the product behind it as the parts run them, against the kernel that folds them: the same bits on either side of the rows (13 to 16) and widths
