@@ -491,15 +491,16 @@ def gemm_f32_ln(x: torch.Tensor, ln_weight: Optional[torch.Tensor], ln_bias: Opt
 
 def f32_norm_pays(M: int, N: int, K: int) -> bool:
     """Whether the 32-bit path computes a norm inside the product behind it: every workgroup of 16 rows repeats it (us, inside / norm and product: 768 -> 3,072 4 rows
-    6.1 / 7.4, 8 rows 6.3 / 7.8, 16 rows 7.4 / 8.0, 24 rows 11.1 / 11.3; 1,024 -> 3,072 8 rows 8.5 / 8.9, 16 rows 10.0 / 9.5; 1,600 -> 6,400 4 rows 16.9 / 17.5, 8 rows
-    18.6 / 18.3)."""
+    6.8 / 7.6, 8 rows 6.8 / 7.9, 12 rows 7.5 / 8.3, 16 rows 7.8 / 8.6, 24 rows 11.6 / 10.6; 1,024 -> 3,072 8 rows 8.6 / 8.8, 12 rows 9.3 / 9.1, 16 rows 10.2 / 9.4; 1,600 -> 6,400 4 rows
+    18.0 / 17.8, 8 rows 19.6 / 18.3)."""
     return 0 < M <= 16 and K % 64 == 0 and K <= 2048 and M * K <= 16 * 768
 
 
 def splits_in_product_pay(M: int, splits: int, n_head: int, hd: int) -> bool:
     """Whether attention's splits by position are merged inside the output projection (`gemm_splits`): every workgroup merges all rows (us, inside / merge and
     product: bfloat16, 12 heads of 64, 4 splits, 4 rows 4.8 / 5.6, 8 rows 6.4 / 5.7; 25 heads 1 row 6.3 / 7.0, 4 rows 9.6 / 7.3; 32 bits 12 heads, 2 splits, 4 rows
-    5.6 / 6.6, 8 rows 7.0 / 6.8; 8 splits, 1 row 7.2 / 6.9)."""
+    5.6 / 6.5, 8 rows 7.2 / 6.7; 8 splits, 1 row 7.2 / 6.9). In between, 5 to 7 rows of 12 heads: bfloat16 6.2 / 5.6, 6.5 / 5.6, 6.5 / 5.7, and 3 rows of 16 heads 6.0 / 5.9, 4 7.8 /
+    5.9; in 32 bits the line could be at 6 rows of 768 (5.7 / 6.7, 6.4 / 6.7, 7.1 / 6.7)."""
     return 1 < splits <= 4 and hd % 4 == 0 and (n_head * hd) % 64 == 0 and 0 < M * n_head * hd <= 4 * 768
 
 
