@@ -281,7 +281,7 @@ int launch_dl(const void* a, int64_t lda, const void* w, int M, int N, int K, co
 
 using namespace liyab;
 
-// tile: 2, 6 = 64x64; 7, 8 = 128x128; 9, 11 = 192x128; 15 = 256x256 (gemm_mfma_tile.hip, which also chooses
+// tile: 2, 6 to 9, 11, 15, 21 = from 64x64 to 256x256 (gemm_tile.h lists them; gemm_mfma_tile.hip also chooses
 // among them for 0); 17 = 32x32 on four waves that walk K side by side (a workgroup then brings in a
 // third less of the operands, and twice as many workgroups pull: 64 rows with cold weights, 768 -> 2,304 in
 // 5.05 us against 5.53, 1,024 -> 3,072 in 5.97 against 6.85; for as long as every tile has a compute unit

@@ -5,21 +5,21 @@
 // What bounds it. The matrix cores draw more power than the card has: on random data, nothing but products, 32 x 32 x 16
 // instructions settle at 1.6-1.8 PFLOP/s and 16 x 16 x 32 at 1.9-2.1 (2.4 on zeros), so the blocks are 16 x 16. A compute unit
 // takes operands in at about 113 GB/s, loads alone, when a load covers whole lines of 128 bytes, and at 70 when it covers
-// halves of them (stages of 32 k), so a stage is 64 k; a tile of 256 x 256 then needs 0.6 us a stage for operands and 0.9 for
-// products. A wave that asks for a whole stage at once waits at the load queue before its first product: the loads of the
-// stage ahead go out in two halves, each in front of the products of 32 k. What is left unhidden (a stage's barrier, the
-// first fragments, the outputs) overlaps with another workgroup's products: two workgroups of eight waves a compute unit for
-// the middle tiles, sixteen waves in one for 256 x 256.
-// Measured in prefill steps, us a product, before (32 x 32 x 16 in tiles of 64 x 64, 128 x 128 or 256 x 256, a stage's loads at
-// once) and now, on one box in turn: GPT-2 XL's widths, 7,920 rows: 1,600 -> 4,800 158 -> 126, 1,600 -> 6,400 198 -> 164, the two products
-// back to the stream 138 -> 115 on average; 768 wide, 8,001 rows: 768 -> 2,304 48 -> 40, 768 -> 3,072 58 -> 49, the two back 44 -> 33; 2,048
-// rows: 18.6 -> 16.3, 20.3 -> 20.1 and 18.0 -> 16.3; 1,024 wide, some 780 rows: 1,024 -> 3,072 15.5 -> 14.8, -> 4,096 21.7 -> 15.3.
-// (There the operands come from memory, not from L2: three and four stages, which lose in a product repeated alone, win while
-// every tile has a compute unit of its own.) Alone and repeated, 8,192 cubed runs at 1.32 PFLOP/s (1.19 before, the vendor's library 1.44),
-// 4,096 x 4,096 x 16,384 at 1.28 (1.15).
-// Tried and left: four waves of 128 x 128, eight of 128 x 64, two groups of waves in turn at products and reads (each with
-// 32 x 32 blocks: 173-200 us for 6,400 -> 1,600 alone, 160 here), stages of 32 k four deep (190), fragments read a step ahead in
-// registers of their own or strung between the products by hand (slower than the compiler's order); 128 x 192, 128 x 64, 64 x 128.
+// halves of them (stages of 32 k), so a stage is 64 k. Beside the loads LDS hands the fragments out, 128 bytes a cycle: of the small tiles that is the larger
+// part (a stage of 64 x 64: 384 cycles of LDS, 128 of products), and then a chain of barrier, reads and products whose length the reads' latency sets: all of a
+// stage's fragments are read at once (780 rows, 4,096 -> 1,024, cold weights: 22.8 us in halves, 20.7 at once; 400 rows of 1,024 -> 1,024 8.4 and 7.4). Of tiles
+// whose waves would stand at the load queue the loads go out in two halves, each in front of the products of 32 k. What is left unhidden (a stage's barrier,
+// the first fragments, the outputs) overlaps with another workgroup's products: two workgroups of eight waves a compute unit for the middle tiles; 256 x 256
+// has eight waves, whose larger parts read LDS less than sixteen did (7,936 rows: 6,400 -> 1,600 172 -> 160 us, 1,600 -> 1,600 55 -> 53).
+// Alone and repeated, 8,192 cubed ran at 1.32 PFLOP/s on sixteen waves (the vendor's library 1.44).
+// Tried and left, cold weights: rings of six to nine stages for small tiles (no faster: not the latency of memory), fragments a stage or half of one ahead in
+// registers of their own, strung between the products (3 to 30 % slower), some waves
+// that load `a` only and others `w` (in steps 1 to 3 % slower), one wave a SIMD with parts of 96 x 64 to 128 x 128 (15 to 60 % slower); tiles of 128 x 64, 128 x
+// 96, 128 x 160, 192 x 192, 256 x 128, 160 x 256, 256 x 192 and 160 x 320 under a model fitted to 232 products alone (4 % faster there on their average; in steps up to 3 % slower); rows of `w` and `a` 64 elements further apart (no change);
+// bands of columns in the tiles' order, which bring fewer rows of `w` into an XCD's L2 (alone up to 8 % faster, in a step slower: the kernels around them find fewer of their rows there, 8,001 tokens
+// 768 -> 2,304 40.8 -> 46.1). Faster,
+// but with sums in another order, which moves a sampled token where two logits lie within the rounding: groups of waves that walk K side by side (64 x 64 and 64 x 96, 5 to 20 %
+// with a compute unit a tile), XCDs that start an eighth of K apart (they ask for the same rows of `w` at once: 3,072 -> 768 of 2,048 rows 21.8 -> 18.8).
 #include "common.h"
 #include "launchers.h"
 #include "gemm_tile.h"
@@ -36,9 +36,10 @@ constexpr size_t tile_lds_bytes(size_t out_bytes) {
     return stages > staging ? stages : staging;
 }
 
-// WM x WN waves, each with (BM / WM) x (BN / WN) of the tile in blocks of 16 x 16; MIN_WAVES a SIMD: what the registers must leave
-// room for (the workgroups that LDS lets a compute unit hold).
-template <int BM, int BN, int STAGES, typename OutT, int EPI, int WM, int WN, int MIN_WAVES>
+// WM x WN waves, each with (BM / WM) x (BN / WN) of the tile in blocks of 16 x 16; MIN_WAVES a SIMD: what the registers must leave room for (the
+// workgroups that LDS lets a compute unit hold). HALVES: a stage's loads and fragments in two halves of 32 k, for tiles whose waves ask for more than the
+// load queue takes; otherwise all of a stage's fragments are read at once, ahead of its products and of the loads.
+template <int BM, int BN, int STAGES, typename OutT, int EPI, int WM, int WN, int MIN_WAVES, bool HALVES>
 __global__ void __launch_bounds__(64 * WM * WN, MIN_WAVES)
 gemm_mfma_tile_kernel(const bf16_t* __restrict__ a, int64_t lda, const bf16_t* __restrict__ w, int M, int N, int K, EpiParams epi, int vec_ok,
                       int page_shift, PartsParams parts) {
@@ -47,11 +48,12 @@ gemm_mfma_tile_kernel(const bf16_t* __restrict__ a, int64_t lda, const bf16_t* _
     static_assert(A_LOADS * 8 * WAVES == BM && W_LOADS * 8 * WAVES == BN, "whole loads a wave");
     static_assert(STAGES >= 2 && STAGES <= 4 && (STAGES - 2) * LOADS <= 63, "the waits below");
     extern __shared__ __attribute__((aligned(1024))) bf16_t lds[];
-    const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64), wm = wave / WN, wn = wave % WN;
+    const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
+    const int wm = wave / WN, wn = wave % WN;
     int m0, n0;
     tile_place<BM, BN>(M, N, K, m0, n0);
 
-    int units = K / TBK, first = 0;  // stages of k this workgroup walks, and where it starts
+    int units = K / TBK, first = 0;  // units of k this workgroup walks, and where it starts
     if constexpr (EPI == kEpiParts) {
         first = blockIdx.y * parts.kt_per_part;
         units = min(units - first, parts.kt_per_part);
@@ -87,50 +89,67 @@ gemm_mfma_tile_kernel(const bf16_t* __restrict__ a, int64_t lda, const bf16_t* _
         for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     const int li = lane % 16, g = lane / 16, swizzle = (li >> 1) & 7;  // (rows of a block start at multiples of 16)
     const int row_a = (wm * (BM / WM) + li) * TBK, row_w = BM * TBK + (wn * (BN / WN) + li) * TBK;
-    auto multiply = [&](int stage, int half) {  // 32 k
+    struct Frags {
+        bf16x8 a[TM], w[TN];
+    };
+    auto read = [&](Frags& f, int stage, int half) {  // 32 k
         const bf16_t* piece = lds + stage * STAGE + (((4 * half + g) ^ swizzle) * 8);
-        bf16x8 fa[TM], fw[TN];
 #pragma unroll
-        for (int j = 0; j < TN; ++j) fw[j] = *reinterpret_cast<const bf16x8*>(piece + row_w + j * 16 * TBK);
+        for (int j = 0; j < TN; ++j) f.w[j] = *reinterpret_cast<const bf16x8*>(piece + row_w + j * 16 * TBK);
 #pragma unroll
-        for (int i = 0; i < TM; ++i) fa[i] = *reinterpret_cast<const bf16x8*>(piece + row_a + i * 16 * TBK);
+        for (int i = 0; i < TM; ++i) f.a[i] = *reinterpret_cast<const bf16x8*>(piece + row_a + i * 16 * TBK);
+    };
+    auto multiply = [&](const Frags& f) {
 #pragma unroll
         for (int i = 0; i < TM; ++i)
 #pragma unroll
-            for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw[j], fa[i], acc[i][j], 0, 0, 0);
+            for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f.w[j], f.a[i], acc[i][j], 0, 0, 0);
     };
 
 #pragma unroll
     for (int p = 0; p < STAGES - 1; ++p)
         if (p < units) issue(0, LOADS, p, p);
     for (int u = 0, stage = 0, next = STAGES - 1; u < units; ++u) {
-        // unit u must have landed; the loads of the units after it may be in flight (a wave's loads complete in order)
+        // stage u must have landed; the loads of the stages after it may be in flight (a wave's loads complete in order)
         const int later = min(units - 1 - u, STAGES - 2);
         if (STAGES > 3 && later >= 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(STAGES > 3 ? 2 * LOADS : 0) : "memory");
         else if (STAGES > 2 && later >= 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(STAGES > 2 ? LOADS : 0) : "memory");
         else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        // everyone's loads of unit u are in LDS, everyone is done reading unit u - 1: its stage takes unit u + STAGES - 1
+        // everyone's loads of stage u are in LDS, everyone is done reading stage u - 1: its place takes stage u + STAGES - 1
         __builtin_amdgcn_s_barrier();
         __builtin_amdgcn_sched_barrier(0);
         const bool more = u + STAGES - 1 < units;
-        if (more) issue(0, (LOADS + 1) / 2, u + STAGES - 1, next);
-        multiply(stage, 0);
-        __builtin_amdgcn_sched_barrier(0);
-        if (more) issue((LOADS + 1) / 2, LOADS, u + STAGES - 1, next);
-        multiply(stage, 1);
-        __builtin_amdgcn_sched_barrier(0);
+        Frags f[2];
+        if constexpr (HALVES) {
+            if (more) issue(0, (LOADS + 1) / 2, u + STAGES - 1, next);
+            read(f[0], stage, 0);
+            multiply(f[0]);
+            __builtin_amdgcn_sched_barrier(0);
+            if (more) issue((LOADS + 1) / 2, LOADS, u + STAGES - 1, next);
+            read(f[1], stage, 1);
+            multiply(f[1]);
+            __builtin_amdgcn_sched_barrier(0);
+        } else {
+            read(f[0], stage, 0);
+            read(f[1], stage, 1);
+            if (more) issue(0, LOADS, u + STAGES - 1, next);
+            __builtin_amdgcn_sched_barrier(0);
+            multiply(f[0]);
+            multiply(f[1]);
+            __builtin_amdgcn_sched_barrier(0);  // (its products, and with them the reads they wait for, stay ahead of the next barrier)
+        }
         stage = stage + 1 == STAGES ? 0 : stage + 1;
         next = next + 1 == STAGES ? 0 : next + 1;
     }
     store_tile<BM, BN, OutT, EPI, WM, WN>(acc, lds, epi, parts, m0, n0, M, N, vec_ok, page_shift, wave, wm, wn, lane);
 }
 
-template <int BM, int BN, int STAGES, int WM, int WN, int MIN_WAVES, typename OutT, int EPI>
+template <int BM, int BN, int STAGES, int WM, int WN, int MIN_WAVES, bool HALVES, typename OutT, int EPI>
 int launch_tile_as(const bf16_t* a, int64_t lda, const bf16_t* w, int M, int N, int K, const EpiParams& epi, int kparts, const PartsParams& parts,
                    hipStream_t stream) {
     constexpr size_t smem = tile_lds_bytes<BM, BN, STAGES, WM, WN>(sizeof(OutT));
     static_assert(smem <= 160 * 1024, "a workgroup's LDS");
-    auto kern = gemm_mfma_tile_kernel<BM, BN, STAGES, OutT, EPI, WM, WN, MIN_WAVES>;
+    auto kern = gemm_mfma_tile_kernel<BM, BN, STAGES, OutT, EPI, WM, WN, MIN_WAVES, HALVES>;
     static bool ready = false;  // once per instantiation, outside any stream capture's first use
     if (!ready) {
         hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(smem));
@@ -144,9 +163,9 @@ int launch_tile_as(const bf16_t* a, int64_t lda, const bf16_t* w, int M, int N, 
     return check_launch("gemm_mfma_tile");
 }
 
-template <int BM, int BN, int STAGES, int WM, int WN, int MIN_WAVES>
+template <int BM, int BN, int STAGES, int WM, int WN, int MIN_WAVES, bool HALVES>
 int launch_tile_epi(const bf16_t* a, int64_t lda, const bf16_t* w, int M, int N, int K, const EpiParams& epi, hipStream_t stream) {
-#define LIYAB_TILE(T, E) launch_tile_as<BM, BN, STAGES, WM, WN, MIN_WAVES, T, E>(a, lda, w, M, N, K, epi, 1, PartsParams{}, stream)
+#define LIYAB_TILE(T, E) launch_tile_as<BM, BN, STAGES, WM, WN, MIN_WAVES, HALVES, T, E>(a, lda, w, M, N, K, epi, 1, PartsParams{}, stream)
     if (epi.mode == kEpiResidual) return LIYAB_TILE(float, kEpiResidual);
     if (epi.out_dtype == kF32) return epi.mode == kEpiNone ? LIYAB_TILE(float, kEpiNone) : LIYAB_TILE(float, -1);
     switch (epi.mode) {
@@ -165,9 +184,9 @@ int choose_gemm_tile(int M, int N, int K) {
     // 256 tile overlaps nothing), in us; a last round that is not full runs at the lower occupancy's time.
     struct Shape { int tile, bm, bn, fit; float unit[3], round; };
     constexpr Shape shapes[] = {
-        {15, 256, 256, 1, {1.45f, 0, 0}, 10.0f}, {9, 192, 128, 2, {0.68f, 1.3f, 0}, 5.0f},  {11, 192, 128, 1, {0.62f, 0, 0}, 4.5f},
-        {8, 128, 128, 2, {0.60f, 1.0f, 0}, 4.0f}, {7, 128, 128, 1, {0.50f, 0, 0}, 3.7f},    {6, 64, 64, 2, {0.30f, 0.45f, 0}, 2.0f},
-        {2, 64, 64, 3, {0.30f, 0.45f, 0.62f}, 2.0f}};
+        {15, 256, 256, 1, {1.38f, 0, 0}, 11.0f}, {9, 192, 128, 2, {0.68f, 1.3f, 0}, 5.0f},  {11, 192, 128, 1, {0.62f, 0, 0}, 4.5f},
+        {21, 128, 192, 1, {0.62f, 0, 0}, 4.5f},  {8, 128, 128, 2, {0.60f, 1.0f, 0}, 4.0f},  {7, 128, 128, 1, {0.50f, 0, 0}, 3.7f},
+        {6, 64, 64, 2, {0.26f, 0.45f, 0}, 2.0f}, {2, 64, 64, 3, {0.30f, 0.45f, 0.62f}, 2.0f}};
     constexpr int kUnits = 256;  // compute units
     int best = 0;
     float best_us = 0.0f;
@@ -181,7 +200,8 @@ int choose_gemm_tile(int M, int N, int K) {
             best_us = us;
         }
     }
-    // Tiles of 64 x 64 in three stages and in four cost the same here. With a compute unit each, two on every unit, or a long K the fourth
+    // 128 x 192 is here for the products whose columns it divides better (2,048 rows of 768 -> 3,072: 256 tiles, 18.4 us in a step; 384 of 128 x 128 20.3).
+    // Tiles of 64 x 64 in three stages and in four cost nearly the same here. With a compute unit each, two on every unit, or a long K the fourth
     // stage is worth its LDS (780 rows, 5,120 -> 1,280 33.4 us against 35.2 in three; 361 rows, 1,280 -> 5,120 14.7 against 14.9); a round
     // in between with a short K takes three (512 rows: 768 -> 2,304 8.9 against 9.7, 1,024 -> 3,072 10.8 against 11.5).
     const int64_t small = static_cast<int64_t>((M + 63) / 64) * ((N + 63) / 64);
@@ -191,20 +211,21 @@ int choose_gemm_tile(int M, int N, int K) {
 
 int launch_gemm_tile(int tile, const bf16_t* a, int64_t lda, const bf16_t* w, int M, int N, int K, const EpiParams& epi, hipStream_t stream) {
     switch (tile) {
-        case 2: return launch_tile_epi<64, 64, 3, 2, 2, 3>(a, lda, w, M, N, K, epi, stream);
-        case 6: return launch_tile_epi<64, 64, 4, 2, 2, 2>(a, lda, w, M, N, K, epi, stream);
-        case 7: return launch_tile_epi<128, 128, 3, 4, 2, 2>(a, lda, w, M, N, K, epi, stream);
-        case 8: return launch_tile_epi<128, 128, 2, 4, 2, 4>(a, lda, w, M, N, K, epi, stream);
-        case 9: return launch_tile_epi<192, 128, 2, 4, 2, 4>(a, lda, w, M, N, K, epi, stream);
-        case 11: return launch_tile_epi<192, 128, 3, 4, 2, 2>(a, lda, w, M, N, K, epi, stream);
-        case 15: return launch_tile_epi<256, 256, 2, 4, 4, 4>(a, lda, w, M, N, K, epi, stream);
+        case 2: return launch_tile_epi<64, 64, 3, 2, 2, 3, false>(a, lda, w, M, N, K, epi, stream);
+        case 6: return launch_tile_epi<64, 64, 4, 2, 2, 2, false>(a, lda, w, M, N, K, epi, stream);
+        case 7: return launch_tile_epi<128, 128, 3, 4, 2, 2, true>(a, lda, w, M, N, K, epi, stream);
+        case 8: return launch_tile_epi<128, 128, 2, 4, 2, 4, true>(a, lda, w, M, N, K, epi, stream);
+        case 9: return launch_tile_epi<192, 128, 2, 4, 2, 4, true>(a, lda, w, M, N, K, epi, stream);
+        case 11: return launch_tile_epi<192, 128, 3, 4, 2, 2, true>(a, lda, w, M, N, K, epi, stream);
+        case 15: return launch_tile_epi<256, 256, 2, 2, 4, 2, false>(a, lda, w, M, N, K, epi, stream);
+        case 21: return launch_tile_epi<128, 192, 3, 2, 4, 2, false>(a, lda, w, M, N, K, epi, stream);
         default: return fail(1, "gemm_mfma_dl: unknown tile %d", tile);
     }
 }
 
 int launch_gemm_tile_parts(const bf16_t* a, int64_t lda, const bf16_t* w, int M, int N, int K, int kparts, const EpiParams& epi, const PartsParams& parts,
                            hipStream_t stream) {
-    return launch_tile_as<64, 64, 4, 2, 2, 2, float, kEpiParts>(a, lda, w, M, N, K, epi, kparts, parts, stream);
+    return launch_tile_as<64, 64, 4, 2, 2, 2, false, float, kEpiParts>(a, lda, w, M, N, K, epi, kparts, parts, stream);
 }
 
 }  // namespace liyab

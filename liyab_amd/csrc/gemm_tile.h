@@ -284,8 +284,8 @@ inline void store_rules(const EpiParams& epi, int N, int& vec_ok, int& page_shif
     vec_ok = vec16 ? 2 : (vec ? 1 : 0);
 }
 
-// gemm_mfma_tile.hip: the tile for a product of these sizes; the product in it (2, 6: 64 x 64, three and four stages; 7, 8: 128 x 128,
-// three and two; 9, 11: 192 x 128, two and three; 15: 256 x 256); and cut over K, in tiles of 64 x 64.
+// gemm_mfma_tile.hip: the tile for a product of these sizes; the product in it (2, 6: 64 x 64, three stages and four; 7, 8: 128 x 128, three and two; 21: 128 x
+// 192; 9, 11: 192 x 128, two and three; 15: 256 x 256: the same bits from each); and cut over K, in tiles of 64 x 64.
 int choose_gemm_tile(int M, int N, int K);
 int launch_gemm_tile(int tile, const bf16_t* a, int64_t lda, const bf16_t* w, int M, int N, int K, const EpiParams& epi, hipStream_t stream);
 int launch_gemm_tile_parts(const bf16_t* a, int64_t lda, const bf16_t* w, int M, int N, int K, int kparts, const EpiParams& epi, const PartsParams& parts,
