@@ -26,6 +26,7 @@
 // rounding only. Scores, exponentials and sums are 32-bit.
 #include <type_traits>
 
+#include "attention_partial.h"
 #include "common.h"
 #include "launchers.h"
 
@@ -58,27 +59,6 @@ __device__ __forceinline__ void unpack8(const Raw8F& v, float* f) {
 }
 template <typename T> struct Raw8 { typedef u32x4 type; };
 template <> struct Raw8<float> { typedef Raw8F type; };
-// exponentials of scores: the fast one beside bfloat16 data, the library's beside 32-bit data
-template <typename T> __device__ __forceinline__ float exp_for(float x) { return __expf(x); }
-template <> __device__ __forceinline__ float exp_for<float>(float x) { return expf(x); }
-
-struct Partial {
-    float m, l;
-    float acc[8];
-};
-
-// this <- merge(this, other): both rescaled to the larger maximum; this comes first.
-template <typename T>
-__device__ __forceinline__ void merge_partial(Partial& a, float mo, float lo, const float* acco) {
-    const float M = fmaxf(a.m, mo);
-    const float wa = a.m == -INFINITY ? 0.0f : exp_for<T>(a.m - M);
-    const float wb = mo == -INFINITY ? 0.0f : exp_for<T>(mo - M);
-    a.l = wa * a.l + wb * lo;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) a.acc[e] = wa * a.acc[e] + wb * acco[e];
-    a.m = M;
-}
-
 // A sink joins a row's softmax: a learned logit a head that stands in the denominator once, as a key would whose score it is,
 // and has no value. (m, l, acc): the row's maximum, sum and weighted values, rescaled to the larger of m and the sink.
 template <typename T, int N = 8>

@@ -44,6 +44,7 @@ VGPR_MFMA = ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]
 FILE_FLAGS = {
     "attention_prefill.hip": VGPR_MFMA,
     "attention_prefill_direct.hip": VGPR_MFMA,
+    "attention_rows.hip": VGPR_MFMA,
     "gemm_simple.hip": VGPR_MFMA,
 }
 

@@ -65,6 +65,9 @@ int liyab_attention_decode(void* out, int64_t out_stride, const void* q, int64_t
                            float scale, int window, int n_head, int n_kv_head, int hd, int page_size, int n_splits, int chunk,
                            int waves, int rows_are_requests, float* partials, int leave_splits, int num_pages, int reach,
                            hipStream_t stream);
+int liyab_attention_rows(float* out, int64_t out_stride, const float* q, int64_t q_stride, const float* kc, const float* vc, const int* block_tables,
+                         int max_blocks, const int* work, int n_tiles, int tile, float scale, int n_head, int n_kv_head, int page_size, int n_splits,
+                         float* partials, int num_pages, hipStream_t stream);
 int liyab_attention_merge(void* out, int out_dtype, int64_t out_stride, const float* partials, int n, int n_head, int hd, int n_splits,
                           hipStream_t stream);
 int liyab_attention_prefill(void* out, int64_t out_stride, const void* q, int64_t q_stride, const void* kc, const void* vc,

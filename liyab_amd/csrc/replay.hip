@@ -94,6 +94,7 @@ static const Entry kEntries[] = {
     LIYAB_ENTRY(liyab_attention_generic),
     LIYAB_ENTRY(liyab_attention_decode),
     LIYAB_ENTRY(liyab_attention_merge),
+    LIYAB_ENTRY(liyab_attention_rows),
     LIYAB_ENTRY(liyab_attention_prefill),
     LIYAB_ENTRY(liyab_rmsnorm),
     LIYAB_ENTRY(liyab_gated_norm_add),

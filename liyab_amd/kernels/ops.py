@@ -1010,6 +1010,31 @@ def attention_merge(out: torch.Tensor, partials: torch.Tensor) -> None:
     _lib.call("liyab_attention_merge", out.data_ptr(), dtype_code(out.dtype), os_, partials.data_ptr(), n, H, hd4 - 4, S, _stream())
 
 
+def attention_rows(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, block_tables: torch.Tensor, work: torch.Tensor,
+                   n_tiles: int, *, n_head: int, scale: float, tile: int, n_splits: int = 1, partials: Optional[torch.Tensor] = None,
+                   num_pages: Optional[int] = None) -> None:
+    """Tiles of up to `tile` consecutive queries of one request over its 32-bit cache, heads of 64: the bits of `attention_decode(..., chunk=256)`, whose splits they
+    are cut into: one leaves its rows in `out`; more leave `partials` [rows, heads, splits, 68] for `attention_merge`. work: as for `attention_prefill`."""
+    if k_cache.dim() != 4 or k_cache.shape != v_cache.shape or not k_cache.is_contiguous() or not v_cache.is_contiguous():
+        raise KernelError("attention: caches must be contiguous [pages, kv_heads, page_size, head_dim] of one shape")
+    _, hkv, page, hd = k_cache.shape
+    os_, qs = _rows(out, "out"), _rows(q, "q")
+    if q.shape[0] != out.shape[0] or q.shape[1] < n_head * hd or out.shape[1] != n_head * hd:
+        raise KernelError(f"attention: q {tuple(q.shape)} / out {tuple(out.shape)} do not fit {n_head} heads of {hd}")
+    if not (q.dtype == out.dtype == k_cache.dtype == v_cache.dtype == torch.float32) or hd != 64:
+        raise KernelError("attention_rows: q, out and the caches must be float32, heads of 64")
+    _dev(block_tables, "block_tables")
+    if block_tables.dim() != 2 or block_tables.dtype != torch.int32 or not block_tables.is_contiguous():
+        raise KernelError("attention: block_tables must be contiguous int32 [requests, max_blocks]")
+    _i32(work, "work", 4 * n_tiles)
+    if n_splits > 1:
+        need = out.shape[0] * n_head * n_splits * (hd + 4)
+        if partials is None or partials.dtype != torch.float32 or partials.numel() < need or not partials.is_contiguous():
+            raise KernelError(f"attention_rows: {n_splits} splits need {need} float32 of partials")
+    _lib.call("liyab_attention_rows", out.data_ptr(), os_, q.data_ptr(), qs, k_cache.data_ptr(), v_cache.data_ptr(), block_tables.data_ptr(), block_tables.shape[1],
+              work.data_ptr(), n_tiles, int(tile), float(scale), n_head, hkv, page, n_splits, _ptr(partials), _pages(k_cache, num_pages), _stream())
+
+
 def attention_prefill(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
                       block_tables: torch.Tensor, work: torch.Tensor, n_tiles: int, *, n_head: int, scale: float,
                       window: int = 0, tile: int = 128, ksplit: int = 1, num_pages: Optional[int] = None, softcap: float = 0.0,
@@ -1120,6 +1145,18 @@ def invariant_chunk(reach: int) -> int:
     return chunk
 
 
+# (token, head) pairs of a step of prompt portions in 32 bits from which attention_rows takes it (us token by token / there, 12 heads: one portion of 200 tokens 16.1 / 17.2, of 500
+# 52 / 27, four of 48 12.9 / 11.2, ten of 30 16.9 / 11.2; 25 heads: one of 300 47 / 26)
+ROWS_FROM_PAIRS = 3000
+ROWS_MAX_PARTIALS = 32 << 20  # floats of splits left for the merge
+
+
+def rows_pay(plan, q, hd: int, n: int, n_head: int, splits: int, chunk: int) -> bool:
+    """Whether a step of prompt portions in 32 bits goes to the kernel that takes 32 queries to 256 keys (attention_rows): the same bits as token by token."""
+    return (q.dtype == torch.float32 and hd == 64 and chunk == 256 and plan.mode == "prefill" and plan.n_single == 0 and plan.n_tiles > 0
+            and n * n_head >= ROWS_FROM_PAIRS and splits <= 64 and n * n_head * splits * (hd + 4) <= ROWS_MAX_PARTIALS)
+
+
 def attention_takes(head_dim: int) -> bool:
     """Whether some attention kernel of the library takes this head size, in either precision."""
     return 0 < head_dim <= ATTENTION_MAX_HEAD_DIM
@@ -1170,6 +1207,12 @@ def attention(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor, v_cache
         reach = block_tables.shape[1] * k_cache.shape[2] if window <= 0 else min(window + keep_first, block_tables.shape[1] * k_cache.shape[2])
         chunk = invariant_chunk(reach)
         splits = max(1, -(-min(plan.context_bucket, reach) // chunk))
+        if rows_pay(plan, q, hd, n, n_head, splits, chunk) and window <= 0 and not scored:
+            partials = ctx.workspace.get("attn_partials", (n, n_head, splits, hd + 4), torch.float32) if splits > 1 else None
+            attention_rows(out, q, k_cache, v_cache, block_tables, plan.work, plan.n_tiles, n_head=n_head, scale=scale, tile=plan.tile, n_splits=splits, partials=partials)
+            if splits > 1:
+                attention_merge(out, partials)
+            return None
         # many tokens: a workgroup walks its token's splits in turn (the same bits: the kernel merges them
         # as the merge kernel does), which saves the splits' traffic and leaves the chip as full
         if n * n_head * splits > INVARIANT_SPLIT_WORK:
