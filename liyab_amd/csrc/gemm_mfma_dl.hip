@@ -288,7 +288,8 @@ using namespace liyab;
 // of its own: 1,600 -> 4,800 in 13.9 against 9.7); 16 = 64x32 on four groups of two waves that walk K side by side, three stages of
 // four units (for one tile of rows: 8.2 us for 64 x 4,800 x 1,600 where two waves walking K alone, four
 // stages deep, took 10.3; deeper rings for those took longer, 11.1 with eight stages: the walk waits on
-// its own chain of load, barrier, fragments and products, not on the loads in flight).
+// its own chain of load, barrier, fragments and products, not on the loads in flight); 18 = the same bits for up to 64 rows from waves
+// with rings of their own (gemm_mfma_waves.hip; more rows than 64 are taken tile by tile).
 extern "C" int liyab_gemm_mfma_dl(const void* a, int64_t lda, const void* w, int M, int N, int K, int tile,
                                   const EpiParams* epi_in, hipStream_t stream) {
     LIYAB_REQUIRE(a && w && epi_in, "gemm: null operand");
@@ -303,6 +304,7 @@ extern "C" int liyab_gemm_mfma_dl(const void* a, int64_t lda, const void* w, int
     switch (tile) {
         case 16: return launch_dl<64, 32, 3, 2, 1, 4>(a, lda, w, M, N, K, epi, stream);
         case 17: return launch_dl<32, 32, 3, 1, 1, 4>(a, lda, w, M, N, K, epi, stream);
+        case 18: return launch_gemm_waves(static_cast<const bf16_t*>(a), lda, static_cast<const bf16_t*>(w), M, N, K, epi, 1, nullptr, stream);
         // 102, 106, 108: tiles of 64 x 64 and 128 x 128 with four sums by unit of K, whose results are those of 16 and 17 bit for bit
         case 102: return launch_dl<64, 64, 3, 2, 2, 1, 4>(a, lda, w, M, N, K, epi, stream);
         case 106: return launch_dl<64, 64, 4, 2, 2, 1, 4>(a, lda, w, M, N, K, epi, stream);
@@ -314,7 +316,7 @@ extern "C" int liyab_gemm_mfma_dl(const void* a, int64_t lda, const void* w, int
 // The same product cut over K: parts[p * part_stride + m * N + n] = sum over the p-th of `kparts` parts
 // of K (whole tiles of 64) of a[m, k] w[n, k]. With `base` (n_base planes [M, N], base_stride floats
 // apart, not overlapping `parts`) the first plane also takes bias[n] and base[0] + base[1] + ...;
-// without it `bias` must be null. tile: 6 = 64x64 tiles, 16 = 64x32 (for one tile of rows), 17 = 32x32.
+// without it `bias` must be null. tile: 6 = 64x64 tiles, 16 = 64x32 (for one tile of rows), 17 = 32x32, 18 = gemm_mfma_waves.hip.
 extern "C" int liyab_gemm_mfma_dl_parts(const void* a, int64_t lda, const void* w, int M, int N, int K, int kparts, int tile,
                                         float* parts, int64_t part_stride, const float* bias, const float* base, int n_base,
                                         int64_t base_stride, hipStream_t stream) {
@@ -349,5 +351,6 @@ extern "C" int liyab_gemm_mfma_dl_parts(const void* a, int64_t lda, const void* 
     if (tile == 6) return launch_gemm_tile_parts(pa, lda, pw, M, N, K, kparts, epi, pp, stream);
     if (tile == 16) return launch_dl_parts<64, 32, 3, 2, 1, 4>(pa, lda, pw, M, N, K, kparts, epi, pp, stream);
     if (tile == 17) return launch_dl_parts<32, 32, 3, 1, 1, 4>(pa, lda, pw, M, N, K, kparts, epi, pp, stream);
-    return fail(1, "gemm_mfma_dl_parts: unknown tile %d (6, 16 or 17)", tile);
+    if (tile == 18) return launch_gemm_waves(pa, lda, pw, M, N, K, epi, kparts, &pp, stream);
+    return fail(1, "gemm_mfma_dl_parts: unknown tile %d (6, 16, 17 or 18)", tile);
 }

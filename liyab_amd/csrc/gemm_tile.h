@@ -291,4 +291,7 @@ int launch_gemm_tile(int tile, const bf16_t* a, int64_t lda, const bf16_t* w, in
 int launch_gemm_tile_parts(const bf16_t* a, int64_t lda, const bf16_t* w, int M, int N, int K, int kparts, const EpiParams& epi, const PartsParams& parts,
                            hipStream_t stream);
 
+// gemm_mfma_waves.hip: products of 17 to 64 rows (more are taken, row tile by row tile), whole (parts null) or cut over K.
+int launch_gemm_waves(const bf16_t* a, int64_t lda, const bf16_t* w, int M, int N, int K, const EpiParams& epi, int kparts, const PartsParams* parts, hipStream_t stream);
+
 }  // namespace liyab

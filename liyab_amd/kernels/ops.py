@@ -656,7 +656,7 @@ def gemm_mfma_dl_parts(a: torch.Tensor, w: torch.Tensor, planes: torch.Tensor, *
                        base: Optional[torch.Tensor] = None, tile: int = 6) -> None:
     """The tiled matrix-core product cut over K (K a multiple of 64), as `gemm_skinny_parts` for
     any number of rows: planes float32 [parts, M, N]; with `base` the first plane also takes
-    `bias` and the rows of `base`. tile: 6 = 64 x 64 tiles, 16 = 64 x 32, 17 = 32 x 32."""
+    `bias` and the rows of `base`. tile: 6 = 64 x 64 tiles, 16 = 64 x 32, 17 = 32 x 32, 18 = the bits of these two for up to 64 rows (`waves_pay`)."""
     lda = _rows(a, "a")
     M, K = a.shape
     _dev(w, "w")
@@ -833,6 +833,13 @@ def compute_units() -> int:
     return _compute_units
 
 
+def waves_pay(M: int, K: int, parts: int = 1) -> bool:
+    """Whether a product of 17 to 64 rows that the tiles of 32 x 32 and 64 x 32 would take (`gemm_mfma_dl`'s 16 and 17) goes to the kernel that leaves their bits from
+    waves with rings of their own (csrc/gemm_mfma_waves.hip, 18). us, cold weights, those / it: 15 to 35 % less at 24 to 64 rows of 13 shapes from 640 -> 2,560 to 2,048 -> 6,144;
+    3,200 -> 2,176 at 64 rows 11.5 / 9.8, 4,096 -> 4,096 at 24, 48 and 64 rows 13.2 / 10.3, 12.5 / 13.2, 14.0 / 13.5."""
+    return K % 64 == 0 and 16 < M <= 64 and K <= (4096 if M <= 32 else 3200) * parts
+
+
 def skinny_ln_pays(M: int, N: int, K: int) -> bool:
     """Whether folding the norm into the product beats the norm kernel followed by the plain
     product. The folded kernel keeps a row in registers, so one workgroup fills a compute unit:
@@ -907,8 +914,9 @@ def gemm(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], *, out:
             # tiles of 32 x 32 while each has a compute unit of its own: a workgroup brings in a third
             # less of the operands and twice as many pull (64 rows, cold weights: 5.05 against 5.53 us
             # for 768 -> 2,304, 5.97 against 6.85 for 1,024 -> 3,072; 13.9 against 9.7 for 1,600 -> 4,800)
+            # (up to 64 rows the same bits come faster from waves with rings of their own: waves_pay)
             small = (M + 31) // 32 * ((N + 31) // 32) <= compute_units()
-            gemm_mfma_dl(a, w, bias, out=out, residual=residual, epilogue=epilogue, kv=kv, tile=17 if small else 16)
+            gemm_mfma_dl(a, w, bias, out=out, residual=residual, epilogue=epilogue, kv=kv, tile=18 if waves_pay(M, a.shape[1]) else 17 if small else 16)
         elif M <= 16 or (M <= 64 and N <= 8192):
             # few tokens: stream the weights (for a huge N and more than 16 tokens the tiled
             # kernel's shared loads beat every workgroup re-reading the tokens); 11 to 16 tokens and

@@ -132,6 +132,8 @@ def linear_deferred(a, w: torch.Tensor, bias: Optional[torch.Tensor], ctx, name:
             tile = 17 if M <= 32 else 6
         else:
             tile = 17 if fewer else (16 if M <= 64 or few else 6)
+        if tile != 6 and ops.waves_pay(M, K, parts):
+            tile = 18  # (their bits)
         ops.gemm_mfma_dl_parts(a, w, planes, bias=bias, base=base, tile=tile)
     else:
         ops.gemm_skinny_parts(a, w, planes, bias=bias, base=base)

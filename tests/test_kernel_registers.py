@@ -9,7 +9,7 @@ import pytest
 from liyab_amd.csrc import build
 
 
-@pytest.mark.parametrize("source", ["attention_prefill_direct.hip", "sampling.hip", "gemm_skinny_ln.hip", "gemm_skinny.hip", "gemm_rows.hip", "grouped_product.hip"])
+@pytest.mark.parametrize("source", ["attention_prefill_direct.hip", "sampling.hip", "gemm_skinny_ln.hip", "gemm_skinny.hip", "gemm_rows.hip", "grouped_product.hip", "gemm_mfma_waves.hip"])
 def test_no_kernel_spills(source, tmp_path):
     """A spilled register goes to memory and back in the walk over the keys, and counts among the loads that its waits count; in the sampler, whose threads
     hold a row, in every pass over it; in the norm's product, which is as short as the trips it waits for, in the middle of them. The kernels with rings in LDS wait for
