@@ -14,15 +14,16 @@ struct Partial {
     float acc[8];
 };
 
-// this <- merge(this, other): both rescaled to the larger maximum; this comes first.
-template <typename T>
+// this <- merge(this, other): both rescaled to the larger maximum; this comes first. Which product of a value is rounded by itself ahead of the sum is part of a
+// kernel's bits: the other's (OTHER_FIRST), or this one's; a sum's is the other's.
+template <typename T, bool OTHER_FIRST>
 __device__ __forceinline__ void merge_partial(Partial& a, float mo, float lo, const float* acco) {
     const float M = fmaxf(a.m, mo);
     const float wa = a.m == -INFINITY ? 0.0f : exp_for<T>(a.m - M);
     const float wb = mo == -INFINITY ? 0.0f : exp_for<T>(mo - M);
-    a.l = wa * a.l + wb * lo;
+    a.l = fmaf(wa, a.l, wb * lo);
 #pragma unroll
-    for (int e = 0; e < 8; ++e) a.acc[e] = wa * a.acc[e] + wb * acco[e];
+    for (int e = 0; e < 8; ++e) a.acc[e] = OTHER_FIRST ? fmaf(wa, a.acc[e], wb * acco[e]) : fmaf(wb, acco[e], wa * a.acc[e]);
     a.m = M;
 }
 

@@ -42,6 +42,7 @@ FLAGS = [
 # by default they land in accumulation registers and every such use costs a move each way.
 VGPR_MFMA = ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]
 FILE_FLAGS = {
+    "attention_mixed.hip": VGPR_MFMA,
     "attention_prefill.hip": VGPR_MFMA,
     "attention_prefill_direct.hip": VGPR_MFMA,
     "attention_rows.hip": VGPR_MFMA,

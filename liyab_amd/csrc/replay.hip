@@ -96,6 +96,7 @@ static const Entry kEntries[] = {
     LIYAB_ENTRY(liyab_attention_merge),
     LIYAB_ENTRY(liyab_attention_rows),
     LIYAB_ENTRY(liyab_attention_prefill),
+    LIYAB_ENTRY(liyab_attention_mixed),
     LIYAB_ENTRY(liyab_rmsnorm),
     LIYAB_ENTRY(liyab_gated_norm_add),
     LIYAB_ENTRY(liyab_causal_conv),
