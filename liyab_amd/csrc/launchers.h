@@ -98,6 +98,9 @@ int liyab_moe_route(const float* logits, int64_t ld, int n, int n_experts, int t
 int liyab_moe_route_align(const float* logits, int64_t ld, int n, int n_experts, int top, int* ids, float* weights, int block,
                           int* rows_list, int* tile_group, int max_tiles, int mode, int n_groups, int keep, const float* correction,
                           float scale, int n_listed, int extra, hipStream_t stream);
+int liyab_moe_router(const void* a, int64_t lda, const void* w, const float* bias, int columns, int K, float* logits, int64_t ld, int n, int n_experts, int top, int* ids,
+                     float* weights, int block, int* rows_list, int* tile_group, int max_tiles, int mode, int n_groups, int keep, const float* correction, float scale,
+                     int n_listed, int extra, hipStream_t stream);
 int liyab_moe_align(const int* ids, int n_entries, int n_experts, int block, int* rows_list, int* tile_group, int max_tiles,
                     hipStream_t stream);
 

@@ -191,11 +191,11 @@ __device__ __forceinline__ void route_wave(const float* __restrict__ z, const Ro
     }
 }
 
-// The same for one group of at most 64 outputs: an output a lane, its score in a register; zl is the lane's logit, and with `extra` lane 0 knows the
-// token's own one. No trip through LDS.
+// The same for at most 64 outputs: an output a lane, its score in a register; zl is the lane's logit, and with `extra` lane 0 knows the
+// token's own one. No trip through LDS. Groups of a power of two of outputs: their two largest meet in a butterfly.
 __device__ __forceinline__ void route_wave_lane(float zl, float own, const RouteArgs& ra, int E, int top, int* __restrict__ ids, float* __restrict__ weights) {
     const int lane = threadIdx.x % kWave;
-    const bool real = lane < E;
+    const bool real = lane < E, grouped = ra.keep < ra.n_groups;
     float s;
     if (ra.mode == 3) {
         const float v = real ? expf(zl - wave_max(real ? zl : -INFINITY)) : 0.0f;
@@ -204,9 +204,29 @@ __device__ __forceinline__ void route_wave_lane(float zl, float own, const Route
         s = 1.0f / (1.0f + expf(-zl));
     }
     float c = real ? s + (ra.correction != nullptr ? ra.correction[lane] : 0.0f) : -INFINITY;
+    if (grouped) {
+        const int per = E / ra.n_groups;
+        float a = fmaxf(-INFINITY, c), b = -INFINITY;  // the two largest so far
+        for (int off = 1; off < per; off <<= 1) {
+            const float ao = __shfl_xor(a, off, kWave), bo = __shfl_xor(b, off, kWave);
+            b = fmaxf(fminf(a, ao), fmaxf(b, bo));
+            a = fmaxf(a, ao);
+        }
+        float score = __shfl(per > 1 ? a + b : a, (lane * per) % kWave, kWave);  // lane g: group g's
+        if (lane >= ra.n_groups) score = -INFINITY;
+        uint64_t kept = 0;
+        for (int k = 0; k < ra.keep; ++k) {
+            float bv = score;
+            int bi = lane < ra.n_groups ? lane : kMaxGroups + lane;
+            wave_argmax(bv, bi);
+            kept |= uint64_t(1) << (bi % kMaxGroups);
+            if (lane == bi) score = -INFINITY;
+        }
+        if (!(c > -INFINITY) || !((kept >> (lane / per)) & 1)) c = -INFINITY;
+    }
     for (int k = 0; k < top; ++k) {
         float bv = c;
-        int bi = real ? lane : kWave + lane;
+        int bi = grouped ? (c > -INFINITY ? lane : E) : real ? lane : kWave + lane;
         wave_argmax(bv, bi);
         const int best = min(bi, E - 1);
         if (lane == best) {
@@ -220,7 +240,10 @@ __device__ __forceinline__ void route_wave_lane(float zl, float own, const Route
         weights[top] = 1.0f / (1.0f + expf(-own));
     }
 }
-__device__ __forceinline__ bool routes_in_lanes(const RouteArgs& ra, int E) { return E <= kWave && ra.keep == ra.n_groups; }
+__device__ __forceinline__ __host__ bool routes_in_lanes(const RouteArgs& ra, int E) {
+    const int per = E / ra.n_groups;
+    return E <= kWave && (ra.keep == ra.n_groups || (per & (per - 1)) == 0);
+}
 
 // a wave a token, four waves a workgroup
 __global__ void __launch_bounds__(256)
@@ -338,29 +361,93 @@ moe_route_softmax_kernel(const float* __restrict__ logits, int64_t ld, int n, in
     route_wave_softmax(logits[static_cast<int64_t>(t) * ld + min(static_cast<int>(threadIdx.x) % kWave, E - 1)], E, top, ids + at, weights + at);
 }
 
-// Choices (mode 0) and lists of a step of at most kWaveRouteTokens tokens, few experts and entries (a decoding step): one workgroup, whose time is the trips of
-// what one thread writes and another reads. A wave chooses for a token, an expert a lane; ids, counts and lists stay in LDS, an expert's first place is
-// summed up by whoever needs it, and everything leaves once at the end. (The kernel below has a thread choose, clears the lists in memory, reads the ids back from there
-// twice and has one thread lay out the tiles: 4 tokens, 2 of 8 experts 6.7 -> 4.9 us, 8 of 64 235 -> 17.5.)
+// Choices (modes 0, 2 and 3) and lists of a step of at most kWaveRouteTokens tokens, few experts and entries (a decoding step): one workgroup, whose time is the trips of
+// what one thread writes and another reads. A wave chooses for a token, an expert a lane; ids, counts and lists stay in LDS, every wave sums up the experts'
+// first places by itself, an expert a lane, and everything leaves once at the end. (The kernel below has a thread choose, or a wave with its scores in LDS, clears the lists in memory,
+// reads the ids back from there twice and has one thread lay out the tiles: 4 tokens, 2 of 8 experts
+// 6.7 -> 4.9 us, 8 of 64 235 -> 17.5; with the product ahead, a layer's step of 4 tokens at GPT-2 small's width gains 4.1 us with groups of experts, 3.1 with softmax scores over
+// all, 1.0 with the largest logits, the last two of whose choices were as short before.)
 constexpr int kSmallExperts = 64, kSmallEntries = 1024, kSmallPlaces = 4096;
 
+// The router's own product ahead of that, for up to 16 tokens and outputs: the logits are one strip of gemm_skinny.hip's streaming kernel, one workgroup, and this one takes it
+// over with that kernel's waves, order of sums and bits. K: whole units of 64; 1 << split_shift waves share it, two units a trip.
+struct RouterProduct {
+    const bf16_t* a;
+    int64_t lda;
+    const bf16_t* w;
+    const float* bias;
+    int columns, K, split_shift;
+    float* logits;
+};
+typedef __attribute__((ext_vector_type(8))) __bf16 moe_bf16x8;
+typedef __attribute__((ext_vector_type(4))) float moe_f32x4;
+constexpr int kRouterSide = 16;
+
+template <bool PRODUCT>
 __global__ void __launch_bounds__(1024)
 moe_route_align_small_kernel(const float* __restrict__ logits, int64_t ld, int n, int E, int top, int* __restrict__ ids, float* __restrict__ weights,
-                             int block, int* __restrict__ rows_list, int* __restrict__ tile_group, int max_tiles) {
+                             int block, int* __restrict__ rows_list, int* __restrict__ tile_group, int max_tiles, RouteArgs ra, RouterProduct rp) {
     extern __shared__ int list[];  // [places]
     __shared__ int ids_of[kSmallEntries], counts[kSmallExperts];
     __shared__ float weights_of[kSmallEntries];
-    const int t = threadIdx.x, wave = t / kWave, entries = n * top, places = max_tiles * block;
+    const int t = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(t / kWave), lane = t % kWave, each = top + ra.extra, entries = n * each, places = max_tiles * block;
     constexpr int kEach = kWaveRouteTokens / (1024 / kWave);  // tokens a wave: all their logits are asked for together
-    float zl[kEach];
+    float zl[kEach], own[kEach];
+    if constexpr (PRODUCT) {
+        __shared__ float sums[1024 / kWave][kRouterSide * kRouterSide], z[kRouterSide][kRouterSide];
+        const int i = lane % 16, g = lane / 16, splits = 1 << rp.split_shift, units = rp.K / 64, trips = (units + 1) / 2;
+        const int live = min(splits, trips);
+        if (wave < live) {
+            const bf16_t* const w = rp.w + static_cast<int64_t>(min(i, rp.columns - 1)) * rp.K + g * 8;
+            const bf16_t* const a = rp.a + static_cast<int64_t>(min(i, n - 1)) * rp.lda + g * 8;
+            moe_f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+            for (int trip = wave; trip < trips; trip += splits) {
+                moe_bf16x8 x[4], y[4];
 #pragma unroll
-    for (int j = 0; j < kEach; ++j) zl[j] = logits[static_cast<int64_t>(min(wave + j * (1024 / kWave), n - 1)) * ld + min(t % kWave, E - 1)];
-    for (int i = t; i < places; i += 1024) list[i] = -1;
-    if (t < kSmallExperts) counts[t] = 0;
+                for (int h = 0; h < 4; ++h) {
+                    const int k = min(trip * 128 + 32 * h, rp.K - 32);  // (a unit past the end: read and not multiplied)
+                    x[h] = *reinterpret_cast<const moe_bf16x8*>(w + k);
+                    y[h] = *reinterpret_cast<const moe_bf16x8*>(a + k);
+                }
 #pragma unroll
-    for (int j = 0; j < kEach; ++j) {
+                for (int h = 0; h < 4; ++h)
+                    if (h < 2 || 2 * trip + 1 < units) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x[h], y[h], acc, 0, 0, 0);
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) sums[wave][i * 16 + 4 * g + r] = acc[r];
+        }
+        for (int q = t; q < places; q += 1024) list[q] = -1;
+        if (t < kSmallExperts) counts[t] = 0;
+        const int m = t / 16, c = t % 16;
+        const bool mine = t < 256 && m < n && c < rp.columns;
+        const float bias = rp.bias != nullptr ? rp.bias[min(c, rp.columns - 1)] : 0.0f;
+        lds_barrier();
+        if (mine) {
+            float v = 0.0f;
+            for (int q = 0; q < live; ++q) v += sums[q][t];
+            v += bias;
+            z[m][c] = v;
+            rp.logits[static_cast<int64_t>(m) * ld + c] = v;
+        }
+        lds_barrier();
+        zl[0] = z[min(wave, n - 1)][min(lane, E - 1)];
+        own[0] = z[min(wave, n - 1)][ra.extra ? E : 0];
+    } else {
+#pragma unroll
+        for (int j = 0; j < kEach; ++j) {
+            const float* const z = logits + static_cast<int64_t>(min(wave + j * (1024 / kWave), n - 1)) * ld;
+            zl[j] = z[min(lane, E - 1)];
+            own[j] = z[ra.extra ? E : 0];
+        }
+        for (int i = t; i < places; i += 1024) list[i] = -1;
+        if (t < kSmallExperts) counts[t] = 0;
+    }
+#pragma unroll
+    for (int j = 0; j < (PRODUCT ? 1 : kEach); ++j) {
         const int i = wave + j * (1024 / kWave);
-        if (i < n) route_wave_softmax(zl[j], E, top, ids_of + i * top, weights_of + i * top);
+        if (i >= n) continue;
+        if (ra.mode == 0) route_wave_softmax(zl[j], E, top, ids_of + i * each, weights_of + i * each);
+        else route_wave_lane(zl[j], own[j], ra, E, top, ids_of + i * each, weights_of + i * each);
     }
     lds_barrier();
     int e = -1, rank = 0;
@@ -368,19 +455,21 @@ moe_route_align_small_kernel(const float* __restrict__ logits, int64_t ld, int n
         e = ids_of[t];
         ids[t] = e;
         weights[t] = weights_of[t];
-        rank = atomicAdd(&counts[e], 1);
+        if (e >= 0) rank = atomicAdd(&counts[e], 1);
     }
     lds_barrier();
-    // tile t's expert, and the first place of this thread's entry's
-    int group = -1, first = 0, at = 0;
-    for (int x = 0; x < E; ++x) {
-        const int tiles = (counts[x] + block - 1) / block;
-        if (x == e) first = at * block;
-        if (t >= at && t < at + tiles) group = x;
-        at += tiles;
+    const int tiles = (counts[lane] + block - 1) / block;  // of expert `lane` (past the experts: none)
+    int up_to = tiles;
+    for (int off = 1; off < kWave; off <<= 1) {
+        const int before = __shfl_up(up_to, off, kWave);
+        if (lane >= off) up_to += before;
     }
-    if (e >= 0 && first + rank < places) list[first + rank] = t;
-    if (t < max_tiles) tile_group[t] = group;
+    const int at = up_to - tiles, used = __shfl(up_to, kWave - 1, kWave), place = __shfl(at, max(e, 0), kWave) * block + rank;
+    if (e >= 0 && place < places) list[place] = t;
+    if (wave == 0) {
+        for (int i = at; i < min(up_to, max_tiles); ++i) tile_group[i] = lane;
+        for (int i = used + lane; i < max_tiles; i += kWave) tile_group[i] = -1;
+    }
     lds_barrier();
     for (int i = t; i < places; i += 1024) rows_list[i] = list[i];
 }
@@ -458,7 +547,8 @@ extern "C" int liyab_moe_align(const int* ids, int n_entries, int n_experts, int
     return check_launch("moe_align");
 }
 
-extern "C" int liyab_moe_route_align(const float* logits, int64_t ld, int n, int n_experts, int top, int* ids, float* weights, int block,
+// `rp`: the router's product ahead of the choice (or null).
+static int route_align(const RouterProduct* rp, const float* logits, int64_t ld, int n, int n_experts, int top, int* ids, float* weights, int block,
                                      int* rows_list, int* tile_group, int max_tiles, int mode, int n_groups, int keep, const float* correction,
                                      float scale, int n_listed, int extra, hipStream_t stream) {
     LIYAB_REQUIRE(n <= 1024, "moe_route_align: %d tokens; one workgroup routes at most 1,024 (moe_route and moe_align take more)", n);
@@ -474,11 +564,36 @@ extern "C" int liyab_moe_route_align(const float* logits, int64_t ld, int n, int
     // More than a token a wave and few experts: a thread a token is faster (64 tokens, 2 of 8 experts 7.2 us against 10.6; 8 of 64 246 against 36), and from some
     // ten tokens on where it has little to scan (16 tokens, 1 of 2 3.3 against 3.7, 1 of 4 3.8 and 4.1, 2 of 4 5.0 and 4.8; 8 tokens, 1 of 2 3.3 and 3.3).
     const int64_t places = static_cast<int64_t>(max_tiles) * block;
-    if (mode == 0 && n <= kWaveRouteTokens && n_experts > 1 && n_experts <= kSmallExperts && n * top <= kSmallEntries && places <= kSmallPlaces && max_tiles <= 1024 &&
-        (n <= 8 || (n <= 1024 / kWave && n_experts * top > 4) || n_experts * top > 64)) {
-        moe_route_align_small_kernel<<<1, 1024, static_cast<size_t>(places) * sizeof(int), stream>>>(logits, ld, n, n_experts, top, ids, weights, block, rows_list, tile_group, max_tiles);
+    const bool small = n <= kWaveRouteTokens && n_experts > 1 && n_experts <= kSmallExperts && listed <= kSmallExperts && n * (top + extra) <= kSmallEntries && places <= kSmallPlaces;
+    if (small && (mode == 0 ? n <= 8 || (n <= 1024 / kWave && n_experts * top > 4) || n_experts * top > 64 : mode >= 2 && routes_in_lanes(ra, n_experts))) {
+        if (rp != nullptr)
+            moe_route_align_small_kernel<true><<<1, 1024, static_cast<size_t>(places) * sizeof(int), stream>>>(logits, ld, n, n_experts, top, ids, weights, block, rows_list, tile_group, max_tiles, ra, *rp);
+        else
+            moe_route_align_small_kernel<false><<<1, 1024, static_cast<size_t>(places) * sizeof(int), stream>>>(logits, ld, n, n_experts, top, ids, weights, block, rows_list, tile_group, max_tiles, ra, RouterProduct{});
         return check_launch("moe_route_align");
     }
+    LIYAB_REQUIRE(rp == nullptr, "moe_router: %d tokens of %d experts are not taken with the router's product", n, n_experts);
     moe_route_align_kernel<<<1, 1024, smem, stream>>>(logits, ld, n, n_experts, top, ids, weights, block, rows_list, tile_group, max_tiles, ra);
     return check_launch("moe_route_align");
+}
+
+extern "C" int liyab_moe_route_align(const float* logits, int64_t ld, int n, int n_experts, int top, int* ids, float* weights, int block,
+                                     int* rows_list, int* tile_group, int max_tiles, int mode, int n_groups, int keep, const float* correction,
+                                     float scale, int n_listed, int extra, hipStream_t stream) {
+    return route_align(nullptr, logits, ld, n, n_experts, top, ids, weights, block, rows_list, tile_group, max_tiles, mode, n_groups, keep, correction, scale, n_listed, extra, stream);
+}
+
+// The same behind the router's product, logits = a . w^T + bias for a [n <= 16, K] and w [columns <= 16, K] in bfloat16, K whole units of 64 and not of 16,384: the logits of
+// liyab_gemm_skinny, bit for bit, whose launch goes. columns: n_experts, or more (of which the choice sees the first n_experts and, with `extra`, the one behind them).
+extern "C" int liyab_moe_router(const void* a, int64_t lda, const void* w, const float* bias, int columns, int K, float* logits, int64_t ld, int n, int n_experts, int top, int* ids,
+                                float* weights, int block, int* rows_list, int* tile_group, int max_tiles, int mode, int n_groups, int keep, const float* correction, float scale,
+                                int n_listed, int extra, hipStream_t stream) {
+    LIYAB_REQUIRE(a && w, "moe_router: null operand");
+    LIYAB_REQUIRE(n <= kRouterSide && columns <= kRouterSide && columns >= n_experts + extra && ld >= columns && K > 0 && K % 64 == 0 && K % 16384 != 0 && lda >= K && lda % 8 == 0,
+                  "moe_router: bad sizes n=%d columns=%d of %d experts K=%d", n, columns, n_experts, K);
+    LIYAB_REQUIRE((reinterpret_cast<uintptr_t>(a) & 15) == 0 && (reinterpret_cast<uintptr_t>(w) & 15) == 0, "moe_router: operands must be 16-byte aligned");
+    int split_shift = 0;  // the waves that gemm_skinny.hip's choice has for one strip (choose_ksplit)
+    while (split_shift < 4 && K / 64 > (2 << split_shift)) ++split_shift;
+    const RouterProduct rp{static_cast<const bf16_t*>(a), lda, static_cast<const bf16_t*>(w), bias, columns, K, split_shift, logits};
+    return route_align(&rp, logits, ld, n, n_experts, top, ids, weights, block, rows_list, tile_group, max_tiles, mode, n_groups, keep, correction, scale, n_listed, extra, stream);
 }

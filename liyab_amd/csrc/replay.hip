@@ -106,6 +106,7 @@ static const Entry kEntries[] = {
     LIYAB_ENTRY(liyab_moe_route),
     LIYAB_ENTRY(liyab_moe_align),
     LIYAB_ENTRY(liyab_moe_route_align),
+    LIYAB_ENTRY(liyab_moe_router),
     LIYAB_ENTRY(liyab_attention_decode_scored),
     LIYAB_ENTRY(liyab_attention_prefill_scored),
     LIYAB_ENTRY(liyab_gate_rows),

@@ -91,6 +91,7 @@ _SIGNATURES = {
                               c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_float, c_float, P],
     "liyab_moe_route": [P, c_int64, c_int, c_int, c_int, P, P, c_int, c_int, c_int, P, c_float, c_int, c_int, P],
     "liyab_moe_align": [P, c_int, c_int, c_int, P, P, c_int, P],
+    "liyab_moe_router": [P, c_int64, P, P, c_int, c_int, P, c_int64, c_int, c_int, c_int, P, P, c_int, P, P, c_int, c_int, c_int, c_int, P, c_float, c_int, c_int, P],
     "liyab_moe_route_align": [P, c_int64, c_int, c_int, c_int, P, P, c_int, P, P, c_int, c_int, c_int, c_int, P, c_float, c_int, c_int, P],
     "liyab_attention_decode_scored": [P, c_int64, P, c_int64, P, P, c_int, P, c_int, P, P, P, c_int, c_float, c_int, c_int, c_int,
                                       c_int, c_int, c_int, c_int, c_int, c_int, P, c_int, c_int, c_int, c_float, P, c_int, P, c_int, P],

@@ -1506,9 +1506,22 @@ MOE_MAX_WAVE_EXPERTS = 2048  # with logistic scores (csrc/moe.hip: kMaxWaveExper
 MOE_WAVE_TOKENS = 64  # tokens such a choice and its lists take in one launch (kWaveRouteTokens)
 
 
+def router_product_pays(a: torch.Tensor, w: torch.Tensor, n: int, n_experts: int, top: int, groups: Optional[tuple] = None, scores: str = "softmax") -> bool:
+    """Whether the choice's kernel makes the router's logits itself (csrc/moe.hip: liyab_moe_router): few tokens and outputs, whose product `gemm` would leave to one
+    workgroup of the streaming kernel, a link of its own in a decode step's chain; and a choice that the kernel of small steps takes (short replies of four
+    requests at GPT-2 small's width, 8 experts: 32 such layers 5,730 -> 5,598 us with groups, 5,782 -> 5,683 with softmax scores over all; 96 with the largest logits 8,540 -> 8,447)."""
+    if _invariant or not 0 < n <= 16 or not 1 < n_experts <= w.shape[0] <= 16 or not mfma_takes(a, w) or w.shape[1] % 64 != 0 or w.shape[1] % 16384 == 0 or w.dtype != torch.bfloat16:
+        return False
+    if scores == "softmax":
+        return groups is None and (n <= 8 or n_experts * top > 4)
+    per = n_experts // groups[0] if groups is not None and groups[1] < groups[0] else 1
+    return per & (per - 1) == 0
+
+
 def moe_route(logits: torch.Tensor, top: int, ids: torch.Tensor, weights: torch.Tensor, rows_list: torch.Tensor,
               tile_group: torch.Tensor, block: int = GROUPED_ROWS, groups: Optional[tuple] = None, scores: str = "softmax",
-              correction: Optional[torch.Tensor] = None, scale: float = 1.0, identity: int = 0, extra: bool = False, n_lists: int = 0) -> None:
+              correction: Optional[torch.Tensor] = None, scale: float = 1.0, identity: int = 0, extra: bool = False, n_lists: int = 0,
+              router: Optional[tuple] = None) -> None:
     """From float32 router logits [n, experts] (rows may be strided): ids int32 and weights float32 [n,
     top] (the experts with the largest logits, softmax over those alone), and the entries t * top + k
     listed by expert in tiles of `block` places: rows_list int32 [tiles * block] (-1: empty), tile_group
@@ -1519,7 +1532,8 @@ def moe_route(logits: torch.Tensor, top: int, ids: torch.Tensor, weights: torch.
     chosen s as they are. "softmax_all": the same with s = softmax(logits) over all outputs and weights scale * s. With either of these, the last
     `identity` outputs are identity experts: an entry that takes one gets the id -1 and stands in no list; and `extra`: the logits have one
     column more, and a token one more entry behind its `top`, of the expert behind the listed ones, weighted sigmoid(that logit). `n_lists`: the
-    experts that `tile_group` and `rows_list` are made for, where they are more than the router lists."""
+    experts that `tile_group` and `rows_list` are made for, where they are more than the router lists. `router` = (a [n, K], w [columns, K], bias or None), where
+    `router_product_pays`: the logits, and what stands beside them in their rows, are not there yet but a . w^T + bias."""
     ld = _rows(logits, "logits")
     n, E = logits.shape
     E -= 1 if extra else 0
@@ -1555,6 +1569,15 @@ def moe_route(logits: torch.Tensor, top: int, ids: torch.Tensor, weights: torch.
     elif correction is not None:
         raise KernelError("moe_route: a correction goes with logistic scores")
     more = (float(scale), E - identity, 1 if extra else 0)
+    if router is not None:
+        a, w, bias = router
+        lda, columns = _rows(a, "a"), w.shape[0]
+        if not router_product_pays(a, w, n, E, top, groups, scores) or a.shape != (n, w.shape[1]) or not w.is_contiguous() or columns < logits.shape[1] or ld < columns:
+            raise KernelError(f"moe_route: a router of {tuple(w.shape)} over {tuple(a.shape)} is not taken here")
+        _f32vec(bias, "bias", columns)
+        _lib.call("liyab_moe_router", a.data_ptr(), lda, w.data_ptr(), _ptr(bias), columns, w.shape[1], logits.data_ptr(), ld, n, E, top, ids.data_ptr(), weights.data_ptr(), block,
+                  rows_list.data_ptr(), tile_group.data_ptr(), tiles, mode, count, keep, _ptr(correction), *more, _stream())
+        return
     if n <= (1024 if mode < 2 else MOE_WAVE_TOKENS if E <= 512 else 0):  # one launch: the tokens are routed, then the workgroup lists the entries
         _lib.call("liyab_moe_route_align", logits.data_ptr(), ld, n, E, top, ids.data_ptr(), weights.data_ptr(), block,
                   rows_list.data_ptr(), tile_group.data_ptr(), tiles, mode, count, keep, _ptr(correction), *more, _stream())

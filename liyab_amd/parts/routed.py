@@ -118,9 +118,13 @@ class RoutedFFN:
             z = ws.get("router_shared", (n, self.joint_in.shape[0]), torch.float32)
             linear(h, self.joint_in, None, out=z)
             logits, shared_pre = z[:, :columns], z[:, self.shared_col:]
+        router = None
         if logits is None:
             logits = ws.get("router_logits", (n, columns), torch.float32)
-            linear(h, self.router, self.router_bias, out=logits)
+            if ops.router_product_pays(h, self.router, n, E + self.identity, top, self.groups, self.scores):
+                router = (h, self.router, self.router_bias)  # (the choice's kernel makes the logits)
+            else:
+                linear(h, self.router, self.router_bias, out=logits)
         rows = self.rows_a_token
         entries = rows if listed else top  # of a token, as the router lists them
         groups = self.up.shape[0]
@@ -130,7 +134,7 @@ class RoutedFFN:
         rows_list = ws.get("routed_rows", (tiles * block,), torch.int32)
         tile_group = ws.get("routed_tiles", (tiles,), torch.int32)
         ops.moe_route(logits if listed or not self.weighed else logits[:, :columns - 1], top, ids, weights, rows_list, tile_group, block=block, groups=self.groups,
-                      scores=self.scores, correction=self.correction, scale=self.scale, identity=self.identity, extra=listed, n_lists=groups)
+                      scores=self.scores, correction=self.correction, scale=self.scale, identity=self.identity, extra=listed, n_lists=groups, router=router)
         inner = ws.get("routed_inner", (n * entries, self.inner), self.dtype)
         if self.gated:
             ops.moe_product(inner, h, self.gate, self.up, rows_list, tile_group, a_div=entries, block=block, clamp=self.clamp)
