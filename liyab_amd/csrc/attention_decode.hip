@@ -180,6 +180,11 @@ int launch_attention_decode(void* out, int64_t out_stride, const void* q, int64_
     }
     return 0;
 }
+int merge_decode_splits(bf16_t* out, int64_t out_stride, const int* tok_list, const float* partials, int n, int n_head, int hd, int n_splits, hipStream_t stream) {
+    attention_merge_kernel<bf16_t><<<dim3(n, n_head), ((hd + 63) / 64) * 64, 0, stream>>>(out, out_stride, tok_list, partials, n_head, hd, n_splits);
+    return check_launch("attention_merge");
+}
+
 }  // namespace liyab
 
 using namespace liyab;

@@ -52,6 +52,9 @@ __device__ __forceinline__ void add_sink(float& m, float& l, float (&acc)[N], fl
 // softmax's denominator where the row's sums are final; with a window, the first `keep_first` positions may stay visible: the
 // walk goes over places first - kept .. position, of which those ahead of `first` are positions 0 .. kept - 1. Without SCORED these arguments are not read, and the kernel is the one it was.
 // AHEAD: the next trip's keys are on their way while this one's are absorbed (where it pays: next_trip_ahead_pays).
+// Splits of rows tok_list[0..n) in bfloat16, merged in their order (attention_decode.hip).
+int merge_decode_splits(bf16_t* out, int64_t out_stride, const int* tok_list, const float* partials, int n, int n_head, int hd, int n_splits, hipStream_t stream);
+
 template <int LPK, int AD_WAVES>
 struct DecodeLds {
     float sums[2][AD_WAVES][LPK][10];  // the waves' sums, for the first wave to merge; two of them in turn, so that one barrier a split is enough

@@ -75,7 +75,7 @@ int liyab_attention_prefill(void* out, int64_t out_stride, const void* q, int64_
                             int window, int n_head, int n_kv_head, int hd, int page_size, int num_pages, hipStream_t stream);
 int liyab_attention_mixed(void* out, int64_t out_stride, const void* q, int64_t q_stride, const void* kc, const void* vc, const int* block_tables,
                           int max_blocks, const int* work, int n_tiles, int tile, int ksplit, const int* tok_list, const int* tok_seq, const int* tok_pos,
-                          int n, float scale, int window, int n_head, int n_kv_head, int page_size, int num_pages, hipStream_t stream);
+                          int n, int n_splits, int waves, float* partials, float scale, int window, int n_head, int n_kv_head, int page_size, int num_pages, hipStream_t stream);
 
 int liyab_rmsnorm(void* out, int out_dtype, const float* x, const float* w, const int* rows, int n, int d, float eps, hipStream_t stream);
 int liyab_gated_norm_add(float* x, void* cast_out, int cast_dtype, const float* y, int n_sum, const float* gate, int64_t gate_stride,

@@ -75,7 +75,7 @@ _SIGNATURES = {
     "liyab_gemm_att_parts": [P, c_int, c_int, c_int, P, c_int, c_int, c_int, P, c_int64, P, P, c_int, c_int64, P],
     "liyab_gemm_skinny_ln": [P, c_int, c_int64, P, P, c_float, P, c_int, c_int, c_int, c_int, _EPI_PTR, P],
     "liyab_gemm_skinny_dyt": [P, c_int, c_int64, P, P, P, P, c_int, c_int, c_int, c_int, _EPI_PTR, P],
-    "liyab_attention_mixed": [P, c_int64, P, c_int64, P, P, P, c_int, P, c_int, c_int, c_int, P, P, P, c_int, c_float, c_int, c_int, c_int, c_int, c_int, P],
+    "liyab_attention_mixed": [P, c_int64, P, c_int64, P, P, P, c_int, P, c_int, c_int, c_int, P, P, P, c_int, c_int, c_int, P, c_float, c_int, c_int, c_int, c_int, c_int, P],
     "liyab_attention_prefill": [P, c_int64, P, c_int64, P, P, P, c_int, P, c_int, c_int, c_int, c_float, c_int, c_int,
                                 c_int, c_int, c_int, c_int, P],
     "liyab_argmax": [P, P, c_int64, c_int, c_int, P, P, P, P, P],

@@ -1045,8 +1045,9 @@ def attention_rows(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor, v_
 
 def attention_mixed(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, block_tables: torch.Tensor, work: torch.Tensor,
                     n_tiles: int, tok_list: torch.Tensor, n_tokens: int, tok_seq: torch.Tensor, tok_pos: torch.Tensor, *, n_head: int, scale: float, window: int = 0,
-                    tile: int = 64, ksplit: int = 4, num_pages: Optional[int] = None) -> None:
-    """`attention_prefill`'s tiles and the rows `tok_list` as `attention_decode` takes them uncut, on tile / 32 * ksplit waves, in one launch: bfloat16, heads of 64."""
+                    tile: int = 64, ksplit: int = 4, n_splits: int = 1, waves: int = 8, partials: Optional[torch.Tensor] = None, num_pages: Optional[int] = None) -> None:
+    """`attention_prefill`'s tiles and the rows `tok_list` as `attention_decode` takes them (in `n_splits` on `waves` waves) in one launch: bfloat16, heads of 64, the forms
+    that `mixed_pays` names."""
     if k_cache.dim() != 4 or k_cache.shape != v_cache.shape or not k_cache.is_contiguous() or not v_cache.is_contiguous():
         raise KernelError("attention: caches must be contiguous [pages, kv_heads, page_size, head_dim] of one shape")
     _, hkv, page, hd = k_cache.shape
@@ -1063,16 +1064,20 @@ def attention_mixed(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor, v
     _i32(tok_list, "tok_list", n_tokens)
     _i32(tok_seq, "tok_seq", rows)
     _i32(tok_pos, "tok_pos", rows)
+    if n_splits > 1:
+        need = n_tokens * n_head * n_splits * (hd + 4)
+        if partials is None or partials.dtype != torch.float32 or partials.numel() < need or not partials.is_contiguous():
+            raise KernelError(f"attention_mixed: {n_splits} splits need {need} float32 of partials")
     _lib.call("liyab_attention_mixed", out.data_ptr(), os_, q.data_ptr(), qs, k_cache.data_ptr(), v_cache.data_ptr(), block_tables.data_ptr(), block_tables.shape[1],
-              work.data_ptr(), n_tiles, int(tile), int(ksplit), tok_list.data_ptr(), tok_seq.data_ptr(), tok_pos.data_ptr(), n_tokens, float(scale), int(window),
+              work.data_ptr(), n_tiles, int(tile), int(ksplit), tok_list.data_ptr(), tok_seq.data_ptr(), tok_pos.data_ptr(), n_tokens, n_splits, waves, _ptr(partials), float(scale), int(window),
               n_head, hkv, page, _pages(k_cache, num_pages), _stream())
 
 
-def mixed_pays(dtype: torch.dtype, hd: int, page: int, tile: int, ksplit: int, splits: int, waves: int) -> bool:
-    """Whether a step's tiles of prompt portions and its single tokens (`decode_plan`'s splits and waves) are attended in one launch: where the two kernels' workgroups
-    have as many waves and the single tokens' keys are not cut, so that every row keeps its bits."""
-    return (dtype == torch.bfloat16 and hd == 64 and page >= 8 and page & (page - 1) == 0 and (tile, ksplit) in ((64, 2), (64, 4), (128, 1))
-            and splits == 1 and waves == tile // 32 * ksplit)
+def mixed_pays(dtype: torch.dtype, hd: int, page: int, tile: int, ksplit: int, waves: int) -> bool:
+    """Whether a step's tiles of prompt portions and its single tokens (on `decode_plan`'s waves) are attended in one launch: the kernel's forms, all of which keep the
+    bits of two. Tiles of 128 with two waves a query group are left alone: their registers leave a compute unit no room for another workgroup."""
+    return (dtype == torch.bfloat16 and hd == 64 and page >= 8 and page & (page - 1) == 0
+            and (waves in (4, 8) if (tile, ksplit) in ((64, 2), (64, 4)) else waves == 4 and (tile, ksplit) == (128, 1)))
 
 
 def attention_prefill(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
@@ -1289,10 +1294,13 @@ def attention(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor, v_cache
             # 217 us for 16 x 1,024 tokens of 12 heads. Straight into LDS one wave a group is the faster past some 500 workgroups, 80 against 101 for
             # these, 34.5 and 34.0 for 4 x 1,000 of 16, 29.8 and 24.5 for 2 x 1,000 of 12; the line has stayed, since the other form adds in another order)
             ksplit = (4 if plan.tile == 64 and hd <= 64 and work <= PREFILL_KSPLIT4_WORK else 2) if work <= 256 or hd > 96 else 1
-            if plan.n_single and not scored and mixed_pays(q.dtype, hd, k_cache.shape[2], plan.tile, ksplit, *decode_plan(plan.n_single, n_head, longest())):
-                attention_mixed(out, q, k_cache, v_cache, block_tables, plan.work, plan.n_tiles, plan.single_rows, plan.n_single, ctx.tok_seq, ctx.positions,
-                                n_head=n_head, scale=scale, window=window, tile=plan.tile, ksplit=ksplit)
-                return None
+            if plan.n_single and not scored:
+                splits, waves = decode_plan(plan.n_single, n_head, longest())
+                if mixed_pays(q.dtype, hd, k_cache.shape[2], plan.tile, ksplit, waves):
+                    partials = ctx.workspace.get("attn_partials", (plan.n_single * n_head * splits * (hd + 4),), torch.float32) if splits > 1 else None
+                    attention_mixed(out, q, k_cache, v_cache, block_tables, plan.work, plan.n_tiles, plan.single_rows, plan.n_single, ctx.tok_seq, ctx.positions, n_head=n_head,
+                                    scale=scale, window=window, tile=plan.tile, ksplit=ksplit, n_splits=splits, waves=waves, partials=partials)
+                    return None
             attention_prefill(out, q, k_cache, v_cache, block_tables, plan.work, plan.n_tiles, n_head=n_head,
                               scale=scale, window=window, tile=plan.tile, ksplit=ksplit, **scored)
         if plan.n_single:
