@@ -52,20 +52,22 @@ __device__ __forceinline__ int64_t qkv_row_base(const EpiParams& p, int slot_wor
 // store, since the compiler cannot know that outputs and bias do not overlap.
 __device__ __forceinline__ float epilogue_bias(const EpiParams& p, int n) { return p.bias != nullptr ? p.bias[n] : 0.0f; }
 
-template <typename OutT, int MODE = -1>
+// EXACT: whether `exact` is looked at. Kernels whose operands are bfloat16 are never asked for it, and the double-precision erf, unrolled over a wave's sums, is most of
+// a tile's code.
+template <typename OutT, int MODE = -1, bool EXACT = true>
 __device__ __forceinline__ void epilogue_store_biased(const EpiParams& p, int m, int n, float v);
 
-template <typename OutT, int MODE = -1>
+template <typename OutT, int MODE = -1, bool EXACT = true>
 __device__ __forceinline__ void epilogue_store(const EpiParams& p, int m, int n, float v) {
-    epilogue_store_biased<OutT, MODE>(p, m, n, v + epilogue_bias(p, n));
+    epilogue_store_biased<OutT, MODE, EXACT>(p, m, n, v + epilogue_bias(p, n));
 }
 
 // `v` already holds the bias.
-template <typename OutT, int MODE>
+template <typename OutT, int MODE, bool EXACT>
 __device__ __forceinline__ void epilogue_store_biased(const EpiParams& p, int m, int n, float v) {
     switch (MODE >= 0 ? MODE : p.mode) {
-        case kEpiGeluTanh: v = p.exact ? gelu_tanh(v) : gelu_tanh_fast(v); break;
-        case kEpiGeluErf: v = p.exact ? gelu_erf_exact(v) : gelu_erf_fast(v); break;
+        case kEpiGeluTanh: v = EXACT && p.exact ? gelu_tanh(v) : gelu_tanh_fast(v); break;
+        case kEpiGeluErf: v = EXACT && p.exact ? gelu_erf_exact(v) : gelu_erf_fast(v); break;
         case kEpiResidual:
             p.residual[static_cast<int64_t>(m) * p.ldr + n] += v;
             return;

@@ -10,7 +10,7 @@
 // stage's fragments are read at once (780 rows, 4,096 -> 1,024, cold weights: 22.8 us in halves, 20.7 at once; 400 rows of 1,024 -> 1,024 8.4 and 7.4). Of tiles
 // whose waves would stand at the load queue the loads go out in two halves, each in front of the products of 32 k. What is left unhidden (a stage's barrier,
 // the first fragments, the outputs) overlaps with another workgroup's products: two workgroups of eight waves a compute unit for the middle tiles; 256 x 256
-// has eight waves, whose larger parts read LDS less than sixteen did (7,936 rows: 6,400 -> 1,600 172 -> 160 us, 1,600 -> 1,600 55 -> 53).
+// has eight waves or sixteen (launch_tile_256).
 // Alone and repeated, 8,192 cubed ran at 1.32 PFLOP/s on sixteen waves (the vendor's library 1.44).
 // Tried and left, cold weights: rings of six to nine stages for small tiles (no faster: not the latency of memory), fragments a stage or half of one ahead in
 // registers of their own, strung between the products (3 to 30 % slower), some waves
@@ -163,19 +163,44 @@ int launch_tile_as(const bf16_t* a, int64_t lda, const bf16_t* w, int M, int N, 
     return check_launch("gemm_mfma_tile");
 }
 
-template <int BM, int BN, int STAGES, int WM, int WN, int MIN_WAVES, bool HALVES>
-int launch_tile_epi(const bf16_t* a, int64_t lda, const bf16_t* w, int M, int N, int K, const EpiParams& epi, hipStream_t stream) {
+// (each epilogue a kernel: one that chooses as it stores is too long a loop to unroll over 128 sums a lane, which then lie in memory)
 #define LIYAB_TILE(T, E) launch_tile_as<BM, BN, STAGES, WM, WN, MIN_WAVES, HALVES, T, E>(a, lda, w, M, N, K, epi, 1, PartsParams{}, stream)
-    if (epi.mode == kEpiResidual) return LIYAB_TILE(float, kEpiResidual);
-    if (epi.out_dtype == kF32) return epi.mode == kEpiNone ? LIYAB_TILE(float, kEpiNone) : LIYAB_TILE(float, -1);
+template <int BM, int BN, int STAGES, int WM, int WN, int MIN_WAVES, bool HALVES>
+int launch_tile_gelu(const bf16_t* a, int64_t lda, const bf16_t* w, int M, int N, int K, const EpiParams& epi, hipStream_t stream) {
+    const bool f32 = epi.out_dtype == kF32;
+    if (epi.mode == kEpiGeluTanh) return f32 ? LIYAB_TILE(float, kEpiGeluTanh) : LIYAB_TILE(bf16_t, kEpiGeluTanh);
+    return f32 ? LIYAB_TILE(float, kEpiGeluErf) : LIYAB_TILE(bf16_t, kEpiGeluErf);
+}
+
+template <int BM, int BN, int STAGES, int WM, int WN, int MIN_WAVES, bool HALVES>
+int launch_tile_plain(const bf16_t* a, int64_t lda, const bf16_t* w, int M, int N, int K, const EpiParams& epi, hipStream_t stream) {
+    const bool f32 = epi.out_dtype == kF32;
     switch (epi.mode) {
-        case kEpiNone: return LIYAB_TILE(bf16_t, kEpiNone);
-        case kEpiGeluTanh: return LIYAB_TILE(bf16_t, kEpiGeluTanh);
-        case kEpiGeluErf: return LIYAB_TILE(bf16_t, kEpiGeluErf);
-        case kEpiQkvPaged: return LIYAB_TILE(bf16_t, kEpiQkvPaged);
+        case kEpiResidual: return LIYAB_TILE(float, kEpiResidual);
+        case kEpiNone: return f32 ? LIYAB_TILE(float, kEpiNone) : LIYAB_TILE(bf16_t, kEpiNone);
+        case kEpiQkvPaged: return f32 ? LIYAB_TILE(float, kEpiQkvPaged) : LIYAB_TILE(bf16_t, kEpiQkvPaged);
         default: return fail(1, "gemm: unknown epilogue %d", epi.mode);
     }
+}
 #undef LIYAB_TILE
+
+inline bool is_gelu(const EpiParams& epi) { return epi.mode == kEpiGeluTanh || epi.mode == kEpiGeluErf; }
+
+template <int BM, int BN, int STAGES, int WM, int WN, int MIN_WAVES, bool HALVES>
+int launch_tile_epi(const bf16_t* a, int64_t lda, const bf16_t* w, int M, int N, int K, const EpiParams& epi, hipStream_t stream) {
+    return is_gelu(epi) ? launch_tile_gelu<BM, BN, STAGES, WM, WN, MIN_WAVES, HALVES>(a, lda, w, M, N, K, epi, stream)
+                        : launch_tile_plain<BM, BN, STAGES, WM, WN, MIN_WAVES, HALVES>(a, lda, w, M, N, K, epi, stream);
+}
+
+// 256 x 256. Eight waves of 128 x 64 read LDS less than sixteen of 64 x 64, which counts the more the longer K is; sixteen have twice as many at an activation's
+// arithmetic, which two a SIMD don't hide. us, sixteen / eight, cold weights: 7,900 rows back to the stream, 1,600 -> 1,600 57.0 / 55.2, 4,096 -> 1,024 110.4 / 103.5, 6,400 ->
+// 1,600 171 / 163; no activation, 1,600 -> 4,800 129.5 / 129.4, 1,024 -> 3,072 60.3 / 60.6; tanh, 1,600 -> 6,400 189.9 / 187.5, 2,048 -> 8,192 248 / 241, but 1,280 -> 5,120
+// 122.0 / 122.5 and of 3,800 rows of 1,280 -> 3,840 44.3 / 44.9; erf, 1,600 -> 6,400 222 / 238, 1,024 -> 4,096 of 3,800 rows 47.3 / 51.6.
+int launch_tile_256(const bf16_t* a, int64_t lda, const bf16_t* w, int M, int N, int K, const EpiParams& epi, hipStream_t stream) {
+    if (epi.mode == kEpiGeluTanh && epi.out_dtype == kBF16 && K >= 1536)
+        return launch_tile_as<256, 256, 2, 2, 4, 2, false, bf16_t, kEpiGeluTanh>(a, lda, w, M, N, K, epi, 1, PartsParams{}, stream);
+    return is_gelu(epi) ? launch_tile_gelu<256, 256, 2, 4, 4, 4, true>(a, lda, w, M, N, K, epi, stream)
+                        : launch_tile_plain<256, 256, 2, 2, 4, 2, false>(a, lda, w, M, N, K, epi, stream);
 }
 
 int choose_gemm_tile(int M, int N, int K) {
@@ -217,7 +242,7 @@ int launch_gemm_tile(int tile, const bf16_t* a, int64_t lda, const bf16_t* w, in
         case 8: return launch_tile_epi<128, 128, 2, 4, 2, 4, true>(a, lda, w, M, N, K, epi, stream);
         case 9: return launch_tile_epi<192, 128, 2, 4, 2, 4, true>(a, lda, w, M, N, K, epi, stream);
         case 11: return launch_tile_epi<192, 128, 3, 4, 2, 2, true>(a, lda, w, M, N, K, epi, stream);
-        case 15: return launch_tile_epi<256, 256, 2, 2, 4, 2, false>(a, lda, w, M, N, K, epi, stream);
+        case 15: return launch_tile_256(a, lda, w, M, N, K, epi, stream);
         case 21: return launch_tile_epi<128, 192, 3, 2, 4, 2, false>(a, lda, w, M, N, K, epi, stream);
         default: return fail(1, "gemm_mfma_dl: unknown tile %d", tile);
     }

@@ -165,7 +165,7 @@ gemm_waves_kernel(const bf16_t* __restrict__ a, int64_t lda, const bf16_t* __res
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     if constexpr (EPI == kEpiGeluTanh) v[r] = gelu_tanh_fast(v[r]);
-                    if constexpr (EPI == kEpiGeluErf) v[r] = epi.exact ? gelu_erf_exact(v[r]) : gelu_erf_fast(v[r]);
+                    if constexpr (EPI == kEpiGeluErf) v[r] = gelu_erf_fast(v[r]);
                 }
                 store4<OutT>(static_cast<OutT*>(epi.out) + static_cast<int64_t>(m) * epi.ldo + n, v);
             }
@@ -184,7 +184,7 @@ gemm_waves_kernel(const bf16_t* __restrict__ a, int64_t lda, const bf16_t* __res
                 }
                 (static_cast<float*>(epi.out) + blockIdx.y * parts.part_stride)[static_cast<int64_t>(m) * N + n + r] = y;
             } else {
-                epilogue_store<OutT, EPI>(epi, m, n + r, x);
+                epilogue_store<OutT, EPI, false>(epi, m, n + r, x);
             }
         }
     }

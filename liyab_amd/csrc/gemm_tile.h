@@ -113,7 +113,7 @@ __device__ __forceinline__ void store_tile(Sums (&acc)[TM][TN], bf16_t* lds, con
                             for (int e = 0; e < 4; ++e) {
                                 v[e] = acc[i][j][4 * q + e] + b4[e];
                                 if constexpr (EPI == kEpiGeluTanh) v[e] = gelu_tanh_fast(v[e]);
-                                if constexpr (EPI == kEpiGeluErf) v[e] = epi.exact ? gelu_erf_exact(v[e]) : gelu_erf_fast(v[e]);
+                                if constexpr (EPI == kEpiGeluErf) v[e] = gelu_erf_fast(v[e]);
                             }
                             store4<bf16_t>(tile + (i * BLK + li) * LDO + j * BLK + 8 * q + 4 * g, v);
                         }
@@ -221,7 +221,7 @@ __device__ __forceinline__ void store_tile(Sums (&acc)[TM][TN], bf16_t* lds, con
                                 for (int e = 0; e < 4; ++e) v[e] = gelu_tanh_fast(v[e]);
                             } else if constexpr (EPI == kEpiGeluErf) {
 #pragma unroll
-                                for (int e = 0; e < 4; ++e) v[e] = epi.exact ? gelu_erf_exact(v[e]) : gelu_erf_fast(v[e]);
+                                for (int e = 0; e < 4; ++e) v[e] = gelu_erf_fast(v[e]);
                             }
                             store4<OutT>(static_cast<OutT*>(epi.out) + static_cast<int64_t>(m) * epi.ldo + n, v);
                         }
@@ -254,7 +254,7 @@ __device__ __forceinline__ void store_tile(Sums (&acc)[TM][TN], bf16_t* lds, con
                         (static_cast<float*>(epi.out) + blockIdx.y * parts.part_stride)[static_cast<int64_t>(m) * N + n] = v;
                     }
                 } else {
-                    if (n < N) epilogue_store<OutT, EPI>(epi, m, n, acc[i][j][r]);
+                    if (n < N) epilogue_store<OutT, EPI, false>(epi, m, n, acc[i][j][r]);
                 }
             }
     }

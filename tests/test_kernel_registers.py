@@ -9,11 +9,13 @@ import pytest
 from liyab_amd.csrc import build
 
 
-@pytest.mark.parametrize("source", ["attention_prefill_direct.hip", "sampling.hip", "gemm_skinny_ln.hip", "gemm_skinny.hip", "gemm_rows.hip", "grouped_product.hip", "gemm_mfma_waves.hip"])
+@pytest.mark.parametrize("source", ["attention_prefill_direct.hip", "sampling.hip", "gemm_skinny_ln.hip", "gemm_skinny.hip", "gemm_rows.hip", "grouped_product.hip", "gemm_mfma_waves.hip", "gemm_mfma_tile.hip", "gemm_mfma_dl.hip",
+                                    "attention_mixed.hip", "attention_rows.hip"])
 def test_no_kernel_spills(source, tmp_path):
     """A spilled register goes to memory and back in the walk over the keys, and counts among the loads that its waits count; in the sampler, whose threads
     hold a row, in every pass over it; in the norm's product, which is as short as the trips it waits for, in the middle of them. The kernels with rings in LDS wait for
-    their loads by count: one to memory that is not theirs would be counted too."""
+    their loads by count: one to memory that is not theirs would be counted too. Of a tile of 256 x 256 a wave holds 128 sums a lane: a store loop that is not
+    unrolled over them puts them all in memory, in every workgroup."""
     hipcc = build.hipcc_path()
     if hipcc is None:
         pytest.skip("hipcc was not found")

@@ -8,7 +8,7 @@ from test_kernels_gpu import DEV, close, gemm_reference, ops, rnd  # noqa: F401
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("epilogue", ["none", "gelu_tanh", "residual"])
+@pytest.mark.parametrize("epilogue", ["none", "gelu_tanh", "gelu_erf", "residual"])
 @pytest.mark.parametrize("M,N,K", [(1, 8, 64), (65, 97, 64), (330, 680, 128), (161, 321, 192), (300, 264, 832), (129, 1000, 1600), (520, 3000, 128), (2100, 1416, 192), (700, 4200, 1536)])
 def test_tiles_of_every_shape(ops, M, N, K, epilogue):  # noqa: F811
     """Against float64, from one unit of K to more than the rings hold, no whole number of tiles, N with no wide stores (97) and a large
@@ -49,3 +49,27 @@ def test_tiles_write_pages(ops, tile, M, H, Hkv, hd, K, page):  # noqa: F811
         got.append((q, kc, vc))
     for x, y in zip(*got):
         assert torch.equal(x, y)
+
+
+@pytest.mark.parametrize("tile", [2, 6, 7, 8, 9, 11, 15, 21])
+@pytest.mark.parametrize("M,H,Hkv,hd,K,page", [(70, 3, 3, 16, 64, 4), (300, 6, 3, 64, 192, 16), (20, 5, 1, 6, 128, 16)])
+def test_tiles_write_pages_in_32_bits(ops, tile, M, H, Hkv, hd, K, page):  # noqa: F811
+    """bfloat16 operands, queries and caches in 32 bits: the sums that stand in a plain output, in their places, and nothing elsewhere; heads that four outputs
+    side by side do not divide (6) among them."""
+    q_dim, kv_dim = H * hd, Hkv * hd
+    N = q_dim + 2 * kv_dim
+    a, w, bias = rnd(M, K, dtype=torch.bfloat16), rnd(N, K, seed=1, scale=0.2, dtype=torch.bfloat16), rnd(N, seed=2)
+    pages = -(-M // page) + 3
+    slots = torch.randperm(pages * page)[:M].to(torch.int32).to(DEV)
+    slots[1] = -1
+    flat = torch.empty(M, N, device=DEV)
+    ops.gemm_mfma_dl(a, w, bias, out=flat, tile=tile)
+    kc = torch.full((pages, Hkv, page, hd), 7.0, device=DEV)
+    vc, q = kc.clone(), torch.zeros(M, q_dim, device=DEV)
+    want_k, want_v = kc.clone(), vc.clone()
+    ops.gemm_mfma_dl(a, w, bias, out=q, epilogue=ops.EPI_QKV_PAGED, kv=(kc, vc, slots, q_dim), tile=tile)
+    real = (slots >= 0).nonzero()[:, 0]
+    at = slots[real].long()
+    want_k[at // page, :, at % page] = flat[real, q_dim:q_dim + kv_dim].view(-1, Hkv, hd)
+    want_v[at // page, :, at % page] = flat[real, q_dim + kv_dim:].view(-1, Hkv, hd)
+    assert torch.equal(q, flat[:, :q_dim]) and torch.equal(kc, want_k) and torch.equal(vc, want_v)
