@@ -209,7 +209,7 @@ int choose_gemm_tile(int M, int N, int K) {
     // 256 tile overlaps nothing), in us; a last round that is not full runs at the lower occupancy's time.
     struct Shape { int tile, bm, bn, fit; float unit[3], round; };
     constexpr Shape shapes[] = {
-        {15, 256, 256, 1, {1.38f, 0, 0}, 11.0f}, {9, 192, 128, 2, {0.68f, 1.3f, 0}, 5.0f},  {11, 192, 128, 1, {0.62f, 0, 0}, 4.5f},
+        {15, 256, 256, 1, {1.45f, 0, 0}, 10.0f}, {9, 192, 128, 2, {0.68f, 1.3f, 0}, 5.0f},  {11, 192, 128, 1, {0.62f, 0, 0}, 4.5f},
         {21, 128, 192, 1, {0.62f, 0, 0}, 4.5f},  {8, 128, 128, 2, {0.60f, 1.0f, 0}, 4.0f},  {7, 128, 128, 1, {0.50f, 0, 0}, 3.7f},
         {6, 64, 64, 2, {0.26f, 0.45f, 0}, 2.0f}, {2, 64, 64, 3, {0.30f, 0.45f, 0.62f}, 2.0f}};
     constexpr int kUnits = 256;  // compute units
@@ -217,6 +217,7 @@ int choose_gemm_tile(int M, int N, int K) {
     float best_us = 0.0f;
     for (const Shape& s : shapes) {
         const int64_t tiles = static_cast<int64_t>((M + s.bm - 1) / s.bm) * ((N + s.bn - 1) / s.bn);
+        if (s.tile == 21 && tiles > kUnits) continue;
         const int64_t slots = static_cast<int64_t>(kUnits) * s.fit, full = tiles / slots, rest = tiles % slots;
         float us = full * (s.unit[s.fit - 1] * (K / TBK) + s.round);
         if (rest > 0) us += s.unit[(rest + kUnits - 1) / kUnits - 1] * (K / TBK) + s.round;
@@ -225,7 +226,12 @@ int choose_gemm_tile(int M, int N, int K) {
             best_us = us;
         }
     }
-    // 128 x 192 is here for the products whose columns it divides better (2,048 rows of 768 -> 3,072: 256 tiles, 18.4 us in a step; 384 of 128 x 128 20.3).
+    // (256 x 256's times are those of sixteen waves: with the eight waves' own, 1.38 and 11, it took 6,148 to 7,100 rows of 2,048 -> 6,144 from 192 x 128, 154.2 us against 157.2 there at
+    // 6,550 rows, 162.8 against 167.6 with tanh.)
+    // 128 x 192 is here for products that it takes in one round and 128 x 128 in two: 250 to 256 tiles of it save 4 to 28 % (us, 128 x 128 / it, cold weights: 1,274 rows of
+    // 1,600 -> 4,800 29.5 / 25.3, 2,015 of 768 -> 3,072 18.1 / 16.5, 8,125 of 3,072 -> 768 52.7 / 44.7, 4,095 of 512 -> 1,536 12.9 / 12.4). From the second round on, where
+    // nothing overlaps a round's ends, it loses to all three that the times above put behind it (192 x 128: 7,740 rows of 1,600 -> 4,800 122 / 133, 8,115 of 768 -> 2,304 35.6 / 38.9;
+    // 256 x 256: 2,515 of 1,600 -> 4,800 42.2 / 44.2; 128 x 128: 8,115 of 768 -> 3,072 49.3 / 56.2).
     // Tiles of 64 x 64 in three stages and in four cost nearly the same here. With a compute unit each, two on every unit, or a long K the fourth
     // stage is worth its LDS (780 rows, 5,120 -> 1,280 33.4 us against 35.2 in three; 361 rows, 1,280 -> 5,120 14.7 against 14.9); a round
     // in between with a short K takes three (512 rows: 768 -> 2,304 8.9 against 9.7, 1,024 -> 3,072 10.8 against 11.5).
