@@ -5,9 +5,10 @@
 // little arithmetic, all of it on the vector unit. Here 256 keys and values lie in LDS once for 32 queries (136 KB with the queries, so a workgroup a compute unit, and eight waves, whose four parts of a row want more registers than sixteen would leave),
 // and both contractions run on the matrix cores, whose v_mfma_f32_16x16x4_f32 is four fused multiply-adds one after the other. What is left is
 // shared between them (1,152 cycles for 16 keys of 16 queries) and the vector unit (some 900: exponentials, maxima, the sums' trees).
-// Alone, us a layer of 12 heads, token by token / here with the splits' merge: portions of 100, 237, 374 and 511 tokens 94 / 50, four of 511 182 / 79, one of 1,000
-// 147 / 73, one of 500 52 / 27, ten of 30 16.9 / 11.2, one of 200 16.1 / 17.2, of 100 8.9 / 11.6: a workgroup is a chain of some 7 us however few keys it has. (Eight lanes
-// a query and the vector unit alone, as the other kernel, on sixteen waves: 64, 102, 94, 35, 15.4, 24, 15.6.)
+// Alone, us a layer of 12 heads, token by token / here with the splits' merge: portions of 100, 237, 374 and 511 tokens 102 / 50, four of 511 183 / 77, one of 1,000
+// 151 / 70, one of 500 49 / 26, eight of 33 behind 1,500 keys 133 / 84, ten of 30 17.6 / 11.3, one of 200 16.2 / 17.1, of 100 9.0 / 11.4: a workgroup is a chain of some 7 us however few
+// keys it has (with a wait for each page id between the loads, a trip to memory every time, 51.7, 79, 74, 26.8, 90.6, 11.3, 17.4 and 11.8). (Eight lanes a query and the vector unit
+// alone, as the other kernel, on sixteen waves: 64, 102, 94, 35, -, 15.4, 24, 15.6.)
 //
 // The order of a token's sums is that of the other kernel: a score is eight chains of eight dimensions, added in a tree; 32 lane groups take every 32nd
 // key, four at a time, each with a maximum, a sum and weighted values of its own; groups are merged in a tree, eight to a wave, then the four waves in
@@ -103,6 +104,9 @@ attention_rows_kernel(float* __restrict__ out, int64_t out_stride, const float* 
             id[l] = bt[lp];
         }
         const f32x4 mine_q = *reinterpret_cast<const f32x4*>(q + static_cast<int64_t>(row0 + min(tid / 16, nq - 1)) * q_stride + h * kRowsDim + li * 4);
+        // (all ids are waited for here: inside the branches below, where loads into LDS are in flight that nobody can count, each would wait for everything ahead of it)
+#pragma unroll
+        for (int l = 0; l < LOADS; ++l) asm volatile("" : "+v"(id[l]));
 #pragma unroll
         for (int l = 0; l < LOADS; ++l) {
             const int key = (l * kRowsWaves + wave) * 4;  // (a multiple of 4: its four keys differ in key % 4 = u)
@@ -289,7 +293,6 @@ extern "C" int liyab_attention_rows(float* out, int64_t out_stride, const float*
     LIYAB_REQUIRE(n_splits >= 1 && n_splits <= 64 && static_cast<int64_t>(n_tiles) * (tile / kRowsQueries) <= 65535, "attention_rows: %d splits, %d tiles", n_splits, n_tiles);
     LIYAB_REQUIRE(q_stride % 4 == 0 && (reinterpret_cast<uintptr_t>(q) & 15) == 0 && (reinterpret_cast<uintptr_t>(kc) & 15) == 0 && (reinterpret_cast<uintptr_t>(vc) & 15) == 0,
                   "attention_rows: queries and caches must be 16-byte aligned with a query stride that is a multiple of 4");
-    LIYAB_REQUIRE((reinterpret_cast<uintptr_t>(partials) & 15) == 0, "attention_rows: partials must be 16-byte aligned");
     LIYAB_REQUIRE((reinterpret_cast<uintptr_t>(partials) & 15) == 0, "attention_rows: partials must be 16-byte aligned");
     LIYAB_REQUIRE(q_stride >= static_cast<int64_t>(n_head) * kRowsDim && (n_splits > 1 || out_stride >= static_cast<int64_t>(n_head) * kRowsDim), "attention_rows: short rows");
     if (n_tiles == 0) return 0;

@@ -27,3 +27,18 @@ def test_no_kernel_spills(source, tmp_path):
     for k in kernels:
         spilled, scratch = (int(re.search(what + r": (\d+)", k)[1]) for what in ("VGPRs Spill", r"ScratchSize \[bytes/lane\]"))
         assert spilled == 0 and scratch == 0, f"{k.split()[0]}: {spilled} registers spilled, {scratch} bytes of scratch a lane"
+
+
+def test_keys_go_to_lds_without_a_wait_between_them(tmp_path):
+    """attention_rows.hip asks for 256 keys and values in loads that nobody counts: a wait for a register between two of them waits for all of them, a trip to memory each."""
+    hipcc = build.hipcc_path()
+    if hipcc is None:
+        pytest.skip("hipcc was not found")
+    source, out = "attention_rows.hip", tmp_path / "kernel.s"
+    r = subprocess.run([hipcc, *build.FLAGS, *build.FILE_FLAGS.get(source, []), "-I", build.CSRC, "--cuda-device-only", "-S", os.path.join(build.CSRC, source), "-o", str(out)],
+                       capture_output=True, text=True, timeout=600)
+    assert r.returncode == 0, r.stderr[-2000:]
+    blocks = re.split(r"(?m)^\.LBB\S*:|^\s+s_c?branch\S* .*$|^\s+s_barrier.*$", out.read_text())
+    loads = [b for b in blocks if "global_load_lds" in b]
+    assert len(loads) == 8
+    assert not any("vmcnt" in b[:b.rindex("global_load_lds")] for b in loads)
