@@ -9,6 +9,7 @@ library's own kernel. Nothing here runs without the GPU and the library.
 from __future__ import annotations
 
 import ctypes
+import math
 import struct
 from typing import Optional
 
@@ -1190,16 +1191,23 @@ def invariant_chunk(reach: int) -> int:
     return chunk
 
 
-# (token, head) pairs of a step of prompt portions in 32 bits from which attention_rows takes it (us token by token / there, 12 heads: one portion of 200 tokens 16.1 / 17.2, of 500
-# 52 / 27, four of 48 12.9 / 11.2, ten of 30 16.9 / 11.2; 25 heads: one of 300 47 / 26)
+# (token, head) pairs of a step of prompt portions in 32 bits from which attention_rows takes it (us token by token / there, 12 heads: one portion of 200 tokens 16.2 / 17.1, of 250
+# 19.3 / 17.2, of 500 49.5 / 26.2, four of 48 13.2 / 11.3, ten of 30 17.6 / 11.3; 25 heads: one of 120 16.8 / 11.8, of 300 50 / 27)
 ROWS_FROM_PAIRS = 3000
+# Tokens a tile on their average from which it does so for any heads: its workgroups take 32 queries, and one is as long with nine. 12 heads, portions of 9, 12, 16 and 20 tokens: 30, 22, 16 and
+# 13 of them 14.8 / 17.5, 14.9 / 16.8, 14.2 / 16.8, 15.6 / 11.6; 66, 50, 37 and 30 behind 300 keys 90 / 110, 89 / 85, 85 / 65, 79 / 62; one of 200 and forty of 9 (13 a tile) 29.8 / 32.0, one of 300
+# and twenty of 9 (19) 31.3 / 29.8. Where a token on its own finds no neighbour's keys in an XCD's L2 (csrc/attention_decode.hip: heads_first_pays), shorter portions gain too:
+# 25 heads, 30 portions of 9 behind 300 keys 135 / 87, of 12 behind 900 284 / 150; 25 heads behind none, whose keys still fit, 26.8 / 32.1 and 26.9 / 24.4.
+ROWS_TOKENS_A_TILE = 18
 ROWS_MAX_PARTIALS = 32 << 20  # floats of splits left for the merge
 
 
 def rows_pay(plan, q, hd: int, n: int, n_head: int, splits: int, chunk: int) -> bool:
     """Whether a step of prompt portions in 32 bits goes to the kernel that takes 32 queries to 256 keys (attention_rows): the same bits as token by token."""
-    return (q.dtype == torch.float32 and hd == 64 and chunk == 256 and plan.mode == "prefill" and plan.n_single == 0 and plan.n_tiles > 0
-            and n * n_head >= ROWS_FROM_PAIRS and splits <= 64 and n * n_head * splits * (hd + 4) <= ROWS_MAX_PARTIALS)
+    if not (q.dtype == torch.float32 and hd == 64 and chunk == 256 and plan.mode == "prefill" and plan.n_single == 0 and 0 < plan.n_tiles * (plan.tile // 32) <= 65535
+            and n * n_head >= ROWS_FROM_PAIRS and splits <= 64 and n * n_head * splits * (hd + 4) <= ROWS_MAX_PARTIALS):
+        return False
+    return n >= ROWS_TOKENS_A_TILE * plan.n_tiles or n_head // math.gcd(n_head, 8) * plan.context_bucket * hd * 8 > 4 << 20
 
 
 def attention_takes(head_dim: int) -> bool:

@@ -194,3 +194,23 @@ def test_products_of_few_rows_are_within_what_their_kernels_take(ops):
             for heads, hd in ((1, 8), (12, 64), (3, 36), (25, 64), (64, 128)):
                 if ops.splits_in_product_pay(M, splits, heads, hd):
                     assert 1 < splits <= 8 and hd % 4 == 0 and heads * hd % 64 == 0 and heads * hd <= 8192 and 0 < M <= 64
+
+
+def test_prompt_portions_in_32_bits_that_go_32_queries_at_a_time(ops):
+    """Long portions do; many short ones only where their heads' keys do not stay in an L2; and never more tiles than a grid has rows, which token by token has no bound on."""
+    import torch
+
+    from liyab_amd.parts.attention import AttentionStep
+
+    q = torch.empty(1, 64)
+
+    def pays(H, lens, bucket, tile=64, **kw):
+        tiles = sum(-(-n // tile) for n in lens)
+        n = sum(lens)
+        return ops.rows_pay(AttentionStep("prefill", bucket, tiles, tile, **kw), q, 64, n, H, max(1, bucket // 256), 256)
+
+    assert pays(12, [500], 512) and pays(12, [20] * 13, 256) and pays(25, [130], 256) and pays(12, [300] + [9] * 20, 512)
+    assert not pays(12, [200], 256) and not pays(12, [9] * 66, 256) and not pays(12, [9] * 66, 1024) and not pays(12, [200] + [9] * 40, 256)
+    assert pays(25, [9] * 30, 512) and not pays(25, [9] * 30, 256)
+    assert not pays(12, [500], 512, n_single=1)
+    assert pays(1, [100] * 3000, 256, tile=128) and not pays(1, [20] * 16384, 256, tile=128)
