@@ -1074,9 +1074,18 @@ def attention_mixed(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor, v
               n_head, hkv, page, _pages(k_cache, num_pages), _stream())
 
 
-def mixed_pays(dtype: torch.dtype, hd: int, page: int, tile: int, ksplit: int, waves: int) -> bool:
-    """Whether a step's tiles of prompt portions and its single tokens (on `decode_plan`'s waves) are attended in one launch: the kernel's forms, all of which keep the
-    bits of two. Tiles of 128 with two waves a query group are left alone: their registers leave a compute unit no room for another workgroup."""
+# Single tokens' (token, head) pairs up to which short contexts are attended beside tiles of 64: those leave a compute unit two workgroups, which alone hold four of a token's. us in two
+# launches / one, portions of 100 tokens, contexts of up to 250 keys: 20 heads, 48 tokens 16.9 / 13.9, 80 and six portions 24.2 / 23.7, 96 and six 26.0 / 26.8, 128 31.6 / 32.6, 160 35.2 / 38.2; 25 heads,
+# 160 40.2 / 43.0. Longer contexts are bound by the keys' bytes and gain at any number (25 heads, up to 1,000 keys: 64 tokens 60.3 / 50.4, 128 105 / 93), as beside tiles of 128, three a unit.
+MIXED_SHORT_PAIRS = 1792
+
+
+def mixed_pays(dtype: torch.dtype, hd: int, page: int, tile: int, ksplit: int, waves: int, pairs: int = 0, longest: int = 0) -> bool:
+    """Whether a step's tiles of prompt portions and its single tokens (on `decode_plan`'s waves; `pairs` of them with a head, over up to `longest` keys) are attended in one
+    launch: the kernel's forms, all of which keep the bits of two. Tiles of 128 with two waves a query group are left alone: their registers leave a compute unit no room for
+    another workgroup; tiles of 64 with one are not a form of it."""
+    if tile == 64 and longest <= 256 and pairs > MIXED_SHORT_PAIRS:
+        return False
     return (dtype == torch.bfloat16 and hd == 64 and page >= 8 and page & (page - 1) == 0
             and (waves in (4, 8) if (tile, ksplit) in ((64, 2), (64, 4)) else waves == 4 and (tile, ksplit) == (128, 1)))
 
@@ -1304,7 +1313,7 @@ def attention(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor, v_cache
             ksplit = (4 if plan.tile == 64 and hd <= 64 and work <= PREFILL_KSPLIT4_WORK else 2) if work <= 256 or hd > 96 else 1
             if plan.n_single and not scored:
                 splits, waves = decode_plan(plan.n_single, n_head, longest())
-                if mixed_pays(q.dtype, hd, k_cache.shape[2], plan.tile, ksplit, waves):
+                if mixed_pays(q.dtype, hd, k_cache.shape[2], plan.tile, ksplit, waves, plan.n_single * n_head, longest()):
                     partials = ctx.workspace.get("attn_partials", (plan.n_single * n_head * splits * (hd + 4),), torch.float32) if splits > 1 else None
                     attention_mixed(out, q, k_cache, v_cache, block_tables, plan.work, plan.n_tiles, plan.single_rows, plan.n_single, ctx.tok_seq, ctx.positions, n_head=n_head,
                                     scale=scale, window=window, tile=plan.tile, ksplit=ksplit, n_splits=splits, waves=waves, partials=partials)

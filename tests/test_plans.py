@@ -214,3 +214,14 @@ def test_prompt_portions_in_32_bits_that_go_32_queries_at_a_time(ops):
     assert pays(25, [9] * 30, 512) and not pays(25, [9] * 30, 256)
     assert not pays(12, [500], 512, n_single=1)
     assert pays(1, [100] * 3000, 256, tile=128) and not pays(1, [20] * 16384, 256, tile=128)
+
+
+def test_single_tokens_beside_tiles_of_64(ops):
+    """Many of them over short contexts keep a launch of their own, which holds twice as many a compute unit."""
+    import torch
+
+    def pays(tile, ksplit, waves, pairs, longest):
+        return ops.mixed_pays(torch.bfloat16, 64, 16, tile, ksplit, waves, pairs, longest)
+
+    assert pays(64, 4, 4, 1600, 256) and pays(64, 4, 4, 3200, 512) and pays(128, 1, 4, 3200, 256) and pays(64, 2, 8, 240, 256)
+    assert not pays(64, 4, 4, 1920, 256) and not pays(64, 2, 4, 3200, 100)
