@@ -47,11 +47,6 @@ __device__ __forceinline__ void add_sink(float& m, float& l, float (&acc)[N], fl
     m = M;
 }
 
-// SCORED: the score scale * q . k is worked on before the softmax: a soft cap, cap * tanh(score / cap) (softcap > 0), then
-// a bias by distance, bias_table[min(position - key, max_dist), head] (bias_table given); `sinks` (one logit a head) join the
-// softmax's denominator where the row's sums are final; with a window, the first `keep_first` positions may stay visible: the
-// walk goes over places first - kept .. position, of which those ahead of `first` are positions 0 .. kept - 1. Without SCORED these arguments are not read, and the kernel is the one it was.
-// AHEAD: the next trip's keys are on their way while this one's are absorbed (where it pays: next_trip_ahead_pays).
 // Splits of rows tok_list[0..n) in bfloat16, merged in their order (attention_decode.hip).
 int merge_decode_splits(bf16_t* out, int64_t out_stride, const int* tok_list, const float* partials, int n, int n_head, int hd, int n_splits, hipStream_t stream);
 
@@ -62,6 +57,11 @@ struct DecodeLds {
     float stash[AD_LOOP_CHUNKS][LPK][10];
 };
 
+// SCORED: the score scale * q . k is worked on before the softmax: a soft cap, cap * tanh(score / cap) (softcap > 0), then
+// a bias by distance, bias_table[min(position - key, max_dist), head] (bias_table given); `sinks` (one logit a head) join the
+// softmax's denominator where the row's sums are final; with a window, the first `keep_first` positions may stay visible: the
+// walk goes over places first - kept .. position, of which those ahead of `first` are positions 0 .. kept - 1. Without SCORED these arguments are not read.
+// AHEAD: the next trip's keys are on their way while this one's are absorbed (where it pays: next_trip_ahead_pays).
 template <typename T, int LPK, int AD_WAVES, int AD_U, bool SCORED, bool AHEAD>
 __device__ __forceinline__ void attention_decode_walk(DecodeLds<LPK, AD_WAVES>& shared, int slot, int h, int z,
                         T* __restrict__ out, int64_t out_stride, const T* __restrict__ q, int64_t q_stride,
