@@ -192,7 +192,8 @@ __device__ __forceinline__ void route_wave(const float* __restrict__ z, const Ro
 }
 
 // The same for at most 64 outputs: an output a lane, its score in a register; zl is the lane's logit, and with `extra` lane 0 knows the
-// token's own one. No trip through LDS. Groups of a power of two of outputs: their two largest meet in a butterfly.
+// token's own one. No trip through LDS. Groups of a power of two of outputs: their two largest meet in a butterfly, where a score that is no number brings the largest ahead
+// of it in its group, which is what it leaves for the second largest in route_wave's order.
 __device__ __forceinline__ void route_wave_lane(float zl, float own, const RouteArgs& ra, int E, int top, int* __restrict__ ids, float* __restrict__ weights) {
     const int lane = threadIdx.x % kWave;
     const bool real = lane < E, grouped = ra.keep < ra.n_groups;
@@ -207,6 +208,14 @@ __device__ __forceinline__ void route_wave_lane(float zl, float own, const Route
     if (grouped) {
         const int per = E / ra.n_groups;
         float a = fmaxf(-INFINITY, c), b = -INFINITY;  // the two largest so far
+        if (__builtin_amdgcn_ballot_w64(c != c) != 0) {
+            float ahead = a;  // the largest up to this lane's, of its group
+            for (int off = 1; off < per; off <<= 1) {
+                const float before = __shfl_up(ahead, off, kWave);
+                if (lane % per >= off) ahead = fmaxf(ahead, before);
+            }
+            if (c != c) b = ahead;
+        }
         for (int off = 1; off < per; off <<= 1) {
             const float ao = __shfl_xor(a, off, kWave), bo = __shfl_xor(b, off, kWave);
             b = fmaxf(fminf(a, ao), fmaxf(b, bo));

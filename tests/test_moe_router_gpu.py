@@ -45,6 +45,17 @@ def test_the_routers_product_inside(ops, n, E, K, bias, kw):  # noqa: F811
     assert torch.equal(got, want) and all(torch.equal(x, y) for x, y in zip(first, second))
 
 
+def group_score(values):
+    """The two largest, in the order of the kernel that walks a group."""
+    a = b = float("-inf")
+    for v in values:
+        if v != v:
+            b = max(b, a)
+        else:
+            b, a = max(b, min(a, v)), max(a, v)
+    return a + b if len(values) > 1 else a
+
+
 @pytest.mark.parametrize("n", [1, 5, 64])
 @pytest.mark.parametrize("E,groups,top", [(2, (2, 1), 1), (8, (4, 2), 2), (64, (8, 3), 6), (64, (64, 7), 7), (48, (3, 2), 4), (32, (2, 2), 8)])
 def test_groups_of_experts_in_lanes(ops, n, E, groups, top):  # noqa: F811
@@ -60,12 +71,30 @@ def test_groups_of_experts_in_lanes(ops, n, E, groups, top):  # noqa: F811
     score = 1.0 / (1.0 + torch.exp(-z.cpu()))
     per = E // groups[0]
     for t in range(n):
-        # (what is no number is never chosen)
-        key = [(v if v == v else float("-inf")) for v in (score[t] + c.cpu()).tolist()]
-        best2 = [sum(sorted(key[g * per:(g + 1) * per])[-2:]) for g in range(groups[0])]
+        # (what is no number is never chosen; in its group's score the largest ahead of it stands again)
+        raw = (score[t] + c.cpu()).tolist()
+        key = [(v if v == v else float("-inf")) for v in raw]
+        best2 = [group_score(raw[g * per:(g + 1) * per]) for g in range(groups[0])]
         kept = sorted(range(groups[0]), key=lambda g: (-best2[g], g))[:groups[1]]
         want = sorted((e for e in range(E) if e // per in kept), key=lambda e: (-key[e], e))[:top]
         got = ids[t * top:(t + 1) * top].tolist()
         # (scores that the two exponentials round apart may change places)
         assert all(abs(key[x] - key[y]) < 1e-6 for x, y in zip(got, want)), (got, want)
         torch.testing.assert_close(weights[t * top:(t + 1) * top].cpu(), score[t][got], rtol=1e-6, atol=1e-7)
+
+
+@pytest.mark.parametrize("groups", [(32, 9), (32, 5), (16, 3), (8, 2), (4, 3), (2, 1)])
+def test_logits_that_are_no_numbers_choose_the_same_groups_in_lanes_and_in_a_walk(ops, groups):  # noqa: F811
+    """64 experts, an expert a lane, against 64 and one group more that is never kept, which the kernel that walks takes: the same choices and weights, with none to five logits a
+    token that are no numbers, and infinities."""
+    n, E, per, top = 64, 64, 64 // groups[0], 5
+    more, wide = per, (groups[0] + 1, groups[1])
+    z, c = rnd(n, E, seed=7), rnd(E, seed=8, scale=0.1)
+    g = torch.Generator().manual_seed(9)
+    for t in range(n):
+        z[t, torch.randperm(E, generator=g)[:t % 6].to(DEV)] = float("nan")
+    z[3, 5], z[4, 9] = float("inf"), float("-inf")
+    z2, c2 = torch.cat([z, torch.zeros(n, more, device=DEV)], 1).contiguous(), torch.cat([c, torch.full((more,), -10.0, device=DEV)])
+    a = route(ops, z, n, E, top, 16, scores="logistic", groups=groups, correction=c)
+    b = route(ops, z2, n, E + more, top, 16, scores="logistic", groups=wide, correction=c2)
+    assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1])
