@@ -112,8 +112,9 @@ class Attention:
 
     @property
     def takes_padding_rows(self) -> bool:
-        """Rows behind the step's tokens (token 0 at position 0 of the first request, slot -1) are computed
-        and never read: their keys and values are not written, and no other row attends to them."""
+        """Rows behind the step's tokens (token 0 at position 0 of the first request, slot -1) are carried along and never
+        read: their keys and values are not written, and no other row attends to them. Where tokens are taken tile by
+        tile, their own rows of attention's output hold whatever the workspace held."""
         return self.position is None or bool(getattr(self.position, "takes_padding_rows", False))
 
     def __init__(self, spec, store, dtype: torch.dtype):

@@ -28,7 +28,7 @@ class RoutedFFN:
     weight one or a logistic weight of its own, whose result is one more row a token for the reader to add."""
 
     replayable = True
-    takes_padding_rows = True  # (they are routed and computed like token 0; nobody reads them)
+    takes_padding_rows = True  # (they are routed by whatever their rows hold, numbers or not, to some expert; nobody reads them)
 
     def __init__(self, spec, store, dtype: torch.dtype):
         self.dtype = dtype

@@ -208,6 +208,41 @@ def test_prompts_of_one_padded_size_share_a_graph(dtype, model_dirs):
     assert core.manager.pages_in_use() == 0
 
 
+def test_what_lies_in_padding_rows_reaches_no_other_in_32_bits(tmp_path):
+    """A padded prompt in 32 bits whose attention leaves the padding rows out (32 queries at a time, two splits merged): whatever the workspace held, the tokens' logits and
+    those behind them are the bits of an engine that pads nothing."""
+    import torch
+
+    from liyab_amd.engine import EngineCore, StepItem
+    from liyab_amd.kernels import ops
+    from liyab_amd.weights import write_random_model
+
+    cfg = {"architectures": ["GPT2LMHeadModel"], "activation_function": "gelu_new", "layer_norm_epsilon": 1e-5, "n_layer": 2, "n_embd": 768, "n_head": 12, "n_inner": 192,
+           "vocab_size": 211, "n_positions": 512}
+    write_random_model(str(tmp_path), cfg, 17)
+    cores = [EngineCore(str(tmp_path), dtype="float32", page_size=16, max_tokens=512, max_requests=2, use_graphs=graphs) for graphs in (False, True)]
+    assert cores[1].step_fn.pads_rows and not cores[0].step_fn.pads_rows
+    calls, rows_kernel = [], ops.attention_rows
+    ops.attention_rows = lambda out, *a, **kw: (calls.append((out.shape[0], kw["n_splits"])), rows_kernel(out, *a, **kw))[1]
+    try:
+        for n in (300, 290, 310, 301, 261):
+            toks = tt.random_tokens(n, n, 211)
+            got = []
+            for c in cores:
+                c.open("r")
+                logits = c.step([StepItem("r", toks, [0, n // 2, n - 1])]).float().cpu().numpy().copy()
+                got.append((logits, c.step([StepItem("r", [toks[0]], [0])]).float().cpu().numpy().copy()))
+                c.close("r")
+            assert np.array_equal(got[0][0], got[1][0]) and np.array_equal(got[0][1], got[1][1]) and np.isfinite(got[1][0]).all(), n
+            for buf in cores[1].step_fn.workspace._bufs.values():
+                if buf.is_floating_point():
+                    buf.fill_(float("nan"))
+            torch.cuda.synchronize()
+    finally:
+        ops.attention_rows = rows_kernel
+    assert (320, 2) in calls and (300, 2) in calls
+
+
 # ---------------------------------------------------------------------------
 # geometries that take the kernels' fallbacks in bfloat16; a head of its own
 # ---------------------------------------------------------------------------
