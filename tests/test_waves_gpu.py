@@ -10,7 +10,8 @@ pytestmark = pytest.mark.gpu
 
 # a row and a tile's edge, one unit of K to more than eight, no whole number of strips, N with no wide stores (97), each of the four tiles (32 x 16 and 32 x 32 of few
 # strips, 48 x 32, 64 x 32), more than one tile of rows
-SHAPES = [(17, 97, 64), (1, 2064, 128), (33, 1284, 448), (32, 6152, 576), (31, 4808, 512), (48, 6400, 640), (40, 4999, 128), (64, 4808, 1600), (49, 8192, 192), (70, 520, 192)]
+SHAPES = [(17, 97, 64), (1, 2064, 128), (33, 1284, 448), (32, 6152, 576), (31, 4808, 512), (48, 6400, 640), (40, 4999, 128), (64, 4808, 1600), (49, 8192, 192), (70, 520, 192),
+          (48, 6408, 1344), (41, 4999, 1344)]
 
 
 @pytest.mark.parametrize("epilogue", ["none", "gelu_tanh", "gelu_erf", "residual"])
@@ -36,7 +37,8 @@ def test_products_of_a_tile_of_rows(ops, M, N, K, epilogue):  # noqa: F811
         assert torch.equal(run(slice(M // 2, M // 2 + 1)), got[M // 2:M // 2 + 1])
 
 
-@pytest.mark.parametrize("M,H,Hkv,hd,K,page", [(33, 3, 3, 16, 64, 4), (64, 25, 25, 64, 192, 16), (20, 6, 3, 64, 128, 16), (40, 40, 20, 64, 192, 48), (17, 5, 1, 80, 1600, 16)])
+@pytest.mark.parametrize("M,H,Hkv,hd,K,page", [(33, 3, 3, 16, 64, 4), (64, 25, 25, 64, 192, 16), (20, 6, 3, 64, 128, 16), (40, 40, 20, 64, 192, 48), (17, 5, 1, 80, 1600, 16),
+                                                (40, 40, 20, 64, 1344, 48), (64, 25, 25, 64, 1344, 16)])
 def test_they_write_pages(ops, M, H, Hkv, hd, K, page):  # noqa: F811
     """Queries to their rows, keys and values to their slots, and nothing anywhere else; a slot outside the pages is not written."""
     q_dim, kv_dim = H * hd, Hkv * hd
@@ -59,7 +61,7 @@ def test_they_write_pages(ops, M, H, Hkv, hd, K, page):  # noqa: F811
 
 
 @pytest.mark.parametrize("n_base", [0, 1, 4, 6])
-@pytest.mark.parametrize("M,N,K,parts", [(33, 768, 3072, 4), (64, 1600, 6400, 4), (64, 1284, 1280, 1), (24, 4096, 1024, 2), (50, 99, 320, 3)])
+@pytest.mark.parametrize("M,N,K,parts", [(33, 768, 3072, 4), (64, 1600, 6400, 4), (64, 1284, 1280, 1), (24, 4096, 1024, 2), (50, 99, 320, 3), (45, 4099, 1344, 2), (60, 4100, 1344, 2)])
 def test_cut_over_k(ops, M, N, K, parts, n_base):  # noqa: F811
     """The planes add up to base + a . w^T + bias."""
     a, w, bias = rnd(M, K, dtype=torch.bfloat16), rnd(N, K, seed=1, scale=0.2, dtype=torch.bfloat16), rnd(N, seed=2)
