@@ -1531,16 +1531,27 @@ MOE_MAX_WAVE_EXPERTS = 2048  # with logistic scores (csrc/moe.hip: kMaxWaveExper
 MOE_WAVE_TOKENS = 64  # tokens such a choice and its lists take in one launch (kWaveRouteTokens)
 
 
-def router_product_pays(a: torch.Tensor, w: torch.Tensor, n: int, n_experts: int, top: int, groups: Optional[tuple] = None, scores: str = "softmax") -> bool:
-    """Whether the choice's kernel makes the router's logits itself (csrc/moe.hip: liyab_moe_router): few tokens and outputs, whose product `gemm` would leave to one
-    workgroup of the streaming kernel, a link of its own in a decode step's chain; and a choice that the kernel of small steps takes (short replies of four
-    requests at GPT-2 small's width, 8 experts: 32 such layers 5,730 -> 5,598 us with groups, 5,782 -> 5,683 with softmax scores over all; 96 with the largest logits 8,540 -> 8,447)."""
+def router_product_takes(a: torch.Tensor, w: torch.Tensor, n: int, n_experts: int, top: int, groups: Optional[tuple] = None, scores: str = "softmax") -> bool:
+    """Whether the choice's kernel can make the router's logits itself (csrc/moe.hip: liyab_moe_router): few tokens and outputs, whose product `gemm` would leave to one
+    workgroup of the streaming kernel, and a choice that the kernel of small steps takes."""
     if _invariant or not 0 < n <= 16 or not 1 < n_experts <= w.shape[0] <= 16 or not mfma_takes(a, w) or w.shape[1] % 64 != 0 or w.shape[1] % 16384 == 0 or w.dtype != torch.bfloat16:
         return False
     if scores == "softmax":
         return groups is None and (n <= 8 or n_experts * top > 4)
     per = n_experts // groups[0] if groups is not None and groups[1] < groups[0] else 1
     return per & (per - 1) == 0
+
+
+# Elements of rows and weights up to which the choice's workgroup makes the logits: it saves a link of a decode step's chain and reads them with one trip's loads in flight, where the streaming kernel
+# has its ring. us, two kernels / one, weights cold: 4 tokens of 8 experts, 768 wide 6.0 / 4.8 and 2,048 6.7 / 5.9, 4,096 7.2 / 7.8, 8,192 8.4 / 11.3; 1 token of 4, 4,096 7.1 / 6.3, 8,192 8.4 / 8.7; 8 of 16 (4
+# chosen), 768 7.2 / 6.3, 1,600 7.6 / 7.5, 2,048 7.7 / 7.8, 12,288 13.0 / 22.5; 16 of 16 among groups, 768 9.9 / 9.0, 1,600 10.4 / 10.6. (Short replies of four requests at GPT-2 small's width, 8 experts: 32 such
+# layers 5,730 -> 5,598 us with groups, 5,782 -> 5,683 with softmax scores over all; 96 with the largest logits 8,540 -> 8,447.)
+ROUTER_PRODUCT_ELEMENTS = 36000
+
+
+def router_product_pays(a: torch.Tensor, w: torch.Tensor, n: int, n_experts: int, top: int, groups: Optional[tuple] = None, scores: str = "softmax") -> bool:
+    """Whether the choice's kernel makes the router's logits: where it can and is the faster."""
+    return (n + w.shape[0]) * w.shape[1] <= ROUTER_PRODUCT_ELEMENTS and router_product_takes(a, w, n, n_experts, top, groups, scores)
 
 
 def moe_route(logits: torch.Tensor, top: int, ids: torch.Tensor, weights: torch.Tensor, rows_list: torch.Tensor,
@@ -1558,7 +1569,7 @@ def moe_route(logits: torch.Tensor, top: int, ids: torch.Tensor, weights: torch.
     `identity` outputs are identity experts: an entry that takes one gets the id -1 and stands in no list; and `extra`: the logits have one
     column more, and a token one more entry behind its `top`, of the expert behind the listed ones, weighted sigmoid(that logit). `n_lists`: the
     experts that `tile_group` and `rows_list` are made for, where they are more than the router lists. `router` = (a [n, K], w [columns, K], bias or None), where
-    `router_product_pays`: the logits, and what stands beside them in their rows, are not there yet but a . w^T + bias."""
+    `router_product_takes`: the logits, and what stands beside them in their rows, are not there yet but a . w^T + bias."""
     ld = _rows(logits, "logits")
     n, E = logits.shape
     E -= 1 if extra else 0
@@ -1597,7 +1608,7 @@ def moe_route(logits: torch.Tensor, top: int, ids: torch.Tensor, weights: torch.
     if router is not None:
         a, w, bias = router
         lda, columns = _rows(a, "a"), w.shape[0]
-        if not router_product_pays(a, w, n, E, top, groups, scores) or a.shape != (n, w.shape[1]) or not w.is_contiguous() or columns < logits.shape[1] or ld < columns:
+        if not router_product_takes(a, w, n, E, top, groups, scores) or a.shape != (n, w.shape[1]) or not w.is_contiguous() or columns < logits.shape[1] or ld < columns:
             raise KernelError(f"moe_route: a router of {tuple(w.shape)} over {tuple(a.shape)} is not taken here")
         _f32vec(bias, "bias", columns)
         _lib.call("liyab_moe_router", a.data_ptr(), lda, w.data_ptr(), _ptr(bias), columns, w.shape[1], logits.data_ptr(), ld, n, E, top, ids.data_ptr(), weights.data_ptr(), block,

@@ -37,7 +37,7 @@ def test_the_routers_product_inside(ops, n, E, K, bias, kw):  # noqa: F811
     want = torch.full((n, E + extra), float("nan"), device=DEV)
     ops.gemm_skinny(a, w, b, out=want)
     first = route(ops, want, n, E, top, 16, **more)
-    if not ops.router_product_pays(a, w, n, E, top, kw.get("groups"), kw.get("scores", "softmax")):
+    if not ops.router_product_takes(a, w, n, E, top, kw.get("groups"), kw.get("scores", "softmax")):
         assert kw.get("groups", (1, 1))[0] == 4 and E == 12
         return
     got = torch.full_like(want, float("nan"))

@@ -225,3 +225,14 @@ def test_single_tokens_beside_tiles_of_64(ops):
 
     assert pays(64, 4, 4, 1600, 256) and pays(64, 4, 4, 3200, 512) and pays(128, 1, 4, 3200, 256) and pays(64, 2, 8, 240, 256)
     assert not pays(64, 4, 4, 1920, 256) and not pays(64, 2, 4, 3200, 100)
+
+
+def test_the_routers_product_inside_the_choice_up_to_what_one_trip_reads(ops):
+    import torch
+
+    def pays(n, E, K, **kw):
+        return ops.router_product_pays(torch.empty(n, K, dtype=torch.bfloat16), torch.empty(E, K, dtype=torch.bfloat16), n, E, 2, **kw)
+
+    assert pays(4, 8, 768) and pays(8, 8, 2048) and pays(1, 4, 4096) and pays(8, 16, 768) and pays(16, 8, 768, scores="logistic", groups=(4, 2))
+    assert not pays(4, 8, 4096) and not pays(1, 8, 4096) and not pays(8, 16, 2048) and not pays(16, 16, 1600, scores="softmax_all") and not pays(8, 8, 12288)
+    assert not pays(17, 8, 768) and not pays(4, 17, 768) and not pays(4, 8, 776)
