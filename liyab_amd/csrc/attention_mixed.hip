@@ -35,7 +35,7 @@ attention_mixed_kernel(PrefillArgs p, MixedArgs d, int page_shift) {
     } else {
         if (wave >= QG * KS) return;
         const int t = block - singles;
-        attention_prefill_walk<64, QG, KS, NS, STAGES, false, true>(p, page_shift, ring, t % p.n_head, t / p.n_head);
+        attention_prefill_walk<64, QG, KS, NS, STAGES, false, true>(p, page_shift, t % p.n_head, t / p.n_head);
     }
 }
 

@@ -26,10 +26,9 @@ namespace liyab {
 template <int HD, int QG, int KS, int NS, int STAGES, int MIN_WAVES, bool SCORED, bool BY_LOAD>
 __global__ void __launch_bounds__(64 * QG * KS, MIN_WAVES)
 attention_prefill_direct_kernel(PrefillArgs p, int page_shift) {
-    extern __shared__ __attribute__((aligned(1024))) bf16_t ring[];
     // heads vary fastest: the work list has the longest tiles first, and workgroups start in the
     // grid's order, so that every head's longest tile starts before anybody's short one
-    attention_prefill_walk<HD, QG, KS, NS, STAGES, SCORED, BY_LOAD>(p, page_shift, ring, blockIdx.x, blockIdx.y);
+    attention_prefill_walk<HD, QG, KS, NS, STAGES, SCORED, BY_LOAD>(p, page_shift, blockIdx.x, blockIdx.y);
 }
 
 template <int HD, int QG, int KS, int NS, int STAGES, int MIN_WAVES, bool SCORED, bool BY_LOAD>
