@@ -50,11 +50,12 @@ __device__ __forceinline__ void add_sink(float& m, float& l, float (&acc)[N], fl
 // Splits of rows tok_list[0..n) in bfloat16, merged in their order (attention_decode.hip).
 int merge_decode_splits(bf16_t* out, int64_t out_stride, const int* tok_list, const float* partials, int n, int n_head, int hd, int n_splits, hipStream_t stream);
 
+// (aligned as arrays on their own would be: a part's ten floats are read in pieces of eight bytes)
 template <int LPK, int AD_WAVES>
-struct DecodeLds {
-    float sums[2][AD_WAVES][LPK][10];  // the waves' sums, for the first wave to merge; two of them in turn, so that one barrier a split is enough
-    int pages[AD_MAX_BLOCKS];
-    float stash[AD_LOOP_CHUNKS][LPK][10];
+struct alignas(16) DecodeLds {
+    alignas(16) float sums[2][AD_WAVES][LPK][10];  // the waves' sums, for the first wave to merge; two of them in turn, so that one barrier a split is enough
+    alignas(16) int pages[AD_MAX_BLOCKS];
+    alignas(16) float stash[AD_LOOP_CHUNKS][LPK][10];
 };
 
 // SCORED: the score scale * q . k is worked on before the softmax: a soft cap, cap * tanh(score / cap) (softcap > 0), then

@@ -42,3 +42,17 @@ def test_keys_go_to_lds_without_a_wait_between_them(tmp_path):
     loads = [b for b in blocks if "global_load_lds" in b]
     assert len(loads) == 8
     assert not any("vmcnt" in b[:b.rindex("global_load_lds")] for b in loads)
+
+
+def test_waves_parts_are_read_in_pieces_of_eight_bytes(tmp_path):
+    """Decode attention merges its waves' parts from LDS, ten floats each: single floats, which an array that is known to be aligned to four bytes gets, make eight waves 2 to 10 % slower."""
+    hipcc = build.hipcc_path()
+    if hipcc is None:
+        pytest.skip("hipcc was not found")
+    source, out = "attention_decode.hip", tmp_path / "kernels.s"
+    r = subprocess.run([hipcc, *build.FLAGS, *build.FILE_FLAGS.get(source, []), "-I", build.CSRC, "--cuda-device-only", "-S", os.path.join(build.CSRC, source), "-o", str(out)],
+                       capture_output=True, text=True, timeout=600)
+    assert r.returncode == 0, r.stderr[-2000:]
+    kernels = re.findall(r"(?ms)^_ZN5liyab23attention_decode_kernelI\S*Li8ELi4E\S*:.*?^\.Lfunc_end", out.read_text())  # (eight waves)
+    assert kernels
+    assert all(k.count("ds_read2_b64") > k.count("ds_read2_b32") / 4 for k in kernels), [(k.split(":")[0], k.count("ds_read2_b64"), k.count("ds_read2_b32")) for k in kernels]
