@@ -836,8 +836,9 @@ def compute_units() -> int:
 
 def waves_pay(M: int, K: int, parts: int = 1) -> bool:
     """Whether a product of 17 to 64 rows that the tiles of 32 x 32 and 64 x 32 would take (`gemm_mfma_dl`'s 16 and 17) goes to the kernel that leaves their bits from
-    waves with rings of their own (csrc/gemm_mfma_waves.hip, 18). us, cold weights, those / it: 15 to 35 % less at 24 to 64 rows of 13 shapes from 640 -> 2,560 to 2,048 -> 6,144;
-    3,200 -> 2,176 at 64 rows 11.5 / 9.8, 4,096 -> 4,096 at 24, 48 and 64 rows 13.2 / 10.3, 12.5 / 13.2, 14.0 / 13.5."""
+    waves with rings of their own (csrc/gemm_mfma_waves.hip, 18). us, cold weights, those / it: a median of 14 % less over 211 products of 17 to 64 rows of 40 shapes, whole and cut, 35 % at
+    most (768 -> 2,304 at 48 rows 5.3 / 4.2, 1,600 -> 4,800 at 64 9.8 / 8.8), and up to 2 % more where few long parts meet one tile's second row (33 rows of 6,144 -> 1,536 in four parts 8.5 / 8.7); past its
+    bound on K 4,096 -> 4,096 at 48 and 64 rows 12.5 / 13.2 and 14.0 / 13.5."""
     return K % 64 == 0 and 16 < M <= 64 and K <= (4096 if M <= 32 else 3200) * parts
 
 
@@ -902,13 +903,13 @@ def gemm(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], *, out:
             gemm_mfma_dl(a, w, bias, out=out, residual=residual, epilogue=epilogue, kv=kv, tile=8)
         elif ((M > 32 or (M > 16 and N * a.shape[1] >= 6 << 20)) and a.shape[1] % 64 == 0 and N >= 2048
               and (M + 63) // 64 * ((N + 31) // 32) <= compute_units()):
-            # one tile of 33 to 64 rows and many output features: 64 x 32 tiles share the tokens'
-            # rows through LDS where the streaming kernel's workgroups each read them again (40
-            # rows: 5.2 against 6.4 us for 768 -> 2,304, 8.0 against 10.4 for 1,600 -> 4,800, before the streaming
-            # kernel's rings: 5.0 and 10.1 at 48 rows since, 5.9 and 12.0 at 64; the lines stay, for the two add in different orders; the
+            # one tile of 33 to 64 rows and many output features: a workgroup's 32 or 64 rows share
+            # the weights where the streaming kernel's workgroups each read the rows again (us, cold
+            # weights, it / here at 33, 48 and 64 rows: 768 -> 2,304 4.5 / 3.9, 4.5 / 3.8, 5.6 / 3.9; 1,024 -> 3,072 6.5 /
+            # 4.2, 6.7 / 4.3, 7.3 / 4.5; 1,600 -> 4,800 10.6 / 7.6, 10.9 / 8.1, 12.6 / 8.9; the
             # products back to the model's width, with fewer tiles, stay with the streaming kernel);
-            # the largest matrices already from 17 rows (32 rows, weights cold from HBM: 8.9
-            # against 12.5 us for 1,600 -> 4,800, but 6.6 against 6.1 for 1,024 -> 3,072); more
+            # the largest matrices already from 17 rows (the line is from the tiles that took these rows
+            # before, and the two add in different orders: 32 rows of 1,600 -> 4,800 8.9 against 12.5 us, of 1,024 -> 3,072 6.6 against 6.1); more
             # tiles of rows as long as every tile has a compute unit of its own (the stages fill
             # a unit's LDS; 128 rows: 6.1 against 7.7 us for 768 -> 2,304 in 64 x 64 tiles; with
             # more tiles than units, 400 rows: 10.7 against 8.0)
