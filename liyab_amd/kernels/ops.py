@@ -836,7 +836,7 @@ def compute_units() -> int:
 
 def waves_pay(M: int, K: int, parts: int = 1) -> bool:
     """Whether a product of 17 to 64 rows that the tiles of 32 x 32 and 64 x 32 would take (`gemm_mfma_dl`'s 16 and 17) goes to the kernel that leaves their bits from
-    waves with rings of their own (csrc/gemm_mfma_waves.hip, 18). us, cold weights, those / it: a median of 14 % less over 211 products of 17 to 64 rows of 40 shapes, whole and cut, 35 % at
+    waves with rings of their own (csrc/gemm_mfma_waves.hip, 18). us, cold weights, those / it: a median of 14 % less over 211 products of 17 to 64 rows of 33 shapes, whole and cut, 31 % at
     most (768 -> 2,304 at 48 rows 5.3 / 4.2, 1,600 -> 4,800 at 64 9.8 / 8.8), and up to 2 % more where few long parts meet one tile's second row (33 rows of 6,144 -> 1,536 in four parts 8.5 / 8.7); past its
     bound on K 4,096 -> 4,096 at 48 and 64 rows 12.5 / 13.2 and 14.0 / 13.5."""
     return K % 64 == 0 and 16 < M <= 64 and K <= (4096 if M <= 32 else 3200) * parts
